@@ -236,7 +236,7 @@ struct MergeStats {
   const void *d_out, *o[3];      // [N, Hq, D]
   const void* gate;              // [N, 3]
   const float* lse[3];           // [Hq, N]
-  float2* stat[3];               // [N, Hq] (lse - log2 gate, delta)
+  float2* stat[3];               // [N, Hq] (lse - log2 gate, delta); lse +inf where the row has no probability at all
   void* dl;                      // [N, 3] gradient of the gate's logits
   int64_t n;
   int hq;
@@ -279,7 +279,10 @@ merge_stats_kernel(MergeStats p) {
       const float* lse = sub == 0 ? p.lse[0] : sub == 1 ? p.lse[1] : p.lse[2];
       const float l = sub == 0 ? lg[0] : sub == 1 ? lg[1] : lg[2];
       float2* st = sub == 0 ? p.stat[0] : sub == 1 ? p.stat[1] : p.stat[2];
-      st[n * p.hq + h] = make_float2(lse[(int64_t)h * p.n + n] - l, delta);
+      // No visible key (lse -inf) or a gate that is zero (l -inf): +inf, every probability 0.  The difference of the two
+      // where both hold would be NaN.
+      const float lse_h = lse[(int64_t)h * p.n + n];
+      st[n * p.hq + h] = make_float2(lse_h == -INFINITY || l == -INFINITY ? INFINITY : lse_h - l, delta);
     }
   }
 #pragma unroll
