@@ -726,12 +726,14 @@ cmp_topk_kernel(TopkParams p) {
       if (lane < p.t_out) out[lane] = lane < n_cand ? lane : -1;
       return;
     }
-    uint32_t key[NREG];   // bf16 bits + 1; 0: no candidate
+    // bf16 bits + 1; 0: no candidate.  A NaN is a large score; the largest of them is cut to the 15 bits that the search
+    // below runs over, a key above every threshold would be taken however many there are.
+    uint32_t key[NREG];
 #pragma unroll
     for (int r = 0; r < NREG; ++r) {
       const int b = lane + 64 * r;
       const float sc = (b < p.nblk && (b < n_cand || p.block_score)) ? block_score(b) : 0.f;
-      key[r] = b < n_cand ? (__float_as_uint(sc) >> 16 & 0x7FFFu) + 1u : 0u;   // (a NaN is a large score)
+      key[r] = b < n_cand ? min(__float_as_uint(sc) >> 16 & 0x7FFFu, 0x7FFEu) + 1u : 0u;
     }
     // largest threshold that at least t_out keys reach, bit by bit; counts come from ballots, in scalar registers
     auto count_from = [&](uint32_t t) {

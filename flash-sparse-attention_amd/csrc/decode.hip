@@ -692,8 +692,10 @@ __device__ __forceinline__ void dec_topk_block(const DecTopkParams& p, int b, in
       p.block_score[((int64_t)h * p.batch + b) * p.score_ld + blk] = -INFINITY;
   int32_t* out = p.topk_idx + ((int64_t)h * p.batch + b) * p.topk;
   if constexpr (NREG > 0) {
-    uint32_t key[NREG];   // score bits + 1; 0: no candidate
-    auto key_bits = [](float score) { return (__float_as_uint(score) & 0x7FFFFFFFu) + 1u; };   // (a NaN is a large score)
+    // score bits + 1; 0: no candidate.  A NaN is a large score; the largest of them is cut to the 31 bits that the search
+    // below runs over, a key above every threshold would be taken however many there are.
+    uint32_t key[NREG];
+    auto key_bits = [](float score) { return min(__float_as_uint(score) & 0x7FFFFFFFu, 0x7FFFFFFEu) + 1u; };
     if (na == 2 && ne == 4) {
       // usual geometry: the scores 4 blk - 1 .. 4 blk + 3 with weights 1 2 2 2 1, all loads of a lane in flight at once
       f32x4 x[NREG];
