@@ -773,22 +773,18 @@ cmp_topk_kernel(TopkParams p) {
   } else {
     for (int b = lane; b < p.nblk; b += 64) bs[b] = block_score(b);
     __builtin_amdgcn_wave_barrier();
-    // t_out rounds of arg-max by (value desc, id asc); taken entries are marked -1 (scores are >= 0)
+    // t_out rounds of arg-max by (value desc, id asc).  Scores are >= 0 or NaN, which is a large score, as in the other
+    // form; taken entries are marked -1.  As 64-bit keys, score bits + 1 above (0: taken) and the complement of the id
+    // below, the larger key is the larger score or, on equal scores, the lower id; t_out <= nblk entries are never all taken.
     for (int t = 0; t < p.t_out; ++t) {
-      float best = -2.f;
-      int best_id = 0x7fffffff;
+      uint64_t best = 0;
       for (int b = lane; b < p.nblk; b += 64) {
-        const float vv = bs[b];
-        if (vv > best) {
-          best = vv;
-          best_id = b;
-        }
+        const uint32_t bits = __float_as_uint(bs[b]);
+        const uint64_t k = bits == 0xBF800000u ? 0ull : ((uint64_t)((bits & 0x7FFFFFFFu) + 1u) << 32) | (0xFFFFFFFFu - (uint32_t)b);
+        best = k > best ? k : best;
       }
-      // scores are >= 0 (or the -2 of a lane without blocks): as 64-bit keys, score bits above and the complement
-      // of the id below, the larger key is the larger score or, on equal scores, the lower id
-      const uint64_t mine = best < 0.f ? 0ull : ((uint64_t)__float_as_uint(best) << 32) | (0xFFFFFFFFu - (uint32_t)best_id);
-      const uint64_t top = wave_max_u64(mine);
-      best_id = (int)(0xFFFFFFFFu - (uint32_t)top);
+      const uint64_t top = wave_max_u64(best);
+      const int best_id = (int)(0xFFFFFFFFu - (uint32_t)top);
       if (!BIG && lane == t) my_id = best_id;
       if (lane == 0) {
         bs[best_id] = -1.f;

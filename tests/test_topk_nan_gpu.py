@@ -12,10 +12,13 @@ pytestmark = pytest.mark.gpu
 NAN = 0x7FFFFFFF
 
 
-@pytest.mark.parametrize("n", [640, 5000, 10000, 20000, 60000])   # two to sixteen scores per lane
-def test_prefill_selection(dev, n):
-    h, d, ks, st, bs, topk = 1, 64, 32, 16, 64, 4
-    print(f"case n={n}", flush=True)
+@pytest.mark.parametrize("n,topk,bf16", [
+    (640, 4, 1), (5000, 4, 1), (10000, 4, 1), (20000, 4, 1), (60000, 4, 1),   # two to sixteen scores per lane
+    (640, 4, 0), (5000, 64, 0), (70000, 4, 1), (6000, 70, 0), (6000, 70, 1),  # scores in LDS
+])
+def test_prefill_selection(dev, n, topk, bf16):
+    h, d, ks, st, bs = 1, 64, 32, 16, 64
+    print(f"case n={n} topk={topk} bf16={bf16}", flush=True)
     q = torch.randn(n, h, d, device=dev, dtype=torch.bfloat16)
     nc, nblk = (n - ks) // st + 1, (n + bs - 1) // bs
     ck = torch.randn(nc, h, d, device=dev, dtype=torch.bfloat16)
@@ -27,7 +30,7 @@ def test_prefill_selection(dev, n):
     score = torch.zeros(h, n, nblk, device=dev)
     ws = torch.empty(lib.fsa_cmp_topk_workspace_bytes(n, h, nc // 4 + 1), dtype=torch.uint8, device=dev)
     rc = lib.fsa_cmp_topk(q.data_ptr(), ck.data_ptr(), lse.data_ptr(), 0, h * d, d, h * d, d, cu_q.data_ptr(), cu_k.data_ptr(),
-                          1, n, n, nc, h, h, d, ks, st, bs, topk, 1, 2, 1, 0, 1 / math.sqrt(d), out.data_ptr() + guard * 4,
+                          1, n, n, nc, h, h, d, ks, st, bs, topk, 1, 2, bf16, 0, 1 / math.sqrt(d), out.data_ptr() + guard * 4,
                           score.data_ptr(), ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
     _lib.check(rc, "fsa_cmp_topk")
     torch.cuda.synchronize()
@@ -38,7 +41,8 @@ def test_prefill_selection(dev, n):
     blocks = torch.arange(n, device=dev) // bs
     taken = torch.minimum(blocks + 1, torch.tensor(topk, device=dev))
     assert ((idx >= 0).sum(1) == taken).all() and (idx <= blocks[:, None]).all()
-    assert ((idx[:, 1:] > idx[:, :-1]) | (idx[:, 1:] == -1)).all()
+    ids = idx.masked_fill(idx < 0, nblk).sort(1).values     # distinct but for the padding
+    assert ((ids[:, 1:] > ids[:, :-1]) | (ids[:, 1:] == nblk)).all()
 
 
 @pytest.mark.parametrize("bf16", [True, False])
