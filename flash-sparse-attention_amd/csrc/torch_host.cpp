@@ -624,7 +624,7 @@ void matmul(const fsa_matmul_out* outs, int n, int form, const Tensor& like) {
 }
 
 struct LayerForward {
-  Tensor q, k, v, saved, out, topk_idx, y;   // out: merged heads; y: their projection where w_o is given, otherwise out
+  Tensor q, k, v, saved, out, topk_idx, y;   // out: merged heads; y: their projection
 };
 // `lens`: host copy of cu_seqlens that is on its way (batches of several sequences), waited for when the projections are
 // queued; null: one sequence, as long as x.
@@ -676,9 +676,7 @@ LayerForward layer_forward(const Tensor& x, const Tensor& cu, const Tensor& w_q,
   const int64_t t_out = std::min<int64_t>(shape[6], (z.max_len + shape[5] - 1) / shape[5]);
   f.topk_idx = empty_i32({shape[1], x.size(0), t_out}, x);
   check(api.fsa_layer_forward(&a, f.out.data_ptr(), (int32_t*)i32(f.topk_idx), stream_of(x)), "fsa_layer_forward");
-  if (!w_o.defined()) {
-    f.y = f.out;
-  } else if (own) {
+  if (own) {
     f.y = at::empty({x.size(0), w_o.size(0)}, x.options());
     fsa_matmul_out o = product(f.y);
     add_part(o, f.out, w_o, f.out.size(1));
@@ -689,7 +687,7 @@ LayerForward layer_forward(const Tensor& x, const Tensor& cu, const Tensor& w_q,
   return f;
 }
 
-// Inputs with gradients first: x, w_q, w_k, w_v, w_o (may be undefined), w_gate, w_ck, w_cv, pe.
+// Inputs with gradients first: x, w_q, w_k, w_v, w_o, w_gate, w_ck, w_cv, pe.
 struct LayerCore : torch::autograd::Function<LayerCore> {
   static torch::autograd::variable_list forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& w_q,
                                                 const Tensor& w_k, const Tensor& w_v, const Tensor& w_o, const Tensor& w_gate,
@@ -698,7 +696,7 @@ struct LayerCore : torch::autograd::Function<LayerCore> {
                                                 LayerSizes z, const Tensor* lens, HostCopy* copied) {
     LayerForward f = layer_forward(x, cu, w_q, w_k, w_v, w_o, w_gate, w_ck, w_cv, pe, inv_freq, rope_scale, *shape, z, lens,
                                    copied, true);
-    const Tensor merged = w_o.defined() && w_o.requires_grad() ? f.out : Tensor();
+    const Tensor merged = w_o.requires_grad() ? f.out : Tensor();
     ctx->save_for_backward({x, w_q, w_k, w_v, w_o, w_gate, w_ck, w_cv, pe, cu, inv_freq, f.k, f.v, f.saved, merged});
     ctx->saved_data["shape"] = std::vector<int64_t>(shape->begin(), shape->end());
     ctx->saved_data["sizes"] = std::vector<int64_t>{z.total_ck, z.max_len, z.max_ck};
@@ -719,13 +717,13 @@ struct LayerCore : torch::autograd::Function<LayerCore> {
     const c10::OptionalDeviceGuard guard(x.device());
     const Tensor dy = grads[0].contiguous();
     const bool own = own_products(x.size(0), x.size(1), shape, true) && (uintptr_t)dy.data_ptr() % 16 == 0;
-    Tensor d_out = dy;
-    if (w_o.defined() && own) {
+    Tensor d_out;
+    if (own) {
       d_out = at::empty({dy.size(0), w_o.size(1)}, dy.options());
       fsa_matmul_out o = product(d_out);
       add_part(o, dy, w_o, w_o.size(0));
       matmul(&o, 1, FSA_MM_NN, x);
-    } else if (w_o.defined()) {
+    } else {
       d_out = at::mm(dy, w_o);
     }
     fsa_layer_args a = layer_args(x, cu, w_gate, w_ck, w_cv, pe, s[10], ctx->saved_data["rope_scale"].toDouble(), shape,
@@ -780,7 +778,7 @@ struct LayerCore : torch::autograd::Function<LayerCore> {
 
 // nullopt: sizes, types or layouts the kernels are not built for (the caller composes the layer from the single operators).
 optional<std::pair<Tensor, Tensor>> layer_core(const Tensor& x, const Tensor& cu, const Tensor& w_q, const Tensor& w_k,
-                                               const Tensor& w_v, const optional<Tensor>& w_out, const Tensor& w_gate,
+                                               const Tensor& w_v, const Tensor& w_o, const Tensor& w_gate,
                                                const Tensor& w_ck, const Tensor& w_cv, const Tensor& pe, const Tensor& inv_freq, double rope_scale,
                                                const LayerShape& shape, bool exact_lens) {
   const int64_t hq = shape[0], hkv = shape[1], d = shape[2], ks = shape[3], st = shape[4], bs = shape[5], hidden = shape[10];
@@ -793,10 +791,8 @@ optional<std::pair<Tensor, Tensor>> layer_core(const Tensor& x, const Tensor& cu
       !cu.is_cuda() || cu.scalar_type() != at::kInt || !cu.is_contiguous() || inv_freq.scalar_type() != at::kFloat ||
       inv_freq.device() != x.device())
     return std::nullopt;
-  for (const Tensor* t : {&w_q, &w_k, &w_v, &w_gate, &w_ck, &w_cv, &pe})
+  for (const Tensor* t : {&w_q, &w_k, &w_v, &w_o, &w_gate, &w_ck, &w_cv, &pe})
     if (!ok(*t)) return std::nullopt;
-  const Tensor w_o = w_out ? *w_out : Tensor();
-  if (w_o.defined() && !ok(w_o)) return std::nullopt;
   const c10::OptionalDeviceGuard guard(x.device());
   const int64_t n = x.size(0);
   // Upper bounds are all the kernels need.  One sequence: its length is at most that of x.  More sequences: the same
@@ -815,7 +811,7 @@ optional<std::pair<Tensor, Tensor>> layer_core(const Tensor& x, const Tensor& cu
   }
   const Tensor* lp = lens.defined() ? &lens : nullptr;
   bool grad = false;
-  for (const Tensor* t : {&x, &w_q, &w_k, &w_v, &w_o, &w_gate, &w_ck, &w_cv, &pe}) grad |= t->defined() && t->requires_grad();
+  for (const Tensor* t : {&x, &w_q, &w_k, &w_v, &w_o, &w_gate, &w_ck, &w_cv, &pe}) grad |= t->requires_grad();
   try {
     if (grad && at::GradMode::is_enabled()) {
       const auto out = LayerCore::apply(x, w_q, w_k, w_v, w_o, w_gate, w_ck, w_cv, pe, cu, inv_freq, rope_scale, &shape, z, lp,

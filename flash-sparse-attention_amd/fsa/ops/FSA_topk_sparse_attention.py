@@ -196,6 +196,6 @@ def FSA_topk_sparse_attention(
     """
     # The kernels derive every per-sequence size on the device, so unlike the
     # reference (:1988) no host synchronisation is needed for max_seqlen.  The
-    # autograd node behind this call is native; `FSATopkSparseAttention` is the
-    # same node for callers that use the class.
+    # autograd node behind this call is native; `FSATopkSparseAttention` above is
+    # a Python node over the same kernels, for callers that use the class.
     return _ops.selected_attention(q, k, v, topk_idx, block_size, cu_seqlens, softmax_scale)

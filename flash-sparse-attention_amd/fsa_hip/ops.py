@@ -282,10 +282,9 @@ def is_plain_linear(module) -> bool:
 
 
 def layer_core(x, cu_seqlens, proj, w_gate, w_ck, w_cv, pe, inv_freq, rope_scale, shape, exact_lens):
-    """The layer as one differentiable call (C entry points fsa_layer_*, fsa_matmul): projections, attention core and, where
-    proj = (w_q, w_k, w_v, w_o) has a fourth weight, the output projection.  Returns (output, block ids), the output being
-    the merged heads [N, Hq*D] where w_o is None; or None for sizes or layouts without kernels.  `exact_lens`: the block
-    ids are wanted in the shape that the longest sequence gives (reads cu_seqlens back)."""
+    """The layer as one differentiable call (C entry points fsa_layer_*, fsa_matmul): projections with proj = (w_q, w_k, w_v,
+    w_o) and the attention core between them.  Returns (output [N, hidden], block ids), or None for sizes or layouts without
+    kernels.  `exact_lens`: the block ids are wanted in the shape that the longest sequence gives (reads cu_seqlens back)."""
     return _native.layer_core(x, cu_seqlens, *proj, w_gate, w_ck, w_cv, pe, inv_freq, rope_scale, shape, exact_lens)
 
 
