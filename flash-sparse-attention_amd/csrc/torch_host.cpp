@@ -458,6 +458,31 @@ Tensor compress_window(const Tensor& rows, const Tensor& w, const optional<Tenso
   return y;
 }
 
+// The sizes and places that the fused calls of the layer take for granted.  What does not pass is left to the composition
+// of the single operators, whose own checks refuse it (a projection of another width, a weight on another device) or
+// which serves it.
+bool plain_input(const Tensor& t, const Tensor& x, at::IntArrayRef sizes) {
+  return t.is_cuda() && t.device() == x.device() && t.scalar_type() == x.scalar_type() && t.is_contiguous() &&
+         t.sizes() == sizes && (uintptr_t)t.data_ptr() % 16 == 0;
+}
+bool layer_config_ok(int64_t hq, int64_t hkv, int64_t d, int64_t ks, int64_t st, int64_t hidden) {
+  // (window sizes: what LinearCompress takes)
+  return hidden >= 8 && hidden % 8 == 0 && (d == 64 || d == 128 || d == 256) && hq % hkv == 0 && ks % st == 0 &&
+         (ks == 16 || ks == 32 || ks == 64 || ks == 128);
+}
+bool projections_ok(const Tensor& x, const Tensor& w_q, const Tensor& w_k, const Tensor& w_v, const Tensor& w_gate,
+                    const Tensor& w_o, int64_t hq, int64_t hkv, int64_t d, int64_t hidden) {
+  return plain_input(w_q, x, {hq * d, hidden}) && plain_input(w_k, x, {hkv * d, hidden}) &&
+         plain_input(w_v, x, {hkv * d, hidden}) && plain_input(w_gate, x, {3, hidden}) && plain_input(w_o, x, {hidden, hq * d});
+}
+bool compression_ok(const Tensor& x, const Tensor& w_ck, const Tensor& w_cv, const Tensor& pe, int64_t hkv, int64_t ks, int64_t d) {
+  return plain_input(w_ck, x, {hkv, ks * d, d}) && plain_input(w_cv, x, {hkv, ks * d, d}) && plain_input(pe, x, {hkv, ks, d});
+}
+bool frequencies_ok(const Tensor& x, const Tensor& inv_freq, int64_t d) {
+  return inv_freq.device() == x.device() && inv_freq.scalar_type() == at::kFloat && inv_freq.is_contiguous() &&
+         inv_freq.numel() == d / 2;
+}
+
 // One token of one request through the whole layer.  nullopt: sizes, types or layouts the kernels are not built for (the
 // caller then composes the step from the single operators); otherwise y [1, hidden], the new k and v rows and, if the
 // token completes a compression window, the new compressed rows.
@@ -466,24 +491,23 @@ optional<DecodeLayerOut> decode_layer(const Tensor& x, const std::vector<Tensor>
                                       const Tensor& w_ck, const Tensor& w_cv, const Tensor& pe, const Tensor& inv_freq,
                                       double rope_scale, const std::array<int64_t, 10>& shape) {
   const auto [hq, hkv, d, ks, st, bs, topk, init_blocks, local_blocks, window] = shape;
+  if (caches.size() != 4 || weights.size() != 5 || x.dim() != 2 || x.size(0) != 1) return std::nullopt;
   const Tensor &k = caches[0], &v = caches[1], &ck = caches[2], &cv = caches[3];
-  const auto type = x.scalar_type();
-  auto aligned = [](const Tensor& t) { return (uintptr_t)t.data_ptr() % 16 == 0; };
   auto rows_ok = [&](const Tensor& t) {
-    return t.is_cuda() && t.scalar_type() == type && t.dim() == 3 && t.size(1) == hkv && t.size(2) == d && t.stride(2) == 1 &&
-           t.stride(0) >= 0 && t.stride(1) >= 0 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 && aligned(t);
+    return t.is_cuda() && t.device() == x.device() && t.scalar_type() == x.scalar_type() && t.dim() == 3 && t.size(1) == hkv &&
+           t.size(2) == d && t.stride(2) == 1 && t.stride(0) >= 0 && t.stride(1) >= 0 && t.stride(0) % 8 == 0 &&
+           t.stride(1) % 8 == 0 && (uintptr_t)t.data_ptr() % 16 == 0;
   };
-  auto weight_ok = [&](const Tensor& t) { return t.is_cuda() && t.scalar_type() == type && t.is_contiguous() && aligned(t); };
-  const int64_t L = k.size(0), hidden = x.size(1);
-  if (!x.is_cuda() || !is16(x) || !x.is_contiguous() || !aligned(x) || hidden % 8 || api.fsa_native_head_dim((int32_t)d) != d ||
-      hq % hkv || hq / hkv > 16 || hkv > 1024 || L < ks - 1 || L < 1 || (L + bs) / bs > 16384)
+  const int64_t hidden = x.size(1);
+  if (!is16(x) || !plain_input(x, x, {1, hidden}) || hkv < 1 || hq < 1 || st < 1 || bs < 1 ||
+      !layer_config_ok(hq, hkv, d, ks, st, hidden) || hq / hkv > 16 || hkv > 1024)
     return std::nullopt;
   for (const Tensor& t : caches)
     if (!rows_ok(t)) return std::nullopt;
-  for (const Tensor& t : weights)
-    if (!weight_ok(t)) return std::nullopt;
-  if (!weight_ok(w_ck) || !weight_ok(w_cv) || !weight_ok(pe) || v.size(0) != L || ck.size(0) != cv.size(0) ||
-      inv_freq.scalar_type() != at::kFloat || inv_freq.device() != x.device())
+  const int64_t L = k.size(0);
+  if (L < ks - 1 || L < 1 || (L + bs) / bs > 16384 || v.size(0) != L || ck.size(0) != cv.size(0)) return std::nullopt;
+  if (!projections_ok(x, weights[0], weights[1], weights[2], weights[3], weights[4], hq, hkv, d, hidden) ||
+      !compression_ok(x, w_ck, w_cv, pe, hkv, ks, d) || !frequencies_ok(x, inv_freq, d))
     return std::nullopt;
   const bool completes = (L + 1 - ks) % st == 0;
   if (ck.size(0) + completes < 1) return std::nullopt;
@@ -782,17 +806,12 @@ optional<std::pair<Tensor, Tensor>> layer_core(const Tensor& x, const Tensor& cu
                                                const Tensor& w_ck, const Tensor& w_cv, const Tensor& pe, const Tensor& inv_freq, double rope_scale,
                                                const LayerShape& shape, bool exact_lens) {
   const int64_t hq = shape[0], hkv = shape[1], d = shape[2], ks = shape[3], st = shape[4], bs = shape[5], hidden = shape[10];
-  const auto type = x.scalar_type();
-  auto ok = [&](const Tensor& t) {
-    return t.is_cuda() && t.scalar_type() == type && t.is_contiguous() && (uintptr_t)t.data_ptr() % 16 == 0;
-  };
-  if (!is16(x) || x.dim() != 2 || x.size(0) < 1 || !ok(x) || hidden % 8 || (d != 64 && d != 128 && d != 256) || hq % hkv ||
-      (bs != 32 && bs != 64 && bs != 128) || st < 1 || ks % st || bs % st || ks % 2 || shape[6] < std::max<int64_t>(1, shape[7] + shape[8]) ||
-      !cu.is_cuda() || cu.scalar_type() != at::kInt || !cu.is_contiguous() || inv_freq.scalar_type() != at::kFloat ||
-      inv_freq.device() != x.device())
+  if (!is16(x) || x.dim() != 2 || x.size(0) < 1 || !plain_input(x, x, {x.size(0), hidden}) || hkv < 1 || hq < 1 || st < 1 ||
+      !layer_config_ok(hq, hkv, d, ks, st, hidden) || (bs != 32 && bs != 64 && bs != 128) || bs % st ||
+      shape[6] < std::max<int64_t>(1, shape[7] + shape[8]) || !cu.is_cuda() || cu.device() != x.device() ||
+      cu.scalar_type() != at::kInt || cu.dim() != 1 || cu.numel() < 2 || !cu.is_contiguous() || !frequencies_ok(x, inv_freq, d) ||
+      !projections_ok(x, w_q, w_k, w_v, w_gate, w_o, hq, hkv, d, hidden) || !compression_ok(x, w_ck, w_cv, pe, hkv, ks, d))
     return std::nullopt;
-  for (const Tensor* t : {&w_q, &w_k, &w_v, &w_o, &w_gate, &w_ck, &w_cv, &pe})
-    if (!ok(*t)) return std::nullopt;
   const c10::OptionalDeviceGuard guard(x.device());
   const int64_t n = x.size(0);
   // Upper bounds are all the kernels need.  One sequence: its length is at most that of x.  More sequences: the same

@@ -130,9 +130,9 @@ class FlashSparseAttention(torch.nn.Module):
         max_len = max(lens)
         clens = [(l - self.kernel_size) // self.kernel_stride + 1 if l >= self.kernel_size else 0 for l in lens]
 
-        q = self.proj_q(x).view(-1, self.num_q_heads, self.head_dim)
-        k = self.proj_k(x).view(-1, self.num_kv_heads, self.head_dim)
-        v = self.proj_v(x).view(-1, self.num_kv_heads, self.head_dim)
+        q = self.proj_q(x).view(x.shape[0], self.num_q_heads, self.head_dim)
+        k = self.proj_k(x).view(x.shape[0], self.num_kv_heads, self.head_dim)
+        v = self.proj_v(x).view(x.shape[0], self.num_kv_heads, self.head_dim)
 
         # compressed keys / values are built from the un-rotated k, v
         compressed_k, compressed_cu = linear_compress(k, self.compress_key, cu_seqlens, self.kernel_size,

@@ -394,12 +394,20 @@ def _pad_compress_weight(w, kernel_size: int, d: int, dn: int):
     return w4.reshape(h, kernel_size * dn, dn).contiguous()
 
 
+def _check_compress(w, pe, x, h, kernel_size, d):
+    """The kernels read h * kernel_size * d * d weights and h * kernel_size * d positions whatever is there."""
+    assert w.device == x.device and w.numel() == h * kernel_size * d * d, "w must be [num_heads, kernel_size * head_dim, head_dim]"
+    assert pe is None or (pe.device == x.device and pe.numel() == h * kernel_size * d), \
+        "pe must be [num_heads, kernel_size, head_dim]"
+
+
 def linear_compress_fwd(x, w, cu_x, cu_y, total_y, max_y, kernel_size, kernel_stride, pe=None):
     """y [total_y, H, D] = strided-window projection of x [N, H, D] with w [H, ks*D, D] (+ pe bias)."""
     _require_cuda(x, w, cu_x, cu_y)
     assert x.dtype in _DTYPE and x.dtype == w.dtype and x.stride(2) == 1 and w.is_contiguous()
-    lib = _lib.load()
     n, h, d = x.shape
+    _check_compress(w, pe, x, h, kernel_size, d)
+    lib = _lib.load()
     dn = _native_dim(d)
     if dn != d:
         y = linear_compress_fwd(_pad_d(x, dn), _pad_compress_weight(w, kernel_size, d, dn), cu_x, cu_y, total_y, max_y,
@@ -421,8 +429,9 @@ def linear_compress_fwd(x, w, cu_x, cu_y, total_y, max_y, kernel_size, kernel_st
 def linear_compress_bwd(x, w, dy, cu_x, cu_y, max_x, kernel_size, kernel_stride, pe=None):
     """(dx, dw, dpe or None) of linear_compress_fwd."""
     _require_cuda(x, w, dy, cu_x, cu_y)
-    lib = _lib.load()
     n, h, d = x.shape
+    _check_compress(w, pe, x, h, kernel_size, d)
+    lib = _lib.load()
     dn = _native_dim(d)
     if dn != d:
         dx, dw, dpe = linear_compress_bwd(_pad_d(x, dn), _pad_compress_weight(w, kernel_size, d, dn), _pad_d(dy, dn),

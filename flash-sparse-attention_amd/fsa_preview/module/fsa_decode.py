@@ -97,9 +97,9 @@ class FlashSparseAttentionDecode(torch.nn.Module):
             return (out[0], out[1:]) if return_new_rows else out[0]
         cu_seqlens_q = cu_seqlens_q.to(torch.int32)
         cu_seqlens_k = cu_seqlens_k.to(torch.int32)
-        q = self.proj_q(x).view(-1, self.num_q_heads, self.head_dim)
-        k_new = self.proj_k(x).view(-1, self.num_kv_heads, self.head_dim)
-        v_new = self.proj_v(x).view(-1, self.num_kv_heads, self.head_dim)
+        q = self.proj_q(x).view(x.shape[0], self.num_q_heads, self.head_dim)
+        k_new = self.proj_k(x).view(x.shape[0], self.num_kv_heads, self.head_dim)
+        v_new = self.proj_v(x).view(x.shape[0], self.num_kv_heads, self.head_dim)
         k = torch.cat([k_cache, k_new], dim=0)
         v = torch.cat([v_cache, v_new], dim=0)
         cmp_out, sel_out, win_out, new_c = decode_step_attention(
