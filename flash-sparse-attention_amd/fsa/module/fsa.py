@@ -98,12 +98,13 @@ class FlashSparseAttention(torch.nn.Module):
 
     def _fused_core(self, x, cu_seqlens, exact_lens):
         """The whole layer as one native call, or None where it does not apply: projections that are more than a plain
-        Linear, autocast, head dims, block sizes or layouts without kernels."""
+        Linear, tensor subclasses, autocast, head dims, block sizes or layouts without kernels."""
         gate = self.gate
         layers = (self.proj_q, self.proj_k, self.proj_v, self.proj_o, gate[0])
         if (torch.is_autocast_enabled() or not all(map(_ops.is_plain_linear, layers))
                 or not _ops.is_plain(gate, torch.nn.Sequential) or len(gate) != 2
-                or not _ops.is_plain(gate[1], torch.nn.Sigmoid) or not _ops.is_plain(self.rope, RotaryEmbedding)):
+                or not _ops.is_plain(gate[1], torch.nn.Sigmoid) or not _ops.is_plain(self.rope, RotaryEmbedding)
+                or not _ops.are_plain_tensors(x, cu_seqlens, self.compress_key, self.compress_value, self.intra_block_pe)):
             return None
         q, k, v, o, g = (m.weight for m in layers)
         return _ops.layer_core(x, cu_seqlens, (q, k, v, o), g, self.compress_key, self.compress_value, self.intra_block_pe,

@@ -270,15 +270,31 @@ def decode_selattn(q, k_cache, v_cache, cu_k, topk_idx, block_size, softmax_scal
     return _native.decode_selattn(q, k_cache, v_cache, cu_k, topk_idx, block_size, softmax_scale, seqlens)
 
 
+_module = torch.nn.modules.module
+_GLOBAL_HOOKS = (_module._global_forward_hooks, _module._global_forward_pre_hooks, _module._global_backward_hooks,
+                 _module._global_backward_pre_hooks)
+# the forward that each of these classes was defined with (a module of this package adds its own)
+PLAIN_FORWARD = {c: c.forward for c in (torch.nn.Linear, torch.nn.Sequential, torch.nn.Sigmoid)}
+_TENSOR_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
+def are_plain_tensors(*tensors) -> bool:
+    """Tensors of torch's own types: their memory holds their values.  A subclass (quantised, sharded, wrapped) may keep
+    them elsewhere and has to go through torch."""
+    return all(type(t) in _TENSOR_TYPES for t in tensors)
+
+
 def is_plain(module, cls) -> bool:
-    """A module that is exactly `cls` and has no hooks: its forward can be replaced by the same mathematics."""
+    """A module that is exactly `cls`, without hooks of its own or for all modules, whose forward nobody has replaced, on
+    the instance or on the class: its forward can be replaced by the same mathematics."""
     d = module.__dict__
-    return type(module) is cls and not d["_forward_hooks"] and not d["_forward_pre_hooks"] \
+    return type(module) is cls and "forward" not in d and cls.forward is PLAIN_FORWARD[cls] \
+        and not any(_GLOBAL_HOOKS) and not d["_forward_hooks"] and not d["_forward_pre_hooks"] \
         and not d["_backward_hooks"] and not d.get("_backward_pre_hooks")
 
 
 def is_plain_linear(module) -> bool:
-    return is_plain(module, torch.nn.Linear) and module.bias is None
+    return is_plain(module, torch.nn.Linear) and module.bias is None and type(module.weight) in _TENSOR_TYPES
 
 
 def layer_core(x, cu_seqlens, proj, w_gate, w_ck, w_cv, pe, inv_freq, rope_scale, shape, exact_lens):

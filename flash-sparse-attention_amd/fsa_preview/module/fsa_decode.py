@@ -63,12 +63,14 @@ class FlashSparseAttentionDecode(torch.nn.Module):
 
     def _fused_step(self, x, *caches):
         """The step as one native call (six launches, caches neither copied nor rotated), or None where it does not
-        apply: projections that are more than a plain Linear, head dims or layouts without kernels, no compressed key."""
+        apply: projections that are more than a plain Linear, tensor subclasses, head dims or layouts without kernels, no
+        compressed key."""
         gate = self.gate
         layers = (self.proj_q, self.proj_k, self.proj_v, gate[0], self.proj_o)
         if (any(c is None for c in caches) or torch.is_autocast_enabled() or not all(map(_ops.is_plain_linear, layers))
                 or not _ops.is_plain(gate, torch.nn.Sequential) or len(gate) != 2
-                or not _ops.is_plain(gate[1], torch.nn.Sigmoid) or not _ops.is_plain(self.rope, RotaryEmbedding)):
+                or not _ops.is_plain(gate[1], torch.nn.Sigmoid) or not _ops.is_plain(self.rope, RotaryEmbedding)
+                or not _ops.are_plain_tensors(x, *caches, self.compress_key, self.compress_value, self.intra_block_pe)):
             return None
         return _ops.decode_layer(x, caches, [m.weight for m in layers], self.compress_key, self.compress_value,
                                  self.intra_block_pe, self.rope.table(x.device), self.rope.attention_scaling,

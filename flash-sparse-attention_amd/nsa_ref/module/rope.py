@@ -92,3 +92,6 @@ class RotaryEmbedding(nn.Module):
     def forward(self, x: torch.Tensor, cu_seqlens: torch.Tensor, start: int = 0, stride: int = 1):
         """Token j of every sequence is rotated for position start + j * stride."""
         return _Rotary.apply(x, cu_seqlens, self.table(x.device), self.attention_scaling, start, stride)
+
+
+_ops.PLAIN_FORWARD[RotaryEmbedding] = RotaryEmbedding.forward
