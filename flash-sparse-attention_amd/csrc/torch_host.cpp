@@ -77,6 +77,17 @@ template <typename... Ts> void need_device(const Tensor& t, const Ts&... rest) {
   need_device(rest...);
 }
 
+// The kernels have no forward-mode derivative.  An autograd node says so by itself, but without a gradient to record there
+// is no node, and a tangent would be lost without a word.
+void refuse_tangent(const Tensor& t) {
+  if (t.defined())
+    TORCH_CHECK_NOT_IMPLEMENTED(!t._fw_grad(/*level=*/0).defined(), "fsa_hip: forward-mode differentiation is not implemented");
+}
+template <typename... Ts> void refuse_tangent(const Tensor& t, const Ts&... rest) {
+  refuse_tangent(t);
+  refuse_tangent(rest...);
+}
+
 bool is16(const Tensor& t) { return t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kHalf; }
 int dtype_code(const Tensor& t) { return t.scalar_type() == at::kBFloat16 ? FSA_BF16 : FSA_FP16; }
 void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
@@ -346,6 +357,7 @@ struct SelectedAttention : torch::autograd::Function<SelectedAttention> {
 
 Tensor selected_attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& topk_idx, int64_t block,
                           const Tensor& cu, optional<double> scale_) {
+  refuse_tangent(q, k, v);
   FSA_ASSERT(block == 32 || block == 64 || block == 128 || block == 256, "block_size must be 32, 64, 128 or 256");
   check_qkv(q, k, v);
   check_topk(topk_idx, cu);
@@ -491,6 +503,9 @@ optional<DecodeLayerOut> decode_layer(const Tensor& x, const std::vector<Tensor>
                                       const Tensor& w_ck, const Tensor& w_cv, const Tensor& pe, const Tensor& inv_freq,
                                       double rope_scale, const std::array<int64_t, 10>& shape) {
   const auto [hq, hkv, d, ks, st, bs, topk, init_blocks, local_blocks, window] = shape;
+  refuse_tangent(x, w_ck, w_cv, pe);
+  for (const Tensor& t : caches) refuse_tangent(t);
+  for (const Tensor& t : weights) refuse_tangent(t);
   if (caches.size() != 4 || weights.size() != 5 || x.dim() != 2 || x.size(0) != 1) return std::nullopt;
   const Tensor &k = caches[0], &v = caches[1], &ck = caches[2], &cv = caches[3];
   auto rows_ok = [&](const Tensor& t) {
@@ -806,6 +821,7 @@ optional<std::pair<Tensor, Tensor>> layer_core(const Tensor& x, const Tensor& cu
                                                const Tensor& w_ck, const Tensor& w_cv, const Tensor& pe, const Tensor& inv_freq, double rope_scale,
                                                const LayerShape& shape, bool exact_lens) {
   const int64_t hq = shape[0], hkv = shape[1], d = shape[2], ks = shape[3], st = shape[4], bs = shape[5], hidden = shape[10];
+  refuse_tangent(x, w_q, w_k, w_v, w_o, w_gate, w_ck, w_cv, pe);
   if (!is16(x) || x.dim() != 2 || x.size(0) < 1 || !plain_input(x, x, {x.size(0), hidden}) || hkv < 1 || hq < 1 || st < 1 ||
       !layer_config_ok(hq, hkv, d, ks, st, hidden) || (bs != 32 && bs != 64 && bs != 128) || bs % st ||
       shape[6] < std::max<int64_t>(1, shape[7] + shape[8]) || !cu.is_cuda() || cu.device() != x.device() ||
