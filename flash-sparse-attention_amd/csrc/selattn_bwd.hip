@@ -307,7 +307,7 @@ int fsa::selattn_bwd(const void* q, const void* k, const void* v, const void* o,
   p.cu_seqlens = cu_seqlens; p.cu_blocks = cu_blocks; p.counts = counts; p.starts = starts;
   p.sel_tokens = sel_tokens;
   p.batch = batch; p.max_blocks = max_blocks; p.cap = cap; p.n_tokens = total_tokens; p.g = g; p.g_shift = group_shift(g);
-  p.scale = softmax_scale; p.scale_log2 = softmax_scale * LOG2E;
+  kv_set_scales(p, softmax_scale, dtype, stats != nullptr);
   p.dq_part = wsp + ws.off_dqpart;
   p.dkdv_part = (float*)(wsp + ws.off_kvpart);
   p.dk = dk; p.dv = dv;
