@@ -181,8 +181,10 @@ __device__ __forceinline__ void dec_emit(const DecParams& p, int b, int h, int c
 // Wave = (group of tiles, kv head): the waves of a group read the same cache rows, one kv head each, at about the same
 // time, so that a row (all kv heads, contiguous in memory) is fetched whole instead of in hkv visits of 2 D bytes.
 // cos / sin of x radians, |x| < 2^18: the turns are formed with the rounding error of the product and the low part of
-// 1 / (2 pi), so that the hardware instructions (which take turns) see an argument good to 2^-24
+// 1 / (2 pi), so that the hardware instructions (which take turns) see an argument good to 2^-24.  No contraction: with
+// t - rint(t) fused to x * HI - rint(t) the rounding error of t would be added twice, 6e-3 radians at x = 1e5.
 __device__ __forceinline__ void sincos_turns(float x, float& sn, float& cs) {
+#pragma clang fp contract(off)
   constexpr float HI = 0.15915494f, LO = 6.4206382e-9f;   // HI + LO = 1 / (2 pi)
   const float t = x * HI;
   const float e = __builtin_fmaf(x, HI, -t) + x * LO;
