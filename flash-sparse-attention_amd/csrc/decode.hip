@@ -297,10 +297,12 @@ decode_attn_kernel(DecParams p) {
   };
   // Layer form: rotation of the K rows of a tile in registers (the caches hold un-rotated rows).  The partner of a
   // lane's eight dims, D/2 further, sits D/16 lanes away and needs the same eight angles: each of the two forms four, packs
-  // cosine and sine as two 16-bit numbers, which is what they are rounded to anyway, and they exchange them.  Rows follow
-  // each other RPI positions apart: every fourth angle is formed anew, the others follow by the angle sum, three steps
-  // whose rounding (1e-7 each) is that of the angle itself.  (Sine and cosine of every element in every lane: 12.6
-  // and 8.4 us for the attention launches of a step over 32K tokens, this form 11.5 and 7.3.)
+  // cosine and sine as two 16-bit numbers, which is what they are rounded to anyway, and they exchange them.  Every angle
+  // is fp32 position times fp32 frequency, the product that prefill takes the sine and cosine of.  At position 131072 it
+  // may lie 4e-3 from the exact angle, and an angle that does not lie there with it (one formed by the angle sum from
+  // another row's) gives other 16-bit entries, 7 % of them in bf16.  (The angle sum for three rows of four is 1.1 us of a
+  // step of 54.6 us over 32K tokens.  What the hardware's sine and cosine leave, about 1e-6, changed none of 640 entries
+  // near positions 70000 and 131000.)
   constexpr int RPI = 64 / (D / 8);   // rows per load instruction
   auto partner = [&](uint32_t v) -> uint32_t {
     if constexpr (D == 128) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false);  // row_ror:8
@@ -316,24 +318,16 @@ decode_attn_kernel(DecParams p) {
     if constexpr (LAYER) {
       const DecParams::Source& c = MODE == DEC_MODE_COMPRESSED && r.b == 1 ? p.src[1] : p.src[0];
       const float sign = upper ? 1.f : -1.f;   // second half of the dims: x1 sin + x2 cos
-      float cs[4], sn[4], dc[4], ds[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sincos_turns((float)(RPI * c.pos_step) * freq[e], ds[e], dc[e]);
 #pragma unroll
       for (int j = 0; j < VCH; ++j) {
         const float pos = (float)(c.pos0 + (row0 + lane / (D / 8) + RPI * j) * c.pos_step);
         uint32_t mine[4], theirs[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          if (j % 4 == 0) {
-            sincos_turns(pos * freq[e], sn[e], cs[e]);
-          } else {
-            const float c0 = cs[e];
-            cs[e] = c0 * dc[e] - sn[e] * ds[e];
-            sn[e] = sn[e] * dc[e] + c0 * ds[e];
-          }
+          float cs, sn;
+          sincos_turns(pos * freq[e], sn, cs);
           typedef T pair __attribute__((ext_vector_type(2)));
-          mine[e] = __builtin_bit_cast(uint32_t, (pair){(T)(cs[e] * p.rope_scale), (T)(sn[e] * p.rope_scale)});
+          mine[e] = __builtin_bit_cast(uint32_t, (pair){(T)(cs * p.rope_scale), (T)(sn * p.rope_scale)});
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) theirs[e] = partner(mine[e]);
