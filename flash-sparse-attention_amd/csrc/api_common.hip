@@ -14,6 +14,24 @@ void set_error(const char* fmt, ...) {
   va_end(ap);
 }
 
+int set_lds_limit(const void* kernel, int bytes) {
+  const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e == hipSuccess) return 0;
+  set_error("hipFuncSetAttribute(%d B LDS): %s", bytes, hipGetErrorString(e));
+  return (int)e;
+}
+
+int allow_lds(LdsAllowed& done, const void* kernel, int bytes) {
+  if (bytes <= 48 * 1024) return 0;
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess) dev = -1;
+  const uint64_t bit = dev >= 0 && dev < 64 ? (uint64_t)1 << dev : 0;   // others: set on every call
+  if (done.devices.load(std::memory_order_relaxed) & bit) return 0;
+  const int rc = set_lds_limit(kernel, bytes);
+  if (rc == 0) done.devices.fetch_or(bit, std::memory_order_relaxed);
+  return rc;
+}
+
 struct ProfRec {
   const char* name;
   hipEvent_t start, stop;

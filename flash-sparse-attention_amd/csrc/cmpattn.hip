@@ -814,16 +814,6 @@ cmp_topk_kernel(TopkParams p) {
 }
 
 // -------------------------------------------------------------- host side ----
-template <typename K> static int cmp_set_lds(K kernel, int bytes) {
-  if (bytes <= 48 * 1024) return 0;
-  hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (e != hipSuccess) {
-    set_error("hipFuncSetAttribute(%d B LDS): %s", bytes, hipGetErrorString(e));
-    return (int)e;
-  }
-  return 0;
-}
-
 // rows of all (key tile, query head) pairs: a key tile of a sequence is seen by about half of its queries
 static int cmp_tile_rows(int64_t max_blocks, int64_t max_q, int hq, int g, int d) {
   return kv_tile_rows(max_blocks * max_q * hq / 2, g, d, CMP_BK);
@@ -856,8 +846,8 @@ static CmpBwdWs cmp_bwd_ws(int64_t n, int64_t n_k, int64_t max_q, int batch, int
 
 template <typename T, int D, int MODE>
 static int attn_fwd_launch(CmpParams p, int batch, int hkv, int64_t max_rows, hipStream_t stream) {
-  static const int rc = cmp_set_lds(cmpattn_fwd_kernel<T, D, MODE>, CmpLds<D>::BYTES);
-  if (rc) return rc;
+  static LdsAllowed lds;
+  if (int rc_ = allow_lds(lds, (const void*)cmpattn_fwd_kernel<T, D, MODE>, CmpLds<D>::BYTES)) return rc_;
   p.hkv = hkv;
   p.nx = (int)((max_rows + CMP_ROWS - 1) / CMP_ROWS);
   const unsigned grid = p.nx * batch * hkv;
@@ -878,10 +868,10 @@ template <typename T, int D, int MODE>
 static int attn_bwd_launch(CmpParams p, const SelBwdParams& kv, int batch, int hq, int hkv,
                            int64_t max_rows, int64_t n, hipStream_t stream) {
   constexpr int KVM = MODE == CMP_MODE_WINDOW ? KV_MODE_WINDOW : KV_MODE_COMPRESSED;
-  static const int rc1 = cmp_set_lds(cmpattn_bwd_dq_kernel<T, D, MODE>, CmpLds<D>::BYTES);
-  if (rc1) return rc1;
-  static const int rc2 = cmp_set_lds(attn_bwd_dkdv_kernel<T, D, CMP_BK, KVM>, KvCfg<D, CMP_BK>::BYTES);
-  if (rc2) return rc2;
+  static LdsAllowed lds1;
+  if (int rc_ = allow_lds(lds1, (const void*)cmpattn_bwd_dq_kernel<T, D, MODE>, CmpLds<D>::BYTES)) return rc_;
+  static LdsAllowed lds2;
+  if (int rc_ = allow_lds(lds2, (const void*)attn_bwd_dkdv_kernel<T, D, CMP_BK, KVM>, KvCfg<D, CMP_BK>::BYTES)) return rc_;
   p.hkv = hkv;
   p.nx = (int)((max_rows + CMP_ROWS - 1) / CMP_ROWS);
   {
@@ -912,8 +902,8 @@ static int attn_bwd_launch(CmpParams p, const SelBwdParams& kv, int batch, int h
 
 template <typename T, int D>
 static int pair_fwd_launch(CmpParams a, CmpParams b, int batch, int hkv, int64_t max_rows, hipStream_t stream) {
-  static const int rc = cmp_set_lds(attn_fwd_pair_kernel<T, D>, CmpLds<D>::BYTES);
-  if (rc) return rc;
+  static LdsAllowed lds;
+  if (int rc_ = allow_lds(lds, (const void*)attn_fwd_pair_kernel<T, D>, CmpLds<D>::BYTES)) return rc_;
   a.hkv = b.hkv = hkv;
   a.nx = b.nx = (int)((max_rows + CMP_ROWS - 1) / CMP_ROWS);
   const int tiles = a.nx * batch * hkv;
@@ -924,11 +914,11 @@ static int pair_fwd_launch(CmpParams a, CmpParams b, int batch, int hkv, int64_t
 template <typename T, int D>
 static int pair_bwd_launch(CmpParams a, CmpParams b, const SelBwdParams& ka, const SelBwdParams& kb, const KvTiles& ta,
                            const KvTiles& tb, int batch, int hkv, int64_t max_rows, hipStream_t stream) {
-  static const int rc1 = cmp_set_lds(attn_bwd_dq_pair_kernel<T, D>, CmpLds<D>::BYTES);
-  if (rc1) return rc1;
+  static LdsAllowed lds1;
+  if (int rc_ = allow_lds(lds1, (const void*)attn_bwd_dq_pair_kernel<T, D>, CmpLds<D>::BYTES)) return rc_;
   typedef KvCfg<D, CMP_BK> C;
-  static const int rc2 = cmp_set_lds(attn_bwd_dkdv_pair_kernel<T, D, CMP_BK>, C::BYTES);
-  if (rc2) return rc2;
+  static LdsAllowed lds2;
+  if (int rc_ = allow_lds(lds2, (const void*)attn_bwd_dkdv_pair_kernel<T, D, CMP_BK>, C::BYTES)) return rc_;
   a.hkv = b.hkv = hkv;
   a.nx = b.nx = (int)((max_rows + CMP_ROWS - 1) / CMP_ROWS);
   const int tiles = a.nx * batch * hkv;
@@ -1203,8 +1193,8 @@ extern "C" int fsa_cmp_topk(const void* q, const void* ck, const float* lse, int
     const dim3 grid((unsigned)((total_q + 3) / 4), (unsigned)num_kv_heads);
     if (big) {
       const int lds = (nblk + t_out) * 4;
-      rc = cmp_set_lds(cmp_topk_kernel<0, true>, lds);
-      if (rc) return rc;
+      if (lds > 48 * 1024)
+        if (int rc_ = set_lds_limit((const void*)cmp_topk_kernel<0, true>, lds)) return rc_;
       cmp_topk_kernel<0, true><<<dim3((unsigned)total_q, (unsigned)num_kv_heads), 64, lds, stream>>>(tp);
     } else if (scores_to_bf16 && nblk <= 128) cmp_topk_kernel<2><<<grid, 256, 0, stream>>>(tp);
     else if (scores_to_bf16 && nblk <= 256) cmp_topk_kernel<4><<<grid, 256, 0, stream>>>(tp);

@@ -963,12 +963,8 @@ template <int D> struct DecOne {
 };
 template <typename T, int D, int MODE> static int dec_one_launch(const DecParams& p, int pairs, hipStream_t stream) {
   constexpr int W = DecOne<D>::WAVES, LDS = W * DecLds<D>::BYTES;
-  static const hipError_t attr = hipFuncSetAttribute((const void*)decode_attn_kernel<T, D, MODE, false, W>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-  if (attr != hipSuccess) {
-    set_error("hipFuncSetAttribute(decode_attn_kernel): %s", hipGetErrorString(attr));
-    return (int)attr;
-  }
+  static LdsAllowed allowed;
+  if (int rc_ = allow_lds(allowed, (const void*)decode_attn_kernel<T, D, MODE, false, W>, LDS)) return rc_;
   decode_attn_kernel<T, D, MODE, false, W><<<pairs, WAVE * W, LDS, stream>>>(p);
   return 0;
 }

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <stdint.h>
 #include <stdio.h>
 #include <stdarg.h>
@@ -233,6 +234,15 @@ void set_error(const char* fmt, ...);
       return (int)e__;                                                       \
     }                                                                        \
   } while (0)
+
+// Dynamic LDS beyond 48 KB has to be allowed for every kernel, on every device that runs it: the attribute belongs to the
+// pair.  `done` is a static beside the launch of one kernel with one size and remembers the devices by bits; a failure is
+// reported every time it happens.
+struct LdsAllowed {
+  std::atomic<uint64_t> devices{0};
+};
+int allow_lds(LdsAllowed& done, const void* kernel, int bytes);
+int set_lds_limit(const void* kernel, int bytes);   // for sizes that change from call to call
 
 // Optional per-kernel timing: while fsa_profile_enable(1) is in effect every
 // launch wrapped in a ProfScope is bracketed by HIP events on its stream.

@@ -974,13 +974,10 @@ static int launch_index_once(const int32_t* topk_idx, int64_t stride_h, int64_t 
   while ((1 << key_bits) < nbuckets) ++key_bits;
 #define FSA_ONCE(KB)                                                                                               \
   {                                                                                                                \
-    static const hipError_t attr = hipFuncSetAttribute((const void*)index_once_kernel<KB>,                         \
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize,                 \
-                                                       (IO_MAX_COUNTERS + 2 * (IO_THREADS + 1)) * 4);              \
-    if (attr != hipSuccess) {                                                                                      \
-      set_error("hipFuncSetAttribute(index_once_kernel): %s", hipGetErrorString(attr));                            \
-      return (int)attr;                                                                                            \
-    }                                                                                                              \
+    static LdsAllowed allowed;                                                                                     \
+    if (int rc_ = allow_lds(allowed, (const void*)index_once_kernel<KB>,                                           \
+                            (IO_MAX_COUNTERS + 2 * (IO_THREADS + 1)) * 4))                                         \
+      return rc_;                                                                                                  \
     index_once_kernel<KB><<<dim3(ntiles, hkv), IO_THREADS, lds, stream>>>(                                         \
         topk_idx, stride_h, stride_n, cu_seqlens, batch, block_size, (int)n, topk, q_per_tile, nbuckets, copies,   \
         vec4, cu_blocks, counts, starts, sel_tokens, slot_of, la, lb);                                                   \
@@ -1044,17 +1041,10 @@ static int build_index(const int32_t* topk_idx, int64_t topk_stride_h, int64_t t
     dim3 g_place((c.ntiles + 7) / 8 * 8, num_kv_heads);
 #define FSA_PLACE(KB)                                                                                            \
   {                                                                                                              \
-    static bool attr_done = false;                                                                               \
-    if (!attr_done && lds > 48 * 1024) {                                                                         \
-      hipError_t e = hipFuncSetAttribute((const void*)place_items_kernel<KB>,                                    \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize,                     \
-                                         place_lds_ints(CT_MAX_BUCKETS) * 4);                                    \
-      if (e != hipSuccess) {                                                                                     \
-        set_error("hipFuncSetAttribute(place_items_kernel): %s", hipGetErrorString(e));                          \
-        return (int)e;                                                                                           \
-      }                                                                                                          \
-      attr_done = true;                                                                                          \
-    }                                                                                                            \
+    static LdsAllowed allowed;                                                                                   \
+    if (lds > 48 * 1024)                                                                                         \
+      if (int rc_ = allow_lds(allowed, (const void*)place_items_kernel<KB>, place_lds_ints(CT_MAX_BUCKETS) * 4)) \
+        return rc_;                                                                                              \
     place_items_kernel<KB><<<g_place, CT_THREADS, lds, stream>>>(                                                \
         topk_idx, topk_stride_h, topk_stride_n, cu_seqlens, cu_blocks, batch, total_tokens, topk, c.q_per_tile,  \
         c.ntiles, c.nbuckets, table, totals, starts, sel_tokens, slot_of, la, lb);                               \

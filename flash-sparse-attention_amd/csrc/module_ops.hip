@@ -579,20 +579,12 @@ extern "C" int fsa_rope(const void* x, void* out, int32_t dtype, int64_t x_strid
   return 0;
 }
 
-template <typename K> static int lc_set_lds(K kernel, int bytes) {
-  if (bytes <= 48 * 1024) return 0;
-  hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (e == hipSuccess) return 0;
-  set_error("hipFuncSetAttribute(%d B LDS): %s", bytes, hipGetErrorString(e));
-  return (int)e;
-}
-
 template <typename T, int D, int DN>
 static int launch_lc_fwd(const LcPair& p, dim3 grid, const int32_t* cu_x, const int32_t* cu_y, int h, int ks, int stride,
                          hipStream_t stream) {
   constexpr int BYTES = LcFwdLds<D, DN>::BYTES;
-  static const int rc = lc_set_lds(lc_fwd_kernel<T, D, DN>, BYTES);
-  if (rc) return rc;
+  static LdsAllowed lds;
+  if (int rc_ = allow_lds(lds, (const void*)lc_fwd_kernel<T, D, DN>, BYTES)) return rc_;
   grid.z *= D / DN;
   ProfScope ps_("linear_compress_fwd", stream);
   lc_fwd_kernel<T, D, DN><<<grid, 64 * LCF_WAVES, BYTES, stream>>>(p, cu_x, cu_y, h, ks, stride);
@@ -616,10 +608,10 @@ static int lc_fwd_t(const LcPair& p, int n, const int32_t* cu_x, const int32_t* 
 template <typename T, int D>
 static int lc_bwd_t(const LcPair& p, int n, const int32_t* cu_x, const int32_t* cu_y, int batch, int64_t max_x, int h, int ks,
                     int stride, hipStream_t stream) {
-  static const int rc1 = lc_set_lds(lc_dx_kernel<T, D>, D * (D + 8) * 2);
-  if (rc1) return rc1;
-  static const int rc2 = lc_set_lds(lc_dw_kernel<T, D>, LcDwLds<D>::BYTES);
-  if (rc2) return rc2;
+  static LdsAllowed lds1;
+  if (int rc_ = allow_lds(lds1, (const void*)lc_dx_kernel<T, D>, D * (D + 8) * 2)) return rc_;
+  static LdsAllowed lds2;
+  if (int rc_ = allow_lds(lds2, (const void*)lc_dw_kernel<T, D>, LcDwLds<D>::BYTES)) return rc_;
   {
     ProfScope ps_("linear_compress_dx", stream);
     const int64_t m_per_phase = (max_x + stride - 1) / stride;

@@ -148,22 +148,12 @@ static BwdWs bwd_ws_layout(int64_t n, int hq, int hkv, int d, int topk, int bk, 
   return w;
 }
 
-template <typename K> static int set_lds(K kernel, int bytes) {
-  if (bytes <= 48 * 1024) return 0;
-  hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (e != hipSuccess) {
-    set_error("hipFuncSetAttribute(%d B LDS): %s", bytes, hipGetErrorString(e));
-    return (int)e;
-  }
-  return 0;
-}
-
 template <typename T, int D, int BK>
 static int launch_bwd(const SelBwdParams& pkv, int hkv, int64_t tiles_kv, const DqReduceArgs& red,
                       hipStream_t stream) {
   const unsigned kv_spans = (unsigned)((pkv.max_blocks + KV_REDUCE_SPAN - 1) / KV_REDUCE_SPAN);
-  static const int rc = set_lds(attn_bwd_dkdv_kernel<T, D, BK, KV_MODE_SELECTED, true>, KvCfg<D, BK>::BYTES_FUSED);
-  if (rc) return rc;
+  static LdsAllowed lds;
+  if (int rc_ = allow_lds(lds, (const void*)attn_bwd_dkdv_kernel<T, D, BK, KV_MODE_SELECTED, true>, KvCfg<D, BK>::BYTES_FUSED)) return rc_;
   {
     const HeadOrder order = head_order(hkv, pkv.n_tokens * pkv.g * D * 2);
     ProfScope ps_("selattn_bwd_dqdkdv", stream);

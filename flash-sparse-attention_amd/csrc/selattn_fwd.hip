@@ -445,16 +445,8 @@ static FwdWs fwd_ws_layout(int64_t n_tokens, int hq, int hkv, int d, int topk, i
 template <typename T, int D, int BK>
 static int launch_main(const SelFwdParams& p, int hkv, int64_t max_tiles, hipStream_t stream) {
   constexpr int lds = SelLds<D, BK>::BYTES;
-  static bool attr_done = false;
-  if (!attr_done && lds > 48 * 1024) {
-    hipError_t e = hipFuncSetAttribute((const void*)selattn_fwd_main_kernel<T, D, BK>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (e != hipSuccess) {
-      set_error("hipFuncSetAttribute(%d B LDS): %s", lds, hipGetErrorString(e));
-      return (int)e;
-    }
-    attr_done = true;
-  }
+  static LdsAllowed allowed;
+  if (int rc_ = allow_lds(allowed, (const void*)selattn_fwd_main_kernel<T, D, BK>, lds)) return rc_;
   const HeadOrder order = head_order(hkv, p.n_tokens * p.g * D * 2);
   ProfScope ps_("selattn_fwd_main", stream);
   selattn_fwd_main_kernel<T, D, BK><<<head_tile_grid(max_tiles, order), SelLds<D, BK>::THREADS, lds, stream>>>(p, order);
