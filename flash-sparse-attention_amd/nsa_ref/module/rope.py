@@ -83,11 +83,10 @@ class RotaryEmbedding(nn.Module):
             return inv.to(device)
         c = self.config
         key = (device, c.head_dim, c.rope_theta, tuple(c.rope_scaling.items()) if c.rope_scaling else None)
-        tables = self.__dict__.setdefault("_tables", {})
-        if key not in tables:
-            tables.clear()
-            tables[key] = _inv_freq(c).to(device)
-        return tables[key]
+        kept = self.__dict__.get("_table")   # (key, table), replaced as a whole: other threads may be here as well
+        if kept is None or kept[0] != key:
+            kept = self.__dict__["_table"] = (key, _inv_freq(c).to(device))
+        return kept[1]
 
     def forward(self, x: torch.Tensor, cu_seqlens: torch.Tensor, start: int = 0, stride: int = 1):
         """Token j of every sequence is rotated for position start + j * stride."""
