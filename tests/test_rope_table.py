@@ -17,27 +17,26 @@ def test_table_follows_configuration_and_device():
     assert torch.equal(rope.table(cpu), _inv_freq(rope.config))
 
 
-def test_another_thread_between_any_two_lines():
-    """A second caller with another device comes in before every line of the first one's call (a trace function stands in
-    for it: that is where a thread can be switched)."""
-    cpu, meta = torch.device("cpu"), torch.device("meta")
-    for first in (cpu, meta):
-        rope = RotaryEmbedding(RopeConfig(head_dim=64)).to(torch.bfloat16)
-        if first is meta:
-            rope.table(cpu)
-        visits = []
+def test_another_caller_between_any_two_lines():
+    """A second caller, with another configuration each time, comes in before every line of the first one's call (a trace
+    function stands in for its thread: that is where threads are switched)."""
+    rope = RotaryEmbedding(RopeConfig(head_dim=64, rope_theta=10000)).to(torch.bfloat16)
+    cpu, want = torch.device("cpu"), _inv_freq(rope.config)
+    visits = []
 
-        def tracer(frame, event, arg):
-            if frame.f_code is not RotaryEmbedding.table.__code__:
-                return None
-            if event == "line":
-                visits.append(rope.table(meta if first is cpu else cpu).device)
-            return tracer
+    def tracer(frame, event, arg):
+        if frame.f_code is not RotaryEmbedding.table.__code__:
+            return None
+        if event == "line":
+            rope.config.rope_theta = 20000 + len(visits)
+            visits.append(torch.equal(rope.table(cpu), _inv_freq(rope.config)))
+            rope.config.rope_theta = 10000
+        return tracer
 
-        before = sys.gettrace()
-        sys.settrace(tracer)
-        try:
-            got = rope.table(first)
-        finally:
-            sys.settrace(before)
-        assert got.device == first and len(visits) > 3 and first not in visits
+    before = sys.gettrace()
+    sys.settrace(tracer)
+    try:
+        got = rope.table(cpu)
+    finally:
+        sys.settrace(before)
+    assert torch.equal(got, want) and len(visits) > 3 and all(visits)
