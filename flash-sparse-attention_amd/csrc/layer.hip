@@ -360,15 +360,16 @@ static LayerSaved layer_saved(const fsa_layer_args& a) {
   s.k = b.take(n * hkv * d * e);
   s.ck = b.take((size_t)a.total_ck * hkv * d * e);
   s.cv = b.take((size_t)a.total_ck * hkv * d * e);
-  for (int i = 0; i < 3; ++i) s.o[i] = b.take(n * hq * d * e);
-  for (int i = 0; i < 3; ++i) s.lse[i] = b.take(n * hq * 4);
+  // (inference: the selected branch goes into the gated sum without being stored, and nothing asks for the backward's tiles)
+  for (int i = 0; i < 3; ++i) s.o[i] = b.take(a.inference && i == 1 ? 0 : n * hq * d * e);
+  for (int i = 0; i < 3; ++i) s.lse[i] = b.take(a.inference && i == 1 ? 0 : n * hq * 4);
   s.cu_blocks = b.take((a.batch + 1) * 4);
   s.counts = b.take(hkv * s.max_blocks * 4);
   s.starts = b.take(hkv * (s.max_blocks + 1) * 4);
   s.sel = b.take(hkv * n * s.t_out * 4);
   s.slot = b.take(hkv * n * s.t_out * 4);
   s.tiles_fwd = b.take(fsa_selattn_tiles_bytes(0, n, hq, hkv, d, s.t_out, a.block_size, s.max_blocks));
-  s.tiles_bwd = b.take(fsa_selattn_tiles_bytes(1, n, hq, hkv, d, s.t_out, a.block_size, s.max_blocks));
+  s.tiles_bwd = b.take(a.inference ? 0 : fsa_selattn_tiles_bytes(1, n, hq, hkv, d, s.t_out, a.block_size, s.max_blocks));
   s.total = b.at;
   return s;
 }
@@ -516,7 +517,7 @@ static int layer_forward(const fsa_layer_args& a, void* out, int32_t* topk_idx, 
   merge.out = out;
   FSA_RUN(selattn_fwd(q, k, a.v, a.dtype, qs, d, ks_, d, ks_, d, a.cu_seqlens, a.batch, n, a.num_q_heads, a.num_kv_heads, a.head_dim,
                       s.t_out, a.block_size, s.max_blocks, a.softmax_scale, cu_blocks, counts, starts, sel, slot, tf,
-                      a.inference ? nullptr : sv + s.o[1], qs, d, (float*)(sv + s.lse[1]), ws + w.stage, w.sel_bytes, merge, stream));
+                      a.inference ? nullptr : sv + s.o[1], qs, d, a.inference ? nullptr : (float*)(sv + s.lse[1]), ws + w.stage, w.sel_bytes, merge, stream));
   return 0;
 }
 
@@ -632,6 +633,7 @@ extern "C" int fsa_layer_backward(const fsa_layer_args* args, const fsa_layer_gr
   if (int rc = layer_check(args)) return rc;
   FSA_CHECK_ARG(grads && grads->d_out && grads->dq && grads->dk && grads->dv && grads->dw_gate && grads->dw_ck && grads->dw_cv &&
                     grads->dpe, "fsa_layer_backward: null pointer");
+  FSA_CHECK_ARG(!args->inference, "fsa_layer_backward: the forward ran for inference and kept nothing for a backward");
   if (args->saved_bytes < fsa_layer_saved_bytes(args) || args->workspace_bytes < fsa_layer_workspace_bytes(args, 1)) {
     set_error("fsa_layer_backward: workspace too small");
     return FSA_ERR_WORKSPACE;
