@@ -834,7 +834,7 @@ static CmpBwdWs cmp_bwd_ws(int64_t n, int64_t n_k, int64_t max_q, int batch, int
   w.max_blocks = (n_k + CMP_BK - 1) / CMP_BK + batch;
   // a key tile is seen by at most max_q queries of its sequence; rows = queries * g
   w.tile_rows = cmp_tile_rows(w.max_blocks, max_q, hq, g, d);
-  w.max_tiles = w.max_blocks * ((max_q * g + w.tile_rows - 1) / w.tile_rows + 1);
+  w.max_tiles = w.max_blocks * ((max_q * g + w.tile_rows - 1) / w.tile_rows);
   w.off_delta = 0;
   w.off_cu_tiles = align_up((size_t)n * hq * 4, 256);
   w.off_counts = w.off_cu_tiles + align_up((size_t)(batch + 1) * 4, 256);
@@ -1237,7 +1237,7 @@ static CmpBwdWs win_bwd_ws(int64_t n, int64_t max_q, int window, int batch, int 
   const int g = hq / hkv;
   const int64_t rows = (int64_t)(CMP_BK + window) * g;
   w.tile_rows = win_tile_rows(w.max_blocks, window, hq, g, d);
-  w.max_tiles = w.max_blocks * ((rows + w.tile_rows - 1) / w.tile_rows + 1);
+  w.max_tiles = w.max_blocks * ((rows + w.tile_rows - 1) / w.tile_rows);   // as kv_tiles deals them
   w.total = w.off_part + align_up((size_t)hkv * w.max_tiles * 2 * CMP_BK * d * 4, 256);
   return w;
 }
