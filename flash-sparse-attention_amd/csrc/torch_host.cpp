@@ -638,10 +638,14 @@ struct HostCopy {
   }
 };
 
-// Whether the products of a layer run as fsa_matmul launches instead of library calls.  The line lies where what the
-// library gains on the device (from about 250 tokens at hidden 4096, 2500 at 2048; never at 1024 for a training step)
-// meets what its calls cost the host: 12 of 20-25 us in a training step that needs 0.25 ms beside them, 4 in an inference
-// step.
+// Whether the products of a layer run as fsa_matmul launches instead of library calls: a bound on the operations of q, k and
+// v.  All products of a step issued back to back, ours / library in us, training (13 products) | inference (4); the library's
+// times below 225 | 77 are what its calls cost the host:
+//   hidden 4096, 32 + 8 heads: 250 tokens 176 / 225 | 60 / 78, 500 tokens (25e9) 293 / 263 | 102 / 83
+//   hidden 2048, 16 + 4 heads: 1000 tokens (13e9) 158 / 223 | 53 / 77, 2000 (25e9) 220 / 254 | 72 / 76, 4000 392 / 389 | 125 / 98
+//   hidden 1024,  8 + 2 heads: 8000 tokens (25e9) 226 / 356 | 72 / 77, 16000 434 / 606 | 134 / 90
+// The line suits the wide layer; narrower ones are handed over earlier than they need be (hidden 1024 in training at 7600
+// tokens, where ours would still be faster at 16000).
 bool own_products(int64_t n, int64_t hidden, const LayerShape& shape, bool training) {
   return 2.0 * (double)n * (double)hidden * (double)((shape[0] + 2 * shape[1]) * shape[2]) <= (training ? 24e9 : 10e9);
 }

@@ -2,8 +2,12 @@
 constructor, parameter names / shapes / initialisation and forward contract.
 
 Branches: compressed attention (+ top-k block selection), selected attention, sliding-window
-attention, mixed by a sigmoid gate.  Every attention-side operator runs in the gfx950 library;
-the dense projections are torch.nn.Linear (rocBLAS / hipBLASLt), as in the reference."""
+attention, mixed by a sigmoid gate.  The projections are torch.nn.Linear modules, as in the
+reference.  Where they, the gate and the rotary embedding are plain (no hooks, patches, biases,
+autocast or tensor subclasses) and the sizes have kernels, the whole layer is one native autograd
+node, whose projections are grouped products of the gfx950 library for small batches and BLAS
+library calls beyond; otherwise it is composed of the modules and the single operators.  Every
+attention-side operator runs in the gfx950 library on both routes."""
 from __future__ import annotations
 
 import torch
