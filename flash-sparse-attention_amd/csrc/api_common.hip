@@ -84,8 +84,9 @@ pad_head_dim_kernel(const uint16_t* __restrict__ src, int64_t src_sn, int64_t sr
 }  // namespace fsa
 
 // 200: fsa_decode_topk gained scores_to_bf16 and fsa_decode_selattn gained seqlens (both inside their argument
-// lists); 210: fsa_cmp_topk gained score_head_as_written, fsa_native_head_dim / fsa_pad_head_dim added.
-extern "C" int fsa_version(void) { return 210; }
+// lists); 210: fsa_cmp_topk gained score_head_as_written, fsa_native_head_dim / fsa_pad_head_dim added; 220:
+// fsa_linear_compress_fwd wants pe 16-byte aligned, work-list, layer and matrix-product entry points added.
+extern "C" int fsa_version(void) { return FSA_HIP_VERSION; }
 
 extern "C" int fsa_native_head_dim(int32_t head_dim) {
   if (head_dim < 1 || head_dim > 256) return -1;

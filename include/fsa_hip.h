@@ -42,8 +42,12 @@ extern "C" {
  * older header must check it at load: argument lists changed at
  *   200: fsa_decode_topk (scores_to_bf16 added), fsa_decode_selattn (seqlens added);
  *   210: fsa_cmp_topk (score_head_as_written added); fsa_native_head_dim and
- *        fsa_pad_head_dim are new. */
-#define FSA_HIP_VERSION 210
+ *        fsa_pad_head_dim are new;
+ *   220: no list, but fsa_linear_compress_fwd wants pe 16-byte aligned and no longer
+ *        uses bias_scratch; fsa_build_index_tiles, fsa_selattn_tiles_bytes,
+ *        fsa_selattn_fwd_tiles, fsa_selattn_bwd_tiles, fsa_decode_layer_*,
+ *        fsa_layer_* and fsa_matmul are new. */
+#define FSA_HIP_VERSION 220
 int fsa_version(void);
 /* Human-readable description of the last error on the calling thread. */
 const char* fsa_last_error(void);
