@@ -1117,7 +1117,7 @@ extern "C" int fsa_cmpattn_bwd(const void* q, const void* ck, const void* cv, co
   kv.cu_seqlens = cu_seqlens_q; kv.cu_blocks = cu_tiles; kv.counts = counts; kv.starts = nullptr;
   kv.sel_tokens = nullptr; kv.tile_prefix = tile_prefix;
   kv.batch = batch; kv.max_blocks = ws.max_blocks; kv.cap = 0; kv.n_tokens = total_q; kv.g = g; kv.g_shift = group_shift(g);
-  kv_set_scales(kv, softmax_scale, dtype, false);
+  kv.scale = softmax_scale; kv.scale_log2 = softmax_scale * LOG2E;
   kv.dq_part = nullptr; kv.dkdv_part = (float*)(wsp + ws.off_part); kv.max_tiles = ws.max_tiles;
   kv.dk = dck; kv.dv = dcv; kv.dk_sn = (int64_t)num_kv_heads * head_dim; kv.dk_sh = head_dim;
   kv.cu_seqlens_k = cu_seqlens_k; kv.kernel_size = kernel_size; kv.kernel_stride = kernel_stride;
@@ -1294,7 +1294,7 @@ extern "C" int fsa_winattn_bwd(const void* q, const void* k, const void* v, cons
   kv.v_sn = v_stride_n; kv.v_sh = v_stride_h; kv.do_sn = do_stride_n; kv.do_sh = do_stride_h;
   kv.cu_seqlens = cu_seqlens; kv.cu_blocks = cu_tiles; kv.counts = counts; kv.tile_prefix = tile_prefix;
   kv.batch = batch; kv.max_blocks = ws.max_blocks; kv.n_tokens = total_tokens; kv.g = g; kv.g_shift = group_shift(g);
-  kv_set_scales(kv, softmax_scale, dtype, false);
+  kv.scale = softmax_scale; kv.scale_log2 = softmax_scale * LOG2E;
   kv.dkdv_part = (float*)(wsp + ws.off_part); kv.max_tiles = ws.max_tiles;
   kv.dk = dk; kv.dv = dv; kv.dk_sn = (int64_t)num_kv_heads * head_dim; kv.dk_sh = head_dim;
   kv.cu_seqlens_k = cu_seqlens; kv.kernel_size = 1; kv.kernel_stride = 1; kv.window = window;
@@ -1355,7 +1355,7 @@ int fsa::layer_attn_bwd(const LayerAttn& l, void* workspace, hipStream_t stream)
     k.do_sn = p[i].do_sn; k.do_sh = p[i].do_sh;
     k.cu_seqlens = p[i].cu_q; k.cu_seqlens_k = p[i].cu_k; k.cu_blocks = cu_tiles; k.counts = counts; k.tile_prefix = prefix;
     k.batch = l.batch; k.max_blocks = w[i].max_blocks; k.n_tokens = l.n; k.g = g; k.g_shift = group_shift(g);
-    kv_set_scales(k, l.scale, dtype, true);
+    k.scale = p[i].scale; k.scale_log2 = p[i].scale_log2;
     k.dkdv_part = (float*)(ws + w[i].off_part); k.max_tiles = w[i].max_tiles;
     k.dk = i ? l.dk_win : l.dck; k.dv = i ? l.dv_win : l.dcv; k.dk_sn = p[i].k_sn; k.dk_sh = head_dim;
     k.kernel_size = p[i].kernel_size; k.kernel_stride = p[i].kernel_stride; k.window = p[i].window;

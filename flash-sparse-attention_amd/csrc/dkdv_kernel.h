@@ -39,9 +39,8 @@ struct SelBwdParams {
   int64_t n_tokens;
   int g;
   int g_shift;  // log2 g, or -1 if g is not a power of two
+  float scale;
   float scale_log2;
-  // Probabilities are held times 2^p_shift on their way into the dV product (kv_set_scales); ds_scale and dv_scale undo it.
-  float p_shift, ds_scale, dv_scale;
   void* dq_part;     // [Hkv, cap, g, D]
   float* dkdv_part;  // [Hkv, max_tiles, 2, BK, D]
   int64_t max_tiles;
@@ -53,17 +52,6 @@ struct SelBwdParams {
   int kernel_size, kernel_stride;
   int window;  // sliding-window mode only
 };
-
-// Host.  `gated`: the probabilities carry the gate of their token (statistics from merge_stats), which may be small: in fp16
-// gate times probability falls below the normal range long before gate times gradient would (2048 keys, gate 0.002: error
-// of dV 1.2e-3 against 4.3e-4 at gate 0.5).  Held times 2^15 they reach 2^15 at most, half of fp16's range, and have all
-// their bits down to 2^-29.  A power of two: nothing else changes.
-inline void kv_set_scales(SelBwdParams& p, float softmax_scale, int dtype, bool gated) {
-  p.scale_log2 = softmax_scale * LOG2E;
-  p.p_shift = gated && dtype == FSA_FP16 ? 15.f : 0.f;
-  p.dv_scale = gated && dtype == FSA_FP16 ? 0x1p-15f : 1.f;
-  p.ds_scale = softmax_scale * p.dv_scale;
-}
 
 // Host: the kernels form q / dO row addresses with 32-bit strides - token stride and the whole span of a kv head's
 // q heads must be non-negative and below 2^31 elements.
@@ -181,13 +169,20 @@ template <int D, int BK> struct KvCfg {
 // FUSE_DQ (selected mode): the work-group also produces the partial dQ rows of
 // its (query, block) pairs - dQ^T = K^T dS^T with dS^T exchanged between the
 // waves through LDS - so Q and dO are gathered once for dQ, dK and dV.
-template <typename T, int D, int BK, int MODE, bool FUSE_DQ = false>
+// GATED: the probabilities carry the gate of their token (statistics from merge_stats), which may be small.  In fp16 gate
+// times probability falls below the normal range long before gate times gradient would (1024 keys: error of dV 4.3e-4 at
+// gate 0.5, 1.2e-3 at 0.002, 1.1e-2 at 0.0002).  Held times 2^15 they reach 2^15 at most, half of fp16's range, and keep
+// all their bits down to 2^-29; dS and the dV accumulators undo the factor, a power of two, exactly.  A parameter of the
+// kernel because the few instructions cost the fp16 D = 256 backward without gates 3.7 % (4.14 -> 4.30 ms, 131072 tokens).
+template <typename T, int D, int BK, int MODE, bool FUSE_DQ = false, bool GATED = false>
 __device__ __forceinline__ void attn_bwd_dkdv_tile(const SelBwdParams& p, const int w, const int h) {
   typedef typename Elem<T>::vec8 vec8;
   typedef typename Elem<T>::vec4 vec4;
   typedef KvCfg<D, BK> C;
   constexpr int QS = C::QS, NS = D / 32, NDT = D / 16, NRT = C::NRT, NU = C::KV_R / 32;
-  constexpr bool SHIFTED = std::is_same_v<T, _Float16>;   // p_shift may be set
+  constexpr bool SHIFTED = GATED && std::is_same_v<T, _Float16>;
+  constexpr float P_SHIFT = 15.f, P_UNDO = 0x1p-15f;
+  const float ds_scale = SHIFTED ? p.scale * P_UNDO : p.scale;
   // aligned to the bank line and to the largest swizzled row: group addresses are formed by XOR on byte addresses
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   T* Qs = reinterpret_cast<T*>(smem);
@@ -312,7 +307,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const SelBwdParams& p, const 
           lse_st = p.lse[stat];
           del_st = p.delta[stat];
         }
-        if constexpr (SHIFTED) lse_st -= p.p_shift;
+        if constexpr (SHIFTED) lse_st -= P_SHIFT;
         lim_st = blk.limit(p, token - blk.seq_start);
         llo_st = blk.limit_lo(p, token - blk.seq_start);
       }
@@ -472,7 +467,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const SelBwdParams& p, const 
       for (int i = 0; i < 4; ++i) {
         const bool vis = key <= lim_r[i] && (MODE != KV_MODE_WINDOW || key >= llo_r[i]);
         const float pv = vis ? fast_exp2(sacc[i] * p.scale_log2 - lse_r[i]) : 0.f;
-        const float ds = pv * (dpacc[i] - del_r[i]) * p.ds_scale;
+        const float ds = pv * (dpacc[i] - del_r[i]) * ds_scale;
         pk[rt][i] = (T)pv;
         dsk[rt][i] = (T)ds;
       }
@@ -658,7 +653,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const SelBwdParams& p, const 
   // accumulators: dV^T[d = 16*t + 4*kg + i][key]
   if constexpr (SHIFTED) {
 #pragma unroll
-    for (int t = 0; t < NDT; ++t) dvacc[t] *= p.dv_scale;
+    for (int t = 0; t < NDT; ++t) dvacc[t] *= P_UNDO;
   }
   if (ntile_b == 1) {
     if (key_ok) {
@@ -686,12 +681,12 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const SelBwdParams& p, const 
   }
 }
 
-template <typename T, int D, int BK, int MODE, bool FUSE_DQ = false>
+template <typename T, int D, int BK, int MODE, bool FUSE_DQ = false, bool GATED = false>
 __global__ void __launch_bounds__((KvCfg<D, BK>::NT), (KvCfg<D, BK>::MIN_WAVES))
 attn_bwd_dkdv_kernel(SelBwdParams p, HeadOrder order) {
   int h, w;
   head_tile(order, h, w);
-  attn_bwd_dkdv_tile<T, D, BK, MODE, FUSE_DQ>(p, w, h);
+  attn_bwd_dkdv_tile<T, D, BK, MODE, FUSE_DQ, GATED>(p, w, h);
 }
 // compressed and window attention of one layer in one launch: the first `na` work-groups of a kv head take tiles of a
 template <typename T, int D, int BK>
@@ -699,8 +694,8 @@ __global__ void __launch_bounds__((KvCfg<D, BK>::NT), (KvCfg<D, BK>::MIN_WAVES))
 attn_bwd_dkdv_pair_kernel(SelBwdParams a, SelBwdParams b, int na, HeadOrder order) {
   int h, w;
   head_tile(order, h, w);
-  if (w < na) attn_bwd_dkdv_tile<T, D, BK, KV_MODE_COMPRESSED>(a, w, h);
-  else attn_bwd_dkdv_tile<T, D, BK, KV_MODE_WINDOW>(b, w - na, h);
+  if (w < na) attn_bwd_dkdv_tile<T, D, BK, KV_MODE_COMPRESSED, false, true>(a, w, h);
+  else attn_bwd_dkdv_tile<T, D, BK, KV_MODE_WINDOW, false, true>(b, w - na, h);
 }
 
 // Blocks with no selecting query get zeros; blocks split over several

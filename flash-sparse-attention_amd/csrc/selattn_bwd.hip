@@ -148,16 +148,17 @@ static BwdWs bwd_ws_layout(int64_t n, int hq, int hkv, int d, int topk, int bk, 
   return w;
 }
 
-template <typename T, int D, int BK>
+template <typename T, int D, int BK, bool GATED>
 static int launch_bwd(const SelBwdParams& pkv, int hkv, int64_t tiles_kv, const DqReduceArgs& red,
                       hipStream_t stream) {
   const unsigned kv_spans = (unsigned)((pkv.max_blocks + KV_REDUCE_SPAN - 1) / KV_REDUCE_SPAN);
   static LdsAllowed lds;
-  if (int rc_ = allow_lds(lds, (const void*)attn_bwd_dkdv_kernel<T, D, BK, KV_MODE_SELECTED, true>, KvCfg<D, BK>::BYTES_FUSED)) return rc_;
+  if (int rc_ = allow_lds(lds, (const void*)attn_bwd_dkdv_kernel<T, D, BK, KV_MODE_SELECTED, true, GATED>, KvCfg<D, BK>::BYTES_FUSED))
+    return rc_;
   {
     const HeadOrder order = head_order(hkv, pkv.n_tokens * pkv.g * D * 2);
     ProfScope ps_("selattn_bwd_dqdkdv", stream);
-    attn_bwd_dkdv_kernel<T, D, BK, KV_MODE_SELECTED, true>
+    attn_bwd_dkdv_kernel<T, D, BK, KV_MODE_SELECTED, true, GATED>
         <<<head_tile_grid(tiles_kv, order), KvCfg<D, BK>::NT, KvCfg<D, BK>::BYTES_FUSED, stream>>>(pkv, order);
   }
   constexpr int RPB = 256 / (D / 8);
@@ -173,10 +174,14 @@ static int launch_bwd(const SelBwdParams& pkv, int hkv, int64_t tiles_kv, const 
 }
 
 template <typename T>
-static int dispatch_bwd(int d, int bk, const SelBwdParams& pkv, int hkv, int64_t tiles_kv,
+static int dispatch_bwd(int d, int bk, bool gated, const SelBwdParams& pkv, int hkv, int64_t tiles_kv,
                         const DqReduceArgs& red, hipStream_t stream) {
 #define FSA_CASE(DD, BB) \
-  if (d == DD && bk == BB) return launch_bwd<T, DD, BB>(pkv, hkv, tiles_kv, red, stream);
+  if (d == DD && bk == BB) {                                                                                   \
+    if constexpr (std::is_same_v<T, _Float16>)  /* the two forms differ in fp16 only */                        \
+      if (gated) return launch_bwd<T, DD, BB, true>(pkv, hkv, tiles_kv, red, stream);                          \
+    return launch_bwd<T, DD, BB, false>(pkv, hkv, tiles_kv, red, stream);                                      \
+  }
   FSA_CASE(128, 64)
   FSA_CASE(128, 32)
   FSA_CASE(128, 128)
@@ -297,7 +302,7 @@ int fsa::selattn_bwd(const void* q, const void* k, const void* v, const void* o,
   p.cu_seqlens = cu_seqlens; p.cu_blocks = cu_blocks; p.counts = counts; p.starts = starts;
   p.sel_tokens = sel_tokens;
   p.batch = batch; p.max_blocks = max_blocks; p.cap = cap; p.n_tokens = total_tokens; p.g = g; p.g_shift = group_shift(g);
-  kv_set_scales(p, softmax_scale, dtype, stats != nullptr);
+  p.scale = softmax_scale; p.scale_log2 = softmax_scale * LOG2E;
   p.dq_part = wsp + ws.off_dqpart;
   p.dkdv_part = (float*)(wsp + ws.off_kvpart);
   p.dk = dk; p.dv = dv;
@@ -309,8 +314,8 @@ int fsa::selattn_bwd(const void* q, const void* k, const void* v, const void* o,
   red.dq_part = p.dq_part; red.slot_of = slot_of; red.cap = cap; red.n_tokens = total_tokens;
   red.hq = num_q_heads; red.g = g; red.topk = topk; red.dq = dq; red.epi = epi;
   rc = dtype == FSA_BF16
-           ? dispatch_bwd<__bf16>(head_dim, block_size, p, num_kv_heads, ws.max_tiles_kv, red, stream)
-           : dispatch_bwd<_Float16>(head_dim, block_size, p, num_kv_heads, ws.max_tiles_kv, red, stream);
+           ? dispatch_bwd<__bf16>(head_dim, block_size, stats != nullptr, p, num_kv_heads, ws.max_tiles_kv, red, stream)
+           : dispatch_bwd<_Float16>(head_dim, block_size, stats != nullptr, p, num_kv_heads, ws.max_tiles_kv, red, stream);
   if (rc) return rc;
   FSA_CHECK_LAUNCH("fsa_selattn_bwd dq/dk/dv");
   return 0;
