@@ -21,10 +21,9 @@ int set_lds_limit(const void* kernel, int bytes) {
   return (int)e;
 }
 
-int allow_lds(LdsAllowed& done, const void* kernel, int bytes) {
+int allow_lds(LdsAllowed& done, const void* kernel, int bytes, int dev) {
   if (bytes <= 48 * 1024) return 0;
-  int dev = -1;
-  if (hipGetDevice(&dev) != hipSuccess) dev = -1;
+  if (dev < 0 && hipGetDevice(&dev) != hipSuccess) dev = -1;
   const uint64_t bit = dev >= 0 && dev < 64 ? (uint64_t)1 << dev : 0;   // others: set on every call
   if (done.devices.load(std::memory_order_relaxed) & bit) return 0;
   const int rc = set_lds_limit(kernel, bytes);

@@ -961,20 +961,21 @@ decode_layer_combine_kernel(DecParams p, DecLayerParams lp) {
 template <int D> struct DecOne {
   static constexpr int WAVES = D >= 256 ? 4 : 8;   // what the registers allow
 };
-template <typename T, int D, int MODE> static int dec_one_launch(const DecParams& p, int pairs, hipStream_t stream) {
+template <typename T, int D, int MODE> static int dec_one_launch(const DecParams& p, int pairs, int dev, hipStream_t stream) {
   constexpr int W = DecOne<D>::WAVES, LDS = W * DecLds<D>::BYTES;
   static LdsAllowed allowed;
-  if (int rc_ = allow_lds(allowed, (const void*)decode_attn_kernel<T, D, MODE, false, W>, LDS)) return rc_;
+  if (int rc_ = allow_lds(allowed, (const void*)decode_attn_kernel<T, D, MODE, false, W>, LDS, dev)) return rc_;
   decode_attn_kernel<T, D, MODE, false, W><<<pairs, WAVE * W, LDS, stream>>>(p);
   return 0;
 }
 
-// number of waves that are resident at once on the current device
+// number of waves that are resident at once on the current device, and that device
 template <typename T, int D, int MODE>
-static int dec_grid_waves(int* n_waves) {
+static int dec_grid_waves(int* n_waves, int* device) {
   static int cached[16] = {0};
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
+  *device = e == hipSuccess ? dev : -1;
   if (e == hipSuccess && dev >= 0 && dev < 16 && cached[dev] > 0) {
     *n_waves = cached[dev];
     return 0;
@@ -999,8 +1000,8 @@ static int dec_grid_waves(int* n_waves) {
 // actually reads (q head number h for kv head h) they need a column of their own, so that launch has 15 heads.
 template <typename T, int D, int MODE>
 static int dec_launch(const DecParams& p0, hipStream_t stream) {
-  int n_waves = 0;
-  int rc = dec_grid_waves<T, D, MODE>(&n_waves);
+  int n_waves = 0, dev = -1;
+  int rc = dec_grid_waves<T, D, MODE>(&n_waves, &dev);
   if (rc) return rc;
   ProfScope ps_(MODE == DEC_MODE_COMPRESSED ? "decode_cmpattn" : "decode_selattn", stream);
   DecParams p = p0;
@@ -1024,7 +1025,7 @@ static int dec_launch(const DecParams& p0, hipStream_t stream) {
     p.g = std::min(p0.g - head0, own_col ? 15 : 16);
     p.score_col = own_col ? p.g : 0;
     if (one) {
-      rc = dec_one_launch<T, D, MODE>(p, p.batch * p.hkv, stream);
+      rc = dec_one_launch<T, D, MODE>(p, p.batch * p.hkv, dev, stream);
       if (rc) return rc;
     } else {
       decode_attn_kernel<T, D, MODE><<<grid, WAVE * wg_waves, DecLds<D>::BYTES * wg_waves, stream>>>(p);
@@ -1131,8 +1132,8 @@ static int dec_layer_attend(const fsa_decode_layer_args& a, hipStream_t stream) 
   const DecLayerParams lp = dec_layer_params(a, w);
   char* ws = (char*)a.workspace;
   const int L = (int)a.cache_len, hkv = a.num_kv_heads;
-  int n_waves = 0;
-  int rc = dec_grid_waves<T, D, DEC_MODE_COMPRESSED>(&n_waves);
+  int n_waves = 0, dev = -1;
+  int rc = dec_grid_waves<T, D, DEC_MODE_COMPRESSED>(&n_waves, &dev);
   if (rc) return rc;
   const int max_groups = std::max(1, n_waves / hkv), wg_waves = std::min(hkv, DecOcc<D>::WG_WAVES);
   DecParams p = {};

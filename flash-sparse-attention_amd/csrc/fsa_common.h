@@ -237,11 +237,11 @@ void set_error(const char* fmt, ...);
 
 // Dynamic LDS beyond 48 KB has to be allowed for every kernel, on every device that runs it: the attribute belongs to the
 // pair.  `done` is a static beside the launch of one kernel with one size and remembers the devices by bits; a failure is
-// reported every time it happens.
+// reported every time it happens.  `dev`: the current device where the caller has asked for it already, -1 otherwise.
 struct LdsAllowed {
   std::atomic<uint64_t> devices{0};
 };
-int allow_lds(LdsAllowed& done, const void* kernel, int bytes);
+int allow_lds(LdsAllowed& done, const void* kernel, int bytes, int dev = -1);
 int set_lds_limit(const void* kernel, int bytes);   // for sizes that change from call to call
 
 // Optional per-kernel timing: while fsa_profile_enable(1) is in effect every
