@@ -178,8 +178,6 @@ __device__ __forceinline__ void dec_emit(const DecParams& p, int b, int h, int c
   if (lr == 0) p.lse[(int64_t)hq_i * p.batch + b] = lse;
 }
 
-// Wave = (group of tiles, kv head): the waves of a group read the same cache rows, one kv head each, at about the same
-// time, so that a row (all kv heads, contiguous in memory) is fetched whole instead of in hkv visits of 2 D bytes.
 // cos / sin of x radians, |x| < 2^18: the turns are formed with the rounding error of the product and the low part of
 // 1 / (2 pi), so that the hardware instructions (which take turns) see an argument good to 2^-24.  No contraction: with
 // t - rint(t) fused to x * HI - rint(t) the rounding error of t would be added twice, 6e-3 radians at x = 1e5.
@@ -193,6 +191,8 @@ __device__ __forceinline__ void sincos_turns(float x, float& sn, float& cs) {
   cs = __builtin_amdgcn_cosf(f);
 }
 
+// Wave = (group of tiles, kv head): the waves of a group read the same cache rows, one kv head each, at about the same
+// time, so that a row (all kv heads, contiguous in memory) is fetched whole instead of in hkv visits of 2 D bytes.
 // ONE > 0: a work-group of ONE waves serves one (request, kv head), its waves sharing the tiles and merging their partials
 // in LDS; no partial goes through memory and no merge kernel follows.
 template <typename T, int D, int MODE, bool LAYER = false, int ONE = 0>
