@@ -26,9 +26,8 @@ HBM_PEAK_GBS = 8000.0       # MI355X HBM3E
 
 # Kernels whose least work is a dense 16-bit contraction are priced against the MFMA peak (with the HBM view
 # beside it), the streaming / gathering / integer kernels against the HBM peak.
-MFMA_KERNELS = {"selattn_fwd_main", "selattn_bwd_dqdkdv", "cmpattn_fwd", "cmpattn_bwd_dq", "cmpattn_bwd_dkdv",
-                "winattn_fwd", "winattn_bwd_dq", "winattn_bwd_dkdv", "cmp_score", "linear_compress_fwd",
-                "linear_compress_dx", "linear_compress_dw"}
+MFMA_KERNELS = {"selattn_fwd_main", "selattn_bwd_dqdkdv", "attn_fwd_pair", "attn_bwd_dq_pair", "attn_bwd_dkdv_pair",
+                "cmp_score", "linear_compress_fwd", "linear_compress_dx", "linear_compress_dw"}
 
 # Measured HBM traffic per launch comes from the committed counter summary of this same script (two rocprofv3
 # --pmc passes, FETCH_SIZE and WRITE_SIZE, scaled by what the counters read for a 1 GiB device copy); the file
@@ -265,25 +264,24 @@ def side_workload(args):
         qbytes = n * hq * d * e
         kvbytes = 2 * n * hkv * d * e
         ckv = 2 * nseq * nc * hkv * d * e
+        vis = vis_c + vis_w      # compressed and window attention share their launches
         algo.update({
             "selattn_fwd_main": (4.0 * d * p_key * g, rows * (2 * d * e + 4) + kvbytes),
-            "selattn_fwd_reduce": (0.0, rows * (d * e + 4) + n * hq * (d * e + 4)),
+            # partial rows and the other two branches in; o, lse and the gated sum out
+            "selattn_fwd_reduce": (0.0, rows * (d * e + 4) + 4 * qbytes + 4 * n * hq),
             "selattn_bwd_dqdkdv": (10.0 * d * p_key * g, rows * (3 * d * e + 8) + 2 * kvbytes),
-            "selattn_bwd_dq_reduce": (0.0, rows * d * e + qbytes),
-            "selattn_bwd_delta": (0.0, 2 * qbytes + 12 * n * hq),   # o, dO, lse in; (lse, delta) pairs out
-            "cmpattn_bwd_delta": (0.0, 2 * qbytes + 4 * n * hq),
-            "winattn_bwd_delta": (0.0, 2 * qbytes + 4 * n * hq),
-            "cmpattn_fwd": (4.0 * d * vis_c * hq, 2 * qbytes + ckv),
-            "cmpattn_bwd_dq": (6.0 * d * vis_c * hq, 3 * qbytes + ckv),
-            "cmpattn_bwd_dkdv": (8.0 * d * vis_c * hq, 2 * qbytes + 2 * ckv),
-            "winattn_fwd": (4.0 * d * vis_w * hq, 2 * qbytes + kvbytes),
-            "winattn_bwd_dq": (6.0 * d * vis_w * hq, 3 * qbytes + kvbytes),
-            "winattn_bwd_dkdv": (8.0 * d * vis_w * hq, 2 * qbytes + 2 * kvbytes),
+            "selattn_bwd_dq_reduce": (0.0, rows * d * e + 3 * qbytes),   # ... and dQ of the other branches in
+            "attn_fwd_pair": (4.0 * d * vis * hq, 4 * qbytes + ckv + kvbytes),
+            "attn_bwd_dq_pair": (6.0 * d * vis * hq, 6 * qbytes + ckv + kvbytes),
+            "attn_bwd_dkdv_pair": (8.0 * d * vis * hq, 4 * qbytes + 2 * ckv + 2 * kvbytes),
+            "merge_stats": (0.0, 4.0 * qbytes + 36.0 * n * hq),          # d_out, three outputs, lse in; three pairs out
             "cmp_score": (2.0 * d * vis_c * hkv, n * hkv * d * e + 4.0 * hkv * n * (nc // 4 + 1)),  # q in, fp32 block scores out
             "cmp_topk": (0.0, 4.0 * hkv * n * (nc // 4 + 1) + 4.0 * hkv * n * t),    # ... read back, ids written
-            "rope": (0.0, 2.0 * (2 * qbytes + 2 * n * hkv * d * e + 2 * nseq * nc * hkv * d * e)),  # fwd + bwd, in + out
-            "gate_merge_fwd": (0.0, 4.0 * qbytes),
-            "gate_merge_bwd": (0.0, 7.0 * qbytes),
+            # q, k and the compressed keys in and out; backward: the gradient of the compressed keys
+            "rope": (0.0, 2.0 * qbytes + kvbytes + 2.0 * ckv),
+            "layer_prep": (0.0, n * hidden * e + slen * d * e),
+            "gate_bwd": (0.0, 2.0 * n * hidden * e),
+            "kv_combine": (0.0, 4.0 * kvbytes),
             "linear_compress_fwd": (2 * 2.0 * nseq * nc * ks * d * d * hkv, kvbytes + ckv + 2 * hkv * ks * d * d * e),
             "linear_compress_dx": (2 * 2.0 * nseq * nc * ks * d * d * hkv, kvbytes + ckv + 2 * hkv * ks * d * d * e),
             "linear_compress_dw": (2 * 2.0 * nseq * nc * ks * d * d * hkv, kvbytes + ckv + 2 * hkv * ks * d * d * 4),
