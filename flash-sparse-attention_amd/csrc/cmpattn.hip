@@ -121,12 +121,13 @@ __device__ __forceinline__ void stage_kv_tile(const T* kbase, int64_t k_sn, uint
 
 // Work-group -> (query tile, sequence, kv head).  Consecutive work-groups go to the eight XCDs in turn: with the kv head
 // running fastest an XCD keeps to few heads, whose keys and values then stay in its L2.  The tiles of a sequence run from
-// its end: late queries see the most compressed keys, and the long tiles should not start last.
+// its end: late queries see the most compressed keys, and the long tiles should not start last.  Many sequences and a long
+// one among them: the sequences go into the second dimension of the grid (dense_grid).
 __device__ __forceinline__ void tile_of(const CmpParams& p, int id, int& x, int& s, int& h) {
   h = id % p.hkv;
   const int rest = id / p.hkv;
   x = p.nx - 1 - rest % p.nx;
-  s = rest / p.nx;
+  s = blockIdx.y + rest / p.nx;
 }
 
 // Per-row and per-work-group visible key range [lo, hi] (inclusive) in both modes.
@@ -408,13 +409,13 @@ __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1))
 cmpattn_bwd_dq_kernel(CmpParams p) {
   attn_bwd_dq_tile<T, D, MODE>(p, blockIdx.x);
 }
-// Compressed and window attention of one layer in one launch, the compressed tiles (`na` of them, the longest first) in
-// front.  At small sizes either alone leaves most of the chip idle.
+// Compressed (blockIdx.z == 0, in front) and window attention of one layer in one launch.  At small sizes either alone
+// leaves most of the chip idle.
 template <typename T, int D>
 __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1))
-attn_fwd_pair_kernel(CmpParams a, CmpParams b, int na) {
-  if ((int)blockIdx.x < na) attn_fwd_tile<T, D, CMP_MODE_COMPRESSED>(a, blockIdx.x);
-  else attn_fwd_tile<T, D, CMP_MODE_WINDOW>(b, blockIdx.x - na);
+attn_fwd_pair_kernel(CmpParams a, CmpParams b) {
+  if (blockIdx.z == 0) attn_fwd_tile<T, D, CMP_MODE_COMPRESSED>(a, blockIdx.x);
+  else attn_fwd_tile<T, D, CMP_MODE_WINDOW>(b, blockIdx.x);
 }
 template <typename T, int D>
 __global__ void __launch_bounds__(256)
@@ -511,15 +512,21 @@ kv_tiles_kernel(KvTiles p, int batch, int g) {
   kv_tiles<MODE>(p, batch, g, blockIdx.x);
 }
 
-// dQ of a pair; the first work-groups write the two work lists that the dK/dV launch behind it needs.
+// dQ of a pair; the first 2 hkv work-groups write the two work lists that the dK/dV launch behind it needs (their places in
+// the other rows of the grid stay empty).
 template <typename T, int D>
 __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1))
-attn_bwd_dq_pair_kernel(CmpParams a, CmpParams b, int na, KvTiles ta, KvTiles tb, int batch) {
+attn_bwd_dq_pair_kernel(CmpParams a, CmpParams b, KvTiles ta, KvTiles tb, int batch) {
   const int hkv = a.hkv, id = (int)blockIdx.x - 2 * hkv;
-  if (id < -hkv) kv_tiles<CMP_MODE_COMPRESSED>(ta, batch, a.g, id + 2 * hkv);
-  else if (id < 0) kv_tiles<CMP_MODE_WINDOW>(tb, batch, a.g, id + hkv);
-  else if (id < na) attn_bwd_dq_tile<T, D, CMP_MODE_COMPRESSED>(a, id);
-  else attn_bwd_dq_tile<T, D, CMP_MODE_WINDOW>(b, id - na);
+  if (id < 0) {
+    if (blockIdx.y != 0 || blockIdx.z != 0) return;
+    if (id < -hkv) kv_tiles<CMP_MODE_COMPRESSED>(ta, batch, a.g, id + 2 * hkv);
+    else kv_tiles<CMP_MODE_WINDOW>(tb, batch, a.g, id + hkv);
+  } else if (blockIdx.z == 0) {
+    attn_bwd_dq_tile<T, D, CMP_MODE_COMPRESSED>(a, id);
+  } else {
+    attn_bwd_dq_tile<T, D, CMP_MODE_WINDOW>(b, id);
+  }
 }
 
 // ------------------------------------------------------------------ score ----
@@ -814,6 +821,19 @@ cmp_topk_kernel(TopkParams p) {
 }
 
 // -------------------------------------------------------------- host side ----
+// Grid of 256 threads per tile: one dimension, but not beyond the 2^32 work-items that it may have (600 sequences x 8 kv
+// heads of which one sequence has 131072 tokens x 4 heads).  `lists`: work-groups in front of each row.
+static dim3 dense_grid(int nx, int hkv, int batch, int lists = 0) {
+  const int64_t all = (int64_t)nx * hkv * batch + lists;
+  if (all * 256 < ((int64_t)1 << 32)) return dim3((unsigned)all);
+  return dim3((unsigned)(nx * hkv + lists), (unsigned)batch);
+}
+static dim3 dense_pair_grid(int nx, int hkv, int batch, int lists = 0) {   // both branches of a layer: blockIdx.z
+  dim3 g = dense_grid(nx, hkv, batch, lists);
+  g.z = 2;
+  return g;
+}
+
 // rows of all (key tile, query head) pairs: a key tile of a sequence is seen by about half of its queries
 static int cmp_tile_rows(int64_t max_blocks, int64_t max_q, int hq, int g, int d) {
   return kv_tile_rows(max_blocks * max_q * hq / 2, g, d, CMP_BK);
@@ -850,7 +870,7 @@ static int attn_fwd_launch(CmpParams p, int batch, int hkv, int64_t max_rows, hi
   if (int rc_ = allow_lds(lds, (const void*)cmpattn_fwd_kernel<T, D, MODE>, CmpLds<D>::BYTES)) return rc_;
   p.hkv = hkv;
   p.nx = (int)((max_rows + CMP_ROWS - 1) / CMP_ROWS);
-  const unsigned grid = p.nx * batch * hkv;
+  const dim3 grid = dense_grid(p.nx, hkv, batch);
   ProfScope ps_(MODE == CMP_MODE_WINDOW ? "winattn_fwd" : "cmpattn_fwd", stream);
   cmpattn_fwd_kernel<T, D, MODE><<<grid, 256, CmpLds<D>::BYTES, stream>>>(p);
   return 0;
@@ -882,7 +902,7 @@ static int attn_bwd_launch(CmpParams p, const SelBwdParams& kv, int batch, int h
   }
   {
     ProfScope ps_(MODE == CMP_MODE_WINDOW ? "winattn_bwd_dq" : "cmpattn_bwd_dq", stream);
-    const unsigned grid = p.nx * batch * hkv;
+    const dim3 grid = dense_grid(p.nx, hkv, batch);
     cmpattn_bwd_dq_kernel<T, D, MODE><<<grid, 256, CmpLds<D>::BYTES, stream>>>(p);
   }
   {
@@ -906,9 +926,8 @@ static int pair_fwd_launch(CmpParams a, CmpParams b, int batch, int hkv, int64_t
   if (int rc_ = allow_lds(lds, (const void*)attn_fwd_pair_kernel<T, D>, CmpLds<D>::BYTES)) return rc_;
   a.hkv = b.hkv = hkv;
   a.nx = b.nx = (int)((max_rows + CMP_ROWS - 1) / CMP_ROWS);
-  const int tiles = a.nx * batch * hkv;
   ProfScope ps_("attn_fwd_pair", stream);
-  attn_fwd_pair_kernel<T, D><<<2 * tiles, 256, CmpLds<D>::BYTES, stream>>>(a, b, tiles);
+  attn_fwd_pair_kernel<T, D><<<dense_pair_grid(a.nx, hkv, batch), 256, CmpLds<D>::BYTES, stream>>>(a, b);
   return 0;
 }
 template <typename T, int D>
@@ -921,10 +940,9 @@ static int pair_bwd_launch(CmpParams a, CmpParams b, const SelBwdParams& ka, con
   if (int rc_ = allow_lds(lds2, (const void*)attn_bwd_dkdv_pair_kernel<T, D, CMP_BK>, C::BYTES)) return rc_;
   a.hkv = b.hkv = hkv;
   a.nx = b.nx = (int)((max_rows + CMP_ROWS - 1) / CMP_ROWS);
-  const int tiles = a.nx * batch * hkv;
   {
     ProfScope ps_("attn_bwd_dq_pair", stream);
-    attn_bwd_dq_pair_kernel<T, D><<<2 * (hkv + tiles), 256, CmpLds<D>::BYTES, stream>>>(a, b, tiles, ta, tb, batch);
+    attn_bwd_dq_pair_kernel<T, D><<<dense_pair_grid(a.nx, hkv, batch, 2 * hkv), 256, CmpLds<D>::BYTES, stream>>>(a, b, ta, tb, batch);
   }
   {
     const HeadOrder order = head_order(hkv, ka.n_tokens * ka.g * D * 2);
@@ -957,7 +975,7 @@ static int cmp_score_launch(CmpParams p, int batch, int hkv, int64_t max_q, hipS
   ProfScope ps_("cmp_score", stream);
   p.hkv = hkv;
   p.nx = (int)((max_q + CMP_ROWS - 1) / CMP_ROWS);
-  const unsigned grid = p.nx * batch * hkv;
+  const dim3 grid = dense_grid(p.nx, hkv, batch);
   if (p.rebin) cmp_score_kernel<T, D, true><<<grid, 256, CMP_BK * CmpLds<D>::KS * 2, stream>>>(p);
   else cmp_score_kernel<T, D, false><<<grid, 256, CMP_BK * CmpLds<D>::KS * 2, stream>>>(p);
   return 0;

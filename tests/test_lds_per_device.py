@@ -16,19 +16,24 @@ STUB = r"""
 #include <map>
 #include <utility>
 struct dim3 { uint32_t x, y, z; };
-static int device = 0, failing = 0, large = 0, refused = 0;
+static int device = 0, failing = 0, large = 0, refused = 0, launches = 0, oversized = 0;
 static std::map<std::pair<const void*, int>, int> limit;
 extern "C" {
 void stub_set(int d, int f) { device = d; failing = f; }
 int stub_large() { return large; }       // launches beyond 64 KB
 int stub_refused() { return refused; }   // of those, without an attribute that allows them
+int stub_launches() { return launches; }
+int stub_oversized() { return oversized; }   // launches with 2^32 or more work-items, or no work-group, in a dimension
 int hipGetDevice(int* d) { *d = device; return 0; }
 int hipFuncSetAttribute(const void* f, int, int v) {
   if (failing) return 2;
   limit[{f, device}] = v;
   return 0;
 }
-int hipLaunchKernel(const void* f, dim3, dim3, void**, size_t lds, void*) {
+int hipLaunchKernel(const void* f, dim3 g, dim3 b, void**, size_t lds, void*) {
+  ++launches;
+  auto bad = [](uint32_t n, uint32_t t) { return n == 0 || (uint64_t)n * t >= (1ull << 32); };
+  if (bad(g.x, b.x) || bad(g.y, b.y) || bad(g.z, b.z)) ++oversized;
   if (lds > 65536) {
     ++large;
     auto it = limit.find({f, device});
@@ -39,9 +44,10 @@ int hipLaunchKernel(const void* f, dim3, dim3, void**, size_t lds, void*) {
 int hipGetLastError() { return 0; }
 const char* hipGetErrorString(int) { return "stub error"; }
 static size_t cfg_lds;
-int __hipPushCallConfiguration(dim3, dim3, size_t lds, void*) { cfg_lds = lds; return 0; }
+static dim3 cfg_grid, cfg_block;
+int __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, void*) { cfg_grid = g; cfg_block = b; cfg_lds = lds; return 0; }
 int __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, void** s) {
-  *g = *b = {1, 1, 1}; *lds = cfg_lds; *s = nullptr; return 0;
+  *g = cfg_grid; *b = cfg_block; *lds = cfg_lds; *s = nullptr; return 0;
 }
 int hipDeviceGetAttribute(int* v, int, int) { *v = 256; return 0; }
 int hipOccupancyMaxActiveBlocksPerMultiprocessor(int* v, const void*, int, size_t) { *v = 8; return 0; }
