@@ -403,9 +403,9 @@ static LayerBwdWs layer_bwd_ws(const fsa_layer_args& a, const LayerSaved& s) {
   const size_t kv = n * hkv * d * e, ck = (size_t)a.total_ck * hkv * d * e;
   for (int i = 0; i < 3; ++i) w.stat[i] = b.take(n * hq * 8);
   w.dl = b.take(n * 3 * e);
-  // two work-groups per CU for the pass over x, at least 8 tokens each
+  // two work-groups per CU for the pass over x, at least 8 tokens each and no more than LDS holds without asking (48 KB)
   const int64_t col_groups = (a.hidden + GATE_COLS - 1) / GATE_COLS;
-  w.chunk = (int)std::max<int64_t>(8, (a.total_tokens * col_groups + 511) / 512);
+  w.chunk = (int)std::min<int64_t>(4096, std::max<int64_t>(8, (a.total_tokens * col_groups + 511) / 512));
   w.chunks = (int)((a.total_tokens + w.chunk - 1) / w.chunk);
   w.gate_part = b.take((size_t)w.chunks * 3 * a.hidden * 4);
   w.dq_cmp = b.take(n * hq * d * e);

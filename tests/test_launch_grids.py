@@ -52,6 +52,7 @@ cases = {
   "dense_one": lambda: dense(1, 1 << 20),
   "layer_one_long_of_600": lambda: layer(600, 131072, 131072 + 600 * 200),
   "layer_one": lambda: layer(1, 1 << 19, 1 << 19),
+  "layer_wide": lambda: layer(1, 800000, 800000, hq=8, hkv=2, hidden=8192),   # chunks of the gate's pass over x
   "layer_d256": lambda: layer(3, 4000, 5000, hq=4, hkv=2, d=256),
 }
 stub.stub_set(0, 0)
@@ -64,7 +65,7 @@ os._exit(0)
 
 
 @pytest.mark.parametrize("name", ["dense_one_long_of_600", "dense_100000_short", "dense_one", "layer_one_long_of_600",
-                                  "layer_one", "layer_d256"])
+                                  "layer_one", "layer_wide", "layer_d256"])
 def test_grids_of_large_problems(stub, name):  # noqa: F811
     r = subprocess.run([sys.executable, "-c", CHILD, stub, ROOT, name], capture_output=True, text=True, timeout=120,
                        env={**os.environ, "HIP_VISIBLE_DEVICES": ""})
