@@ -327,6 +327,14 @@ int selattn_fwd(const void* q, const void* k, const void* v, int32_t dtype, int6
                 int64_t o_stride_n, int64_t o_stride_h, float* lse, void* workspace, size_t workspace_bytes,
                 const MergeEpilogue& merge, hipStream_t stream);
 
+bool selattn_direct_preferred(int64_t n, int64_t max_len, int hq, int d, int topk, int bk);
+int selattn_direct_fwd(const void* q, const void* k, const void* v, int32_t dtype, int64_t q_stride_n, int64_t q_stride_h,
+                       int64_t k_stride_n, int64_t k_stride_h, int64_t v_stride_n, int64_t v_stride_h, const int32_t* topk_idx,
+                       int64_t idx_stride_h, int64_t idx_stride_n, const int32_t* cu_seqlens, int32_t batch,
+                       int64_t total_tokens, int64_t max_len, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                       int32_t topk, int32_t block_size, float softmax_scale, void* o, int64_t o_stride_n, int64_t o_stride_h,
+                       float* lse, const MergeEpilogue& merge, hipStream_t stream);
+
 // What the end of the selected backward adds to dQ before it is stored: gradients of the same queries from other branches,
 // and the inverse rotation of the sum (cos / sin pairs [position][D/2] in the tensor's type).  All null: nothing.
 struct DqEpilogue {

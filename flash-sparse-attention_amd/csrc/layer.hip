@@ -346,6 +346,7 @@ struct LayerSaved {
   size_t cu_ck, table, gates, q, k, ck, cv, o[3], lse[3], cu_blocks, counts, starts, sel, slot, tiles_fwd, tiles_bwd, total;
   int64_t max_blocks;
   int t_out;
+  bool direct, index;   // selected forward from the block lists; whether the inverted index is built
 };
 static LayerSaved layer_saved(const fsa_layer_args& a) {
   LayerSaved s;
@@ -353,6 +354,9 @@ static LayerSaved layer_saved(const fsa_layer_args& a) {
   const size_t e = 2, n = a.total_tokens, d = a.head_dim, hq = a.num_q_heads, hkv = a.num_kv_heads;
   s.t_out = (int)std::min<int64_t>(a.topk, (a.max_len + a.block_size - 1) / a.block_size);
   s.max_blocks = (a.total_tokens + a.block_size - 1) / a.block_size + a.batch;
+  s.direct = a.total_tokens * a.num_kv_heads * a.head_dim < (int64_t)1 << 30 &&
+             selattn_direct_preferred(a.total_tokens, a.max_len, a.num_q_heads, a.head_dim, s.t_out, a.block_size);
+  s.index = !s.direct || !a.inference;
   s.cu_ck = b.take((a.batch + 1) * 4);
   s.table = b.take((size_t)a.max_len * d * e);
   s.gates = b.take(n * 3 * e);
@@ -364,11 +368,11 @@ static LayerSaved layer_saved(const fsa_layer_args& a) {
   for (int i = 0; i < 3; ++i) s.o[i] = b.take(a.inference && i == 1 ? 0 : n * hq * d * e);
   for (int i = 0; i < 3; ++i) s.lse[i] = b.take(a.inference && i == 1 ? 0 : n * hq * 4);
   s.cu_blocks = b.take((a.batch + 1) * 4);
-  s.counts = b.take(hkv * s.max_blocks * 4);
-  s.starts = b.take(hkv * (s.max_blocks + 1) * 4);
-  s.sel = b.take(hkv * n * s.t_out * 4);
-  s.slot = b.take(hkv * n * s.t_out * 4);
-  s.tiles_fwd = b.take(fsa_selattn_tiles_bytes(0, n, hq, hkv, d, s.t_out, a.block_size, s.max_blocks));
+  s.counts = b.take(!s.index ? 0 : hkv * s.max_blocks * 4);
+  s.starts = b.take(!s.index ? 0 : hkv * (s.max_blocks + 1) * 4);
+  s.sel = b.take(!s.index ? 0 : hkv * n * s.t_out * 4);
+  s.slot = b.take(!s.index ? 0 : hkv * n * s.t_out * 4);
+  s.tiles_fwd = b.take(!s.index ? 0 : fsa_selattn_tiles_bytes(0, n, hq, hkv, d, s.t_out, a.block_size, s.max_blocks));
   s.tiles_bwd = b.take(a.inference ? 0 : fsa_selattn_tiles_bytes(1, n, hq, hkv, d, s.t_out, a.block_size, s.max_blocks));
   s.total = b.at;
   return s;
@@ -385,8 +389,8 @@ static LayerFwdWs layer_fwd_ws(const fsa_layer_args& a, const LayerSaved& s) {
   w.stage = b.at;
   const bool rebin = a.kernel_size == 2 * a.kernel_stride && a.block_size == 4 * a.kernel_stride;
   w.topk_bytes = fsa_cmp_topk_workspace_bytes(a.total_tokens, a.num_kv_heads, rebin ? a.max_ck / 4 + 1 : a.max_ck);
-  w.index_bytes = fsa_index_workspace_bytes(a.total_tokens, s.t_out, a.num_kv_heads, s.max_blocks);
-  w.sel_bytes = fsa_selattn_fwd_workspace_bytes(a.total_tokens, a.num_q_heads, a.num_kv_heads, a.head_dim, s.t_out, s.max_blocks);
+  w.index_bytes = !s.index ? 0 : fsa_index_workspace_bytes(a.total_tokens, s.t_out, a.num_kv_heads, s.max_blocks);
+  w.sel_bytes = s.direct ? 0 : fsa_selattn_fwd_workspace_bytes(a.total_tokens, a.num_q_heads, a.num_kv_heads, a.head_dim, s.t_out, s.max_blocks);
   w.total = w.stage + align_up(std::max({w.topk_bytes, w.index_bytes, w.sel_bytes}), 256);
   return w;
 }
@@ -507,7 +511,8 @@ static int layer_forward(const fsa_layer_args& a, void* out, int32_t* topk_idx, 
                        a.local_blocks, 1, 0, a.softmax_scale, topk_idx, nullptr, ws + w.stage, w.topk_bytes, stream));
   int32_t *cu_blocks = (int32_t*)(sv + s.cu_blocks), *counts = (int32_t*)(sv + s.counts), *starts = (int32_t*)(sv + s.starts),
           *sel = (int32_t*)(sv + s.sel), *slot = (int32_t*)(sv + s.slot), *tf = (int32_t*)(sv + s.tiles_fwd), *tb = a.inference ? nullptr : (int32_t*)(sv + s.tiles_bwd);
-  FSA_RUN(fsa_build_index_tiles(topk_idx, n * s.t_out, s.t_out, a.cu_seqlens, a.batch, n, a.num_kv_heads, s.t_out, a.block_size,
+  if (s.index)
+    FSA_RUN(fsa_build_index_tiles(topk_idx, n * s.t_out, s.t_out, a.cu_seqlens, a.batch, n, a.num_kv_heads, s.t_out, a.block_size,
                                 s.max_blocks, cu_blocks, counts, starts, sel, slot, a.num_q_heads, a.head_dim, tf, tb,
                                 ws + w.stage, w.index_bytes, stream));
   MergeEpilogue merge;
@@ -515,6 +520,13 @@ static int layer_forward(const fsa_layer_args& a, void* out, int32_t* topk_idx, 
   merge.c = sv + s.o[2];
   merge.gate = sv + s.gates;
   merge.out = out;
+  if (s.direct) {
+    FSA_RUN(selattn_direct_fwd(q, k, a.v, a.dtype, qs, d, ks_, d, ks_, d, topk_idx, n * s.t_out, s.t_out, a.cu_seqlens, a.batch, n,
+                               a.max_len, a.num_q_heads, a.num_kv_heads, a.head_dim, s.t_out, a.block_size, a.softmax_scale,
+                               a.inference ? nullptr : sv + s.o[1], qs, d, a.inference ? nullptr : (float*)(sv + s.lse[1]), merge,
+                               stream));
+    return 0;
+  }
   FSA_RUN(selattn_fwd(q, k, a.v, a.dtype, qs, d, ks_, d, ks_, d, a.cu_seqlens, a.batch, n, a.num_q_heads, a.num_kv_heads, a.head_dim,
                       s.t_out, a.block_size, s.max_blocks, a.softmax_scale, cu_blocks, counts, starts, sel, slot, tf,
                       a.inference ? nullptr : sv + s.o[1], qs, d, a.inference ? nullptr : (float*)(sv + s.lse[1]), ws + w.stage, w.sel_bytes, merge, stream));

@@ -36,7 +36,7 @@ namespace {
   X(fsa_decode_cmpattn) X(fsa_decode_topk) X(fsa_decode_selattn) X(fsa_decode_layer_workspace_bytes)                   \
   X(fsa_decode_layer_project) X(fsa_decode_layer_attend) X(fsa_linear_compress_fwd)                                    \
   X(fsa_layer_saved_bytes) X(fsa_layer_workspace_bytes) X(fsa_layer_forward) X(fsa_layer_backward) \
-  X(fsa_matmul)
+  X(fsa_matmul) X(fsa_selattn_direct_preferred) X(fsa_selattn_direct_fwd)
 struct Api {
 #define FSA_FIELD(f) decltype(&::f) f = nullptr;
   FSA_API(FSA_FIELD)
@@ -217,10 +217,13 @@ struct Index {
 };
 
 // Blocks of 256 keys run as pairs of 128-key blocks (the same key set for every query).
-Index kernel_index(const Tensor& topk_in, const Tensor& cu, int64_t block, int64_t hq, int64_t d, bool backward) {
-  check_topk(topk_in, cu);
-  const Tensor topk_idx = block == 256 ? split_topk_blocks(topk_in, cu, 256, 2) : topk_in;
-  if (block == 256) block = 128;
+Tensor kernel_blocks(const Tensor& topk_idx, const Tensor& cu, int64_t& block) {
+  check_topk(topk_idx, cu);
+  if (block != 256) return topk_idx;
+  block = 128;
+  return split_topk_blocks(topk_idx, cu, 256, 2);
+}
+Index kernel_index(const Tensor& topk_idx, const Tensor& cu, int64_t block, int64_t hq, int64_t d, bool backward) {
   Index x;
   x.cu = cu;
   x.hkv = topk_idx.size(0);
@@ -270,6 +273,29 @@ std::pair<Tensor, Tensor> selattn_fwd_native(const Tensor& q, const Tensor& k, c
                             (int32_t)hkv, (int32_t)d, (int32_t)x.topk, (int32_t)x.block, x.max_blocks, (float)scale,
                             x.cu_blocks, x.counts, x.starts, x.sel, x.slot, x.tiles_fwd, o.data_ptr(), hq * d, d, f32(lse),
                             ws.data_ptr(), bytes, stream_of(q)),
+        "fsa_selattn_fwd");
+  return {o, lse};
+}
+
+// Short sequences: from the block lists (kernel_blocks), without an index
+bool direct(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& topk_idx, int64_t block) {
+  const int64_t n = q.size(0), d = q.size(2);
+  auto rows_ok = [&](const Tensor& t) {   // they go to LDS by 16-byte buffer loads
+    return t.stride(0) >= d && t.stride(0) * n < (int64_t)1 << 30 && (uintptr_t)t.data_ptr() % 16 == 0;
+  };
+  return n >= 1 && topk_idx.size(0) == k.size(1) && topk_idx.size(1) == n && rows_ok(k) && rows_ok(v) &&
+         api.fsa_selattn_direct_preferred(n, n, (int32_t)q.size(1), (int32_t)d, (int32_t)topk_idx.size(2), (int32_t)block);
+}
+std::pair<Tensor, Tensor> selattn_direct(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& topk_idx, const Tensor& cu,
+                                         int64_t block, double scale) {
+  const int64_t n = q.size(0), hq = q.size(1), d = q.size(2), hkv = k.size(1);
+  const c10::OptionalDeviceGuard guard(q.device());
+  Tensor o = at::empty({n, hq, d}, q.options()), lse = empty_f32({hq, n}, q);
+  check(api.fsa_selattn_direct_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), dtype_code(q), q.stride(0), q.stride(1), k.stride(0),
+                                   k.stride(1), v.stride(0), v.stride(1), i32(topk_idx), topk_idx.stride(0), topk_idx.stride(1),
+                                   i32(cu), (int32_t)cu.numel() - 1, n, n, (int32_t)hq, (int32_t)hkv, (int32_t)d,
+                                   (int32_t)topk_idx.size(2), (int32_t)block, (float)scale, o.data_ptr(), hq * d, d, f32(lse),
+                                   stream_of(q)),
         "fsa_selattn_fwd");
   return {o, lse};
 }
@@ -335,9 +361,11 @@ struct SelectedAttention : torch::autograd::Function<SelectedAttention> {
   static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v,
                         const Tensor& topk_idx, int64_t block, const Tensor& cu, double scale) {
     const int64_t d = q.size(2), dn = native_dim(d);
-    const Index x = kernel_index(topk_idx, cu, block, q.size(1), dn, true);
+    const Tensor ids = kernel_blocks(topk_idx, cu, block);
+    const Index x = kernel_index(ids, cu, block, q.size(1), dn, true);
     const Tensor qn = resize_d(q, dn), kn = resize_d(k, dn), vn = resize_d(v, dn);
-    auto [on, lse] = selattn_fwd_native(qn, kn, vn, x.view(), scale);
+    auto [on, lse] = direct(qn, kn, vn, ids, block) ? selattn_direct(qn, kn, vn, ids, cu, block, scale)
+                                                    : selattn_fwd_native(qn, kn, vn, x.view(), scale);
     ctx->save_for_backward({qn, kn, vn, on, lse, x.cu, x.mem});
     ctx->saved_data["ints"] = std::vector<int64_t>{d, x.n, x.hkv, x.topk, x.block, x.max_blocks, x.hq, x.d};
     ctx->saved_data["scale"] = scale;
@@ -365,8 +393,10 @@ Tensor selected_attention(const Tensor& q, const Tensor& k, const Tensor& v, con
   if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()))
     return SelectedAttention::apply(q, k, v, topk_idx, block, cu, scale);
   const int64_t d = q.size(2), dn = native_dim(d);
-  const Index x = kernel_index(topk_idx, cu, block, q.size(1), dn, false);
-  return resize_d(selattn_fwd_native(resize_d(q, dn), resize_d(k, dn), resize_d(v, dn), x.view(), scale).first, d);
+  const Tensor ids = kernel_blocks(topk_idx, cu, block), qn = resize_d(q, dn), kn = resize_d(k, dn), vn = resize_d(v, dn);
+  if (direct(qn, kn, vn, ids, block)) return resize_d(selattn_direct(qn, kn, vn, ids, cu, block, scale).first, d);
+  const Index x = kernel_index(ids, cu, block, q.size(1), dn, false);
+  return resize_d(selattn_fwd_native(qn, kn, vn, x.view(), scale).first, d);
 }
 
 // ---- one-step decode ----

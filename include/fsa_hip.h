@@ -186,6 +186,21 @@ int fsa_selattn_fwd_tiles(const void* q, const void* k, const void* v, int32_t d
                           void* o, int64_t o_stride_n, int64_t o_stride_h, float* lse,
                           void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same result from the block lists alone, without index and workspace: one query-major launch that visits, for every 32
+ * rows, the union of the blocks they selected.  For short sequences: max_len (any upper bound of the longest sequence) is at
+ * most 1024 blocks, rows of k and v do not overlap.  A block that a list names several times counts as often, as above.
+ * fsa_selattn_direct_preferred: 1 where this is the faster one of the two. */
+int fsa_selattn_direct_preferred(int64_t total_tokens, int64_t max_len, int32_t num_q_heads, int32_t head_dim,
+                                 int32_t topk, int32_t block_size);
+int fsa_selattn_direct_fwd(const void* q, const void* k, const void* v, int32_t dtype,
+                           int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h,
+                           int64_t v_stride_n, int64_t v_stride_h,
+                           const int32_t* topk_idx, int64_t idx_stride_h, int64_t idx_stride_n,
+                           const int32_t* cu_seqlens, int32_t batch, int64_t total_tokens, int64_t max_len,
+                           int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32_t topk,
+                           int32_t block_size, float softmax_scale,
+                           void* o, int64_t o_stride_n, int64_t o_stride_h, float* lse, void* stream);
+
 /* ------------------------------------------------------------------------
  * Selected attention backward.
  * Replaces _topk_sparse_attention_bwd_opt (backward_sum_o_do, backward_dkdv,
