@@ -10,6 +10,7 @@
 #pragma once
 #include "fsa_common.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace fsa {
@@ -115,7 +116,15 @@ static inline int kv_tile_rows(int64_t rows_total, int g, int d, int bk) {
   const int r = 1024 + 2048 * g;
   // head_dim 256 with 128-key blocks: 32-row passes of eight waves, fewer, longer tiles
   const int cap = (d >= 256 && bk >= 128) || r > KV_TILE_ROWS_MAX ? KV_TILE_ROWS_MAX : r;
-  return balanced_tile_rows(rows_total, d <= 128 && bk <= 64 ? 2 : 1, cap);
+  const int per_cu = d <= 128 && bk <= 64 ? 2 : 1;
+  const int two = balanced_tile_rows(rows_total, per_cu, cap);   // work-groups for each of the chip's slots
+  if (d < 128) return two;
+  // Every work-group of a shared block leaves 2 * bk * d fp32 partial sums to be added: as long as the tiles are short, one
+  // work-group per slot.  Backward (us, two per slot -> one): 2000 tokens x 8 heads, 8 blocks of 64, 69 -> 51, 8 blocks of
+  // 128, 82 -> 63; 4096 x 4, 16 blocks of 64, 94 -> 88; 4000 x 8 of 256, 8 blocks of 128, 240 -> 209.  (2000 x 32, 16 blocks
+  // of 64, tiles of 2000 rows, 205 -> 215: too few for an even end.  head_dim 64, where more than two fit on a CU: 3001 x 8,
+  // 8 blocks of 32, 36 -> 42.)
+  return std::max(two, balanced_tile_rows(2 * rows_total, per_cu, per_cu == 2 ? 512 : 1024));
 }
 
 // Element offset of element `col` (a multiple of 4) of row `row` in an unpadded LDS tile with rows of W 16-bit
