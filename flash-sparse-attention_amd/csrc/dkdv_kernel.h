@@ -137,11 +137,15 @@ static inline int kv_tile_rows(int64_t rows_total, int g, int d, int bk) {
 // 16 different slots).  Measured on gfx950 (ds_read_b64 / ds_read_b64_tr_b16, 8 waves per CU): both patterns at
 // the full rate of 1.04 ns per wave instruction, where rows padded to 272 bytes give 1.04 / 1.86 (the
 // transposing reads two-way conflicted) and rows of 288 bytes 1.86 / 1.04.
-template <int W> __device__ __forceinline__ int swz(int row, int col) {
+// HALVES false: the natural fragments are read 16 bytes at a time.  Such a read is served in groups of 16 lanes (0-3, 12-15,
+// 20-23 and 24-27 make the first): rows 0-3 and 12-15 of one 16-byte column with rows 4-11 of its neighbour.  The swapped
+// halves would put these on the same slots (8.0 instead of 4.0 clocks per wave instruction); the groups alone keep them
+// apart.  (head_dim 256, blocks of 128, 131072 tokens: fused backward 2150 -> 2055 us.)
+template <int W, bool HALVES = true> __device__ __forceinline__ int swz(int row, int col) {
   static_assert(W >= 32 && (W & (W - 1)) == 0, "row length");
   constexpr int L = W >= 128 ? 1 : 128 / W;          // rows per 256-byte bank line
   constexpr int XM = W / 16 - 1 < 7 ? W / 16 - 1 : 7;  // 32-byte groups per row - 1, at most 8 take part
-  const int x = (row / L) & XM, hb = (row >> 3) & 1;
+  const int x = (row / L) & XM, hb = HALVES ? (row >> 3) & 1 : 0;
   return row * W + ((((col >> 4) ^ x) << 4) | ((((col >> 3) & 1) ^ hb) << 3) | (col & 7));
 }
 
@@ -257,7 +261,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const SelBwdParams& p, const 
       const int row = c / (D / 8), cc = c % (D / 8);
       vec8 x = zero8<T>();
       if (row < blk.n_keys_valid) x = load16<vec8>(kb + (int64_t)(blk.key_row0 + row) * p.k_sn + cc * 8);
-      store16(&Kl[swz<D>(row, cc * 8)], x);
+      store16(&Kl[swz<D, SPLIT>(row, cc * 8)], x);
     }
   }
   const int32_t* toks = MODE == KV_MODE_SELECTED ? p.sel_tokens + (int64_t)h * p.cap + start : nullptr;
@@ -322,12 +326,12 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const SelBwdParams& p, const 
       }
     }
   };
-  const int st_off = swz<D>(ld_row, ld_col * 8);
+  const int st_off = swz<D, SPLIT>(ld_row, ld_col * 8);
   auto stash = [&]() {
 #pragma unroll
     for (int j = 0; j < C::CPT; ++j) {
       // the swizzle of a row repeats every 16 rows
-      const int off = C::ROW_STEP % 16 == 0 ? st_off + C::ROW_STEP * j * QS : swz<D>(ld_row + C::ROW_STEP * j, ld_col * 8);
+      const int off = C::ROW_STEP % 16 == 0 ? st_off + C::ROW_STEP * j * QS : swz<D, SPLIT>(ld_row + C::ROW_STEP * j, ld_col * 8);
       store16(&Qs[off], qst[j]);
       store16(&Os[off], dost[j]);
     }
@@ -353,8 +357,8 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const SelBwdParams& p, const 
   // offset of group 0 XOR 16 g elements, so a lane keeps one offset per access pattern:
   // byte addresses inside the Q tile, 32-byte group 0: the row part of a swizzled offset repeats every 16 rows,
   // and group g of a row sits at the address of group 0 XOR 32 g (the tiles start on multiples of the row size)
-  const uint32_t a_addr00 = lds_addr(Qs + swz<D>(l16, (SPLIT ? 4 : 8) * kg));            // + rt*16 rows
-  const uint32_t tr_addr00 = lds_addr(Qs + swz<D>(4 * kg + (l16 >> 2), 4 * (l16 & 3)));  // + 32*u rows (+ 16 rows)
+  const uint32_t a_addr00 = lds_addr(Qs + swz<D, SPLIT>(l16, (SPLIT ? 4 : 8) * kg));            // + rt*16 rows
+  const uint32_t tr_addr00 = lds_addr(Qs + swz<D, SPLIT>(4 * kg + (l16 >> 2), 4 * (l16 & 3)));  // + 32*u rows (+ 16 rows)
   constexpr int ROW_BYTES = QS * 2, O_BYTES = C::KV_R * ROW_BYTES;                        // Os - Qs
   constexpr int K_BYTES = 2 * O_BYTES + C::KV_R * 16;                                     // Kl - Qs
 
@@ -397,7 +401,7 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const SelBwdParams& p, const 
       }
 #pragma unroll
       for (int s_ = 0; s_ < NS; ++s_) {
-        const vec8 kfrag = KLDS ? load16<vec8>(&Kl[swz<D>(key, 32 * s_ + 8 * kg)]) : kf[KLDS ? 0 : s_];
+        const vec8 kfrag = KLDS ? load16<vec8>(&Kl[swz<D, SPLIT>(key, 32 * s_ + 8 * kg)]) : kf[KLDS ? 0 : s_];
 #pragma unroll
         for (int rt = 0; rt < NRT; ++rt) {
           vec8 qa = load16<vec8>(lds_ptr<T>((a_addr0 ^ (64u * s_)) + rt * 16 * ROW_BYTES));
