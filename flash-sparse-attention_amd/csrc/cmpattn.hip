@@ -190,6 +190,7 @@ __device__ __forceinline__ void attn_fwd_tile(const CmpParams& p, int id) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
 
+  constexpr int KAHEAD = 2, VAHEAD = 3;
   constexpr bool PREFETCH = D <= 128;  // the next tile waits in registers where the budget allows
   KvTileRegs<T, D> nxt;
   if (PREFETCH && jt0 < n_keys) kv_tile_load<T, D>(nxt, kbase, p.k_sn, k_off, vbase, p.v_sn, v_off, k0 + jt0, nc - jt0, tid);
@@ -208,13 +209,27 @@ __device__ __forceinline__ void attn_fwd_tile(const CmpParams& p, int id) {
     for (int a = 0; a < NA; ++a)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[a][i] = 0.f;
+    // Fragments are requested KAHEAD k-steps before their products, and in this order: left to itself the compiler asks for
+    // them right before, and the wave waits for LDS at every pair of products (5003 tokens, 32 + 8 heads: 111 -> 107 us for
+    // both branches).
+    vec8 kf[KAHEAD + 1][NA];
+    auto k_read = [&](int ks) {
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks)
+      for (int a = 0; a < NA; ++a) kf[ks % (KAHEAD + 1)][a] = load16<vec8>(&Ks[(a * 32 + col) * KS + hh * (D / 2) + ks * 8]);
+    };
 #pragma unroll
-      for (int a = 0; a < NA; ++a) {  // consecutive products on different accumulators
-        vec8 kf = load16<vec8>(&Ks[(a * 32 + col) * KS + hh * (D / 2) + ks * 8]);
-        acc[a] = Elem<T>::mfma32(kf, qreg[ks], acc[a]);
-      }
+    for (int ks = 0; ks < KAHEAD; ++ks) k_read(ks);
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+      if (ks + KAHEAD < NKS) k_read(ks + KAHEAD);
+#pragma unroll
+      for (int a = 0; a < NA; ++a) acc[a] = Elem<T>::mfma32(kf[ks % (KAHEAD + 1)][a], qreg[ks], acc[a]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    vec8 vf[VAHEAD + 1];
+    auto v_read = [&](int i) { vf[i % (VAHEAD + 1)] = lds_read_tr8<T>(vtr + 16 * (i / NDT) * VS + i % NDT * 32, 8 * VS); };
+#pragma unroll
+    for (int i = 0; i < VAHEAD; ++i) v_read(i);   // (they arrive during the softmax)
     const int limit = jmax - jt, limit_lo = jmin - jt;
     float mx = m;
     // tiles that every row of the wave sees completely need no mask
@@ -258,12 +273,10 @@ __device__ __forceinline__ void attn_fwd_tile(const CmpParams& p, int id) {
       }
     l += lsum;   // the lane's own keys: the two lanes of a row are added behind the loop
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-#pragma unroll
-      for (int dt = 0; dt < NDT; ++dt) {
-        vec8 vf = lds_read_tr8<T>(vtr + 16 * j * VS + dt * 32, 8 * VS);
-        oacc[dt] = Elem<T>::mfma32(vf, pk[j], oacc[dt]);
-      }
+    for (int i = 0; i < NJ * NDT; ++i) {
+      if (i + VAHEAD < NJ * NDT) v_read(i + VAHEAD);
+      oacc[i % NDT] = Elem<T>::mfma32(vf[i % (VAHEAD + 1)], pk[i / NDT], oacc[i % NDT]);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
   l = sum32(l);

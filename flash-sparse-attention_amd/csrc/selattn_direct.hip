@@ -39,21 +39,6 @@ template <int D, int KG> struct DirectLds {
   static constexpr int bytes(int max_blk) { return KG * WAVE_BYTES + STATS + 16 + 6 * max_blk; }
 };
 
-// Chunk of 16 bytes that a tile keeps in the place of chunk c of row r: c ^ direct_swizzle(r).  Fragments are read by b128 (16
-// rows of one column at a time: all 16 chunks of a 256-byte bank line differ) and, transposing, four rows of 64 bytes at a time
-// (their 64-byte groups differ).  head_dim 64: two rows per bank line.
-template <int D> __device__ __forceinline__ int direct_swizzle(int r) {
-  return D >= 128 ? (r & 3) << 2 | (r >> 2 & 3) : (r >> 1 & 1) << 2 | (r >> 2 & 3);
-}
-
-// Transposed fragment: rows 16 j + (0..3, 8..11) of the lane's column.  `addr`: the lane's address in row 0; rows that are 8
-// apart differ in bit 1 of the swizzle.
-template <typename T, int D> __device__ __forceinline__ typename Elem<T>::vec8 direct_tr_frag(uint32_t addr, int j) {
-  const typename Elem<T>::vec4 lo = lds_read_tr4<T>(lds_ptr<T>(addr + 16 * j * D * 2));
-  const typename Elem<T>::vec4 hi = lds_read_tr4<T>(lds_ptr<T>((addr ^ 32u) + (16 * j + 8) * D * 2));
-  return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-}
-
 // Four KB of a tile, global memory to LDS: lane l's 16 bytes at voff[j](l) + soff + 1024 j of the buffer land at LDS byte
 // `lds` + 1024 j + 16 l (the instruction's offset moves both addresses).  The compiler does not count these loads: vm_wait
 // orders them.
@@ -178,14 +163,14 @@ selattn_direct_fwd_kernel(DirectParams p) {
   const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<T*>(reinterpret_cast<const T*>(p.v) + (int64_t)q0 * p.v_sn + (int64_t)h * p.v_sh), 0, -1, 0x00020000);
   const uint32_t k_lds = lds_addr(smem + wv * L::WAVE_BYTES), v_lds = k_lds + L::TILE;
-  // Rows are unpadded; chunk c of row r sits at chunk c ^ swizzle(r), the loading lane picks its source accordingly
+  // (the loading lane picks its source so that the chunks land where chunk_swizzle wants them)
   const int ld_row = lane / CPR, ld_chunk = lane % CPR;
   uint32_t k_voff[NLD], v_voff[NLD];
 #pragma unroll
   for (int j = 0; j < NLD; ++j) {   // (host: rows are at least 2 D bytes apart, so the difference is not negative)
     const int r = j * RPI + ld_row;
-    k_voff[j] = r * k_row + (ld_chunk ^ direct_swizzle<D>(r)) * 16 - (j & 3) * 1024;
-    v_voff[j] = r * v_row + (ld_chunk ^ direct_swizzle<D>(r)) * 16 - (j & 3) * 1024;
+    k_voff[j] = r * k_row + (ld_chunk ^ chunk_swizzle<D>(r)) * 16 - (j & 3) * 1024;
+    v_voff[j] = r * v_row + (ld_chunk ^ chunk_swizzle<D>(r)) * 16 - (j & 3) * 1024;
   }
   auto issue = [&](__amdgpu_buffer_rsrc_t rsrc, uint32_t row_bytes, const uint32_t* voff, uint32_t to, int key) {
     if (key + 32 <= len) {
@@ -196,7 +181,7 @@ selattn_direct_fwd_kernel(DirectParams p) {
 #pragma unroll 1
       for (int j = 0; j < NLD; ++j) {
         const int r = j * RPI + ld_row;
-        const uint32_t off = (uint32_t)min(key + r, len - 1) * row_bytes + (ld_chunk ^ direct_swizzle<D>(r)) * 16;
+        const uint32_t off = (uint32_t)min(key + r, len - 1) * row_bytes + (ld_chunk ^ chunk_swizzle<D>(r)) * 16;
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
                      :: "v"(off), "s"(rsrc), "s"(to + j * 1024) : "memory");
       }
@@ -205,11 +190,11 @@ selattn_direct_fwd_kernel(DirectParams p) {
   auto issue_k = [&](int key) { issue(k_rsrc, k_row, k_voff, k_lds, key); };
   auto issue_v = [&](int key) { issue(v_rsrc, v_row, v_voff, v_lds, key); };
   // lane addresses of the fragments
-  const uint32_t kf_addr = k_lds + col * (D * 2) + (((hh * (D / 16)) ^ direct_swizzle<D>(col)) << 4);   // k-step ks: ^ 16 ks
+  const uint32_t kf_addr = k_lds + col * (D * 2) + (((hh * (D / 16)) ^ chunk_swizzle<D>(col)) << 4);   // k-step ks: ^ 16 ks
   const int vr = 4 * hh + ((lane & 15) >> 2);
-  const uint32_t vf_addr = v_lds + vr * (D * 2) + (((2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ direct_swizzle<D>(vr)) << 4) + (lane & 1) * 8;
+  const uint32_t vf_addr = v_lds + vr * (D * 2) + (((2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ chunk_swizzle<D>(vr)) << 4) + (lane & 1) * 8;
   auto k_frag = [&](int ks) { return load16<vec8>(lds_ptr<T>(kf_addr ^ (16u * ks))); };
-  auto v_frag = [&](int j, int dt) { return direct_tr_frag<T, D>(vf_addr ^ (64u * dt), j); };   // keys 16 j .., dims 32 dt ..
+  auto v_frag = [&](int j, int dt) { return swizzled_tr_frag<T, D>(vf_addr ^ (64u * dt), j); };   // keys 16 j .., dims 32 dt ..
 
   float m = -INFINITY, mref = 0.f, l = 0.f;   // reference maximum (raw scores), the same scaled (0 while there is none)
   f32x16 oacc[NDT];
