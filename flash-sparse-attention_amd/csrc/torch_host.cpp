@@ -327,12 +327,18 @@ IndexView view_of(const std::vector<Tensor>& t, int64_t topk, int64_t block, int
           t[5].size(1), t[5].size(0), topk, block, max_blocks};
 }
 
+// `lists`: the block lists of the index, where short sequences may run from them as the operator's do
 std::pair<Tensor, Tensor> selattn_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const std::vector<Tensor>& index,
-                                      int64_t topk, int64_t block, int64_t max_blocks, optional<double> scale_) {
+                                      int64_t topk, int64_t block, int64_t max_blocks, optional<double> scale_,
+                                      const optional<Tensor>& lists) {
   check_qkv(q, k, v);
+  if (lists) check_topk(*lists, index[0]);
   const int64_t d = q.size(2), dn = native_dim(d);
-  auto [o, lse] = selattn_fwd_native(resize_d(q, dn), resize_d(k, dn), resize_d(v, dn),
-                                     view_of(index, topk, block, max_blocks), default_scale(scale_, d));
+  const double scale = default_scale(scale_, d);
+  const Tensor qn = resize_d(q, dn), kn = resize_d(k, dn), vn = resize_d(v, dn);
+  auto [o, lse] = lists && direct(qn, kn, vn, *lists, block)
+                      ? selattn_direct(qn, kn, vn, *lists, index[0], block, scale)
+                      : selattn_fwd_native(qn, kn, vn, view_of(index, topk, block, max_blocks), scale);
   return {resize_d(o, d), lse};
 }
 

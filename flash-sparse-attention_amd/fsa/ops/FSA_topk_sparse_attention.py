@@ -74,13 +74,26 @@ class PermuteResults(list):
         return super().__iter__()
 
 
-def _build_kernel_index(topk_idx, cu_seqlens, block_size):
-    """Index the kernels run on.  Blocks of 256 keys are handled as pairs of 128-key blocks (the same key set
-    for every query); the dicts of `PermuteResults` are still built for the caller's block size."""
+def _kernel_lists(topk_idx, cu_seqlens, block_size):
+    """(lists, block_size) the kernels run on: blocks of 256 keys are pairs of 128-key blocks (the same key set for
+    every query)."""
     if block_size == 256:
-        split = _ops.split_topk_blocks(topk_idx, cu_seqlens, 256, 2)
-        return _ops.build_index(split, cu_seqlens, 128), (topk_idx, cu_seqlens, 256)
-    return _ops.build_index(topk_idx, cu_seqlens, block_size), None
+        return _ops.split_topk_blocks(topk_idx, cu_seqlens, 256, 2), 128
+    return topk_idx, block_size
+
+
+def _build_kernel_index(topk_idx, cu_seqlens, block_size):
+    """Index the kernels run on; the dicts of `PermuteResults` are still built for the caller's block size."""
+    lists, size = _kernel_lists(topk_idx, cu_seqlens, block_size)
+    return _ops.build_index(lists, cu_seqlens, size), (topk_idx, cu_seqlens, 256) if block_size == 256 else None
+
+
+def _forward(q, k, v, topk_idx, cu_seqlens, block_size, sm_scale):
+    """(o, lse, index, see _build_kernel_index) by the kernels that the operator itself would take."""
+    lists, size = _kernel_lists(topk_idx, cu_seqlens, block_size)
+    index = _ops.build_index(lists, cu_seqlens, size)
+    o, lse = _ops.selattn_fwd(q, k, v, index, sm_scale, lists)
+    return o, lse, index, (topk_idx, cu_seqlens, 256) if block_size == 256 else None
 
 
 def _topk_sparse_attention_fwd_opt(
@@ -102,8 +115,7 @@ def _topk_sparse_attention_fwd_opt(
     assert block_size in _BLOCK_SIZES
     assert q.shape[1] % k.shape[1] == 0
     assert causal, "selected attention is causal"
-    index, ref_args = _build_kernel_index(topk_idx, cu_seqlens_q, block_size)
-    o, lse = _ops.selattn_fwd(q, k, v, index, sm_scale)
+    o, lse, index, ref_args = _forward(q, k, v, topk_idx, cu_seqlens_q, block_size, sm_scale)
     return o, lse, PermuteResults(index, ref_args)
 
 

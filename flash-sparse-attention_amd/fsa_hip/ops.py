@@ -117,10 +117,11 @@ def _check_qkv(q, k, v):
     assert k.shape == v.shape and q.shape[0] == k.shape[0] and q.shape[2] == k.shape[2]
 
 
-def selattn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, index: SelIndex,
-                softmax_scale: Optional[float] = None) -> Tuple[torch.Tensor, torch.Tensor]:
-    """Selected attention forward: returns (o [N,Hq,D], lse [Hq,N] fp32 base 2)."""
-    return _native.selattn_fwd(q, k, v, index.arrays(), index.topk, index.block_size, index.max_blocks, softmax_scale)
+def selattn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, index: SelIndex, softmax_scale: Optional[float] = None,
+                lists: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Selected attention forward: returns (o [N,Hq,D], lse [Hq,N] fp32 base 2).  `lists`: the topk_idx that the index was
+    built from; with it, short sequences take the kernel that `selected_attention` takes for them."""
+    return _native.selattn_fwd(q, k, v, index.arrays(), index.topk, index.block_size, index.max_blocks, softmax_scale, lists)
 
 
 def selattn_bwd(q, k, v, o, do, lse, index: SelIndex, softmax_scale: Optional[float] = None):

@@ -19,7 +19,7 @@ from typing import Any, Optional
 
 import torch
 
-from fsa.ops.FSA_topk_sparse_attention import _BLOCK_SIZES, _build_kernel_index
+from fsa.ops.FSA_topk_sparse_attention import _BLOCK_SIZES, _build_kernel_index, _forward
 from fsa_hip import ops as _ops
 
 
@@ -40,8 +40,7 @@ def _topk_sparse_attention_fwd(
     assert cu_seqlens_q.dtype == torch.int32 and cu_seqlens_k.dtype == torch.int32
     assert block_size in _BLOCK_SIZES
     assert q.shape[1] % k.shape[1] == 0
-    index, _ = _build_kernel_index(topk_idx, cu_seqlens_q, block_size)
-    return _ops.selattn_fwd(q, k, v, index, sm_scale)
+    return _forward(q, k, v, topk_idx, cu_seqlens_q, block_size, sm_scale)[:2]
 
 
 def _topk_sparse_attention_bwd(
