@@ -294,12 +294,18 @@ __device__ __forceinline__ int div_small(int i, int d, float rcp) {
 }
 
 // Block ids of CT_ROUNDS entries of a tile: entry numbers idx[r] (negative: none).  All loads are issued together,
-// without branches, and before anything that waits for another load.
+// without branches, and before anything that waits for another load.  Lists that lie end to end need no division.
 __device__ __forceinline__ void load_block_ids(const int32_t* __restrict__ topk_idx, int64_t stride_h,
                                                int64_t stride_n, int h, int tok0, int topk, int n_it,
                                                const int* idx, int* raw) {
   const float rcp = 1.0f / (float)topk;
   const int32_t* base = topk_idx + h * stride_h;
+  if (stride_n == topk) {
+    base += (int64_t)tok0 * topk;
+#pragma unroll
+    for (int r = 0; r < CT_ROUNDS; ++r) raw[r] = base[min(max(idx[r], 0), n_it - 1)];
+    return;
+  }
 #pragma unroll
   for (int r = 0; r < CT_ROUNDS; ++r) {
     const int i = min(max(idx[r], 0), n_it - 1);
@@ -335,17 +341,28 @@ __device__ __forceinline__ void ids_to_buckets(const int32_t* __restrict__ cu_se
   }
 }
 
-// table[h][tile][bucket] = entries of the tile that fall into the bucket (a tile writes one contiguous row)
+// log2 of the copies of a counter in count_tiles_kernel: what 32 KB hold (five work-groups per CU), one per lane at most
+__host__ __device__ inline int count_copies(int nbuckets) {
+  int c = 6;
+  while (c > 0 && (nbuckets << c) > 8448) --c;
+  return c;
+}
+
+// table[h][tile][bucket] = entries of the tile that fall into the bucket (a tile writes one contiguous row).  Bound by the LDS
+// atomics: lanes that add to one word or one bank are served one after the other, some two clocks each, and the blocks that
+// every query takes are in every list.  A counter therefore has copies, taken in turn by the lanes: 8192 queries x 16 slots x
+// 32 heads 17.5 us with one copy, 9.4 with 64; 65536 x 16 x 4 18.6, with 8 copies 10.6.
 __global__ void __launch_bounds__(CT_THREADS)
 count_tiles_kernel(const int32_t* __restrict__ topk_idx, int64_t stride_h, int64_t stride_n,
                    const int32_t* __restrict__ cu_seqlens, int32_t* __restrict__ cu_blocks_out, int batch,
                    int block_size, int64_t n_tokens, int topk, int q_per_tile, int ntiles, int nbuckets,
-                   int32_t* __restrict__ table) {
-  extern __shared__ int hist[];
+                   int copies, int32_t* __restrict__ table) {
+  extern __shared__ int hist[];   // [nbuckets][1 << copies]
   __shared__ int cu_l[CT_THREADS + 1], cub_l[CT_THREADS + 1];
   const int h = blockIdx.y, tile = blockIdx.x, tid = threadIdx.x;
   const int64_t tok0 = (int64_t)tile * q_per_tile;
   const int n_q = (int)min((int64_t)q_per_tile, n_tokens - tok0);
+  const int mine = (tid + tid / 16) & ((1 << copies) - 1);   // (the same slot of neighbouring queries: different copies)
   int key[CT_ROUNDS], idx[CT_ROUNDS];  // the tile has at most CT_ITEMS entries (host check)
 #pragma unroll
   for (int r = 0; r < CT_ROUNDS; ++r) {
@@ -353,7 +370,7 @@ count_tiles_kernel(const int32_t* __restrict__ topk_idx, int64_t stride_h, int64
     idx[r] = i < n_q * topk ? i : -1;
   }
   load_block_ids(topk_idx, stride_h, stride_n, h, (int)tok0, topk, n_q * topk, idx, key);
-  for (int b = tid; b < nbuckets; b += CT_THREADS) hist[b] = 0;   // while the ids are on their way
+  for (int b = tid; b < nbuckets << copies; b += CT_THREADS) hist[b] = 0;   // while the ids are on their way
   if (batch <= CT_THREADS) {  // no kernel has written cu_blocks yet: the first work-group does
     sequence_table<CT_THREADS>(cu_seqlens, batch, block_size, cu_l, cub_l);
     if (h == 0 && tile == 0)
@@ -367,9 +384,13 @@ count_tiles_kernel(const int32_t* __restrict__ topk_idx, int64_t stride_h, int64
   }
 #pragma unroll
   for (int r = 0; r < CT_ROUNDS; ++r)
-    if (key[r] >= 0) atomicAdd(&hist[key[r]], 1);
+    if (key[r] >= 0) atomicAdd(&hist[(key[r] << copies) + mine], 1);
   __syncthreads();
-  for (int b = tid; b < nbuckets; b += CT_THREADS) table[((int64_t)h * ntiles + tile) * nbuckets + b] = hist[b];
+  for (int b = tid; b < nbuckets; b += CT_THREADS) {
+    int sum = 0;
+    for (int c = 0; c < 1 << copies; ++c) sum += hist[(b << copies) + ((c + tid) & ((1 << copies) - 1))];   // (lanes apart)
+    table[((int64_t)h * ntiles + tile) * nbuckets + b] = sum;
+  }
 }
 
 // Exclusive scan of the table over the tiles, bucket by bucket; the total of a bucket is its entry count.  A
@@ -483,8 +504,12 @@ __host__ __device__ inline int place_lds_ints(int nbuckets) {
 // KEY_BITS: bits of a bucket id that the lanes of a wave are matched on (2^KEY_BITS >= nbuckets); a constant, so
 // that the matching below is straight-line code - as a loop over a run-time count it spends as much on the loop as
 // on the ballots.
+// What bounds it is the serial chain of a tile (loads, 16 rounds of matching, two scans, two scattered stores; 15 us), so all
+// tiles of a call should run at once: with room for 16 waves per CU the 1024 tiles of 4 M entries are one wave of work-groups.
+// (Three work-groups per CU left a few tiles to a second wave: 8192 queries x 16 slots x 32 heads 38 us, now 25.5; 65536 x
+// 16 x 4 42.5, now 29.6.)
 template <int KEY_BITS>
-__global__ void __launch_bounds__(CT_THREADS)
+__global__ void __launch_bounds__(CT_THREADS, KEY_BITS > 11 ? 1 : 4)
 place_items_kernel(const int32_t* __restrict__ topk_idx, int64_t stride_h, int64_t stride_n,
                    const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ cu_blocks, int batch,
                    int64_t n_tokens, int topk, int q_per_tile, int ntiles, int nbuckets,
@@ -501,8 +526,31 @@ place_items_kernel(const int32_t* __restrict__ topk_idx, int64_t stride_h, int64
   // lines of sel_tokens: tiles are dealt so that an XCD gets a contiguous eighth of them (gridDim.x is a multiple
   // of eight), and the pieces of a line meet in one L2 instead of leaving eight of them as partial lines.
   const int h = blockIdx.y, tid = threadIdx.x;
-  const int tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) - 2;
   if (tile >= ntiles) return;
+  constexpr int BPT = KEY_BITS > 8 ? (1 << KEY_BITS) / CT_THREADS : 1;
+  const int per = (nbuckets + CT_THREADS - 1) / CT_THREADS;   // <= BPT: thread t has buckets [t * per, (t + 1) * per)
+  const int32_t* tot = bucket_total + h * nbuckets;
+  int tot_r[BPT];
+  auto load_totals = [&] {
+#pragma unroll
+    for (int j = 0; j < BPT; ++j) {
+      const int b = tid * per + j;
+      tot_r[j] = j < per && b < nbuckets ? tot[b] : 0;
+    }
+  };
+  if (tile < 0) {
+    // two work-groups of a head write the work lists meanwhile (behind the placing of a tile that was 5 us at the end)
+    const TileList& l = tile == -1 ? lb : la;
+    if (!l.prefix) return;
+    load_totals();
+    write_work_list<CT_THREADS>(l, h, nbuckets - 1, per, tot_r, lds, [](int v) {
+      int ea, eb;
+      block_exclusive_scan2(v, 0, &ea, &eb);
+      return ea;
+    });
+    return;
+  }
   const int lane = tid & (WAVE - 1), w = tid / WAVE;
   const int64_t tok0 = (int64_t)tile * q_per_tile;
   const int n_q = (int)min((int64_t)q_per_tile, n_tokens - tok0);
@@ -556,21 +604,17 @@ place_items_kernel(const int32_t* __restrict__ topk_idx, int64_t stride_h, int64
     }
   }
   __syncthreads();
-  // Thread t finishes buckets [t * per, (t + 1) * per): two exclusive scans over the buckets - of the bucket totals
+  // Thread t finishes its buckets: two exclusive scans over the buckets - of the bucket totals
   // (start of the bucket in sel_tokens) and of the tile's own counts (start of the bucket in the sorted tile).
-  constexpr int BPT = CT_MAX_BUCKETS / CT_THREADS;
-  const int per = (nbuckets + CT_THREADS - 1) / CT_THREADS;   // <= BPT
-  const int32_t* tot = bucket_total + h * nbuckets;
   const int32_t* trow = table + ((int64_t)h * ntiles + tile) * nbuckets;
-  int tot_r[BPT], tab_r[BPT];
+  int tab_r[BPT];
   int sum_tot = 0, sum_tile = 0;
+  load_totals();
 #pragma unroll
   for (int j = 0; j < BPT; ++j) {
     const int b = tid * per + j;
-    tot_r[j] = 0;
     tab_r[j] = 0;
     if (j < per && b < nbuckets) {
-      tot_r[j] = tot[b];
       tab_r[j] = trow[b];
       sum_tot += tot_r[j];
 #pragma unroll
@@ -628,18 +672,6 @@ place_items_kernel(const int32_t* __restrict__ topk_idx, int64_t stride_h, int64
   for (int r = 0; r < CT_ROUNDS; ++r) {
     const int j = tid + r * CT_THREADS;
     if (j < n_it) st[sorted_pos[j]] = j < n_real ? (int32_t)(tok0 + div_small((int)sorted_item[j], topk, rcp)) : -1;
-  }
-  // every work-group has the totals: two of them write the work lists
-  for (int k = 0; k < 2; ++k) {
-    const TileList& l = k ? lb : la;
-    if (tile == k % ntiles && l.prefix) {
-      __syncthreads();
-      write_work_list<CT_THREADS>(l, h, nbuckets - 1, per, tot_r, lds, [](int v) {
-        int ea, eb;
-        block_exclusive_scan2(v, 0, &ea, &eb);
-        return ea;
-      });
-    }
   }
 }
 
@@ -1032,13 +1064,14 @@ static int build_index(const int32_t* topk_idx, int64_t topk_stride_h, int64_t t
     int key_bits = 1;
     while ((1 << key_bits) < c.nbuckets) ++key_bits;
     dim3 g_tiles(c.ntiles, num_kv_heads);
-    count_tiles_kernel<<<g_tiles, CT_THREADS, (size_t)c.nbuckets * 4, stream>>>(
+    const int copies = count_copies(c.nbuckets);
+    count_tiles_kernel<<<g_tiles, CT_THREADS, ((size_t)c.nbuckets << copies) * 4, stream>>>(
         topk_idx, topk_stride_h, topk_stride_n, cu_seqlens, cu_blocks, batch, block_size, total_tokens, topk,
-        c.q_per_tile, c.ntiles, c.nbuckets, table);
+        c.q_per_tile, c.ntiles, c.nbuckets, copies, table);
     scan_tiles_kernel<<<dim3((c.nbuckets + WAVE - 1) / WAVE, num_kv_heads), ST_WAVES * WAVE, 0, stream>>>(
         table, c.ntiles, c.nbuckets, max_blocks, counts, totals);
     const size_t lds = (size_t)place_lds_ints(c.nbuckets) * 4;
-    dim3 g_place((c.ntiles + 7) / 8 * 8, num_kv_heads);
+    dim3 g_place((c.ntiles + 2 + 7) / 8 * 8, num_kv_heads);
 #define FSA_PLACE(KB)                                                                                            \
   {                                                                                                              \
     static LdsAllowed allowed;                                                                                   \
