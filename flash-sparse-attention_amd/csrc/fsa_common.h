@@ -174,6 +174,13 @@ template <typename T, int D> __device__ __forceinline__ typename Elem<T>::vec8 s
   return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
+// Loads that go to LDS past the registers are not counted by the compiler: vm_wait<N> waits until only the N youngest memory
+// operations of the wave are still on the way.
+template <int N> __device__ __forceinline__ void vm_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
+}
+__device__ __forceinline__ void lds_reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 // 2^x by the hardware instruction alone (1 ulp; results below 2^-126 flush to zero, -inf gives 0): the
 // library exp2f adds a denormal-range rescaling that costs several VALU operations per element
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }

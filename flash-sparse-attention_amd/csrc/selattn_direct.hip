@@ -40,8 +40,7 @@ template <int D, int KG> struct DirectLds {
 };
 
 // Four KB of a tile, global memory to LDS: lane l's 16 bytes at voff[j](l) + soff + 1024 j of the buffer land at LDS byte
-// `lds` + 1024 j + 16 l (the instruction's offset moves both addresses).  The compiler does not count these loads: vm_wait
-// orders them.
+// `lds` + 1024 j + 16 l (the instruction's offset moves both addresses).
 __device__ __forceinline__ void lds_dma4(__amdgpu_buffer_rsrc_t rsrc, const uint32_t* voff, uint32_t soff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %6\n\ts_nop 0\n\t"
                "buffer_load_dwordx4 %0, %4, %5 offen lds\n\t"
@@ -50,11 +49,6 @@ __device__ __forceinline__ void lds_dma4(__amdgpu_buffer_rsrc_t rsrc, const uint
                "buffer_load_dwordx4 %3, %4, %5 offen offset:3072 lds"
                :: "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(rsrc), "s"(soff), "s"(lds) : "memory");
 }
-template <int N> __device__ __forceinline__ void vm_wait() {
-  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
-}
-__device__ __forceinline__ void lds_reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-
 // Sequence and row tile of work-group `id`; false: past the last tile.  The late tiles of a sequence, which see the most
 // blocks, come first.
 __device__ __forceinline__ bool direct_tile(const int32_t* __restrict__ cu, int batch, int g, int id, int& s, int& tile) {

@@ -675,15 +675,14 @@ struct HostCopy {
 };
 
 // Whether the products of a layer run as fsa_matmul launches instead of library calls: a bound on the operations of q, k and
-// v.  All products of a step issued back to back, ours / library in us, training (13 products) | inference (4); the library's
-// times below 225 | 77 are what its calls cost the host:
-//   hidden 4096, 32 + 8 heads: 250 tokens 176 / 225 | 60 / 78, 500 tokens (25e9) 293 / 263 | 102 / 83
-//   hidden 2048, 16 + 4 heads: 1000 tokens (13e9) 158 / 223 | 53 / 77, 2000 (25e9) 220 / 254 | 72 / 76, 4000 392 / 389 | 125 / 98
-//   hidden 1024,  8 + 2 heads: 8000 tokens (25e9) 226 / 356 | 72 / 77, 16000 434 / 606 | 134 / 90
-// The line suits the wide layer; narrower ones are handed over earlier than they need be (hidden 1024 in training at 7600
-// tokens, where ours would still be faster at 16000).
-bool own_products(int64_t n, int64_t hidden, const LayerShape& shape, bool training) {
-  return 2.0 * (double)n * (double)hidden * (double)((shape[0] + 2 * shape[1]) * shape[2]) <= (training ? 24e9 : 10e9);
+// v.  A whole pass of one sequence, library / ours in us (below some 225 us in training and 77 in inference the library's
+// products cost the host more than the device):
+//   hidden 4096, 32 + 8 heads: inference 300 tokens (15e9) 129 / 127, 700 (35e9) 171 / 174; training 700 tokens 586 / 584
+//   hidden 2048, 16 + 4 heads: inference 1000 tokens (13e9) 122 / 112, 2000 (25e9) 167 / 162; training 2500 (31e9) 744 / 709
+//   hidden 1024,  8 + 2 heads: inference 5000 tokens (16e9) 216 / 206, 8000 (25e9) 331 / 322; training 9000 (28e9) 1357 / 1192
+// The line suits the wide layer; narrower ones are handed over earlier than they need be.
+bool own_products(int64_t n, int64_t hidden, const LayerShape& shape) {
+  return 2.0 * (double)n * (double)hidden * (double)((shape[0] + 2 * shape[1]) * shape[2]) <= 24e9;
 }
 
 fsa_matmul_out product(const Tensor& c, const Tensor* add = nullptr) {
@@ -712,7 +711,7 @@ LayerForward layer_forward(const Tensor& x, const Tensor& cu, const Tensor& w_q,
                            const Tensor& inv_freq, double rope_scale, const LayerShape& shape, LayerSizes& z,
                            const Tensor* lens, HostCopy* copied, bool training) {
   LayerForward f;
-  const bool own = own_products(x.size(0), x.size(1), shape, training);
+  const bool own = own_products(x.size(0), x.size(1), shape);
   if (own) {
     Tensor* y[3] = {&f.q, &f.k, &f.v};
     const Tensor* w[3] = {&w_q, &w_k, &w_v};
@@ -795,7 +794,7 @@ struct LayerCore : torch::autograd::Function<LayerCore> {
     std::copy(shape_v.begin(), shape_v.end(), shape.begin());
     const c10::OptionalDeviceGuard guard(x.device());
     const Tensor dy = grads[0].contiguous();
-    const bool own = own_products(x.size(0), x.size(1), shape, true) && (uintptr_t)dy.data_ptr() % 16 == 0;
+    const bool own = own_products(x.size(0), x.size(1), shape) && (uintptr_t)dy.data_ptr() % 16 == 0;
     Tensor d_out;
     if (own) {
       d_out = at::empty({dy.size(0), w_o.size(1)}, dy.options());
