@@ -116,8 +116,11 @@ static inline int kv_tile_rows(int64_t rows_total, int g, int d, int bk) {
   const int r = 1024 + 2048 * g;
   // head_dim 256 with 128-key blocks: 32-row passes of eight waves, fewer, longer tiles
   const int cap = (d >= 256 && bk >= 128) || r > KV_TILE_ROWS_MAX ? KV_TILE_ROWS_MAX : r;
-  const int per_cu = d <= 128 && bk <= 64 ? 2 : 1;
-  const int two = balanced_tile_rows(rows_total, per_cu, cap);   // work-groups for each of the chip's slots
+  return balanced_tile_rows(rows_total, d <= 128 && bk <= 64 ? 2 : 1, cap);   // two work-groups for each of the chip's slots
+}
+// Selected attention
+static inline int sel_kv_tile_rows(int64_t rows_total, int g, int d, int bk) {
+  const int two = kv_tile_rows(rows_total, g, d, bk), per_cu = d <= 128 && bk <= 64 ? 2 : 1;
   if (d < 128) return two;
   // Every work-group of a shared block leaves 2 * bk * d fp32 partial sums to be added: as long as the tiles are short, one
   // work-group per slot.  Backward (us, two per slot -> one): 2000 tokens x 8 heads, 8 blocks of 64, 69 -> 51, 8 blocks of

@@ -138,7 +138,7 @@ static BwdWs bwd_ws_layout(int64_t n, int hq, int hkv, int d, int topk, int bk, 
   BwdWs w;
   const int g = hq / hkv;
   const size_t cap = (size_t)n * topk;
-  w.max_tiles_kv = fsa_max_tiles(n, topk, g, kv_tile_rows((int64_t)cap * hq, g, d, bk), max_blocks);
+  w.max_tiles_kv = fsa_max_tiles(n, topk, g, sel_kv_tile_rows((int64_t)cap * hq, g, d, bk), max_blocks);
   w.off_delta = 0;
   w.off_dqpart = align_up((size_t)n * hq * 8, 256);
   w.off_tiles_kv = w.off_dqpart + align_up(cap * hkv * g * d * 2, 256);
@@ -222,7 +222,7 @@ TileList selattn_tiles(bool backward, int64_t n_tokens, int hq, int hkv, int d, 
                        int32_t* mem) {
   TileList l;
   l.g = hq / hkv;
-  l.rows = backward ? kv_tile_rows(n_tokens * topk * hq, l.g, d, bk) : sel_tile_rows(n_tokens, topk, hkv, l.g, d, bk);
+  l.rows = backward ? sel_kv_tile_rows(n_tokens * topk * hq, l.g, d, bk) : sel_tile_rows(n_tokens, topk, hkv, l.g, d, bk);
   l.max_tiles = fsa_max_tiles(n_tokens, topk, l.g, l.rows, max_blocks);
   l.prefix = mem;
   l.block = mem ? mem + (int64_t)hkv * (max_blocks + 1) : nullptr;
@@ -280,7 +280,7 @@ int fsa::selattn_bwd(const void* q, const void* k, const void* v, const void* o,
     tiles_kv = (int32_t*)(wsp + ws.off_tiles_kv);
     tile_block = (int32_t*)(wsp + ws.off_tile_block);
     rc = build_tiles(counts, num_kv_heads, max_blocks, g,
-                     kv_tile_rows(total_tokens * topk * num_q_heads, g, head_dim, block_size), (int32_t*)tiles_kv,
+                     sel_kv_tile_rows(total_tokens * topk * num_q_heads, g, head_dim, block_size), (int32_t*)tiles_kv,
                      (int32_t*)tile_block, ws.max_tiles_kv, stream);
     if (rc) return rc;
   }
