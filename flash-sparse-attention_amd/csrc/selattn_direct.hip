@@ -434,6 +434,7 @@ int selattn_direct_fwd(const void* q, const void* k, const void* v, int32_t dtyp
                 "fsa_selattn_direct_fwd: bad sizes");
   FSA_CHECK_ARG((q_stride_n | q_stride_h | k_stride_n | k_stride_h | v_stride_n | v_stride_h | o_stride_n | o_stride_h) % 8 == 0,
                 "fsa_selattn_direct_fwd: strides must be multiples of 8 elements (16-byte rows)");
+  FSA_CHECK_ARG(((uintptr_t)k | (uintptr_t)v) % 16 == 0, "fsa_selattn_direct_fwd: k and v must be 16-byte aligned");
   FSA_CHECK_ARG(k_stride_n >= head_dim && v_stride_n >= head_dim && total_tokens * 2 * k_stride_n < ((int64_t)1 << 31) &&
                     total_tokens * 2 * v_stride_n < ((int64_t)1 << 31), "fsa_selattn_direct_fwd: k / v strides out of range");
   FSA_CHECK_ARG(block_size >= 1 && max_len <= (int64_t)block_size * DIR_MAX_BLOCKS && total_tokens * num_q_heads < ((int64_t)1 << 31),
@@ -477,5 +478,6 @@ extern "C" int fsa_selattn_direct_fwd(const void* q, const void* k, const void* 
 
 extern "C" int fsa_selattn_direct_preferred(int64_t total_tokens, int64_t max_len, int32_t num_q_heads, int32_t head_dim,
                                             int32_t topk, int32_t block_size) {
+  FSA_CHECK_ARG(total_tokens >= 1 && max_len >= 1 && num_q_heads >= 1 && topk >= 1, "fsa_selattn_direct_preferred: bad sizes");
   return selattn_direct_preferred(total_tokens, max_len, num_q_heads, head_dim, topk, block_size);
 }

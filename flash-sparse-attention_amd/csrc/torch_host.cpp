@@ -284,7 +284,7 @@ bool direct(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& top
     return t.stride(0) >= d && t.stride(0) * n < (int64_t)1 << 30 && (uintptr_t)t.data_ptr() % 16 == 0;
   };
   return n >= 1 && topk_idx.size(0) == k.size(1) && topk_idx.size(1) == n && rows_ok(k) && rows_ok(v) &&
-         api.fsa_selattn_direct_preferred(n, n, (int32_t)q.size(1), (int32_t)d, (int32_t)topk_idx.size(2), (int32_t)block);
+         api.fsa_selattn_direct_preferred(n, n, (int32_t)q.size(1), (int32_t)d, (int32_t)topk_idx.size(2), (int32_t)block) == 1;
 }
 std::pair<Tensor, Tensor> selattn_direct(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& topk_idx, const Tensor& cu,
                                          int64_t block, double scale) {
