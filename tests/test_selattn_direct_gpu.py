@@ -175,3 +175,21 @@ def test_refuses(dev):
         _direct(q, k, v, idx, cu, 64, 257)
     with pytest.raises(ValueError):
         _direct(q, k, v, idx, cu, 48)
+
+
+@pytest.mark.parametrize("hq,hkv,d,block,topk", [(2, 1, 128, 64, 3), (4, 4, 64, 32, 20), (1, 1, 256, 128, 3), (80, 80, 128, 64, 6)])
+@pytest.mark.parametrize("kind", ["own", "none", "late"])
+def test_first_blocks_that_nobody_selected(dev, hq, hkv, d, block, topk, kind):
+    """What is requested ahead is not visited: lists of the own block only, of nothing for whole row tiles, of late blocks with
+    more entries than are requested at once."""
+    print(f"case {hq} {hkv} {d} {block} {topk} {kind}", flush=True)
+    n, cu = 641, [0, 641]
+    q, k, v = (x.to(dev) for x in make_qkv(n, hq, hkv, d, torch.bfloat16, seed=5, with_do=False))
+    k[:2 * block], v[:2 * block] = math.nan, math.nan
+    own = torch.arange(n) // block
+    idx = torch.full((hkv, n, topk), -1, dtype=torch.int32)
+    if kind != "none":
+        for t in range(topk if kind == "late" else 1):
+            idx[..., t] = torch.where((own - t >= 2) & (torch.arange(n) % 160 > 70), own - t, -1).int()
+    idx, cut = idx.to(dev), torch.tensor(cu, dtype=torch.int32, device=dev)
+    _check(_direct(q, k, v, idx, cut, block), _reference(q, k, v, idx, cut, block), torch.bfloat16)
