@@ -10,6 +10,7 @@
 #include "fsa_common.h"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace fsa {
@@ -430,17 +431,21 @@ template <typename T, bool MERGE> static int dispatch_direct_fwd(int d, int bk, 
 
 // Whether the forward of `n` tokens in sequences of at most `max_len` takes this path.  Both sides in us on one chip, fitted to
 // the times below: this kernel visits up to half of a sequence for every row, and its longest work-group works through a whole
-// one; the block-major launches work on topk * block keys per row, behind 25 us that do not depend on the size (index, two more
-// launches and their gaps).  head_dim 128, lists of 16 blocks of 64, one sequence; block-major / direct in us:
-//   4096 tokens x 4 heads 61 / 42, x 16 (GQA 4) 135 / 114, x 32 (GQA 4) 244 / 197; 2000 x 8 (GQA 8) 53 / 24, x 32 119 / 61;
-//   8192 x 4 98 / 102, x 32 (GQA 4) 482 / 563, x 32 539 / 722; 16384 x 4 (GQA 4) 170 / 208
-bool selattn_direct_preferred(int64_t n, int64_t max_len, int hq, int d, int topk, int bk) {
+// one; the block-major launches work on topk * block keys per row, behind 33 us that do not depend on the size (index, two more
+// launches and their gaps), 12 of them for the index, which is no loss where the caller builds it all the same (training).
+// Lists of 16 blocks of 64, one sequence; index + block-major / direct / index + direct in us, head_dim 128:
+//   4096 tokens x 4 heads 62 / 37 / 53, x 16 (GQA 4) 131 / 101 / 115, x 32 (GQA 4) 233 / 192 / 208; 5000 x 4 69 / 47 / 65;
+//   5000 x 32 (GQA 4) 283 / 267 / 284; 6000 x 4 79 / 59 / 78, x 32 (GQA 4) 339 / 354; 7000 x 4 83 / 77; 8192 x 4 100 / 100, x 32
+//   505 / 711; 16384 x 4 (GQA 4) 167 / 211
+// head_dim 256, lists of 8: 3000 x 4 64 / 47 / 59, 4096 x 4 85 / 74 / 86, 6000 x 8 164 / 175; 64: 4500 x 8 46 / 35 / 46, 8000 x 8
+// (16 blocks) 93 / 94.
+bool selattn_direct_preferred(int64_t n, int64_t max_len, int hq, int d, int topk, int bk, bool index_needed) {
   if (!(d == 64 || d == 128 || d == 256) || !(bk == 32 || bk == 64 || bk == 128) || topk > 4096 ||
       max_len > (int64_t)bk * DIR_MAX_BLOCKS)
     return false;
   const double rows = (double)n * hq * d / 128, len = (double)max_len;
   const double keys = std::min<double>((double)topk * bk, len);
-  return rows * len / 2.8e6 + 0.0055 * len <= 25 + rows * keys / 4.8e5;
+  return std::hypot(rows * len / 2.95e6, 0.0055 * len) + 5 <= (index_needed ? 21 : 33) + rows * keys / 6.2e5;
 }
 
 int selattn_direct_fwd(const void* q, const void* k, const void* v, int32_t dtype, int64_t q_stride_n, int64_t q_stride_h,
@@ -500,7 +505,7 @@ extern "C" int fsa_selattn_direct_fwd(const void* q, const void* k, const void* 
 }
 
 extern "C" int fsa_selattn_direct_preferred(int64_t total_tokens, int64_t max_len, int32_t num_q_heads, int32_t head_dim,
-                                            int32_t topk, int32_t block_size) {
+                                            int32_t topk, int32_t block_size, int32_t index_needed) {
   FSA_CHECK_ARG(total_tokens >= 1 && max_len >= 1 && num_q_heads >= 1 && topk >= 1, "fsa_selattn_direct_preferred: bad sizes");
-  return selattn_direct_preferred(total_tokens, max_len, num_q_heads, head_dim, topk, block_size);
+  return selattn_direct_preferred(total_tokens, max_len, num_q_heads, head_dim, topk, block_size, index_needed != 0);
 }

@@ -278,13 +278,14 @@ std::pair<Tensor, Tensor> selattn_fwd_native(const Tensor& q, const Tensor& k, c
 }
 
 // Short sequences: from the block lists (kernel_blocks), without an index
-bool direct(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& topk_idx, int64_t block) {
+bool direct(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& topk_idx, int64_t block, bool index_needed) {
   const int64_t n = q.size(0), d = q.size(2);
   auto rows_ok = [&](const Tensor& t) {   // they go to LDS by 16-byte buffer loads
     return t.stride(0) >= d && t.stride(0) * n < (int64_t)1 << 30 && (uintptr_t)t.data_ptr() % 16 == 0;
   };
   return n >= 1 && topk_idx.size(0) == k.size(1) && topk_idx.size(1) == n && rows_ok(k) && rows_ok(v) &&
-         api.fsa_selattn_direct_preferred(n, n, (int32_t)q.size(1), (int32_t)d, (int32_t)topk_idx.size(2), (int32_t)block) == 1;
+         api.fsa_selattn_direct_preferred(n, n, (int32_t)q.size(1), (int32_t)d, (int32_t)topk_idx.size(2), (int32_t)block,
+                                          index_needed) == 1;
 }
 std::pair<Tensor, Tensor> selattn_direct(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& topk_idx, const Tensor& cu,
                                          int64_t block, double scale) {
@@ -336,7 +337,7 @@ std::pair<Tensor, Tensor> selattn_fwd(const Tensor& q, const Tensor& k, const Te
   const int64_t d = q.size(2), dn = native_dim(d);
   const double scale = default_scale(scale_, d);
   const Tensor qn = resize_d(q, dn), kn = resize_d(k, dn), vn = resize_d(v, dn);
-  auto [o, lse] = lists && direct(qn, kn, vn, *lists, block)
+  auto [o, lse] = lists && direct(qn, kn, vn, *lists, block, true)
                       ? selattn_direct(qn, kn, vn, *lists, index[0], block, scale)
                       : selattn_fwd_native(qn, kn, vn, view_of(index, topk, block, max_blocks), scale);
   return {resize_d(o, d), lse};
@@ -370,8 +371,8 @@ struct SelectedAttention : torch::autograd::Function<SelectedAttention> {
     const Tensor ids = kernel_blocks(topk_idx, cu, block);
     const Index x = kernel_index(ids, cu, block, q.size(1), dn, true);
     const Tensor qn = resize_d(q, dn), kn = resize_d(k, dn), vn = resize_d(v, dn);
-    auto [on, lse] = direct(qn, kn, vn, ids, block) ? selattn_direct(qn, kn, vn, ids, cu, block, scale)
-                                                    : selattn_fwd_native(qn, kn, vn, x.view(), scale);
+    auto [on, lse] = direct(qn, kn, vn, ids, block, true) ? selattn_direct(qn, kn, vn, ids, cu, block, scale)
+                                                          : selattn_fwd_native(qn, kn, vn, x.view(), scale);
     ctx->save_for_backward({qn, kn, vn, on, lse, x.cu, x.mem});
     ctx->saved_data["ints"] = std::vector<int64_t>{d, x.n, x.hkv, x.topk, x.block, x.max_blocks, x.hq, x.d};
     ctx->saved_data["scale"] = scale;
@@ -400,7 +401,7 @@ Tensor selected_attention(const Tensor& q, const Tensor& k, const Tensor& v, con
     return SelectedAttention::apply(q, k, v, topk_idx, block, cu, scale);
   const int64_t d = q.size(2), dn = native_dim(d);
   const Tensor ids = kernel_blocks(topk_idx, cu, block), qn = resize_d(q, dn), kn = resize_d(k, dn), vn = resize_d(v, dn);
-  if (direct(qn, kn, vn, ids, block)) return resize_d(selattn_direct(qn, kn, vn, ids, cu, block, scale).first, d);
+  if (direct(qn, kn, vn, ids, block, false)) return resize_d(selattn_direct(qn, kn, vn, ids, cu, block, scale).first, d);
   const Index x = kernel_index(ids, cu, block, q.size(1), dn, false);
   return resize_d(selattn_fwd_native(qn, kn, vn, x.view(), scale).first, d);
 }

@@ -42,7 +42,7 @@ SIGNATURES = {
                                         vp, i32, i64, i32, i32, i32, i32, i32, i64, f32,
                                         vp, vp, vp, vp, vp, vp,
                                         vp, i64, i64, vp, vp, sz, vp]),
-    "fsa_selattn_direct_preferred": (C.c_int, [i64, i64, i32, i32, i32, i32]),
+    "fsa_selattn_direct_preferred": (C.c_int, [i64, i64, i32, i32, i32, i32, i32]),
     "fsa_selattn_direct_fwd": (C.c_int, [vp, vp, vp, i32, i64, i64, i64, i64, i64, i64,
                                          vp, i64, i64, vp, i32, i64, i64, i32, i32, i32, i32, i32, f32,
                                          vp, i64, i64, vp, vp]),

@@ -189,9 +189,10 @@ int fsa_selattn_fwd_tiles(const void* q, const void* k, const void* v, int32_t d
 /* The same result from the block lists alone, without index and workspace: one query-major launch that visits, for every 32
  * rows, the union of the blocks they selected.  For short sequences: max_len (any upper bound of the longest sequence) is at
  * most 1024 blocks, rows of k and v do not overlap and start at multiples of 16 bytes.  A block that a list names several times counts as often, as above.
- * fsa_selattn_direct_preferred: 1 where this is the faster one of the two, else 0 (below 0: bad sizes). */
+ * fsa_selattn_direct_preferred: 1 where this is the faster one of the two, else 0 (below 0: bad sizes); index_needed: the
+ * index is built in any case, for the backward. */
 int fsa_selattn_direct_preferred(int64_t total_tokens, int64_t max_len, int32_t num_q_heads, int32_t head_dim,
-                                 int32_t topk, int32_t block_size);
+                                 int32_t topk, int32_t block_size, int32_t index_needed);
 int fsa_selattn_direct_fwd(const void* q, const void* k, const void* v, int32_t dtype,
                            int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h,
                            int64_t v_stride_n, int64_t v_stride_h,

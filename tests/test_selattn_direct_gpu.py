@@ -158,7 +158,7 @@ def test_strides_and_operator(dev):
     idx = wide[..., :6]
     ref = _reference(q, k, v, idx, cu, 64)
     _check(_direct(q, k, v, idx, cu, 64), ref, torch.bfloat16)
-    assert _lib.load().fsa_selattn_direct_preferred(n, n, hq, d, 6, 64) == 1
+    assert _lib.load().fsa_selattn_direct_preferred(n, n, hq, d, 6, 64, 1) == 1
     assert (FSA_topk_sparse_attention(q, k, v, idx, 64, cu).double().cpu() - ref[0]).abs().max().item() <= O_TOL[torch.bfloat16]
     idx = make_topk_idx([0, 250, n], hkv, 256, 2, seed=10).to(dev)
     ref = _reference(q, k, v, idx, cu, 256)[0]
@@ -193,3 +193,18 @@ def test_first_blocks_that_nobody_selected(dev, hq, hkv, d, block, topk, kind):
             idx[..., t] = torch.where((own - t >= 2) & (torch.arange(n) % 160 > 70), own - t, -1).int()
     idx, cut = idx.to(dev), torch.tensor(cu, dtype=torch.int32, device=dev)
     _check(_direct(q, k, v, idx, cut, block), _reference(q, k, v, idx, cut, block), torch.bfloat16)
+
+
+def test_line_between_the_forms(dev):
+    """Where an index is built anyway the line lies lower; the two forms agree in between."""
+    lib = _lib.load()
+    sides = [[lib.fsa_selattn_direct_preferred(n, n, 4, 128, 16, 64, needed) for n in range(500, 9000, 500)] for needed in (0, 1)]
+    assert all(x == sorted(x, reverse=True) and x[0] == 1 and x[-1] == 0 for x in sides) and sum(sides[0]) > sum(sides[1])
+    n = 6000
+    assert [lib.fsa_selattn_direct_preferred(n, n, 4, 128, 16, 64, needed) for needed in (0, 1)] == [1, 0]
+    q, k, v = (x.to(dev) for x in make_qkv(n, 4, 4, 128, torch.bfloat16, seed=11, with_do=False))
+    cu = torch.tensor([0, n], dtype=torch.int32, device=dev)
+    idx = make_topk_idx([0, n], 4, 64, 16, seed=12).to(dev)
+    alone = FSA_topk_sparse_attention(q, k, v, idx, 64, cu)
+    trained = FSA_topk_sparse_attention(q.requires_grad_(), k, v, idx, 64, cu)
+    assert (alone.float() - trained.float()).abs().max().item() <= O_TOL[torch.bfloat16]
