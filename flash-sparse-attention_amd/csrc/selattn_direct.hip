@@ -32,6 +32,7 @@ struct DirectParams {
 
 constexpr int DIR_ROWS = 32;         // rows per work-group
 constexpr int DIR_MAX_BLOCKS = 1024; // of a sequence: size of the tables in LDS
+constexpr uint32_t DIR_BUFFER = 1u << 31;  // bytes of the K / V buffer descriptors (host: a head's rows span less)
 
 template <int D, int KG> struct DirectLds {
   static constexpr int TILE = 32 * D * 2;                   // 32 K or V rows, bytes
@@ -50,13 +51,23 @@ __device__ __forceinline__ void lds_dma4(__amdgpu_buffer_rsrc_t rsrc, const uint
                "buffer_load_dwordx4 %3, %4, %5 offen offset:3072 lds"
                :: "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(rsrc), "s"(soff), "s"(lds) : "memory");
 }
-// Sequence and row tile of work-group `id`; false: past the last tile.  The late tiles of a sequence, which see the most
+// The rows of the whole buffer, so that none of o and lse stays unwritten where the sequences do not fill it: segment i runs
+// from cu[i - 1] to cu[i], with the start of the buffer in front and its end behind.  Segment 0, in front of the first
+// sequence, has no keys; the last one holds the last sequence and, as queries at the positions behind it, the tokens that
+// follow it, which is where the inverted index counts them too.
+__device__ __forceinline__ int segment_begin(const int32_t* __restrict__ cu, int i) { return i > 0 ? cu[i - 1] : 0; }
+__device__ __forceinline__ int segment_end(const int32_t* __restrict__ cu, int batch, int64_t n_tokens, int i) {
+  return i < batch ? cu[i] : (int)n_tokens;
+}
+// Segment and row tile of work-group `id`; false: past the last tile.  The late tiles of a segment, which see the most
 // blocks, come first.
-__device__ __forceinline__ bool direct_tile(const int32_t* __restrict__ cu, int batch, int g, int id, int& s, int& tile) {
+__device__ __forceinline__ bool direct_tile(const int32_t* __restrict__ cu, int batch, int64_t n_tokens, int g, int id, int& s,
+                                            int& tile) {
   const int lane = threadIdx.x & (WAVE - 1);
-  for (int s0 = 0; s0 < batch; s0 += WAVE) {
+  for (int s0 = 0; s0 <= batch; s0 += WAVE) {
     const int si = s0 + lane;
-    const int n = si < batch ? (int)(((int64_t)(cu[si + 1] - cu[si]) * g + DIR_ROWS - 1) / DIR_ROWS) : 0;
+    const int n =
+        si <= batch ? (int)(((int64_t)(segment_end(cu, batch, n_tokens, si) - segment_begin(cu, si)) * g + DIR_ROWS - 1) / DIR_ROWS) : 0;
     int inc = n;
 #pragma unroll
     for (int o = 1; o < WAVE; o <<= 1) {
@@ -92,11 +103,11 @@ selattn_direct_fwd_kernel(DirectParams p) {
 
   const int h = blockIdx.x % p.hkv;
   int s, tile;
-  if (!direct_tile(p.cu, p.batch, p.g, blockIdx.x / p.hkv, s, tile)) return;
-  const int q0 = p.cu[s], len = p.cu[s + 1] - q0;
-  const int rows = len * p.g, row0 = tile * DIR_ROWS;
+  if (!direct_tile(p.cu, p.batch, p.n_tokens, p.g, blockIdx.x / p.hkv, s, tile)) return;
+  const int q0 = segment_begin(p.cu, s), len = s > 0 ? p.cu[s] - q0 : 0;   // len: keys
+  const int rows = (segment_end(p.cu, p.batch, p.n_tokens, s) - q0) * p.g, row0 = tile * DIR_ROWS;
   const int q_first = div_group(row0, p.g, p.g_shift), q_last = div_group(min(rows, row0 + DIR_ROWS) - 1, p.g, p.g_shift);
-  const int n_blk = q_last / BK + 1;
+  const int n_blk = min(q_last / BK + 1, (len + BK - 1) / BK);
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31, hh = lane >> 5;
 
@@ -114,9 +125,9 @@ selattn_direct_fwd_kernel(DirectParams p) {
   // ---- K / V tiles ----
   const uint32_t k_row = (uint32_t)p.k_sn * 2, v_row = (uint32_t)p.v_sn * 2;   // bytes (host: a head's rows span < 2^31)
   const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<T*>(reinterpret_cast<const T*>(p.k) + (int64_t)q0 * p.k_sn + (int64_t)h * p.k_sh), 0, -1, 0x00020000);
+      const_cast<T*>(reinterpret_cast<const T*>(p.k) + (int64_t)q0 * p.k_sn + (int64_t)h * p.k_sh), 0, (int)DIR_BUFFER, 0x00020000);
   const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<T*>(reinterpret_cast<const T*>(p.v) + (int64_t)q0 * p.v_sn + (int64_t)h * p.v_sh), 0, -1, 0x00020000);
+      const_cast<T*>(reinterpret_cast<const T*>(p.v) + (int64_t)q0 * p.v_sn + (int64_t)h * p.v_sh), 0, (int)DIR_BUFFER, 0x00020000);
   const uint32_t k_lds = lds_addr(smem + wv * L::WAVE_BYTES), v_lds = k_lds + L::TILE;
   // (the loading lane picks its source so that the chunks land where chunk_swizzle wants them)
   const int ld_row = lane / CPR, ld_chunk = lane % CPR;
@@ -132,11 +143,13 @@ selattn_direct_fwd_kernel(DirectParams p) {
 #pragma unroll
       for (int j = 0; j < NLD; j += 4) lds_dma4(rsrc, &voff[j], (uint32_t)key * row_bytes, to + j * 1024);
     } else {
-      // a tile that reaches behind the end: its last row again in the place of the others, which no query sees
+      // A tile that reaches behind the end: zeros there (an offset behind the end of the buffer).  No query of the sequence
+      // sees them; one at a position behind it does, with score 0, as in the block-major kernels.
 #pragma unroll 1
       for (int j = 0; j < NLD; ++j) {
         const int r = j * RPI + ld_row;
-        const uint32_t off = (uint32_t)min(key + r, len - 1) * row_bytes + (ld_chunk ^ chunk_swizzle<D>(r)) * 16;
+        const uint32_t off =
+            key + r < len ? (uint32_t)(key + r) * row_bytes + (ld_chunk ^ chunk_swizzle<D>(r)) * 16 : DIR_BUFFER;
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
                      :: "v"(off), "s"(rsrc), "s"(to + j * 1024) : "memory");
       }
@@ -168,7 +181,7 @@ selattn_direct_fwd_kernel(DirectParams p) {
   if (tid < 2) info[tid] = 0;
   __syncthreads();
   auto visit = [&](int q, int b) {
-    if (b < 0 || b > (q_first + q) / BK) return;   // (a block behind the query's own holds no key it may see)
+    if (b < 0 || b >= n_blk || b > (q_first + q) / BK) return;   // (a block behind the query's own holds no key it may see)
     if (atomicOr(&sel[b], 1u << q) >> q & 1) info[1] = 1;
   };
 #pragma unroll
@@ -401,7 +414,7 @@ static int launch_direct_fwd(const DirectParams& p, int64_t tiles, hipStream_t s
     return rc;
   ProfScope ps_("selattn_direct_fwd", stream);
   selattn_direct_fwd_kernel<T, D, BK, KG, MERGE>
-      <<<(unsigned)(tiles * p.hkv), 64 * KG, DirectLds<D, KG>::bytes(p.max_blk), stream>>>(p);
+      <<<(unsigned)((tiles + 1) * p.hkv), 64 * KG, DirectLds<D, KG>::bytes(p.max_blk), stream>>>(p);
   return 0;
 }
 // Two waves per work-group where there are enough of them to fill the chip: less to merge, and more work-groups in different
