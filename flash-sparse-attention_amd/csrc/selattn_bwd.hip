@@ -48,10 +48,11 @@ selattn_bwd_delta_kernel(const T* __restrict__ o, int64_t o_sn, int64_t o_sh,
 // EPI: the epilogue of DqEpilogue - in a layer dQ of the three branches and the inverse rotation meet here, on rows that
 // are in registers anyway, instead of in two elementwise sums and a rotation over the whole tensor (32K tokens x 32 heads
 // of 128: 347 us).
+// The dK / dV rows of tokens that belong to no sequence, which no block holds, are written here: zeros.
 template <typename T, int D, bool EPI>
-__device__ __forceinline__ void dq_reduce_block(const T* __restrict__ dq_part, const int32_t* __restrict__ slot_of,
-                                                int64_t cap, int64_t n_tokens, int hq, int g, int topk,
-                                                T* __restrict__ dq /* contiguous [N, Hq, D] */, int64_t block,
+__device__ __forceinline__ void dq_reduce_block(const SelBwdParams& p, const T* __restrict__ dq_part,
+                                                const int32_t* __restrict__ slot_of, int64_t cap, int64_t n_tokens, int hq,
+                                                int g, int topk, T* __restrict__ dq /* contiguous [N, Hq, D] */, int64_t block,
                                                 const DqEpilogue& epi) {
   typedef typename Elem<T>::vec8 vec8;
   constexpr int LPR = D / 8, RPB = 256 / LPR;
@@ -62,6 +63,7 @@ __device__ __forceinline__ void dq_reduce_block(const T* __restrict__ dq_part, c
   const int hq_i = (int)(R - tok * hq);
   const int kh = hq_i / g, head = hq_i - kh * g;
   const int32_t* so = slot_of + ((int64_t)kh * n_tokens + tok) * topk;
+  const int seq_lo = p.cu_seqlens[0], seq_hi = p.cu_seqlens[p.batch];
   float accv[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) accv[e] = 0.f;
@@ -102,6 +104,11 @@ __device__ __forceinline__ void dq_reduce_block(const T* __restrict__ dq_part, c
 #pragma unroll
   for (int e = 0; e < 8; ++e) out[e] = (T)accv[e];
   store16_stream(dq + (tok * hq + hq_i) * D + sub * 8, out);
+  if (head == 0 && (tok < seq_lo || tok >= seq_hi)) {
+    const int64_t at = tok * p.dk_sn + kh * p.dk_sh + sub * 8;
+    store16(reinterpret_cast<T*>(p.dk) + at, zero8<T>());
+    store16(reinterpret_cast<T*>(p.dv) + at, zero8<T>());
+  }
 }
 
 // The two reductions that end the fused backward in one launch: the first n_kv work-groups add up the fp32 dK / dV
@@ -123,7 +130,7 @@ selattn_bwd_reduce_kernel(SelBwdParams p, DqReduceArgs a, int n_kv, int split, i
     const int bz = b % split, h = (b / split) % hkv, bx = b / (split * hkv);
     dkdv_reduce_block<T, D, BK, KV_MODE_SELECTED, 4>(p, bx, h, bz, split);
   } else {
-    dq_reduce_block<T, D, EPI>((const T*)a.dq_part, a.slot_of, a.cap, a.n_tokens, a.hq, a.g, a.topk, (T*)a.dq,
+    dq_reduce_block<T, D, EPI>(p, (const T*)a.dq_part, a.slot_of, a.cap, a.n_tokens, a.hq, a.g, a.topk, (T*)a.dq,
                                (int64_t)(b - n_kv), a.epi);
   }
 }
