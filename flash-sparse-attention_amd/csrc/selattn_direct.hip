@@ -51,23 +51,22 @@ __device__ __forceinline__ void lds_dma4(__amdgpu_buffer_rsrc_t rsrc, const uint
                "buffer_load_dwordx4 %3, %4, %5 offen offset:3072 lds"
                :: "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(rsrc), "s"(soff), "s"(lds) : "memory");
 }
-// The rows of the whole buffer, so that none of o and lse stays unwritten where the sequences do not fill it: segment i runs
-// from cu[i - 1] to cu[i], with the start of the buffer in front and its end behind.  Segment 0, in front of the first
-// sequence, has no keys; the last one holds the last sequence and, as queries at the positions behind it, the tokens that
-// follow it, which is where the inverted index counts them too.
-__device__ __forceinline__ int segment_begin(const int32_t* __restrict__ cu, int i) { return i > 0 ? cu[i - 1] : 0; }
-__device__ __forceinline__ int segment_end(const int32_t* __restrict__ cu, int batch, int64_t n_tokens, int i) {
-  return i < batch ? cu[i] : (int)n_tokens;
-}
-// Segment and row tile of work-group `id`; false: past the last tile.  The late tiles of a segment, which see the most
-// blocks, come first.
-__device__ __forceinline__ bool direct_tile(const int32_t* __restrict__ cu, int batch, int64_t n_tokens, int g, int id, int& s,
-                                            int& tile) {
+// A row tile.  The rows of the whole buffer are dealt out, so that none of o and lse stays unwritten where the sequences do not
+// fill it: segment i runs from cu[i - 1] to cu[i], with the start of the buffer in front and its end behind.  Segment 0, in
+// front of the first sequence, has no keys; the last one holds the last sequence and, as queries at the positions behind it,
+// the tokens that follow it, which is where the inverted index counts them too.
+struct DirectTile {
+  int q0, n_q, len;   // first token, queries and keys of its segment
+  int tile;           // of the segment
+};
+// Row tile of work-group `id`; false: past the last tile.  The late tiles of a segment, which see the most blocks, come first.
+__device__ __forceinline__ bool direct_tile(const int32_t* __restrict__ cu, int batch, int n_tokens, int g, int id, DirectTile& t) {
   const int lane = threadIdx.x & (WAVE - 1);
   for (int s0 = 0; s0 <= batch; s0 += WAVE) {
     const int si = s0 + lane;
-    const int n =
-        si <= batch ? (int)(((int64_t)(segment_end(cu, batch, n_tokens, si) - segment_begin(cu, si)) * g + DIR_ROWS - 1) / DIR_ROWS) : 0;
+    const int a = cu[min(max(si - 1, 0), batch)], b = cu[min(si, batch)];
+    const int q0 = si > 0 ? a : 0, n_q = (si < batch ? b : n_tokens) - q0;
+    const int n = si <= batch ? (int)(((int64_t)n_q * g + DIR_ROWS - 1) / DIR_ROWS) : 0;
     int inc = n;
 #pragma unroll
     for (int o = 1; o < WAVE; o <<= 1) {
@@ -77,8 +76,10 @@ __device__ __forceinline__ bool direct_tile(const int32_t* __restrict__ cu, int 
     const uint64_t m = __ballot(inc > id);
     if (m) {
       const int at = __ffsll((unsigned long long)m) - 1;
-      s = __builtin_amdgcn_readfirstlane(s0 + at);
-      tile = __builtin_amdgcn_readfirstlane(__shfl(inc, at, WAVE) - 1 - id);
+      t.q0 = __builtin_amdgcn_readlane(q0, at);
+      t.n_q = __builtin_amdgcn_readlane(n_q, at);
+      t.len = s0 + at > 0 ? __builtin_amdgcn_readlane(b - a, at) : 0;
+      t.tile = __builtin_amdgcn_readlane(inc, at) - 1 - id;
       return true;
     }
     id -= __builtin_amdgcn_readlane(inc, WAVE - 1);
@@ -102,10 +103,9 @@ selattn_direct_fwd_kernel(DirectParams p) {
   uint16_t* list = reinterpret_cast<uint16_t*>(sel + p.max_blk);   // visited blocks
 
   const int h = blockIdx.x % p.hkv;
-  int s, tile;
-  if (!direct_tile(p.cu, p.batch, p.n_tokens, p.g, blockIdx.x / p.hkv, s, tile)) return;
-  const int q0 = segment_begin(p.cu, s), len = s > 0 ? p.cu[s] - q0 : 0;   // len: keys
-  const int rows = (segment_end(p.cu, p.batch, p.n_tokens, s) - q0) * p.g, row0 = tile * DIR_ROWS;
+  DirectTile t;
+  if (!direct_tile(p.cu, p.batch, (int)p.n_tokens, p.g, blockIdx.x / p.hkv, t)) return;
+  const int q0 = t.q0, len = t.len, rows = t.n_q * p.g, row0 = t.tile * DIR_ROWS;
   const int q_first = div_group(row0, p.g, p.g_shift), q_last = div_group(min(rows, row0 + DIR_ROWS) - 1, p.g, p.g_shift);
   const int n_blk = min(q_last / BK + 1, (len + BK - 1) / BK);
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
