@@ -369,7 +369,7 @@ selattn_direct_fwd_kernel(DirectParams p) {
       mw[w] = mx == -INFINITY ? 0.f : fast_exp2(mw[w] - mx);
       sum += mw[w] * st_l[w * DIR_ROWS + r];
     }
-    const float inv = sum > 0.f ? 1.f / sum : sum != sum ? sum : 0.f;
+    const float inv = sum == 0.f ? 0.f : 1.f / sum;   // (a sum that is NaN, from a NaN in q or a key, makes the row NaN)
     float out[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) out[e] = 0.f;
@@ -402,7 +402,7 @@ selattn_direct_fwd_kernel(DirectParams p) {
       if (!p.o) continue;
     }
     store16(reinterpret_cast<T*>(p.o) + tok * p.o_sn + (int64_t)hq_i * p.o_sh + sub * 8, x);
-    if (sub == 0) p.lse[(int64_t)hq_i * p.n_tokens + tok] = sum > 0.f ? mx + log2f(sum) : -INFINITY;
+    if (sub == 0) p.lse[(int64_t)hq_i * p.n_tokens + tok] = sum == 0.f ? -INFINITY : mx + log2f(sum);
   }
 }
 

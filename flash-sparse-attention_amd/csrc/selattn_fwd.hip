@@ -279,7 +279,8 @@ selattn_fwd_main_kernel(SelFwdParams p, HeadOrder order) {
       }
     }
     __builtin_amdgcn_wave_barrier();
-    if (valid && hh == 0) __builtin_nontemporal_store(l > 0.f ? mref + log2f(l) : -INFINITY, &p.lse_part[prow]);
+    // (a sum that is NaN stays NaN)
+    if (valid && hh == 0) __builtin_nontemporal_store(l == 0.f ? -INFINITY : mref + log2f(l), &p.lse_part[prow]);
   };
 
   int sub = row_lo + wv * 32;
@@ -360,25 +361,25 @@ selattn_fwd_reduce_kernel(const T* __restrict__ o_part, const float* __restrict_
   }
 #pragma unroll
   for (int o_ = LPR / 2; o_ >= 1; o_ >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o_, LPR));
+  // A partial whose sum is NaN (a NaN in q or a selected key) makes the row and its log-sum-exp NaN; fmaxf has passed over it.
+  if (mx == -INFINITY) mx = 0.f;   // no key, or nothing but NaN
   float sum = 0.f;
-  if (mx > -INFINITY) {
 #pragma unroll
-    for (int c = 0; c < MAXC; ++c)
-      if (c < nchunk) sum += fast_exp2(lse_c[c] - mx);  // -inf -> 0
-    for (int t = MAXC * LPR + sub; t < topk; t += LPR) {
-      const int pidx = so[t];
-      if (pidx >= 0) sum += fast_exp2(lse_part[(pbase + pidx) * g + head] - mx);
-    }
+  for (int c = 0; c < MAXC; ++c)
+    if (c < nchunk) sum += fast_exp2(lse_c[c] - mx);  // -inf -> 0
+  for (int t = MAXC * LPR + sub; t < topk; t += LPR) {
+    const int pidx = so[t];
+    if (pidx >= 0) sum += fast_exp2(lse_part[(pbase + pidx) * g + head] - mx);
   }
 #pragma unroll
   for (int o_ = LPR / 2; o_ >= 1; o_ >>= 1) sum += __shfl_xor(sum, o_, LPR);
-  const float lse_tot = sum > 0.f ? mx + log2f(sum) : -INFINITY;
+  const float lse_tot = sum == 0.f ? -INFINITY : mx + log2f(sum);
 
   // weighted sum of the partial rows
   float accv[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) accv[e] = 0.f;
-  if (sum > 0.f) {
+  if (sum != 0.f) {
 #pragma unroll
     for (int c = 0; c < MAXC; ++c) {
       if (c < nchunk) {  // uniform

@@ -20,6 +20,11 @@
  * The packed varlen layout is the reference's: q[N,Hq,D], k/v[N,Hkv,D],
  * topk_idx[Hkv,N,T] int32, cu_seqlens[B+1] int32, lse[Hq,N] fp32 base 2
  * (fsa/ops/FSA_topk_sparse_attention.py:1887-1932).
+ * Selected attention: a query without a visible key has o = 0 and lse = -inf; a
+ * NaN score (from q, or from a key that the query sees) makes both NaN.  Tokens of
+ * the buffer in front of cu_seqlens[0] see no key, tokens behind cu_seqlens[B]
+ * count as queries of the last sequence at the positions behind its end; dK and
+ * dV of either are zero.
  */
 #ifndef FSA_HIP_H
 #define FSA_HIP_H
