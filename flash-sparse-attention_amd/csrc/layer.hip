@@ -331,6 +331,16 @@ kv_combine_kernel(KvCombine p) {
   store16(reinterpret_cast<T*>(p.dv_out) + at, v);
 }
 
+// `chunks` times eight 16-bit elements from an address that is aligned to one element only
+__global__ void __launch_bounds__(256) copy_aligned_kernel(const uint16_t* __restrict__ src, void* __restrict__ dst, int64_t chunks) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= chunks) return;
+  uint32_t x[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x[e] = src[8 * i + 2 * e] | (uint32_t)src[8 * i + 2 * e + 1] << 16;
+  reinterpret_cast<uint4*>(dst)[i] = make_uint4(x[0], x[1], x[2], x[3]);
+}
+
 // -------------------------------------------------------------- host side ----
 struct Bump {
   size_t at = 0;
@@ -380,7 +390,7 @@ static LayerSaved layer_saved(const fsa_layer_args& a) {
 
 // Forward workspace: the stages run one after the other and share it, beside the un-rotated compressed keys.
 struct LayerFwdWs {
-  size_t ck_raw, stage, total, topk_bytes, index_bytes, sel_bytes;
+  size_t ck_raw, stage, total, topk_bytes, index_bytes, sel_bytes, kv_bytes;
 };
 static LayerFwdWs layer_fwd_ws(const fsa_layer_args& a, const LayerSaved& s) {
   LayerFwdWs w;
@@ -391,7 +401,8 @@ static LayerFwdWs layer_fwd_ws(const fsa_layer_args& a, const LayerSaved& s) {
   w.topk_bytes = fsa_cmp_topk_workspace_bytes(a.total_tokens, a.num_kv_heads, rebin ? a.max_ck / 4 + 1 : a.max_ck);
   w.index_bytes = !s.index ? 0 : fsa_index_workspace_bytes(a.total_tokens, s.t_out, a.num_kv_heads, s.max_blocks);
   w.sel_bytes = s.direct ? 0 : fsa_selattn_fwd_workspace_bytes(a.total_tokens, a.num_q_heads, a.num_kv_heads, a.head_dim, s.t_out, s.max_blocks);
-  w.total = w.stage + align_up(std::max({w.topk_bytes, w.index_bytes, w.sel_bytes}), 256);
+  w.kv_bytes = align_up((size_t)a.total_tokens * a.num_kv_heads * a.head_dim * 2, 256);
+  w.total = w.stage + align_up(std::max({w.topk_bytes, w.index_bytes, w.sel_bytes, s.direct ? 2 * w.kv_bytes + 16 : 0}), 256);
   return w;
 }
 
@@ -521,7 +532,18 @@ static int layer_forward(const fsa_layer_args& a, void* out, int32_t* topk_idx, 
   merge.gate = sv + s.gates;
   merge.out = out;
   if (s.direct) {
-    FSA_RUN(selattn_direct_fwd(q, k, a.v, a.dtype, qs, d, ks_, d, ks_, d, topk_idx, n * s.t_out, s.t_out, a.cu_seqlens, a.batch, n,
+    // its K and V go to LDS by 16-byte loads, which want aligned rows; the other kernels do without
+    const void* kv[2] = {k, a.v};
+    char* copies = (char*)align_up((uintptr_t)(ws + w.stage), 16);
+    for (int i = 0; i < 2; ++i) {
+      if ((uintptr_t)kv[i] % 16 == 0) continue;
+      ProfScope ps_("copy_aligned", stream);
+      const int64_t chunks = n * ks_ / 8;
+      copy_aligned_kernel<<<(unsigned)((chunks + 255) / 256), 256, 0, stream>>>((const uint16_t*)kv[i], copies + i * w.kv_bytes, chunks);
+      FSA_CHECK_LAUNCH("fsa_layer copy");
+      kv[i] = copies + i * w.kv_bytes;
+    }
+    FSA_RUN(selattn_direct_fwd(q, kv[0], kv[1], a.dtype, qs, d, ks_, d, ks_, d, topk_idx, n * s.t_out, s.t_out, a.cu_seqlens, a.batch, n,
                                a.max_len, a.num_q_heads, a.num_kv_heads, a.head_dim, s.t_out, a.block_size, a.softmax_scale,
                                a.inference ? nullptr : sv + s.o[1], qs, d, a.inference ? nullptr : (float*)(sv + s.lse[1]), merge,
                                stream));
