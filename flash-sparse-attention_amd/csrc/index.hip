@@ -1148,7 +1148,7 @@ extern "C" int fsa_build_index_tiles(const int32_t* topk_idx, int64_t topk_strid
                                      int32_t* cu_blocks, int32_t* counts, int32_t* starts, int32_t* sel_tokens,
                                      int32_t* slot_of, int32_t num_q_heads, int32_t head_dim, int32_t* tiles_fwd,
                                      int32_t* tiles_bwd, void* workspace, size_t workspace_bytes, void* stream_) {
-  FSA_CHECK_ARG(tiles_fwd, "fsa_build_index_tiles: null pointer");
+  FSA_CHECK_ARG(tiles_fwd || tiles_bwd, "fsa_build_index_tiles: null pointer");
   FSA_CHECK_ARG(num_kv_heads >= 1 && num_q_heads % num_kv_heads == 0 && topk >= 1 && total_tokens >= 1 && max_blocks >= 1,
                 "fsa_build_index_tiles: bad sizes");
   const TileList la = selattn_tiles(false, total_tokens, num_q_heads, num_kv_heads, head_dim, topk, block_size, max_blocks, tiles_fwd);

@@ -382,7 +382,7 @@ static LayerSaved layer_saved(const fsa_layer_args& a) {
   s.starts = b.take(!s.index ? 0 : hkv * (s.max_blocks + 1) * 4);
   s.sel = b.take(!s.index ? 0 : hkv * n * s.t_out * 4);
   s.slot = b.take(!s.index ? 0 : hkv * n * s.t_out * 4);
-  s.tiles_fwd = b.take(!s.index ? 0 : fsa_selattn_tiles_bytes(0, n, hq, hkv, d, s.t_out, a.block_size, s.max_blocks));
+  s.tiles_fwd = b.take(s.direct ? 0 : fsa_selattn_tiles_bytes(0, n, hq, hkv, d, s.t_out, a.block_size, s.max_blocks));
   s.tiles_bwd = b.take(a.inference ? 0 : fsa_selattn_tiles_bytes(1, n, hq, hkv, d, s.t_out, a.block_size, s.max_blocks));
   s.total = b.at;
   return s;
@@ -521,7 +521,7 @@ static int layer_forward(const fsa_layer_args& a, void* out, int32_t* topk_idx, 
                        a.num_kv_heads, a.head_dim, a.kernel_size, a.kernel_stride, a.block_size, a.topk, a.init_blocks,
                        a.local_blocks, 1, 0, a.softmax_scale, topk_idx, nullptr, ws + w.stage, w.topk_bytes, stream));
   int32_t *cu_blocks = (int32_t*)(sv + s.cu_blocks), *counts = (int32_t*)(sv + s.counts), *starts = (int32_t*)(sv + s.starts),
-          *sel = (int32_t*)(sv + s.sel), *slot = (int32_t*)(sv + s.slot), *tf = (int32_t*)(sv + s.tiles_fwd), *tb = a.inference ? nullptr : (int32_t*)(sv + s.tiles_bwd);
+          *sel = (int32_t*)(sv + s.sel), *slot = (int32_t*)(sv + s.slot), *tf = s.direct ? nullptr : (int32_t*)(sv + s.tiles_fwd), *tb = a.inference ? nullptr : (int32_t*)(sv + s.tiles_bwd);
   if (s.index)
     FSA_RUN(fsa_build_index_tiles(topk_idx, n * s.t_out, s.t_out, a.cu_seqlens, a.batch, n, a.num_kv_heads, s.t_out, a.block_size,
                                 s.max_blocks, cu_blocks, counts, starts, sel, slot, a.num_q_heads, a.head_dim, tf, tb,

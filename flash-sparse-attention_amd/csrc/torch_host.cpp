@@ -177,7 +177,7 @@ Tensor split_topk_blocks(const Tensor& topk_idx, const Tensor& cu, int64_t block
 struct Index {
   Tensor cu, mem;
   int64_t n, hkv, topk, block, max_blocks, hq, d;
-  bool backward;   // the work list of the backward is there too
+  bool forward, backward;   // whose work lists are there
 
   IndexView view() const {
     const int64_t batch = cu.numel() - 1;
@@ -195,7 +195,7 @@ struct Index {
     v.starts = part(hkv * (max_blocks + 1));
     v.sel = part(hkv * n * topk);
     v.slot = part(hkv * n * topk);
-    v.tiles_fwd = part(tile_ints(false));
+    v.tiles_fwd = forward ? part(tile_ints(false)) : nullptr;
     v.tiles_bwd = backward ? part(tile_ints(true)) : nullptr;
     v.batch = batch;
     v.n = n;
@@ -211,8 +211,8 @@ struct Index {
   }
   int64_t total_ints() const {
     auto r = [](int64_t x) { return (x + 63) / 64 * 64; };
-    return r(cu.numel()) + r(hkv * max_blocks) + r(hkv * (max_blocks + 1)) + 2 * r(hkv * n * topk) + r(tile_ints(false)) +
-           (backward ? r(tile_ints(true)) : 0);
+    return r(cu.numel()) + r(hkv * max_blocks) + r(hkv * (max_blocks + 1)) + 2 * r(hkv * n * topk) +
+           (forward ? r(tile_ints(false)) : 0) + (backward ? r(tile_ints(true)) : 0);
   }
 };
 
@@ -223,7 +223,7 @@ Tensor kernel_blocks(const Tensor& topk_idx, const Tensor& cu, int64_t& block) {
   block = 128;
   return split_topk_blocks(topk_idx, cu, 256, 2);
 }
-Index kernel_index(const Tensor& topk_idx, const Tensor& cu, int64_t block, int64_t hq, int64_t d, bool backward) {
+Index kernel_index(const Tensor& topk_idx, const Tensor& cu, int64_t block, int64_t hq, int64_t d, bool forward, bool backward) {
   Index x;
   x.cu = cu;
   x.hkv = topk_idx.size(0);
@@ -233,6 +233,7 @@ Index kernel_index(const Tensor& topk_idx, const Tensor& cu, int64_t block, int6
   x.max_blocks = (x.n + block - 1) / block + cu.numel() - 1;
   x.hq = hq;
   x.d = d;
+  x.forward = forward;
   x.backward = backward;
   const c10::OptionalDeviceGuard guard(topk_idx.device());
   x.mem = empty_i32({x.total_ints()}, topk_idx);
@@ -343,6 +344,19 @@ std::pair<Tensor, Tensor> selattn_fwd(const Tensor& q, const Tensor& k, const Te
   return {resize_d(o, d), lse};
 }
 
+// The same from the lists alone, for callers that keep no index: (o, lse) of the forward that training takes
+std::pair<Tensor, Tensor> selattn_fwd_lists(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& topk_idx, int64_t block,
+                                            const Tensor& cu, optional<double> scale_) {
+  check_qkv(q, k, v);
+  const int64_t d = q.size(2), dn = native_dim(d);
+  const double scale = default_scale(scale_, d);
+  const Tensor ids = kernel_blocks(topk_idx, cu, block), qn = resize_d(q, dn), kn = resize_d(k, dn), vn = resize_d(v, dn);
+  auto [o, lse] = direct(qn, kn, vn, ids, block, true)
+                      ? selattn_direct(qn, kn, vn, ids, cu, block, scale)
+                      : selattn_fwd_native(qn, kn, vn, kernel_index(ids, cu, block, q.size(1), dn, true, false).view(), scale);
+  return {resize_d(o, d), lse};
+}
+
 void check_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& d_o, const Tensor& lse) {
   check_qkv(q, k, v);
   need_device(o, d_o, lse);
@@ -369,12 +383,12 @@ struct SelectedAttention : torch::autograd::Function<SelectedAttention> {
                         const Tensor& topk_idx, int64_t block, const Tensor& cu, double scale) {
     const int64_t d = q.size(2), dn = native_dim(d);
     const Tensor ids = kernel_blocks(topk_idx, cu, block);
-    const Index x = kernel_index(ids, cu, block, q.size(1), dn, true);
     const Tensor qn = resize_d(q, dn), kn = resize_d(k, dn), vn = resize_d(v, dn);
-    auto [on, lse] = direct(qn, kn, vn, ids, block, true) ? selattn_direct(qn, kn, vn, ids, cu, block, scale)
-                                                          : selattn_fwd_native(qn, kn, vn, x.view(), scale);
+    const bool from_lists = direct(qn, kn, vn, ids, block, true);
+    const Index x = kernel_index(ids, cu, block, q.size(1), dn, !from_lists, true);
+    auto [on, lse] = from_lists ? selattn_direct(qn, kn, vn, ids, cu, block, scale) : selattn_fwd_native(qn, kn, vn, x.view(), scale);
     ctx->save_for_backward({qn, kn, vn, on, lse, x.cu, x.mem});
-    ctx->saved_data["ints"] = std::vector<int64_t>{d, x.n, x.hkv, x.topk, x.block, x.max_blocks, x.hq, x.d};
+    ctx->saved_data["ints"] = std::vector<int64_t>{d, x.n, x.hkv, x.topk, x.block, x.max_blocks, x.hq, x.d, x.forward};
     ctx->saved_data["scale"] = scale;
     return resize_d(on, d);
   }
@@ -383,7 +397,7 @@ struct SelectedAttention : torch::autograd::Function<SelectedAttention> {
     const auto s = ctx->get_saved_variables();
     const auto ints = ctx->saved_data["ints"].toIntVector();
     const Tensor d_o = resize_d(grads[0], s[0].size(2));
-    const Index x{s[5], s[6], ints[1], ints[2], ints[3], ints[4], ints[5], ints[6], ints[7], true};
+    const Index x{s[5], s[6], ints[1], ints[2], ints[3], ints[4], ints[5], ints[6], ints[7], ints[8] != 0, true};
     auto [dq, dk, dv] =
         selattn_bwd_native(s[0], s[1], s[2], s[3], d_o, s[4], x.view(), ctx->saved_data["scale"].toDouble());
     return {resize_d(dq, ints[0]), resize_d(dk, ints[0]), resize_d(dv, ints[0]), Tensor(), Tensor(), Tensor(), Tensor()};
@@ -402,7 +416,7 @@ Tensor selected_attention(const Tensor& q, const Tensor& k, const Tensor& v, con
   const int64_t d = q.size(2), dn = native_dim(d);
   const Tensor ids = kernel_blocks(topk_idx, cu, block), qn = resize_d(q, dn), kn = resize_d(k, dn), vn = resize_d(v, dn);
   if (direct(qn, kn, vn, ids, block, false)) return resize_d(selattn_direct(qn, kn, vn, ids, cu, block, scale).first, d);
-  const Index x = kernel_index(ids, cu, block, q.size(1), dn, false);
+  const Index x = kernel_index(ids, cu, block, q.size(1), dn, true, false);
   return resize_d(selattn_fwd_native(qn, kn, vn, x.view(), scale).first, d);
 }
 
@@ -915,6 +929,7 @@ PYBIND11_MODULE(_native, m) {
   m.def("build_index", &build_index);
   m.def("split_topk_blocks", &split_topk_blocks);
   m.def("selattn_fwd", &selattn_fwd);
+  m.def("selattn_fwd_lists", &selattn_fwd_lists);
   m.def("selattn_bwd", &selattn_bwd);
   m.def("selected_attention", &selected_attention);
   m.def("decode_cmpattn", &decode_cmpattn);

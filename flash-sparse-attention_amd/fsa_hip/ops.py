@@ -124,6 +124,11 @@ def selattn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, index: SelInd
     return _native.selattn_fwd(q, k, v, index.arrays(), index.topk, index.block_size, index.max_blocks, softmax_scale, lists)
 
 
+def selattn_fwd_lists(q, k, v, topk_idx, block_size, cu_seqlens, softmax_scale: Optional[float] = None):
+    """The same without an index: one is built only where the kernels that run need it."""
+    return _native.selattn_fwd_lists(q, k, v, topk_idx, block_size, cu_seqlens, softmax_scale)
+
+
 def selattn_bwd(q, k, v, o, do, lse, index: SelIndex, softmax_scale: Optional[float] = None):
     """Selected attention backward: returns (dq, dk, dv) in the input dtype."""
     return _native.selattn_bwd(q, k, v, o, do, lse, index.arrays(), index.topk, index.block_size, index.max_blocks,

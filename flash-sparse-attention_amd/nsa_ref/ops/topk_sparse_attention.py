@@ -19,7 +19,7 @@ from typing import Any, Optional
 
 import torch
 
-from fsa.ops.FSA_topk_sparse_attention import _BLOCK_SIZES, _build_kernel_index, _forward
+from fsa.ops.FSA_topk_sparse_attention import _BLOCK_SIZES, _build_kernel_index
 from fsa_hip import ops as _ops
 
 
@@ -40,7 +40,7 @@ def _topk_sparse_attention_fwd(
     assert cu_seqlens_q.dtype == torch.int32 and cu_seqlens_k.dtype == torch.int32
     assert block_size in _BLOCK_SIZES
     assert q.shape[1] % k.shape[1] == 0
-    return _forward(q, k, v, topk_idx, cu_seqlens_q, block_size, sm_scale)[:2]
+    return _ops.selattn_fwd_lists(q, k, v, topk_idx, block_size, cu_seqlens_q, sm_scale)
 
 
 def _topk_sparse_attention_bwd(

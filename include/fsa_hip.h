@@ -110,9 +110,9 @@ int fsa_build_index(const int32_t* topk_idx, int64_t topk_stride_h, int64_t topk
                     int32_t* cu_blocks, int32_t* counts, int32_t* starts, int32_t* sel_tokens,
                     int32_t* slot_of, void* workspace, size_t workspace_bytes, void* stream);
 
-/* The same together with the work lists of the forward (tiles_fwd) and, where
- * tiles_bwd is not null, the backward main kernel of selected attention with
- * num_q_heads heads of head_dim dims, for fsa_selattn_fwd_tiles /
+/* The same together with the work lists of the main kernels of selected attention
+ * with num_q_heads heads of head_dim dims, forward (tiles_fwd) and backward
+ * (tiles_bwd), one of which may be null, for fsa_selattn_fwd_tiles /
  * fsa_selattn_bwd_tiles: two launches fewer than letting those build them.
  * A work list has fsa_selattn_tiles_bytes bytes. */
 int fsa_build_index_tiles(const int32_t* topk_idx, int64_t topk_stride_h, int64_t topk_stride_n,
