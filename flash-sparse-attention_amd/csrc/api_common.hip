@@ -84,7 +84,8 @@ pad_head_dim_kernel(const uint16_t* __restrict__ src, int64_t src_sn, int64_t sr
 
 // 200: fsa_decode_topk gained scores_to_bf16 and fsa_decode_selattn gained seqlens (both inside their argument
 // lists); 210: fsa_cmp_topk gained score_head_as_written, fsa_native_head_dim / fsa_pad_head_dim added; 220:
-// fsa_linear_compress_fwd wants pe 16-byte aligned, work-list, layer and matrix-product entry points added.
+// fsa_linear_compress_fwd wants pe 16-byte aligned, work-list, layer and matrix-product entry points added; 230:
+// fsa_selattn_direct_* added, fsa_build_index_tiles takes one list, other sizes of the layer's buffers.
 extern "C" int fsa_version(void) { return FSA_HIP_VERSION; }
 
 extern "C" int fsa_native_head_dim(int32_t head_dim) {

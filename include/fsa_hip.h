@@ -51,8 +51,12 @@ extern "C" {
  *   220: no list, but fsa_linear_compress_fwd wants pe 16-byte aligned and no longer
  *        uses bias_scratch; fsa_build_index_tiles, fsa_selattn_tiles_bytes,
  *        fsa_selattn_fwd_tiles, fsa_selattn_bwd_tiles, fsa_decode_layer_*,
- *        fsa_layer_* and fsa_matmul are new. */
-#define FSA_HIP_VERSION 220
+ *        fsa_layer_* and fsa_matmul are new;
+ *   230: no list; fsa_selattn_direct_preferred and fsa_selattn_direct_fwd are new,
+ *        fsa_build_index_tiles takes one work list alone, rows of no sequence and
+ *        NaN scores are defined (above), fsa_layer_saved_bytes and
+ *        fsa_layer_workspace_bytes answer with other sizes. */
+#define FSA_HIP_VERSION 230
 int fsa_version(void);
 /* Human-readable description of the last error on the calling thread. */
 const char* fsa_last_error(void);
@@ -192,8 +196,9 @@ int fsa_selattn_fwd_tiles(const void* q, const void* k, const void* v, int32_t d
                           void* workspace, size_t workspace_bytes, void* stream);
 
 /* The same result from the block lists alone, without index and workspace: one query-major launch that visits, for every 32
- * rows, the union of the blocks they selected.  For short sequences: max_len (any upper bound of the longest sequence) is at
- * most 1024 blocks, rows of k and v do not overlap and start at multiples of 16 bytes.  A block that a list names several times counts as often, as above.
+ * rows, the union of the blocks they selected.  For short sequences: max_len, an upper bound of the longest sequence that is
+ * no larger than total_tokens, is at most 1024 blocks; rows of k and v do not overlap and start at multiples of 16 bytes; the
+ * rows of one kv head span less than 2^31 bytes.  A block that a list names several times counts as often, as above.
  * fsa_selattn_direct_preferred: 1 where this is the faster one of the two, else 0 (below 0: bad sizes); index_needed: the
  * index is built in any case, for the backward. */
 int fsa_selattn_direct_preferred(int64_t total_tokens, int64_t max_len, int32_t num_q_heads, int32_t head_dim,
@@ -530,8 +535,8 @@ int fsa_gate_merge_bwd(const void* d_out, const void* a, const void* b, const vo
  * gated sum.  q [N,Hq,D], k / v [N,Hkv,D] are the un-rotated projections of
  * x [N, hidden], all tensors contiguous, head_dim one of 64 / 128 / 256,
  * block_size 32 / 64 / 128.  max_len / max_ck / total_ck are upper bounds (longest
- * sequence, longest compressed sequence, compressed rows in all), at least one
- * compressed row must fit.  `saved` is written by the forward and read by the
+ * sequence, no more than total_tokens; longest compressed sequence; compressed
+ * rows in all), at least one compressed row must fit.  `saved` is written by the forward and read by the
  * backward of the same arguments; with `inference` set no backward may follow.
  *   forward:  out [N, Hq*D]; topk_idx [Hkv, N, min(topk, ceil(max_len / block_size))]
  *   backward: from d_out the gradients of q, k, v, of the parameters, and the
