@@ -190,7 +190,12 @@ __device__ __forceinline__ void attn_fwd_tile(const CmpParams& p, int id) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
 
-  constexpr int KAHEAD = 2, VAHEAD = 3;
+  // K and V fragments that are requested ahead of their products.  At head_dim 64 the registers for them would take the
+  // compressed branch on its own from three waves per SIMD to two (168 -> 178 registers; 32 + 8 heads, ahead / not: 5003
+  // tokens 21.6 / 20.1 us, 16384 109 / 98; window 118.1 / 118.7, both branches in one launch 214.5 / 214.5).  At head_dim 256
+  // (8 + 2 heads) ahead is 8 % faster in the window and 5 % at 16384 tokens of the compressed branch (130 / 138 us), but 5 %
+  // slower at 5003 (26.1 / 24.9).
+  constexpr int KAHEAD = D == 64 ? 0 : 2, VAHEAD = D == 64 ? 0 : 3;
   constexpr bool PREFETCH = D <= 128;  // the next tile waits in registers where the budget allows
   KvTileRegs<T, D> nxt;
   if (PREFETCH && jt0 < n_keys) kv_tile_load<T, D>(nxt, kbase, p.k_sn, k_off, vbase, p.v_sn, v_off, k0 + jt0, nc - jt0, tid);
@@ -210,8 +215,8 @@ __device__ __forceinline__ void attn_fwd_tile(const CmpParams& p, int id) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[a][i] = 0.f;
     // Fragments are requested KAHEAD k-steps before their products, and in this order: left to itself the compiler asks for
-    // them right before, and the wave waits for LDS at every pair of products (5003 tokens, 32 + 8 heads: 111 -> 107 us for
-    // both branches).
+    // them right before, and the wave waits for LDS at every pair of products (5003 tokens, 32 + 8 heads of 128: 111 -> 107 us
+    // for both branches).
     vec8 kf[KAHEAD + 1][NA];
     auto k_read = [&](int ks) {
 #pragma unroll
@@ -224,7 +229,7 @@ __device__ __forceinline__ void attn_fwd_tile(const CmpParams& p, int id) {
       if (ks + KAHEAD < NKS) k_read(ks + KAHEAD);
 #pragma unroll
       for (int a = 0; a < NA; ++a) acc[a] = Elem<T>::mfma32(kf[ks % (KAHEAD + 1)][a], qreg[ks], acc[a]);
-      __builtin_amdgcn_sched_barrier(0);
+      if (KAHEAD > 0) __builtin_amdgcn_sched_barrier(0);
     }
     vec8 vf[VAHEAD + 1];
     auto v_read = [&](int i) { vf[i % (VAHEAD + 1)] = lds_read_tr8<T>(vtr + 16 * (i / NDT) * VS + i % NDT * 32, 8 * VS); };
@@ -276,7 +281,7 @@ __device__ __forceinline__ void attn_fwd_tile(const CmpParams& p, int id) {
     for (int i = 0; i < NJ * NDT; ++i) {
       if (i + VAHEAD < NJ * NDT) v_read(i + VAHEAD);
       oacc[i % NDT] = Elem<T>::mfma32(vf[i % (VAHEAD + 1)], pk[i / NDT], oacc[i % NDT]);
-      __builtin_amdgcn_sched_barrier(0);
+      if (VAHEAD > 0) __builtin_amdgcn_sched_barrier(0);
     }
   }
   l = sum32(l);
