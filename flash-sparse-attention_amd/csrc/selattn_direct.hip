@@ -169,7 +169,8 @@ selattn_direct_fwd_kernel(DirectParams p) {
     id[i] = ids[qo[i] * p.i_sn + (e - qo[i] * p.topk)];
   }
   // The first keys of every wave are requested before it is known which blocks are visited: the first blocks of the
-  // sequence, as where the union of the lists has no gap at its start.  4096 tokens x 4 heads 40.5 -> 39.3 us.
+  // sequence, as where the union of the lists has no gap at its start.  4096 tokens x 4 heads 40.5 -> 39.3 us.  (The
+  // compiler's waits for id[] below do not count these loads, which are younger, and so wait for most of them as well.)
   int guess = wv / UPB * BK + wv % UPB * 32;
   if (guess + 32 <= len) {
     issue_k(guess);
@@ -228,6 +229,8 @@ selattn_direct_fwd_kernel(DirectParams p) {
   f32x16 oacc[NDT];
   // CAREFUL: a block that a query did not select must not reach it at all (a key or value of it that is infinite or NaN makes
   // 0 * x NaN in the products), and a block that a list names several times counts as often.
+  // At head_dim 128 this pass is 16 registers short: it puts them into scratch (68 bytes) in front of its loop, which the other
+  // pass does not touch.
   auto attend = [&](auto careful_, int loaded) {   // loaded: the key of the tiles that are in LDS or on their way there, or -1
     constexpr bool CAREFUL = decltype(careful_)::value;
     m = -INFINITY;
@@ -243,10 +246,14 @@ selattn_direct_fwd_kernel(DirectParams p) {
       issue_k(cur.key);
       issue_v(cur.key);
     }
+    // The counts of vm_wait leave the tile that was requested last on its way, and at head_dim 64 that is what runs.  At 128
+    // and 256 the compiler settles qreg, ordinary loads whose first use is in this loop, by waits of its own between the
+    // products of S: they run in every step, down to no operation outstanding, so that K of the next step and V of this one
+    // are awaited there in full and a step takes the latency of a tile (about 1 us at head_dim 128).
     for (int t = 0;; ++t) {
       const bool more = t + 1 < n_steps;
       const Unit nxt = unit(more ? t + 1 : t);
-      vm_wait<NLD>();   // K of this step (its V may still be on the way)
+      vm_wait<NLD>();   // K of this step, not its V
       vec8 kf[NKS];
 #pragma unroll
       for (int ks = 0; ks < NKS; ++ks) kf[ks] = k_frag(ks);
@@ -307,7 +314,7 @@ selattn_direct_fwd_kernel(DirectParams p) {
         pk[i >> 3][i & 7] = (T)pv;
       }
       l += sum;   // the lane's own keys: the two lanes of a row are added behind the loop
-      if (more) vm_wait<NLD>();   // V of this step (K of the next may still be on the way)
+      if (more) vm_wait<NLD>();   // V of this step, not K of the next (but see above)
       else vm_wait<0>();
 #pragma unroll
       for (int j = 0; j < 2; ++j)

@@ -169,7 +169,10 @@ selattn_fwd_main_kernel(SelFwdParams p, HeadOrder order) {
   };
   // one sub-tile: rows sub.. of the block (direct mode: tok_next = token ids of the next sub-tile)
   // staged mode: `qbuf` holds the rows of this sub-tile on entry and, once they are parked in LDS, takes the rows
-  // of the sub-tile after the next (token ids tok_next): the gathers of two sub-tiles are in flight at a time
+  // of the sub-tile after the next (token ids tok_next).  The gathers are requested two sub-tiles ahead; how long they stay
+  // in flight is up to the compiler's waits: gathers, token loads and row stores stand behind branches, so where the rows of
+  // an even sub-tile are parked it assumes that nothing younger was issued and counts 7 ... 0, which also waits for the odd
+  // sub-tile's gathers and the last row stores.  The memory queue is empty once per two sub-tiles.
   auto step = [&](vec8 (&qbuf)[NLD], int token, int sub, int tok_next) {
     const int r = sub + col;
     const bool valid = r < row_hi;

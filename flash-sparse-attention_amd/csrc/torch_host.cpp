@@ -278,7 +278,9 @@ std::pair<Tensor, Tensor> selattn_fwd_native(const Tensor& q, const Tensor& k, c
   return {o, lse};
 }
 
-// Short sequences: from the block lists (kernel_blocks), without an index
+// Short sequences: from the block lists (kernel_blocks), without an index.  The lengths are on the device and are not read
+// back, so that a packed batch is priced as one sequence as long as all of it: eight documents of 1000 tokens take the
+// block-major kernels although each of them is short.
 bool direct(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& topk_idx, int64_t block, bool index_needed) {
   const int64_t n = q.size(0), d = q.size(2);
   auto rows_ok = [&](const Tensor& t) {   // they go to LDS by 16-byte buffer loads
