@@ -458,7 +458,8 @@ template <typename T, bool MERGE> static int dispatch_direct_fwd(int d, int bk, 
 //   5000 x 32 (GQA 4) 283 / 267 / 284; 6000 x 4 79 / 59 / 78, x 32 (GQA 4) 339 / 354; 7000 x 4 83 / 77; 8192 x 4 100 / 100, x 32
 //   505 / 711; 16384 x 4 (GQA 4) 167 / 211
 // head_dim 256, lists of 8: 3000 x 4 64 / 47 / 59, 4096 x 4 85 / 74 / 86, 6000 x 8 164 / 175; 64: 4500 x 8 46 / 35 / 46, 8000 x 8
-// (16 blocks) 93 / 94.
+// (16 blocks) 93 / 94.  All of them, and the waves per work-group above, with the kernel's loads drained in every step (see the
+// loop): a step that takes less moves the line towards longer sequences.
 bool selattn_direct_preferred(int64_t n, int64_t max_len, int hq, int d, int topk, int bk, bool index_needed) {
   if (!(d == 64 || d == 128 || d == 256) || !(bk == 32 || bk == 64 || bk == 128) || topk > 4096 ||
       max_len > (int64_t)bk * DIR_MAX_BLOCKS)

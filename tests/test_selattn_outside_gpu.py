@@ -25,6 +25,7 @@ CASES = [
     ([0, 65, 640], 1000, 2, 2, 256, 64, 8, torch.bfloat16),      # the end is at the edge of a block
     ([0, 10], 500, 2, 1, 64, 128, 3, torch.bfloat16),            # positions behind the end that see the whole last block
     ([33, 33], 90, 2, 1, 128, 64, 2, torch.bfloat16),            # no token in a sequence
+    ([3 + 5 * i for i in range(101)], 520, 2, 2, 64, 32, 2, torch.float16),   # more sequences than a wave has lanes
 ]
 
 
