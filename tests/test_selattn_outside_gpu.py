@@ -79,3 +79,40 @@ def test_rows_of_no_sequence(dev, cu, n, hq, hkv, d, block, topk, dtype, lists):
     for a, b in zip(got, want):
         _close(a, b, O_TOL[dtype], ULP[dtype])
     assert all((t[outside] == 0).all() for t in got[1:])
+
+
+def test_recorded_step_with_lengths_on_the_device(dev):
+    """A step recorded for the whole buffer and replayed on shorter sequences, which only the device knows: every replay equals
+    the eager step on those lengths, whatever the outputs held before."""
+    n, hq, hkv, d, block, topk, dtype = 600, 4, 2, 128, 64, 4, torch.bfloat16
+    q, k, v, do = (x.to(dev) for x in make_qkv(n, hq, hkv, d, dtype, seed=3))
+    cut = torch.tensor([0, 250, n], dtype=torch.int32, device=dev)
+    idx = make_topk_idx([0, 250, n], hkv, block, topk, seed=4).to(dev)
+
+    def step():
+        index = ops.build_index(idx, cut, block)
+        o, lse = ops.selattn_fwd(q, k, v, index, None, idx)
+        return o, lse, *ops.selattn_bwd(q, k, v, o, do, lse, index)
+
+    assert _lib.load().fsa_selattn_direct_preferred(n, n, hq, d, topk, block, 1) == 1
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    with torch.cuda.graph(graph):
+        out = step()
+    for rep, cu in enumerate(([0, 100, 500], [0, 33, 64], [40, 300, 590], [0, 250, n])):
+        print(f"replay {rep} {cu}", flush=True)
+        cut.copy_(torch.tensor(cu, dtype=torch.int32))
+        idx.fill_(-1)
+        idx[:, cu[0]:cu[-1]] = make_topk_idx([c - cu[0] for c in cu], hkv, block, topk, seed=5 + rep).to(dev)
+        for t in out:
+            t.fill_(math.nan)
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [t.clone() for t in out]
+        want = step()
+        torch.cuda.synchronize()
+        for name, a, b in zip(("o", "lse", "dq", "dk", "dv"), got, want):
+            assert torch.equal(a, b) and not torch.isnan(a).any(), f"replay {rep}: {name}"
