@@ -193,8 +193,11 @@ __device__ __forceinline__ void attn_fwd_tile(const CmpParams& p, int id) {
   // K and V fragments that are requested ahead of their products.  At head_dim 64 the registers for them would take the
   // compressed branch on its own from three waves per SIMD to two (168 -> 178 registers; 32 + 8 heads, ahead / not: 5003
   // tokens 21.6 / 20.1 us, 16384 109 / 98; window 118.1 / 118.7, both branches in one launch 214.5 / 214.5).  At head_dim 256
-  // (8 + 2 heads) ahead is 8 % faster in the window and 5 % at 16384 tokens of the compressed branch (130 / 138 us), but 5 %
-  // slower at 5003 (26.1 / 24.9).
+  // (8 + 2 heads) ahead is 9-10 % faster in the window (5003 tokens 68.2 / 75.9 us) and 5-9 % for both branches in one launch;
+  // the compressed branch on its own is 6 % faster at 16384 tokens (129 / 138), 2-3 % slower at 2000 and 5003 (26.3 / 25.7): of
+  // the other form the compiler peels the first tile.  That is why the first tile skips the rescaling below, without which it
+  // is 5 % slower there (27.1).  At head_dim 64 that skip would let the window run three waves per SIMD (5003 tokens x 32
+  // heads, both branches 66 -> 59 us, but 2000 tokens 28.6 -> 30.7).
   constexpr int KAHEAD = D == 64 ? 0 : 2, VAHEAD = D == 64 ? 0 : 3;
   constexpr bool PREFETCH = D <= 128;  // the next tile waits in registers where the budget allows
   KvTileRegs<T, D> nxt;
@@ -255,7 +258,9 @@ __device__ __forceinline__ void attn_fwd_tile(const CmpParams& p, int id) {
     // The reference maximum m moves only when some row of the wave outgrows it by more than 2^8: until then
     // the probabilities are taken relative to the older, smaller maximum (at most 256, exact in the final
     // quotient) and the accumulators need no rescaling.  (-inf) - (-inf) is NaN and compares false.
-    if (__any((mx - m) * p.scale_log2 > 8.f)) {
+    if (D == 256 && jt == jt0) {
+      m = mx;   // nothing to rescale yet
+    } else if (__any((mx - m) * p.scale_log2 > 8.f)) {
       // m = -inf -> 0; a row that keeps its maximum -> 1; a row that has seen no key yet has nothing to rescale
       const float alpha = mx == -INFINITY ? 1.f : exp2f((m - mx) * p.scale_log2);
       l *= alpha;
