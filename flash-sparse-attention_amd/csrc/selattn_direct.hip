@@ -4,9 +4,12 @@
 // may see, and a query-major kernel that visits the union of their blocks does little more arithmetic than the block-major
 // pair (selattn_fwd_main / _reduce) while it reads q once and writes o once.
 //
-// A work-group takes 32 rows; its KG waves share out the visited keys, 32 at a time, each with all 32 rows and K / V buffers of
-// its own that it fills by itself (buffer loads straight into LDS), so there is no barrier between the first step and the merge
-// of the partial results in LDS.
+// Two kernels.  What a wave does in a step is the same in both: 32 rows against 32 keys, K and V from LDS tiles that buffer loads
+// fill past the registers.
+//
+//   narrow  few row tiles: a work-group takes one, its KG waves share out the visited keys, each with K / V buffers of its own,
+//           so there is no barrier between the first step and the merge of the partial results in LDS.
+//   wide    many row tiles: a work-group takes RT of them, whose waves go through the keys together and share every tile.
 #include "fsa_common.h"
 
 #include <algorithm>
@@ -22,6 +25,7 @@ struct DirectParams {
   int64_t i_sh, i_sn;
   const int32_t* cu;
   int batch, hkv, g, g_shift, topk, max_blk;   // max_blk: blocks of the longest sequence the tables hold
+  int bk_shift;                                // log2 of the block size
   int64_t n_tokens;
   float scale_log2;
   void* o;
@@ -29,27 +33,17 @@ struct DirectParams {
   MergeEpilogue merge;
 };
 
-
-constexpr int DIR_ROWS = 32;         // rows per work-group
 constexpr int DIR_MAX_BLOCKS = 1024; // of a sequence: size of the tables in LDS
-constexpr uint32_t DIR_BUFFER = 1u << 31;  // bytes of the K / V buffer descriptors (host: a head's rows span less)
 
-template <int D, int KG> struct DirectLds {
-  static constexpr int TILE = 32 * D * 2;                   // 32 K or V rows, bytes
-  static constexpr int WAVE_BYTES = 2 * TILE;               // K and V of a wave; at the end its fp32 partial [32][D]
-  static constexpr int STATS = 2 * KG * DIR_ROWS * 4;       // (m, l) of every wave
-  static constexpr int bytes(int max_blk) { return KG * WAVE_BYTES + STATS + 16 + 6 * max_blk; }
-};
-
-// Four KB of a tile, global memory to LDS: lane l's 16 bytes at voff[j](l) + soff + 1024 j of the buffer land at LDS byte
+// Four KB of a tile, global memory to LDS: lane l's 16 bytes at voff[j](l) + 1024 j of the buffer land at LDS byte
 // `lds` + 1024 j + 16 l (the instruction's offset moves both addresses).
-__device__ __forceinline__ void lds_dma4(__amdgpu_buffer_rsrc_t rsrc, const uint32_t* voff, uint32_t soff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %6\n\ts_nop 0\n\t"
-               "buffer_load_dwordx4 %0, %4, %5 offen lds\n\t"
-               "buffer_load_dwordx4 %1, %4, %5 offen offset:1024 lds\n\t"
-               "buffer_load_dwordx4 %2, %4, %5 offen offset:2048 lds\n\t"
-               "buffer_load_dwordx4 %3, %4, %5 offen offset:3072 lds"
-               :: "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(rsrc), "s"(soff), "s"(lds) : "memory");
+__device__ __forceinline__ void lds_dma4(__amdgpu_buffer_rsrc_t rsrc, const uint32_t* voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %5\n\ts_nop 0\n\t"
+               "buffer_load_dwordx4 %0, %4, 0 offen lds\n\t"
+               "buffer_load_dwordx4 %1, %4, 0 offen offset:1024 lds\n\t"
+               "buffer_load_dwordx4 %2, %4, 0 offen offset:2048 lds\n\t"
+               "buffer_load_dwordx4 %3, %4, 0 offen offset:3072 lds"
+               :: "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(rsrc), "s"(lds) : "memory");
 }
 // A row tile.  The rows of the whole buffer are dealt out, so that none of o and lse stays unwritten where the sequences do not
 // fill it: segment i runs from cu[i - 1] to cu[i], with the start of the buffer in front and its end behind.  Segment 0, in
@@ -59,14 +53,16 @@ struct DirectTile {
   int q0, n_q, len;   // first token, queries and keys of its segment
   int tile;           // of the segment
 };
-// Row tile of work-group `id`; false: past the last tile.  The late tiles of a segment, which see the most blocks, come first.
-__device__ __forceinline__ bool direct_tile(const int32_t* __restrict__ cu, int batch, int n_tokens, int g, int id, DirectTile& t) {
+// Row tile of work-group `id`, `per_tile` rows each; false: past the last one.  The late tiles of a segment, which see the most
+// blocks, come first.
+__device__ __forceinline__ bool direct_tile(const int32_t* __restrict__ cu, int batch, int n_tokens, int g, int per_tile, int id,
+                                            DirectTile& t) {
   const int lane = threadIdx.x & (WAVE - 1);
   for (int s0 = 0; s0 <= batch; s0 += WAVE) {
     const int si = s0 + lane;
     const int a = cu[min(max(si - 1, 0), batch)], b = cu[min(si, batch)];
     const int q0 = si > 0 ? a : 0, n_q = (si < batch ? b : n_tokens) - q0;
-    const int n = si <= batch ? (int)(((int64_t)n_q * g + DIR_ROWS - 1) / DIR_ROWS) : 0;
+    const int n = si <= batch ? (int)(((int64_t)n_q * g + per_tile - 1) / per_tile) : 0;
     int inc = n;
 #pragma unroll
     for (int o = 1; o < WAVE; o <<= 1) {
@@ -87,76 +83,279 @@ __device__ __forceinline__ bool direct_tile(const int32_t* __restrict__ cu, int 
   return false;
 }
 
-template <typename T, int D, int BK, int KG, bool MERGE>
-__global__ void __launch_bounds__(64 * KG, D <= 128 ? 2 : 1)
-selattn_direct_fwd_kernel(DirectParams p) {
+// Tiles of 32 K or V rows of a sequence and kv head on their way to LDS.
+template <typename T, int D> struct DirectLoads {
+  static constexpr int CPR = D / 8, RPI = 64 / CPR, N = 32 / RPI;   // 16-byte chunks per row, rows per load, loads per tile
+  static constexpr int NV = RPI >= 4 ? 4 : 16 / RPI;   // lane offsets: 16 rows or more, after which chunk_swizzle repeats itself
+  static constexpr int BYTES = 32 * D * 2;
+  const char* base;
+  uint32_t row_bytes, voff[NV];   // (host: a head's rows span < 2^31 bytes)
+  int len;
+  __device__ __forceinline__ DirectLoads(const void* x, int64_t sn, int64_t sh, int q0, int h, int len_) : len(len_) {
+    base = reinterpret_cast<const char*>(reinterpret_cast<const T*>(x) + (int64_t)q0 * sn + (int64_t)h * sh);
+    row_bytes = (uint32_t)sn * 2;
+    const int lane = threadIdx.x & 63, ld_row = lane / CPR, ld_chunk = lane % CPR;
+    // The loading lane picks its source so that the chunks land where chunk_swizzle wants them.  (host: rows are at least 2 D
+    // bytes apart, so the difference is not negative)
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int r = j * RPI + ld_row;
+      voff[j] = r * row_bytes + (ld_chunk ^ chunk_swizzle<D>(r)) * 16 - (j & 3) * 1024;
+    }
+  }
+  // PARTS > 1: one of as many equal shares of the loads.  Rows behind the end of the sequence are out of the range of the
+  // descriptors and arrive as zeros: no query of the sequence sees them; one at a position behind it does, with score 0, as in
+  // the block-major kernels.
+  template <int PARTS = 1> __device__ __forceinline__ void issue(int key, uint32_t to, int part = 0) const {
+    static_assert(N / PARTS >= NV, "a share has whole descriptors");
+#pragma unroll
+    for (int i = 0; i < N / PARTS; i += NV) {
+      const int j0 = part * (N / PARTS) + i, first = key + j0 * RPI;
+      const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<char*>(base + (uint64_t)(uint32_t)first * row_bytes), 0, (int)((uint32_t)max(len - first, 0) * row_bytes), 0x00020000);
+#pragma unroll
+      for (int j = 0; j < NV; j += 4) lds_dma4(rsrc, &voff[j], to + (j0 + j) * 1024);
+    }
+  }
+};
+
+// Fragments of the tiles, relative to a tile's start: k-step ks of K at k ^ 16 ks, 32 dims from 32 dt of V at v ^ 64 dt.
+template <int D> struct DirectFrags {
+  uint32_t k, v;
+  __device__ __forceinline__ DirectFrags() {
+    const int lane = threadIdx.x & 63, col = lane & 31, hh = lane >> 5, vr = 4 * hh + ((lane & 15) >> 2);
+    k = col * (D * 2) + (((hh * (D / 16)) ^ chunk_swizzle<D>(col)) << 4);
+    v = vr * (D * 2) + (((2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ chunk_swizzle<D>(vr)) << 4) + (lane & 1) * 8;
+  }
+};
+
+// What a wave keeps of its row tile: one row per pair of lanes (col, col + 32).
+template <typename T, int D> struct DirectRows {
   typedef typename Elem<T>::vec8 vec8;
-  typedef DirectLds<D, KG> L;
-  constexpr int NKS = D / 16, NDT = D / 32, NT = 64 * KG;
-  constexpr int CPR = D / 8, RPI = 64 / CPR, NLD = 32 / RPI;   // 16-byte chunks per row, rows and number of loads of a tile
-  constexpr int UPB = BK / 32;                                 // steps of 32 keys per block
+  static constexpr int NKS = D / 16, NDT = D / 32;
+  float scale_log2;
+  int qpos;               // position of the lane's query
+  vec8 q[NKS];            // dims hh D/2 + 8 ks .. + 7
+  float mref, l;          // reference maximum (scaled scores), sum
+  f32x16 o[NDT];
+
+  __device__ __forceinline__ void load_q(const DirectParams& p, int q0, int h, int row) {
+    const T* r = reinterpret_cast<const T*>(p.q) + (int64_t)(q0 + qpos) * p.q_sn + (int64_t)(h * p.g + row - qpos * p.g) * p.q_sh +
+                 ((threadIdx.x & 63) >> 5) * (D / 2);
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) q[ks] = load16<vec8>(r + ks * 8);
+  }
+  // q settled: otherwise the compiler waits for it where it is used first, inside the loop and in every step of it, and with it
+  // for the tile that was requested a moment before
+  __device__ __forceinline__ void settle_q() {
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) asm volatile("" : "+v"(q[ks]));
+  }
+  __device__ __forceinline__ void clear() {
+    mref = -INFINITY;
+    l = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
+  }
+  __device__ __forceinline__ void causal(f32x16& s, int key) const {
+    const int limit = qpos - key, hh = (threadIdx.x & 63) >> 5;
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if (8 * (i >> 2) + 4 * hh + (i & 3) > limit) s[i] = -INFINITY;
+  }
+  static __device__ __forceinline__ float lane_max(const f32x16& s) {
+    float mx = s[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+    return mx;
+  }
+  // the reference maximum after scores whose maximum over the lane's own keys is mx
+  __device__ __forceinline__ void raise(float mx, bool on) {
+    mx = max32(mx) * scale_log2;
+    asm volatile("" : "+v"(mx));   // (a select, not a branch over what was computed above)
+    mx = on ? mx : -INFINITY;
+    // a row that has seen no key yet takes its first maximum as it is: there is nothing to rescale
+    mref = mref == -INFINITY ? mx : mref;
+    // as in the dense kernels: the reference maximum moves only when some row outgrows it by more than 2^8
+    if (__builtin_expect(__any(mx > mref + 8.f), 0)) {
+      const float top = fmaxf(mref, mx), alpha = top == -INFINITY ? 1.f : fast_exp2(mref - top);
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
+      mref = top;
+    }
+  }
+  __device__ __forceinline__ float reference(bool on) const { return !on ? INFINITY : mref == -INFINITY ? 0.f : mref; }   // 2^(s - inf) = 0
+  __device__ __forceinline__ bool has_nan() const {
+    float x = l;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x += o[dt][i];
+    return x != x;
+  }
+  // A step of the second pass, K and V through the wave's own 2 tiles at LDS address `own`: a block that a query did not select
+  // must not reach it at all (a key or value of it that is infinite or NaN makes 0 * x NaN in the products), and a block that a
+  // list names several times (`times`) counts as often.
+  __device__ __forceinline__ void step_carefully(const DirectLoads<T, D>& k, const DirectLoads<T, D>& v, const DirectFrags<D>& f, uint32_t own,
+                                                 int key, bool on, float times) {
+    k.issue(key, own);
+    v.issue(key, own + k.BYTES);
+    vm_wait<0>();
+    f32x16 s;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) s = Elem<T>::mfma32(load16<vec8>(lds_ptr<T>(own + (f.k ^ (16u * ks)))), q[ks], s);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = on ? s[i] : -INFINITY;
+    causal(s, key);
+    raise(lane_max(s), on);
+    const float ref = reference(on);
+    vec8 pk[2];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float pv = on ? fast_exp2(s[i] * scale_log2 - ref) * times : 0.f;
+      l += pv;
+      pk[i >> 3][i & 7] = (T)pv;
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) {
+        const f32x16 x = Elem<T>::mfma32(swizzled_tr_frag<T, D>(own + k.BYTES + (f.v ^ (64u * dt)), j), pk[j], o[dt]);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[dt][i] = on ? x[i] : o[dt][i];
+      }
+    lds_reads_done();
+  }
+  // the wave's partial result: [32][D] fp32, 16-byte chunk c of row r at c ^ r; reference and sum to st_m[r], st_l[r]
+  static constexpr int XM = D / 4 - 1 < 31 ? D / 4 - 1 : 31;
+  __device__ __forceinline__ void park(float* part, float* st_m, float* st_l) const {
+    const int lane = threadIdx.x & 63, col = lane & 31, hh = lane >> 5;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int qd = 0; qd < 4; ++qd) {
+        const int c = (dt * 8 + 2 * qd + hh) ^ (col & XM);
+        *reinterpret_cast<f32x4*>(part + col * D + c * 4) = f32x4{o[dt][4 * qd], o[dt][4 * qd + 1], o[dt][4 * qd + 2], o[dt][4 * qd + 3]};
+      }
+    if (hh == 0) {
+      st_m[col] = mref;
+      st_l[col] = l;
+    }
+  }
+};
+
+// Chunk `sub` (8 dims) of row r of a row tile, from the partial results of KG waves: partial w at part + w * part_step bytes,
+// its statistics at st_m + w * st_step.
+template <typename T, int D, bool MERGE, int KG>
+__device__ __forceinline__ void direct_store(const DirectParams& p, int h, int q0, int row, int r, int sub, const unsigned char* part, int part_step,
+                                             const float* st_m, const float* st_l, int st_step) {
+  typedef typename Elem<T>::vec8 vec8;
+  constexpr int XM = DirectRows<T, D>::XM;
+  float mw[KG], mx = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < KG; ++w) {
+    mw[w] = st_m[w * st_step + r];
+    mx = fmaxf(mx, mw[w]);
+  }
+  float sum = 0.f, out[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) out[e] = 0.f;
+#pragma unroll
+  for (int w = 0; w < KG; ++w) {
+    mw[w] = mx == -INFINITY ? 0.f : fast_exp2(mw[w] - mx);
+    sum += mw[w] * st_l[w * st_step + r];
+    const float* pw = reinterpret_cast<const float*>(part + w * part_step) + r * D;
+    const f32x4 x0 = *reinterpret_cast<const f32x4*>(pw + ((2 * sub) ^ (r & XM)) * 4);
+    const f32x4 x1 = *reinterpret_cast<const f32x4*>(pw + ((2 * sub + 1) ^ (r & XM)) * 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      out[e] += mw[w] * x0[e];
+      out[4 + e] += mw[w] * x1[e];
+    }
+    }
+  const float inv = sum == 0.f ? 0.f : 1.f / sum;   // (a sum that is NaN, from a NaN in q or a key, makes the row NaN)
+  vec8 x;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = (T)(out[e] * inv);
+  const int qi = div_group(row, p.g, p.g_shift), hq_i = h * p.g + row - qi * p.g;
+  const int64_t tok = q0 + qi;
+  if constexpr (MERGE) {
+    const int64_t at = (tok * (p.hkv * p.g) + hq_i) * D + sub * 8;
+    const vec8 xa = load16_stream<vec8>(reinterpret_cast<const T*>(p.merge.a) + at);
+    const vec8 xc = load16_stream<vec8>(reinterpret_cast<const T*>(p.merge.c) + at);
+    const T* gate = reinterpret_cast<const T*>(p.merge.gate) + tok * 3;
+    const float g0 = (float)gate[0], g1 = (float)gate[1], g2 = (float)gate[2];
+    vec8 y;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) y[e] = (T)(g0 * (float)xa[e] + g1 * (float)x[e] + g2 * (float)xc[e]);
+    store16(reinterpret_cast<T*>(p.merge.out) + at, y);
+    if (!p.o) return;
+  }
+  store16(reinterpret_cast<T*>(p.o) + tok * p.o_sn + (int64_t)hq_i * p.o_sh + sub * 8, x);
+  if (sub == 0) p.lse[(int64_t)hq_i * p.n_tokens + tok] = sum == 0.f ? -INFINITY : mx + log2f(sum);
+}
+
+// How often the lane's query names block b.
+__device__ __forceinline__ float direct_times(const DirectParams& p, int h, int tok, int b) {
+  const int32_t* ids = p.topk_idx + h * p.i_sh + (int64_t)tok * p.i_sn;
+  int c = 0;
+  for (int i = 0; i < p.topk; ++i) c += ids[i] == b;
+  return (float)c;
+}
+
+// ---- narrow: one row tile, KG key groups of one wave -----------------------------------------------------------------------
+// Bound by the chain of a step (products, maximum, exponentials, products: 0.8 us for a wave that is alone on its SIMD) in the
+// longest work-group.  q is settled in front of the loop, and the lists are read a step ahead: without, the compiler waited for q,
+// and with it for the tile just requested, in every step, and a step began with two trips to LDS.  Both: 4096 tokens x 4 heads of
+// 128 39.3 -> 35.0 us, 4500 x 8 of 64 40 -> 38.  Two row tiles per work-group, a long and a short one, shared out over eight waves:
+// 36 and slower elsewhere.
+template <int D, int KG> struct NarrowLds {
+  static constexpr int TILE = 32 * D * 2;
+  static constexpr int WAVE_BYTES = 2 * TILE;               // K and V of a wave; at the end its fp32 partial [32][D]
+  static constexpr int STATS = 2 * KG * 32 * 4;             // (m, l) of every wave
+  static constexpr int bytes(int max_blk) { return KG * WAVE_BYTES + STATS + 16 + 6 * max_blk; }
+};
+
+template <typename T, int D, int KG, bool MERGE>
+__global__ void __launch_bounds__(64 * KG, D <= 128 ? 2 : 1)
+selattn_direct_narrow_kernel(DirectParams p) {
+  typedef typename Elem<T>::vec8 vec8;
+  typedef NarrowLds<D, KG> L;
+  typedef DirectLoads<T, D> Loads;
+  constexpr int NKS = D / 16, NDT = D / 32, NT = 64 * KG, NLD = Loads::N;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   float* st_m = reinterpret_cast<float*>(smem + KG * L::WAVE_BYTES);   // [wave][row]
-  float* st_l = st_m + KG * DIR_ROWS;
-  int* info = reinterpret_cast<int*>(st_l + KG * DIR_ROWS);     // [0] list length, [1] a list names a block twice
+  float* st_l = st_m + KG * 32;
+  int* info = reinterpret_cast<int*>(st_l + KG * 32);           // [0] list length, [1] a list names a block twice
   uint32_t* sel = reinterpret_cast<uint32_t*>(info + 4);        // [block]: bit i = query q_first + i
   uint16_t* list = reinterpret_cast<uint16_t*>(sel + p.max_blk);   // visited blocks
 
   const int h = blockIdx.x % p.hkv;
-  DirectTile t;
-  if (!direct_tile(p.cu, p.batch, (int)p.n_tokens, p.g, blockIdx.x / p.hkv, t)) return;
-  const int q0 = t.q0, len = t.len, rows = t.n_q * p.g, row0 = t.tile * DIR_ROWS;
-  const int q_first = div_group(row0, p.g, p.g_shift), q_last = div_group(min(rows, row0 + DIR_ROWS) - 1, p.g, p.g_shift);
-  const int n_blk = min(q_last / BK + 1, (len + BK - 1) / BK);
-  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int col = lane & 31, hh = lane >> 5;
+  DirectTile t_;
+  if (!direct_tile(p.cu, p.batch, (int)p.n_tokens, p.g, 32, blockIdx.x / p.hkv, t_)) return;
+  const int q0 = t_.q0, len = t_.len, rows = t_.n_q * p.g, row0 = t_.tile * 32, bks = p.bk_shift;
+  const int q_first = div_group(row0, p.g, p.g_shift), q_last = div_group(min(rows, row0 + 32) - 1, p.g, p.g_shift);
+  const int n_blk = min((q_last >> bks) + 1, (len + (1 << bks) - 1) >> bks);
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 31;
 
-  // q fragments: dims hh D/2 + 8 ks .. + 7
-  const int row = min(row0 + col, rows - 1);
-  const int qpos = div_group(row, p.g, p.g_shift), qoff = qpos - q_first;
-  vec8 qreg[NKS];
+  DirectRows<T, D> r;
+  r.scale_log2 = p.scale_log2;
   {
-    const T* qrow = reinterpret_cast<const T*>(p.q) + (int64_t)(q0 + qpos) * p.q_sn + (int64_t)(h * p.g + row - qpos * p.g) * p.q_sh +
-                    hh * (D / 2);
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) qreg[ks] = load16<vec8>(qrow + ks * 8);
+    const int row = min(row0 + col, rows - 1);
+    r.qpos = div_group(row, p.g, p.g_shift);
+    r.load_q(p, q0, h, row);
   }
-
-  // ---- K / V tiles ----
-  const uint32_t k_row = (uint32_t)p.k_sn * 2, v_row = (uint32_t)p.v_sn * 2;   // bytes (host: a head's rows span < 2^31)
-  const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<T*>(reinterpret_cast<const T*>(p.k) + (int64_t)q0 * p.k_sn + (int64_t)h * p.k_sh), 0, (int)DIR_BUFFER, 0x00020000);
-  const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<T*>(reinterpret_cast<const T*>(p.v) + (int64_t)q0 * p.v_sn + (int64_t)h * p.v_sh), 0, (int)DIR_BUFFER, 0x00020000);
+  const int qoff = r.qpos - q_first;
+  const Loads kl(p.k, p.k_sn, p.k_sh, q0, h, len), vl(p.v, p.v_sn, p.v_sh, q0, h, len);
   const uint32_t k_lds = lds_addr(smem + wv * L::WAVE_BYTES), v_lds = k_lds + L::TILE;
-  // (the loading lane picks its source so that the chunks land where chunk_swizzle wants them)
-  const int ld_row = lane / CPR, ld_chunk = lane % CPR;
-  uint32_t k_voff[NLD], v_voff[NLD];
-#pragma unroll
-  for (int j = 0; j < NLD; ++j) {   // (host: rows are at least 2 D bytes apart, so the difference is not negative)
-    const int r = j * RPI + ld_row;
-    k_voff[j] = r * k_row + (ld_chunk ^ chunk_swizzle<D>(r)) * 16 - (j & 3) * 1024;
-    v_voff[j] = r * v_row + (ld_chunk ^ chunk_swizzle<D>(r)) * 16 - (j & 3) * 1024;
-  }
-  auto issue = [&](__amdgpu_buffer_rsrc_t rsrc, uint32_t row_bytes, const uint32_t* voff, uint32_t to, int key) {
-    if (key + 32 <= len) {
-#pragma unroll
-      for (int j = 0; j < NLD; j += 4) lds_dma4(rsrc, &voff[j], (uint32_t)key * row_bytes, to + j * 1024);
-    } else {
-      // A tile that reaches behind the end: zeros there (an offset behind the end of the buffer).  No query of the sequence
-      // sees them; one at a position behind it does, with score 0, as in the block-major kernels.
-#pragma unroll 1
-      for (int j = 0; j < NLD; ++j) {
-        const int r = j * RPI + ld_row;
-        const uint32_t off =
-            key + r < len ? (uint32_t)(key + r) * row_bytes + (ld_chunk ^ chunk_swizzle<D>(r)) * 16 : DIR_BUFFER;
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
-                     :: "v"(off), "s"(rsrc), "s"(to + j * 1024) : "memory");
-      }
-    }
-  };
-  auto issue_k = [&](int key) { issue(k_rsrc, k_row, k_voff, k_lds, key); };
-  auto issue_v = [&](int key) { issue(v_rsrc, v_row, v_voff, v_lds, key); };
+
   // ---- which blocks, and which of the queries selected them ----
   const int32_t* ids = p.topk_idx + h * p.i_sh + (int64_t)(q0 + q_first) * p.i_sn;
   const int n_ids = (q_last - q_first + 1) * p.topk;
@@ -171,10 +370,10 @@ selattn_direct_fwd_kernel(DirectParams p) {
   // The first keys of every wave are requested before it is known which blocks are visited: the first blocks of the
   // sequence, as where the union of the lists has no gap at its start.  4096 tokens x 4 heads 40.5 -> 39.3 us.  (The
   // compiler's waits for id[] below do not count these loads, which are younger, and so wait for most of them as well.)
-  int guess = wv / UPB * BK + wv % UPB * 32;
+  int guess = 32 * wv;
   if (guess + 32 <= len) {
-    issue_k(guess);
-    issue_v(guess);
+    kl.issue(guess, k_lds);
+    vl.issue(guess, v_lds);
   } else {
     guess = -1;
   }
@@ -182,7 +381,7 @@ selattn_direct_fwd_kernel(DirectParams p) {
   if (tid < 2) info[tid] = 0;
   __syncthreads();
   auto visit = [&](int q, int b) {
-    if (b < 0 || b >= n_blk || b > (q_first + q) / BK) return;   // (a block behind the query's own holds no key it may see)
+    if (b < 0 || b >= n_blk || b > (q_first + q) >> bks) return;   // (a block behind the query's own holds no key it may see)
     if (atomicOr(&sel[b], 1u << q) >> q & 1) info[1] = 1;
   };
 #pragma unroll
@@ -192,6 +391,7 @@ selattn_direct_fwd_kernel(DirectParams p) {
     const int q = (uint32_t)e / (uint32_t)p.topk;
     visit(q, ids[q * p.i_sn + (e - q * p.topk)]);
   }
+  r.settle_q();
   __syncthreads();
   if (wv == 0) {   // the visited blocks, in order
     int at = 0;
@@ -206,267 +406,410 @@ selattn_direct_fwd_kernel(DirectParams p) {
   }
   __syncthreads();
   const bool twice = __builtin_amdgcn_readfirstlane(info[1]) != 0;
-  const int n_units = __builtin_amdgcn_readfirstlane(info[0]) * UPB;
+  const int upb_shift = bks - 5;   // log2 of the steps of 32 keys per block
+  const int n_units = __builtin_amdgcn_readfirstlane(info[0]) << upb_shift;
   const int n_steps = (n_units - wv + KG - 1) / KG;   // of this wave
-  struct Unit {
-    int key;         // position of its first key
-    uint32_t mask;   // queries that selected its block
-  };
-  auto unit = [&](int t) {
-    const int u = wv + KG * t;
-    const int b = __builtin_amdgcn_readfirstlane(list[u / UPB]);
-    return Unit{b * BK + u % UPB * 32, (uint32_t)__builtin_amdgcn_readfirstlane((int)sel[b])};
-  };
+  const DirectFrags<D> f;
+  auto place = [&](int t) { return wv + KG * min(t, n_steps - 1); };   // in the list of steps
+  auto key_of = [&](int u, int b) { return (b << bks) + (u & ((1 << upb_shift) - 1)) * 32; };
 
-  // lane addresses of the fragments
-  const uint32_t kf_addr = k_lds + col * (D * 2) + (((hh * (D / 16)) ^ chunk_swizzle<D>(col)) << 4);   // k-step ks: ^ 16 ks
-  const int vr = 4 * hh + ((lane & 15) >> 2);
-  const uint32_t vf_addr = v_lds + vr * (D * 2) + (((2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ chunk_swizzle<D>(vr)) << 4) + (lane & 1) * 8;
-  auto k_frag = [&](int ks) { return load16<vec8>(lds_ptr<T>(kf_addr ^ (16u * ks))); };
-  auto v_frag = [&](int j, int dt) { return swizzled_tr_frag<T, D>(vf_addr ^ (64u * dt), j); };   // keys 16 j .., dims 32 dt ..
-
-  float m = -INFINITY, mref = 0.f, l = 0.f;   // reference maximum (raw scores), the same scaled (0 while there is none)
-  f32x16 oacc[NDT];
-  // CAREFUL: a block that a query did not select must not reach it at all (a key or value of it that is infinite or NaN makes
-  // 0 * x NaN in the products), and a block that a list names several times counts as often.
-  // At head_dim 128 this pass is 16 registers short: it puts them into scratch (68 bytes) in front of its loop, which the other
-  // pass does not touch.
-  auto attend = [&](auto careful_, int loaded) {   // loaded: the key of the tiles that are in LDS or on their way there, or -1
-    constexpr bool CAREFUL = decltype(careful_)::value;
-    m = -INFINITY;
-    mref = l = 0.f;
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
-    if (n_steps <= 0 || unit(0).key != loaded) vm_wait<0>();   // (what is on its way would land in what comes now)
-    if (n_steps <= 0) return;
-    Unit cur = unit(0);
-    if (cur.key != loaded) {
-      issue_k(cur.key);
-      issue_v(cur.key);
+  auto attend = [&]() {
+    r.clear();
+    if (n_steps <= 0) {
+      vm_wait<0>();
+      return;
     }
-    // The counts of vm_wait leave the tile that was requested last on its way, and at head_dim 64 that is what runs.  At 128
-    // and 256 the compiler settles qreg, ordinary loads whose first use is in this loop, by waits of its own between the
-    // products of S: they run in every step, down to no operation outstanding, so that K of the next step and V of this one
-    // are awaited there in full and a step takes the latency of a tile (about 1 us at head_dim 128).
+    int b = __builtin_amdgcn_readfirstlane(list[place(0) >> upb_shift]), b1 = __builtin_amdgcn_readfirstlane(list[place(1) >> upb_shift]);
+    int key = key_of(place(0), b);
+    uint32_t mask = (uint32_t)__builtin_amdgcn_readfirstlane((int)sel[b]);
+    if (key != guess) {
+      vm_wait<0>();   // (what is on its way would land in what comes now)
+      kl.issue(key, k_lds);
+      vl.issue(key, v_lds);
+    }
     for (int t = 0;; ++t) {
       const bool more = t + 1 < n_steps;
-      const Unit nxt = unit(more ? t + 1 : t);
+      const int key1 = key_of(place(t + 1), b1);
       vm_wait<NLD>();   // K of this step, not its V
       vec8 kf[NKS];
 #pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) kf[ks] = k_frag(ks);
+      for (int ks = 0; ks < NKS; ++ks) kf[ks] = load16<vec8>(lds_ptr<T>(k_lds + (f.k ^ (16u * ks))));
+      // asked for here, looked at behind the products: the mask of the next step, the block of the one after
+      const uint32_t mask1 = sel[b1], b2 = list[place(t + 2) >> upb_shift];
       lds_reads_done();
-      if (more) issue_k(nxt.key);
-      f32x16 acc;
+      if (more) kl.issue(key1, k_lds);
+      f32x16 s;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+      for (int i = 0; i < 16; ++i) s[i] = 0.f;
 #pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) acc = Elem<T>::mfma32(kf[ks], qreg[ks], acc);
-      const bool on = (cur.mask >> qoff) & 1;
-      float times = 1.f;
-      if (CAREFUL) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[i] = on ? acc[i] : -INFINITY;
-        if (twice) {
-          const int32_t* ids = p.topk_idx + h * p.i_sh + (int64_t)(q0 + qpos) * p.i_sn;
-          int c = 0;
-          for (int i = 0; i < p.topk; ++i) c += ids[i] == cur.key / BK;
-          times = (float)c;
-        }
-      }
-      if (cur.key + 31 > q_first) {   // some row may see the keys partly
-        const int limit = qpos - cur.key;
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (8 * (i >> 2) + 4 * hh + (i & 3) > limit) acc[i] = -INFINITY;
-      }
-      float mx = acc[0];
-#pragma unroll
-      for (int i = 1; i < 16; ++i) mx = fmaxf(mx, acc[i]);
-      mx = max32(mx);
-      asm volatile("" : "+v"(mx));   // (a select, not a branch over what was computed above)
-      mx = fmaxf(m, on ? mx : -INFINITY);
-      // a row that has seen no key yet takes its first maximum as it is: there is nothing to rescale
-      const bool first = m == -INFINITY;
-      mref = first ? (mx == -INFINITY ? 0.f : mx * p.scale_log2) : mref;
-      m = first ? mx : m;
-      // as in the dense kernels: the reference maximum moves only when some row outgrows it by more than 2^8
-      if (__any((mx - m) * p.scale_log2 > 8.f)) {   // (a row without a key: NaN)
-        const float alpha = mx == -INFINITY ? 1.f : exp2f((m - mx) * p.scale_log2);
-        l *= alpha;
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) oacc[dt][i] *= alpha;
-        m = mx;
-        mref = mx == -INFINITY ? 0.f : mx * p.scale_log2;
-      }
-      const float ref = on ? mref : INFINITY;   // 2^(s - inf) = 0
+      for (int ks = 0; ks < NKS; ++ks) s = Elem<T>::mfma32(kf[ks], r.q[ks], s);
+      const bool on = mask >> qoff & 1;
+      if (__builtin_expect(key + 31 > q_first, 0)) r.causal(s, key);   // some row may see the keys partly
+      r.raise(r.lane_max(s), on);
+      const float ref = r.reference(on);
       float sum = 0.f;
       vec8 pk[2];
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        float pv = fast_exp2(acc[i] * p.scale_log2 - ref);
-        if (CAREFUL) pv = on ? pv * times : 0.f;
+        const float pv = fast_exp2(s[i] * r.scale_log2 - ref);
         sum += pv;
         pk[i >> 3][i & 7] = (T)pv;
       }
-      l += sum;   // the lane's own keys: the two lanes of a row are added behind the loop
-      if (more) vm_wait<NLD>();   // V of this step, not K of the next (but see above)
+      r.l += sum;   // the lane's own keys: the two lanes of a row are added behind the loop
+      if (more) vm_wait<NLD>();   // V of this step, not K of the next
       else vm_wait<0>();
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) {
-          const f32x16 x = Elem<T>::mfma32(v_frag(j, dt), pk[j], oacc[dt]);
-#pragma unroll
-          for (int i = 0; i < 16; ++i) oacc[dt][i] = !CAREFUL || on ? x[i] : oacc[dt][i];
-        }
+        for (int dt = 0; dt < NDT; ++dt) r.o[dt] = Elem<T>::mfma32(swizzled_tr_frag<T, D>(v_lds + (f.v ^ (64u * dt)), j), pk[j], r.o[dt]);
       lds_reads_done();
       if (!more) break;
-      issue_v(nxt.key);
-      cur = nxt;
+      vl.issue(key1, v_lds);
+      key = key1;
+      mask = (uint32_t)__builtin_amdgcn_readfirstlane((int)mask1);
+      b1 = __builtin_amdgcn_readfirstlane((int)b2);
     }
-    l = sum32(l);
   };
   bool careful = twice;
   if (!careful) {
-    attend(std::false_type{}, guess);
-    float x = 0.f;   // NaN if any accumulator is
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) x += oacc[dt][i];
-    careful = __any(x != x || l != l);
+    attend();
+    careful = __any(r.has_nan());
   }
-  if (careful) attend(std::true_type{}, twice ? guess : -1);
+  if (careful) {
+    vm_wait<0>();
+    r.clear();
+    for (int t = 0; t < n_steps; ++t) {
+      const int b = __builtin_amdgcn_readfirstlane(list[place(t) >> upb_shift]);
+      r.step_carefully(kl, vl, f, k_lds, key_of(place(t), b), sel[b] >> qoff & 1, twice ? direct_times(p, h, q0 + r.qpos, b) : 1.f);
+    }
+  }
+  r.l = sum32(r.l);
 
   // ---- merge of the waves ----
-  float* part = reinterpret_cast<float*>(smem + wv * L::WAVE_BYTES);   // [32][D], 16-byte chunk c of row r at c ^ r
-  constexpr int XM = D / 4 - 1 < 31 ? D / 4 - 1 : 31;
+  r.park(reinterpret_cast<float*>(smem + wv * L::WAVE_BYTES), st_m + wv * 32, st_l + wv * 32);
+  __syncthreads();
+  constexpr int CPR = Loads::CPR;
+  for (int wr = tid / CPR; wr < 32 && row0 + wr < rows; wr += NT / CPR)
+    direct_store<T, D, MERGE, KG>(p, h, q0, row0 + wr, wr, tid % CPR, smem, L::WAVE_BYTES, st_m, st_l, 32);
+}
+
+// ---- wide: RT row tiles, KG key groups --------------------------------------------------------------------------------------
+// With tiles of its own a wave brings 16 KB (head_dim 128) into LDS for 32 rows x 32 keys, 512 clocks of products: the L2 delivers
+// about 50 bytes per clock and CU, so a full chip of such waves waits for tiles (5003 tokens x 32 heads, GQA 4, 250 us; without the
+// loads 170).  Here RT row tiles share them, and a wave does not alternate between products and exponentials but always has both:
+// 209 us, 1.0 PFLOP/s of the pairs it visits.  Two thirds of a SIMD's time are products then (timing-only builds: no LDS reads -9 %,
+// no exponentials -2 %).  64 rows per wave at one wave per SIMD, with the same order of work: 273 us, since a single wave issues an
+// instruction in four clocks at best; 64 rows per wave with q in LDS: 290.
+template <int D, int KG, int RT> struct WideLds {
+  static constexpr int WAVES = KG * RT;
+  static constexpr int TILE = 32 * D * 2;
+  static constexpr int WAVE_BYTES = 2 * TILE;               // a wave's part in the second pass and in the merge: its fp32 partial [32][D]
+  static constexpr int GROUP_BYTES = 4 * TILE > RT * WAVE_BYTES ? 4 * TILE : RT * WAVE_BYTES;   // of a key group: two K and two V tiles
+  static constexpr int STATS = 2 * WAVES * 32 * 4;          // (m, l) of every wave
+  static constexpr int bytes(int max_blk) { return KG * GROUP_BYTES + STATS + 16 + (4 * RT + 2) * max_blk; }
+};
+
+template <typename T, int D, int KG, int RT, bool MERGE>
+__global__ void __launch_bounds__(64 * KG * RT, D <= 128 ? 2 : 1)
+selattn_direct_wide_kernel(DirectParams p) {
+  typedef typename Elem<T>::vec8 vec8;
+  typedef WideLds<D, KG, RT> L;
+  typedef DirectLoads<T, D> Loads;
+  constexpr int ROWS = 32 * RT, NKS = D / 16, NDT = D / 32, NT = 64 * L::WAVES;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  float* st_m = reinterpret_cast<float*>(smem + KG * L::GROUP_BYTES);   // [wave][32]
+  float* st_l = st_m + L::WAVES * 32;
+  int* info = reinterpret_cast<int*>(st_l + L::WAVES * 32);     // [0] list length, [1] a list names a block twice, [2] second pass
+  uint32_t* sel = reinterpret_cast<uint32_t*>(info + 4);        // [block][row tile]: bit i = the i-th query of the row tile
+  uint16_t* list = reinterpret_cast<uint16_t*>(sel + RT * p.max_blk);   // visited blocks
+
+  const int h = blockIdx.x % p.hkv;
+  DirectTile t_;
+  if (!direct_tile(p.cu, p.batch, (int)p.n_tokens, p.g, ROWS, blockIdx.x / p.hkv, t_)) return;
+  const int q0 = t_.q0, len = t_.len, rows = t_.n_q * p.g, row0 = t_.tile * ROWS, bks = p.bk_shift;
+  const int q_first = div_group(row0, p.g, p.g_shift), q_last = div_group(min(rows, row0 + ROWS) - 1, p.g, p.g_shift);
+  const int n_blk = min((q_last >> bks) + 1, (len + (1 << bks) - 1) >> bks);
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 31;
+  const int rt = wv % RT, kg = wv / RT;
+
+  DirectRows<T, D> r;
+  r.scale_log2 = p.scale_log2;
+  {
+    const int row = min(row0 + 32 * rt + col, rows - 1);
+    r.qpos = div_group(row, p.g, p.g_shift);
+    r.load_q(p, q0, h, row);
+  }
+  const int q_tile = div_group(min(row0 + 32 * rt, rows - 1), p.g, p.g_shift), qoff = r.qpos - q_tile;
+  const Loads kl(p.k, p.k_sn, p.k_sh, q0, h, len), vl(p.v, p.v_sn, p.v_sh, q0, h, len);
+  const uint32_t k_lds = lds_addr(smem + kg * L::GROUP_BYTES), v_lds = k_lds + 2 * L::TILE;
+  // This wave's share of a K or V tile of its key group: even waves K, odd ones V, each half a tile where there are four.
+  constexpr int PARTS = RT >= 4 && Loads::N >= 2 * Loads::NV ? 2 : 1;
+  auto issue_k = [&](int key, int stage) {
+    if ((rt & 1) == 0 && rt < 2 * PARTS) kl.template issue<PARTS>(key, k_lds + stage * L::TILE, rt >> 1);
+  };
+  auto issue_v = [&](int key, int stage) {
+    if ((rt & 1) == 1 && rt < 2 * PARTS) vl.template issue<PARTS>(key, v_lds + stage * L::TILE, rt >> 1);
+  };
+
+  // ---- which blocks, and which of the queries selected them ----
+  const int32_t* ids = p.topk_idx + h * p.i_sh + (int64_t)(q0 + q_first) * p.i_sn;
+  const int n_ids = (q_last - q_first + 1) * p.topk;
+  constexpr int AHEAD = 512 * RT / NT;   // entries per thread that are requested at once (32 lists of 16 for each row tile)
+  int qo[AHEAD], id[AHEAD];
 #pragma unroll
-  for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-    for (int qd = 0; qd < 4; ++qd) {
-      const int c = (dt * 8 + 2 * qd + hh) ^ (col & XM);
-      *reinterpret_cast<f32x4*>(part + col * D + c * 4) =
-          f32x4{oacc[dt][4 * qd], oacc[dt][4 * qd + 1], oacc[dt][4 * qd + 2], oacc[dt][4 * qd + 3]};
+  for (int i = 0; i < AHEAD; ++i) {
+    const int e = min(tid + i * NT, n_ids - 1);
+    qo[i] = (uint32_t)e / (uint32_t)p.topk;
+    id[i] = ids[qo[i] * p.i_sn + (e - qo[i] * p.topk)];
+  }
+  int guess = 32 * kg;   // as in the paired kernel
+  if (guess + 32 <= len) {
+    issue_k(guess, 0);
+    issue_v(guess, 0);
+  } else {
+    guess = -1;
+  }
+  for (int b = tid; b < RT * n_blk; b += NT) sel[b] = 0;
+  if (tid < 3) info[tid] = 0;
+  __syncthreads();
+  auto visit = [&](int q, int b) {   // q: relative to q_first
+    if (b < 0 || b >= n_blk || b > (q_first + q) >> bks) return;   // (a block behind the query's own holds no key it may see)
+    // the rows of a query may lie in several row tiles
+    const int r_lo = max((q_first + q) * p.g - row0, 0), r_hi = min((q_first + q) * p.g + p.g - row0, ROWS) - 1;
+    for (int x = r_lo >> 5; x <= r_hi >> 5; ++x) {
+      const int off = q_first + q - div_group(row0 + 32 * x, p.g, p.g_shift);
+      if (atomicOr(&sel[RT * b + x], 1u << off) >> off & 1) info[1] = 1;
     }
-  if (hh == 0) {
-    st_m[wv * DIR_ROWS + col] = m == -INFINITY ? -INFINITY : mref;
-    st_l[wv * DIR_ROWS + col] = l;
+  };
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i)
+    if (tid + i * NT < n_ids) visit(qo[i], id[i]);
+  for (int e = tid + AHEAD * NT; e < n_ids; e += NT) {
+    const int q = (uint32_t)e / (uint32_t)p.topk;
+    visit(q, ids[q * p.i_sn + (e - q * p.topk)]);
+  }
+  r.settle_q();
+  __syncthreads();
+  if (wv == 0) {   // the visited blocks, in order
+    int at = 0;
+    for (int b0 = 0; b0 < n_blk; b0 += WAVE) {
+      const int b = b0 + lane;
+      uint32_t any = 0;
+      if (b < n_blk)
+#pragma unroll
+        for (int x = 0; x < RT; ++x) any |= sel[RT * b + x];
+      const uint64_t m = __ballot(any != 0);
+      if (any) list[at + __popcll(m & ((1ull << lane) - 1))] = (uint16_t)b;
+      at += __popcll(m);
+    }
+    if (lane == 0) info[0] = at;
   }
   __syncthreads();
-  constexpr int RPP = NT / CPR;   // rows per pass
-#pragma unroll
-  for (int r0 = 0; r0 < DIR_ROWS; r0 += RPP) {
-    const int r = r0 + tid / CPR, sub = tid % CPR;
-    if (r >= DIR_ROWS || row0 + r >= rows) break;
-    float mw[KG], mx = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < KG; ++w) {
-      mw[w] = st_m[w * DIR_ROWS + r];
-      mx = fmaxf(mx, mw[w]);
+  const bool twice = __builtin_amdgcn_readfirstlane(info[1]) != 0;
+  const int upb_shift = bks - 5;   // log2 of the steps of 32 keys per block
+  const int n_units = __builtin_amdgcn_readfirstlane(info[0]) << upb_shift;
+  const int n_steps = (n_units + KG - 1) / KG;
+  struct Unit {
+    int key;         // position of its first key
+    uint32_t mask;   // queries of the row tile that selected its block
+  };
+  auto unit = [&](int t) {   // (the last steps of the key groups behind the end: some tile, selected by nobody)
+    const int u = kg + KG * t, v = min(u, n_units - 1);
+    const int b = __builtin_amdgcn_readfirstlane(list[v >> upb_shift]);
+    Unit x;
+    x.key = (b << bks) + (v & ((1 << upb_shift) - 1)) * 32;
+    x.mask = (uint32_t)__builtin_amdgcn_readfirstlane((int)sel[RT * b + rt]);
+    if (u >= n_units) x.mask = 0;
+    return x;
+  };
+  const DirectFrags<D> f;
+
+  // S of a step stands beside the exponentials of the step before, the products with V beside the maxima: a wave has work for
+  // the matrix and for the vector unit at any time.
+  auto attend = [&]() {
+    r.clear();
+    if (n_steps <= 0) {
+      vm_wait<0>();
+      return;
     }
-    float sum = 0.f;
-#pragma unroll
-    for (int w = 0; w < KG; ++w) {
-      mw[w] = mx == -INFINITY ? 0.f : fast_exp2(mw[w] - mx);
-      sum += mw[w] * st_l[w * DIR_ROWS + r];
+    constexpr int KA = 2, VA = 3;   // fragments requested ahead
+    Unit cur = unit(0), nx1 = unit(1);
+    if (cur.key != guess) {
+      vm_wait<0>();   // (what is on its way would land in what comes now)
+      issue_k(cur.key, 0);
+      issue_v(cur.key, 0);
     }
-    const float inv = sum == 0.f ? 0.f : 1.f / sum;   // (a sum that is NaN, from a NaN in q or a key, makes the row NaN)
-    float out[8];
+    issue_k(nx1.key, 1);
+    int key2 = unit(2).key, b2 = key2 >> bks;
+    vec8 kf[KA + 1], vf[VA + 1], pk[2];
+    float ref, sum;
+    auto arrived = [&]() {   // the loads of all waves, and the reads of all waves from what is overwritten next
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    };
+    auto scores = [&](f32x16& next, f32x16& s, int stage, auto exps_) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) out[e] = 0.f;
+      for (int i = 0; i < 16; ++i) next[i] = 0.f;
+      auto k_read = [&](int ks) { kf[ks % (KA + 1)] = load16<vec8>(lds_ptr<T>(k_lds + (f.k ^ (16u * ks)) + stage * L::TILE)); };
 #pragma unroll
-    for (int w = 0; w < KG; ++w) {
-      const float* pw = reinterpret_cast<const float*>(smem + w * L::WAVE_BYTES) + r * D;
-      const f32x4 x0 = *reinterpret_cast<const f32x4*>(pw + ((2 * sub) ^ (r & XM)) * 4);
-      const f32x4 x1 = *reinterpret_cast<const f32x4*>(pw + ((2 * sub + 1) ^ (r & XM)) * 4);
+      for (int ks = 0; ks < KA; ++ks) k_read(ks);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        out[e] += mw[w] * x0[e];
-        out[4 + e] += mw[w] * x1[e];
+      for (int ks = 0; ks < NKS; ++ks) {
+        if (ks + KA < NKS) k_read(ks + KA);
+        next = Elem<T>::mfma32(kf[ks % (KA + 1)], r.q[ks], next);
+        if constexpr (decltype(exps_)::value) {
+#pragma unroll
+          for (int i = ks * 16 / NKS; i < (ks + 1) * 16 / NKS; ++i) {
+            const float pv = fast_exp2(s[i] * r.scale_log2 - ref);
+            sum += pv;
+            pk[i >> 3][i & 7] = (T)pv;
+            if ((i & 7) == 7) asm volatile("" : "+v"(pk[i >> 3]), "+v"(sum));   // (here, not in front of its use)
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
-    }
-    vec8 x;
+    };
+    auto step = [&](f32x16& s, f32x16& next, int t) {   // scores of this step in s, those of the next one into `next`
+      const int odd = t & 1;
+      arrived();   // K of the next step, V of this one
+      issue_k(key2, odd);
+      issue_v(nx1.key, odd ^ 1);
+      // asked for here, looked at behind the products: the mask of step t + 2, the block of step t + 3
+      const uint32_t mask2 = sel[RT * b2 + rt], u3 = min(kg + KG * (t + 3), n_units - 1), b3 = list[u3 >> upb_shift];
+      ref = r.reference(cur.mask >> qoff & 1);
+      sum = 0.f;
+      scores(next, s, odd ^ 1, std::true_type{});
+      r.l += sum;   // the lane's own keys: the two lanes of a row are added behind the loop
+      if (__builtin_expect(nx1.key + 31 > q_first, 0)) r.causal(next, nx1.key);   // some row may see the keys partly
+      auto v_read = [&](int i) { vf[i % (VA + 1)] = swizzled_tr_frag<T, D>(v_lds + (f.v ^ (64u * (i % NDT))) + odd * L::TILE, i / NDT); };
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = (T)(out[e] * inv);
-    const int qi = div_group(row0 + r, p.g, p.g_shift), hq_i = h * p.g + row0 + r - qi * p.g;
-    const int64_t tok = q0 + qi;
-    if constexpr (MERGE) {
-      const int64_t at = (tok * (p.hkv * p.g) + hq_i) * D + sub * 8;
-      const vec8 xa = load16_stream<vec8>(reinterpret_cast<const T*>(p.merge.a) + at);
-      const vec8 xc = load16_stream<vec8>(reinterpret_cast<const T*>(p.merge.c) + at);
-      const T* gate = reinterpret_cast<const T*>(p.merge.gate) + tok * 3;
-      const float g0 = (float)gate[0], g1 = (float)gate[1], g2 = (float)gate[2];
-      vec8 y;
+      for (int i = 0; i < VA; ++i) v_read(i);
+      float mx = -INFINITY;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) y[e] = (T)(g0 * (float)xa[e] + g1 * (float)x[e] + g2 * (float)xc[e]);
-      store16(reinterpret_cast<T*>(p.merge.out) + at, y);
-      if (!p.o) continue;
+      for (int i = 0; i < 2 * NDT; ++i) {
+        if (i + VA < 2 * NDT) v_read(i + VA);
+        r.o[i % NDT] = Elem<T>::mfma32(vf[i % (VA + 1)], pk[i / NDT], r.o[i % NDT]);
+#pragma unroll
+        for (int x = i * 8 / NDT; x < (i + 1) * 8 / NDT; ++x) mx = fmaxf(mx, next[x]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      r.raise(mx, nx1.mask >> qoff & 1);
+      cur = nx1;
+      nx1.key = key2;
+      nx1.mask = kg + KG * (t + 2) < n_units ? (uint32_t)__builtin_amdgcn_readfirstlane((int)mask2) : 0u;
+      b2 = __builtin_amdgcn_readfirstlane((int)b3);
+      key2 = (b2 << bks) + (u3 & ((1 << upb_shift) - 1)) * 32;
+    };
+    f32x16 sa, sb;
+    arrived();
+    scores(sa, sb, 0, std::false_type{});
+    if (cur.key + 31 > q_first) r.causal(sa, cur.key);
+    r.raise(r.lane_max(sa), cur.mask >> qoff & 1);
+    for (int t = 0;;) {
+      step(sa, sb, t);
+      if (++t >= n_steps) break;
+      step(sb, sa, t);
+      if (++t >= n_steps) break;
     }
-    store16(reinterpret_cast<T*>(p.o) + tok * p.o_sn + (int64_t)hq_i * p.o_sh + sub * 8, x);
-    if (sub == 0) p.lse[(int64_t)hq_i * p.n_tokens + tok] = sum == 0.f ? -INFINITY : mx + log2f(sum);
+    vm_wait<0>();
+  };
+  bool careful = twice;
+  if (!careful) {
+    attend();
+    if (__any(r.has_nan())) info[2] = 1;
+    __syncthreads();   // (the last reads from the tiles, too)
+    careful = __builtin_amdgcn_readfirstlane(info[2]) != 0;
+  }
+  unsigned char* own = smem + kg * L::GROUP_BYTES + rt * L::WAVE_BYTES;
+  if (careful) {
+    vm_wait<0>();
+    __syncthreads();
+    r.clear();
+    for (int t = 0; t < n_steps; ++t) {
+      const Unit u = unit(t);
+      if (u.mask != 0)
+        r.step_carefully(kl, vl, f, lds_addr(own), u.key, u.mask >> qoff & 1, twice ? direct_times(p, h, q0 + r.qpos, u.key >> bks) : 1.f);
+    }
+  }
+  r.l = sum32(r.l);
+
+  // ---- merge of the key groups ----
+  r.park(reinterpret_cast<float*>(own), st_m + wv * 32, st_l + wv * 32);
+  __syncthreads();
+  constexpr int CPR = Loads::CPR;
+  for (int wr = tid / CPR; wr < ROWS && row0 + wr < rows; wr += NT / CPR) {
+    const int x = wr >> 5;
+    direct_store<T, D, MERGE, KG>(p, h, q0, row0 + wr, wr & 31, tid % CPR, smem + x * L::WAVE_BYTES, L::GROUP_BYTES, st_m + x * 32,
+                                  st_l + x * 32, RT * 32);
   }
 }
 
-template <typename T, int D, int BK, int KG, bool MERGE>
-static int launch_direct_fwd(const DirectParams& p, int64_t tiles, hipStream_t stream) {
+template <typename T, int D, int KG, bool MERGE> static int launch_direct_narrow(const DirectParams& p, hipStream_t stream) {
   static LdsAllowed allowed;
-  if (int rc = allow_lds(allowed, (const void*)selattn_direct_fwd_kernel<T, D, BK, KG, MERGE>,
-                         DirectLds<D, KG>::bytes(DIR_MAX_BLOCKS)))
-    return rc;
+  typedef NarrowLds<D, KG> L;
+  if (int rc = allow_lds(allowed, (const void*)selattn_direct_narrow_kernel<T, D, KG, MERGE>, L::bytes(DIR_MAX_BLOCKS))) return rc;
+  const int64_t tiles = p.n_tokens * p.g / 32 + p.batch + 1;
   ProfScope ps_("selattn_direct_fwd", stream);
-  selattn_direct_fwd_kernel<T, D, BK, KG, MERGE>
-      <<<(unsigned)((tiles + 1) * p.hkv), 64 * KG, DirectLds<D, KG>::bytes(p.max_blk), stream>>>(p);
+  selattn_direct_narrow_kernel<T, D, KG, MERGE><<<(unsigned)(tiles * p.hkv), 64 * KG, L::bytes(p.max_blk), stream>>>(p);
   return 0;
 }
-// Two waves per work-group where there are enough of them to fill the chip: less to merge, and more work-groups in different
-// stages on a CU.  (us with four / two waves: 4096 tokens x 4 heads of 128, 512 work-groups, 42 / 65; 4096 x 16, 2048, 115 /
-// 114; 2000 x 32, 2000, 71 / 61; 4096 x 32 209 / 197.)
-template <typename T, bool MERGE> static int dispatch_direct_fwd(int d, int bk, const DirectParams& p, hipStream_t stream) {
-  const int64_t tiles = p.n_tokens * p.g / DIR_ROWS + p.batch;
-  const bool two = tiles * p.hkv > 1536;
-#define FSA_CASE(DD, BB)                                                                        \
-  if (d == DD && bk == BB) {                                                                    \
-    if (two) return launch_direct_fwd<T, DD, BB, 2, MERGE>(p, tiles, stream);                   \
-    return launch_direct_fwd<T, DD, BB, 4, MERGE>(p, tiles, stream);                            \
-  }
-  FSA_CASE(128, 32)
-  FSA_CASE(128, 64)
-  FSA_CASE(128, 128)
-  FSA_CASE(64, 32)
-  FSA_CASE(64, 64)
-  FSA_CASE(64, 128)
-  FSA_CASE(256, 32)
-  FSA_CASE(256, 64)
-  FSA_CASE(256, 128)
-#undef FSA_CASE
-  set_error("selected attention (direct): head_dim=%d with block_size=%d is not supported", d, bk);
-  return FSA_ERR_UNSUPPORTED;
+template <typename T, int D, int KG, int RT, bool MERGE> static int launch_direct_wide(const DirectParams& p, hipStream_t stream) {
+  static LdsAllowed allowed;
+  typedef WideLds<D, KG, RT> L;
+  if (int rc = allow_lds(allowed, (const void*)selattn_direct_wide_kernel<T, D, KG, RT, MERGE>, L::bytes(DIR_MAX_BLOCKS))) return rc;
+  const int64_t tiles = p.n_tokens * p.g / (32 * RT) + p.batch + 1;
+  ProfScope ps_("selattn_direct_fwd", stream);
+  selattn_direct_wide_kernel<T, D, KG, RT, MERGE><<<(unsigned)(tiles * p.hkv), 64 * KG * RT, L::bytes(p.max_blk), stream>>>(p);
+  return 0;
+}
+// What the kernels take, in us on one chip: a part that grows with rows x keys, a chain of steps through the longest sequence, and
+// what does not depend on the size.  Fitted to 3 x 30 sizes (lists of 16 blocks of 64; head_dim 256: 8 of 128; one sequence).
+// narrow / wide 2 x 2 / wide 1 x 4 in us, head_dim 128, tokens x heads: 1500 x 4 15.9 / 23.7 / 36.6, 3000 x 4 28 / 40 / 62,
+// 1500 x 32 44 / 40 / 41, 3000 x 16 65 / 56 / 66, 3000 x 32 127 / 100 / 97, 5000 x 32 312 / 245 / 222, 8000 x 32 757 / 576 / 503; 64:
+// 5000 x 32 165 / 139 / 136; 256: 3000 x 4 48 / 73 / 109, 3000 x 32 314 / 249 / 210.
+enum DirectForm { DIRECT_NARROW, DIRECT_WIDE_2X2, DIRECT_WIDE_1X4, DIRECT_FORMS };
+static double direct_us(DirectForm form, int d, double rows, double len) {   // rows: of 128 dims
+  struct Fit { double per_us, step, fixed; };
+  static constexpr Fit fits[3][DIRECT_FORMS] = {{{2.55e6, 0.0036, 6}, {3.3e6, 0.0062, 8.5}, {3.75e6, 0.0145, 7}},
+                                                {{2.65e6, 0.0055, 6}, {3.5e6, 0.0095, 9}, {4.3e6, 0.018, 7}},
+                                                {{2.2e6, 0.01, 10}, {2.75e6, 0.021, 12}, {3.8e6, 0.0325, 12}}};
+  const Fit& f = fits[d <= 64 ? 0 : d <= 128 ? 1 : 2][form];
+  return std::hypot(rows * len / f.per_us, f.step * len) + f.fixed;
+}
+static DirectForm direct_form(int d, double rows, double len) {
+  DirectForm best = DIRECT_NARROW;
+  for (int i = 1; i < DIRECT_FORMS; ++i)
+    if (direct_us((DirectForm)i, d, rows, len) < direct_us(best, d, rows, len)) best = (DirectForm)i;
+  return best;
 }
 
-// Whether the forward of `n` tokens in sequences of at most `max_len` takes this path.  Both sides in us on one chip, fitted to
-// the times below: this kernel visits up to half of a sequence for every row, and its longest work-group works through a whole
-// one; the block-major launches work on topk * block keys per row, behind 33 us that do not depend on the size (index, two more
-// launches and their gaps), 12 of them for the index, which is no loss where the caller builds it all the same (training).
-// Lists of 16 blocks of 64, one sequence; index + block-major / direct / index + direct in us, head_dim 128:
-//   4096 tokens x 4 heads 62 / 37 / 53, x 16 (GQA 4) 131 / 101 / 115, x 32 (GQA 4) 233 / 192 / 208; 5000 x 4 69 / 47 / 65;
-//   5000 x 32 (GQA 4) 283 / 267 / 284; 6000 x 4 79 / 59 / 78, x 32 (GQA 4) 339 / 354; 7000 x 4 83 / 77; 8192 x 4 100 / 100, x 32
-//   505 / 711; 16384 x 4 (GQA 4) 167 / 211
-// head_dim 256, lists of 8: 3000 x 4 64 / 47 / 59, 4096 x 4 85 / 74 / 86, 6000 x 8 164 / 175; 64: 4500 x 8 46 / 35 / 46, 8000 x 8
-// (16 blocks) 93 / 94.  All of them, and the waves per work-group above, with the kernel's loads drained in every step (see the
-// loop): a step that takes less moves the line towards longer sequences.
+template <typename T, int D, bool MERGE> static int launch_direct_fwd(const DirectParams& p, int64_t max_len, hipStream_t stream) {
+  switch (direct_form(D, (double)p.n_tokens * p.hkv * p.g * D / 128, (double)max_len)) {
+    case DIRECT_WIDE_2X2: return launch_direct_wide<T, D, 2, 2, MERGE>(p, stream);
+    case DIRECT_WIDE_1X4: return launch_direct_wide<T, D, 1, 4, MERGE>(p, stream);
+    default: return launch_direct_narrow<T, D, 4, MERGE>(p, stream);
+  }
+}
+template <typename T, bool MERGE> static int dispatch_direct_fwd(int d, const DirectParams& p, int64_t max_len, hipStream_t stream) {
+  if (d == 128) return launch_direct_fwd<T, 128, MERGE>(p, max_len, stream);
+  if (d == 64) return launch_direct_fwd<T, 64, MERGE>(p, max_len, stream);
+  return launch_direct_fwd<T, 256, MERGE>(p, max_len, stream);
+}
+
+// Whether the forward of `n` tokens in sequences of at most `max_len` takes this path.  Both sides in us on one chip: these
+// kernels visit up to half of a sequence for every row; the block-major launches work on topk * block keys per row, behind 33 us
+// that do not depend on the size (index, two more launches and their gaps), 12 of them for the index, which is no loss where the
+// caller builds it all the same (training).  index + block-major / direct in us on the sizes above, head_dim 128: 3000 x 4
+// 13 + 40 / 28, 5000 x 4 17 + 54 / 46, 8000 x 4 23 + 77 / 100, 5000 x 32 27 + 288 / 222, 8000 x 32 33 + 460 / 503; GQA 4 5000 x 32
+// 18 + 269 / 212, 8000 x 32 24 + 428 / 485; 64: 8000 x 4 23 + 49 / 55, 5000 x 32 27 + 171 / 136, 8000 x 32 33 + 264 / 302; 256:
+// 3000 x 4 11 + 53 / 48, 3000 x 32 12 + 243 / 210, 5000 x 32 22 + 434 / 512.
 bool selattn_direct_preferred(int64_t n, int64_t max_len, int hq, int d, int topk, int bk, bool index_needed) {
   if (!(d == 64 || d == 128 || d == 256) || !(bk == 32 || bk == 64 || bk == 128) || topk > 4096 ||
       max_len > (int64_t)bk * DIR_MAX_BLOCKS)
     return false;
   const double rows = (double)n * hq * d / 128, len = (double)max_len;
   const double keys = std::min<double>((double)topk * bk, len);
-  return std::hypot(rows * len / 2.95e6, 0.0055 * len) + 5 <= (index_needed ? 21 : 33) + rows * keys / 6.2e5;
+  const double block_major = 33 + rows * keys / (d == 256 ? 7.8e5 : d == 128 ? 6.2e5 : 5.4e5);
+  return direct_us(direct_form(d, rows, len), d, rows, len) <= block_major - (index_needed ? 12 : 0);
 }
 
 int selattn_direct_fwd(const void* q, const void* k, const void* v, int32_t dtype, int64_t q_stride_n, int64_t q_stride_h,
@@ -488,6 +831,10 @@ int selattn_direct_fwd(const void* q, const void* k, const void* v, int32_t dtyp
                     total_tokens * 2 * v_stride_n < ((int64_t)1 << 31), "fsa_selattn_direct_fwd: k / v strides out of range");
   FSA_CHECK_ARG(block_size >= 1 && max_len <= (int64_t)block_size * DIR_MAX_BLOCKS && total_tokens * num_q_heads < ((int64_t)1 << 31),
                 "fsa_selattn_direct_fwd: too many tokens");
+  if ((head_dim != 64 && head_dim != 128 && head_dim != 256) || (block_size != 32 && block_size != 64 && block_size != 128)) {
+    set_error("selected attention (direct): head_dim=%d with block_size=%d is not supported", head_dim, block_size);
+    return FSA_ERR_UNSUPPORTED;
+  }
   DirectParams p = {};
   p.q = q; p.k = k; p.v = v;
   p.q_sn = q_stride_n; p.q_sh = q_stride_h;
@@ -496,13 +843,14 @@ int selattn_direct_fwd(const void* q, const void* k, const void* v, int32_t dtyp
   p.o_sn = o_stride_n; p.o_sh = o_stride_h;
   p.topk_idx = topk_idx; p.i_sh = idx_stride_h; p.i_sn = idx_stride_n;
   p.cu = cu_seqlens; p.batch = batch; p.hkv = num_kv_heads; p.g = num_q_heads / num_kv_heads; p.g_shift = group_shift(p.g);
+  p.bk_shift = block_size == 32 ? 5 : block_size == 64 ? 6 : 7;
   p.topk = topk; p.max_blk = (int)((max_len + block_size - 1) / block_size); p.n_tokens = total_tokens;
   p.scale_log2 = softmax_scale * LOG2E;
   p.o = o; p.lse = lse; p.merge = merge;
-  const int rc = merge.out ? (dtype == FSA_BF16 ? dispatch_direct_fwd<__bf16, true>(head_dim, block_size, p, stream)
-                                                : dispatch_direct_fwd<_Float16, true>(head_dim, block_size, p, stream))
-                           : (dtype == FSA_BF16 ? dispatch_direct_fwd<__bf16, false>(head_dim, block_size, p, stream)
-                                                : dispatch_direct_fwd<_Float16, false>(head_dim, block_size, p, stream));
+  const int rc = merge.out ? (dtype == FSA_BF16 ? dispatch_direct_fwd<__bf16, true>(head_dim, p, max_len, stream)
+                                                : dispatch_direct_fwd<_Float16, true>(head_dim, p, max_len, stream))
+                           : (dtype == FSA_BF16 ? dispatch_direct_fwd<__bf16, false>(head_dim, p, max_len, stream)
+                                                : dispatch_direct_fwd<_Float16, false>(head_dim, p, max_len, stream));
   if (rc) return rc;
   FSA_CHECK_LAUNCH("fsa_selattn_direct_fwd");
   return 0;

@@ -95,6 +95,39 @@ def test_matches_reference(dev, cu, hq, hkv, d, block, topk, dtype):
     _check(_direct(q, k, v, idx, cut, block, longest), _reference(q, k, v, idx, cut, block), dtype)
 
 
+# Sizes that the rule gives to the kernels of many row tiles: two row tiles and two key groups, four row tiles and one group (at
+# least 3e7 rows x keys).  Row tiles that are not full, whose queries lie in two of them, without keys, of several sequences.
+MANY_ROWS = [
+    # cu_seqlens, Hq, Hkv, D, block, T, dtype, kv heads looked at
+    ([0, 1501], 32, 32, 128, 64, 16, torch.bfloat16, [0, 31]),             # 2 x 2
+    ([0, 1990], 12, 12, 256, 128, 4, torch.float16, [0, 11]),              # 2 x 2
+    ([0, 3100], 24, 8, 64, 32, 8, torch.bfloat16, [3]),                    # 2 x 2, a query in two row tiles
+    ([0, 33, 33, 240], 1536, 512, 128, 32, 5, torch.float16, [0, 511]),    # 1 x 4, the same, an empty sequence
+    ([0, 129, 260], 1024, 1024, 128, 64, 3, torch.bfloat16, [0, 1023]),    # 1 x 4, a row tile of one row
+    ([0, 310], 1200, 20, 64, 64, 4, torch.bfloat16, [0, 19]),              # 1 x 4, group larger than a row tile
+    ([0, 190, 383], 384, 384, 256, 128, 2, torch.bfloat16, [0, 383]),      # 1 x 4
+]
+
+
+@pytest.mark.parametrize("cu,hq,hkv,d,block,topk,dtype,heads", MANY_ROWS)
+@pytest.mark.parametrize("kind", ["plain", "twice", "nan"])
+def test_many_row_tiles(dev, cu, hq, hkv, d, block, topk, dtype, heads, kind):
+    print(f"case {cu} {hq} {hkv} {d} {block} {topk} {dtype} {kind}", flush=True)
+    q, k, v = (x.to(dev) for x in make_qkv(cu[-1], hq, hkv, d, dtype, seed=1, with_do=False))
+    cut = torch.tensor(cu, dtype=torch.int32, device=dev)
+    idx = make_topk_idx(cu, hkv, block, topk, seed=2).to(dev)
+    if kind == "twice":
+        idx[:, ::5, -1] = idx[:, ::5, 0]
+    if kind == "nan":
+        s0 = cu[-2]   # first key of a block: every query that selected the block sees it
+        v[s0 + (cu[-1] - s0) // block // 2 * block] = math.nan
+    o, lse = _direct(q, k, v, idx, cut, block, max(b - a for a, b in zip(cu, cu[1:])))
+    g = hq // hkv
+    for h in heads:
+        mine = slice(h * g, h * g + g)
+        _check((o[:, mine], lse[mine]), _reference(q[:, mine], k[:, h:h + 1], v[:, h:h + 1], idx[h:h + 1], cut, block), dtype)
+
+
 def _odd_lists(n, hkv, block, topk, kind):
     g = torch.Generator().manual_seed(3)
     nb = (n + block - 1) // block
