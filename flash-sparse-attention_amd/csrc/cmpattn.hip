@@ -16,7 +16,7 @@
 // to query i iff i >= j*stride + ks - 1, rows without a visible key give O = 0,
 // LSE = -inf), :195-518 (backward), :832-930 (score), :1006-1158 (transform),
 // :1272-1315 (selection).
-#include "fsa_common.h"
+#include "attn_rows.h"
 #include "dkdv_kernel.h"
 
 #include <algorithm>
@@ -143,15 +143,23 @@ template <int MODE> struct KeyRange {
 };
 
 // ---------------------------------------------------------------- forward ----
-template <typename T, int D, int MODE>
+// Four waves of 32 rows share the tiles of K and V, 32 keys a step, two tiles of each in LDS; the products of one step stand beside
+// the exponentials of another.  What a step takes, about 1 us for the two waves of a SIMD, is less than half of it products; a
+// work-group has 6 us in front of and behind its steps, with one other work-group on the CU to cover them.  Hence q and o by way
+// of LDS, too: a load or store instruction of whole rows touches four of them, not 32 (16384 tokens x 8 heads of 256 138 -> 120
+// us).  Against 64-key tiles by way of the registers, products and exponentials in turn, window of 512 / compressed, us: 5003 x 32
+// heads of 128 74 -> 64 / 37 -> 32, 4 x 8192 x 32 400 -> 362 / 248 -> 221, 5003 x 32 of 64 42 -> 36 / 21 -> 18, 16384 x 8 of 256
+// 148 -> 117 / 129 -> 100.
+template <typename T, int D> struct CmpFwdLds {
+  static constexpr int TILE = TileLoads<T, D>::BYTES, BYTES = 8 * TILE;   // two tiles of K, two of V, one of q / o for every wave
+};
+// ANY: keys or values that are not aligned, or whose rows lie on top of each other.
+template <typename T, int D, int MODE, bool ANY>
 __device__ __forceinline__ void attn_fwd_tile(const CmpParams& p, int id) {
   typedef typename Elem<T>::vec8 vec8;
-  typedef typename Elem<T>::vec4 vec4;
-  constexpr int KS = CmpLds<D>::KS, VS = CmpLds<D>::VS;
-  constexpr int NA = CMP_BK / 32, NKS = D / 16, NDT = D / 32, NJ = CMP_BK / 16;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  T* Ks = reinterpret_cast<T*>(smem);
-  T* Vs = Ks + CMP_BK * KS;
+  typedef TileLoads<T, D, ANY> Loads;
+  constexpr int TILE = Loads::BYTES;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
   int bx, s, h;
   tile_of(p, id, bx, s, h);
@@ -161,148 +169,71 @@ __device__ __forceinline__ void attn_fwd_tile(const CmpParams& p, int id) {
   const int rows_total = lq * p.g;
   const int row_lo = bx * CMP_ROWS;
   if (row_lo >= rows_total) return;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int col = lane & 31, hh = lane >> 5;
-  const int r = row_lo + wv * 32 + col;
-  const bool valid = r < rows_total;
-  const int rr = valid ? r : rows_total - 1;
-  const int qi = rr / p.g, head = rr - qi * p.g;
-  const int hq_i = h * p.g + head;
-  const T* qrow = reinterpret_cast<const T*>(p.q) + (int64_t)(q0 + qi) * p.q_sn + (int64_t)hq_i * p.q_sh + hh * (D / 2);
-  vec8 qreg[NKS];
-#pragma unroll
-  for (int ks = 0; ks < NKS; ++ks) qreg[ks] = load16<vec8>(qrow + ks * 8);
-  // keys visible to this row and to the rows of the work-group
-  const int jmax = KeyRange<MODE>::hi(p, qi, nc), jmin = KeyRange<MODE>::lo(p, qi);
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 31, hh = lane >> 5;
+  const int row = row_lo + wv * 32 + col;
+  const bool valid = row < rows_total;
+  const int rr = valid ? row : rows_total - 1;
+  const int qi = rr / p.g, hq_i = h * p.g + rr - qi * p.g;
+  // the range of keys of the work-group, in steps of 32
   const int qi_first = row_lo / p.g, qi_last = (min(rows_total, row_lo + CMP_ROWS) - 1) / p.g;
-  const int n_keys = KeyRange<MODE>::hi(p, qi_last, nc) + 1;                 // end of the work-group's key range
-  const int jt0 = KeyRange<MODE>::lo(p, qi_first) / CMP_BK * CMP_BK;          // its tile-aligned start
-
-  const T* kbase = reinterpret_cast<const T*>(p.k) + (int64_t)h * p.k_sh;
-  const T* vbase = reinterpret_cast<const T*>(p.v) + (int64_t)h * p.v_sh;
-  const uint32_t k_off = kv_tile_offset<T, D>(p.k_sn, tid), v_off = kv_tile_offset<T, D>(p.v_sn, tid);
-  const T* vtr = Vs + (4 * hh + ((lane & 15) >> 2)) * VS + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-
-  float m = -INFINITY, l = 0.f;  // m in raw (unscaled) score units
-  f32x16 oacc[NDT];
-#pragma unroll
-  for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
-
-  // K and V fragments that are requested ahead of their products.  At head_dim 64 the registers for them would take the
-  // compressed branch on its own from three waves per SIMD to two (168 -> 178 registers; 32 + 8 heads, ahead / not: 5003
-  // tokens 21.6 / 20.1 us, 16384 109 / 98; window 118.1 / 118.7, both branches in one launch 214.5 / 214.5).  At head_dim 256
-  // (8 + 2 heads) ahead is 9-10 % faster in the window (5003 tokens 68.2 / 75.9 us) and 5-9 % for both branches in one launch;
-  // the compressed branch on its own is 6 % faster at 16384 tokens (129 / 138), 2-3 % slower at 2000 and 5003 (26.3 / 25.7): of
-  // the other form the compiler peels the first tile.  That is why the first tile skips the rescaling below, without which it
-  // is 5 % slower there (27.1).  At head_dim 64 that skip would let the window run three waves per SIMD (5003 tokens x 32
-  // heads, both branches 66 -> 59 us, but 2000 tokens 28.6 -> 30.7).
-  constexpr int KAHEAD = D == 64 ? 0 : 2, VAHEAD = D == 64 ? 0 : 3;
-  constexpr bool PREFETCH = D <= 128;  // the next tile waits in registers where the budget allows
-  KvTileRegs<T, D> nxt;
-  if (PREFETCH && jt0 < n_keys) kv_tile_load<T, D>(nxt, kbase, p.k_sn, k_off, vbase, p.v_sn, v_off, k0 + jt0, nc - jt0, tid);
-  for (int jt = jt0; jt < n_keys; jt += CMP_BK) {
-    if (jt != jt0) __syncthreads();
-    if (PREFETCH) {
-      kv_tile_store<T, D>(nxt, Ks, Vs, tid);
-      if (jt + CMP_BK < n_keys)
-        kv_tile_load<T, D>(nxt, kbase, p.k_sn, k_off, vbase, p.v_sn, v_off, k0 + jt + CMP_BK, nc - jt - CMP_BK, tid);
-    } else {
-      stage_kv_tile<T, D>(kbase, p.k_sn, k_off, vbase, p.v_sn, v_off, k0 + jt, nc - jt, Ks, Vs, tid);
-    }
-    __syncthreads();
-    f32x16 acc[NA];
-#pragma unroll
-    for (int a = 0; a < NA; ++a)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[a][i] = 0.f;
-    // Fragments are requested KAHEAD k-steps before their products, and in this order: left to itself the compiler asks for
-    // them right before, and the wave waits for LDS at every pair of products (5003 tokens, 32 + 8 heads of 128: 111 -> 107 us
-    // for both branches).
-    vec8 kf[KAHEAD + 1][NA];
-    auto k_read = [&](int ks) {
-#pragma unroll
-      for (int a = 0; a < NA; ++a) kf[ks % (KAHEAD + 1)][a] = load16<vec8>(&Ks[(a * 32 + col) * KS + hh * (D / 2) + ks * 8]);
-    };
-#pragma unroll
-    for (int ks = 0; ks < KAHEAD; ++ks) k_read(ks);
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      if (ks + KAHEAD < NKS) k_read(ks + KAHEAD);
-#pragma unroll
-      for (int a = 0; a < NA; ++a) acc[a] = Elem<T>::mfma32(kf[ks % (KAHEAD + 1)][a], qreg[ks], acc[a]);
-      if (KAHEAD > 0) __builtin_amdgcn_sched_barrier(0);
-    }
-    vec8 vf[VAHEAD + 1];
-    auto v_read = [&](int i) { vf[i % (VAHEAD + 1)] = lds_read_tr8<T>(vtr + 16 * (i / NDT) * VS + i % NDT * 32, 8 * VS); };
-#pragma unroll
-    for (int i = 0; i < VAHEAD; ++i) v_read(i);   // (they arrive during the softmax)
-    const int limit = jmax - jt, limit_lo = jmin - jt;
-    float mx = m;
-    // tiles that every row of the wave sees completely need no mask
-    if (!__all(limit >= CMP_BK - 1 && limit_lo <= 0)) {
-#pragma unroll
-      for (int a = 0; a < NA; ++a)
+  const int jt0 = __builtin_amdgcn_readfirstlane(KeyRange<MODE>::lo(p, qi_first) & ~31);
+  const int n_steps = __builtin_amdgcn_readfirstlane((KeyRange<MODE>::hi(p, qi_last, nc) + 1 - jt0 + 31) >> 5);
+  const Loads kl(p.k, p.k_sn, p.k_sh, k0, h, nc), vl(p.v, p.v_sn, p.v_sh, k0, h, nc);
+  const uint32_t k_lds = lds_addr(smem), v_lds = k_lds + 2 * TILE;
+  // this wave's share of a tile: even waves K, odd ones V, each half a tile where that has loads enough
+  constexpr int PARTS = Loads::N >= 2 * Loads::NV ? 2 : 1;
+  auto issue_k = [&](int t) {
+    if ((wv & 1) == 0 && wv < 2 * PARTS) kl.template issue<PARTS>(jt0 + 32 * t, k_lds + (t & 1) * TILE, wv >> 1);
+  };
+  auto issue_v = [&](int t) {
+    if ((wv & 1) == 1 && wv < 2 * PARTS) vl.template issue<PARTS>(jt0 + 32 * t, v_lds + (t & 1) * TILE, wv >> 1);
+  };
+  AttnRows<T, D> r;
+  r.scale_log2 = p.scale_log2;
+  r.clear();
+  T* rows_lds = reinterpret_cast<T*>(smem + (4 + wv) * TILE);
+  if (n_steps > 0) {
+    issue_k(0);
+    issue_v(0);
+    issue_k(1);
+    const int jmax = KeyRange<MODE>::hi(p, qi, nc) - jt0, jmin = KeyRange<MODE>::lo(p, qi) - jt0;
+    auto mask = [&](f32x16& x, int t) {   // a step that every row of the wave sees completely needs none
+      const int limit = jmax - 32 * t, limit_lo = jmin - 32 * t;
+      if (!__all(limit >= 31 && limit_lo <= 0)) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const int key = a * 32 + 8 * (i >> 2) + 4 * hh + (i & 3);
-          if (!(key <= limit && key >= limit_lo)) acc[a][i] = -INFINITY;
+          const int key = 8 * (i >> 2) + 4 * hh + (i & 3);
+          if (!(key <= limit && key >= limit_lo)) x[i] = -INFINITY;
         }
-    }
-#pragma unroll
-    for (int a = 0; a < NA; ++a)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, acc[a][i]);
-    mx = max32(mx);
-    // The reference maximum m moves only when some row of the wave outgrows it by more than 2^8: until then
-    // the probabilities are taken relative to the older, smaller maximum (at most 256, exact in the final
-    // quotient) and the accumulators need no rescaling.  (-inf) - (-inf) is NaN and compares false.
-    if (D == 256 && jt == jt0) {
-      m = mx;   // nothing to rescale yet
-    } else if (__any((mx - m) * p.scale_log2 > 8.f)) {
-      // m = -inf -> 0; a row that keeps its maximum -> 1; a row that has seen no key yet has nothing to rescale
-      const float alpha = mx == -INFINITY ? 1.f : exp2f((m - mx) * p.scale_log2);
-      l *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) oacc[dt][i] *= alpha;
-      m = mx;
-    }
-    const float mref = (m == -INFINITY) ? 0.f : m * p.scale_log2;
-    float lsum = 0.f;
-    vec8 pk[NJ];
-#pragma unroll
-    for (int a = 0; a < NA; ++a)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float pv = fast_exp2(acc[a][i] * p.scale_log2 - mref);
-        lsum += pv;
-        pk[a * 2 + (i >> 3)][i & 7] = (T)pv;
       }
-    l += lsum;   // the lane's own keys: the two lanes of a row are added behind the loop
-#pragma unroll
-    for (int i = 0; i < NJ * NDT; ++i) {
-      if (i + VAHEAD < NJ * NDT) v_read(i + VAHEAD);
-      oacc[i % NDT] = Elem<T>::mfma32(vf[i % (VAHEAD + 1)], pk[i / NDT], oacc[i % NDT]);
-      if (VAHEAD > 0) __builtin_amdgcn_sched_barrier(0);
+    };
+    const TileFrags<D> f;
+    r.load_q_rows(reinterpret_cast<const T*>(p.q) + (int64_t)(q0 + qi) * p.q_sn + (int64_t)hq_i * p.q_sh, rows_lds, f);
+    vec8 pk[2];
+    auto step = [&](f32x16& x, f32x16& next, int t) {   // scores of this step in x, those of the next one into `next`
+      tiles_arrived();   // K of the next step, V of this one
+      issue_k(t + 2);    // (behind the last key: zeros, and nothing is read)
+      issue_v(t + 1);
+      r.template scores<true>(next, x, r.reference(true), pk, k_lds + ((t + 1) & 1) * TILE, f);
+      mask(next, t + 1);
+      r.raise(r.values(next, pk, v_lds + (t & 1) * TILE, f), true);
+    };
+    f32x16 sa, sb;
+    tiles_arrived();
+    r.template scores<false>(sa, sb, 0.f, pk, k_lds, f);
+    mask(sa, 0);
+    r.raise(r.lane_max(sa), true);
+    for (int t = 0;;) {
+      step(sa, sb, t);
+      if (++t >= n_steps) break;
+      step(sb, sa, t);
+      if (++t >= n_steps) break;
     }
+    vm_wait<0>();
   }
-  l = sum32(l);
-  if (!valid) return;
-  const float inv_l = l > 0.f ? 1.f / l : 0.f;
-  T* orow = reinterpret_cast<T*>(p.o) + (int64_t)(q0 + qi) * p.o_sn + (int64_t)hq_i * p.o_sh + 4 * hh;
-#pragma unroll
-  for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-    for (int qd = 0; qd < 4; ++qd) {
-      vec4 x;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] = (T)(oacc[dt][4 * qd + e] * inv_l);
-      store8(orow + dt * 32 + 8 * qd, x);
-    }
-  if (hh == 0) p.lse[(int64_t)hq_i * p.n_tokens + q0 + qi] = l > 0.f ? m * p.scale_log2 + log2f(l) : -INFINITY;
+  r.l = sum32(r.l);
+  r.store_rows(reinterpret_cast<T*>(p.o) + (int64_t)(q0 + qi) * p.o_sn + (int64_t)hq_i * p.o_sh, valid, r.l > 0.f ? 1.f / r.l : 0.f, rows_lds);
+  if (valid && hh == 0) p.lse[(int64_t)hq_i * p.n_tokens + q0 + qi] = r.l > 0.f ? r.mref + log2f(r.l) : -INFINITY;
 }
 
 // --------------------------------------------------------------------- dq ----
@@ -422,10 +353,10 @@ __device__ __forceinline__ void attn_bwd_dq_tile(const CmpParams& p, int id) {
     }
 }
 
-template <typename T, int D, int MODE>
+template <typename T, int D, int MODE, bool ANY>
 __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1))
 cmpattn_fwd_kernel(CmpParams p) {
-  attn_fwd_tile<T, D, MODE>(p, blockIdx.x);
+  attn_fwd_tile<T, D, MODE, ANY>(p, blockIdx.x);
 }
 template <typename T, int D, int MODE>
 __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1))
@@ -434,11 +365,11 @@ cmpattn_bwd_dq_kernel(CmpParams p) {
 }
 // Compressed (blockIdx.z == 0, in front) and window attention of one layer in one launch.  At small sizes either alone
 // leaves most of the chip idle.
-template <typename T, int D>
+template <typename T, int D, bool ANY>
 __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1))
 attn_fwd_pair_kernel(CmpParams a, CmpParams b) {
-  if (blockIdx.z == 0) attn_fwd_tile<T, D, CMP_MODE_COMPRESSED>(a, blockIdx.x);
-  else attn_fwd_tile<T, D, CMP_MODE_WINDOW>(b, blockIdx.x);
+  if (blockIdx.z == 0) attn_fwd_tile<T, D, CMP_MODE_COMPRESSED, ANY>(a, blockIdx.x);
+  else attn_fwd_tile<T, D, CMP_MODE_WINDOW, ANY>(b, blockIdx.x);
 }
 template <typename T, int D>
 __global__ void __launch_bounds__(256)
@@ -887,16 +818,27 @@ static CmpBwdWs cmp_bwd_ws(int64_t n, int64_t n_k, int64_t max_q, int batch, int
   return w;
 }
 
-template <typename T, int D, int MODE>
-static int attn_fwd_launch(CmpParams p, int batch, int hkv, int64_t max_rows, hipStream_t stream) {
+// Whether keys and values can go to LDS past the registers: rows 16-byte aligned, and none on top of another.
+static bool rows_go_straight(const CmpParams& p, int d) {
+  auto ok = [&](const void* x, int64_t sn, int64_t sh) { return ((uintptr_t)x % 16 | (sn | sh) % 8) == 0 && sn >= d; };
+  return ok(p.k, p.k_sn, p.k_sh) && ok(p.v, p.v_sn, p.v_sh);
+}
+
+template <typename T, int D, int MODE, bool ANY>
+static int attn_fwd_launch_as(CmpParams p, int batch, int hkv, int64_t max_rows, hipStream_t stream) {
   static LdsAllowed lds;
-  if (int rc_ = allow_lds(lds, (const void*)cmpattn_fwd_kernel<T, D, MODE>, CmpLds<D>::BYTES)) return rc_;
+  if (int rc_ = allow_lds(lds, (const void*)cmpattn_fwd_kernel<T, D, MODE, ANY>, CmpFwdLds<T, D>::BYTES)) return rc_;
   p.hkv = hkv;
   p.nx = (int)((max_rows + CMP_ROWS - 1) / CMP_ROWS);
   const dim3 grid = dense_grid(p.nx, hkv, batch);
   ProfScope ps_(MODE == CMP_MODE_WINDOW ? "winattn_fwd" : "cmpattn_fwd", stream);
-  cmpattn_fwd_kernel<T, D, MODE><<<grid, 256, CmpLds<D>::BYTES, stream>>>(p);
+  cmpattn_fwd_kernel<T, D, MODE, ANY><<<grid, 256, CmpFwdLds<T, D>::BYTES, stream>>>(p);
   return 0;
+}
+template <typename T, int D, int MODE>
+static int attn_fwd_launch(const CmpParams& p, int batch, int hkv, int64_t max_rows, hipStream_t stream) {
+  return rows_go_straight(p, D) ? attn_fwd_launch_as<T, D, MODE, false>(p, batch, hkv, max_rows, stream)
+                                : attn_fwd_launch_as<T, D, MODE, true>(p, batch, hkv, max_rows, stream);
 }
 template <typename T, int D>
 static int cmp_fwd_launch(const CmpParams& p, int batch, int hkv, int64_t max_rows, hipStream_t stream) {
@@ -943,15 +885,20 @@ static int attn_bwd_launch(CmpParams p, const SelBwdParams& kv, int batch, int h
   return 0;
 }
 
-template <typename T, int D>
-static int pair_fwd_launch(CmpParams a, CmpParams b, int batch, int hkv, int64_t max_rows, hipStream_t stream) {
+template <typename T, int D, bool ANY>
+static int pair_fwd_launch_as(CmpParams a, CmpParams b, int batch, int hkv, int64_t max_rows, hipStream_t stream) {
   static LdsAllowed lds;
-  if (int rc_ = allow_lds(lds, (const void*)attn_fwd_pair_kernel<T, D>, CmpLds<D>::BYTES)) return rc_;
+  if (int rc_ = allow_lds(lds, (const void*)attn_fwd_pair_kernel<T, D, ANY>, CmpFwdLds<T, D>::BYTES)) return rc_;
   a.hkv = b.hkv = hkv;
   a.nx = b.nx = (int)((max_rows + CMP_ROWS - 1) / CMP_ROWS);
   ProfScope ps_("attn_fwd_pair", stream);
-  attn_fwd_pair_kernel<T, D><<<dense_pair_grid(a.nx, hkv, batch), 256, CmpLds<D>::BYTES, stream>>>(a, b);
+  attn_fwd_pair_kernel<T, D, ANY><<<dense_pair_grid(a.nx, hkv, batch), 256, CmpFwdLds<T, D>::BYTES, stream>>>(a, b);
   return 0;
+}
+template <typename T, int D>
+static int pair_fwd_launch(const CmpParams& a, const CmpParams& b, int batch, int hkv, int64_t max_rows, hipStream_t stream) {
+  return rows_go_straight(a, D) && rows_go_straight(b, D) ? pair_fwd_launch_as<T, D, false>(a, b, batch, hkv, max_rows, stream)
+                                                          : pair_fwd_launch_as<T, D, true>(a, b, batch, hkv, max_rows, stream);
 }
 template <typename T, int D>
 static int pair_bwd_launch(CmpParams a, CmpParams b, const SelBwdParams& ka, const SelBwdParams& kb, const KvTiles& ta,

@@ -10,7 +10,7 @@
 //   narrow  few row tiles: a work-group takes one, its KG waves share out the visited keys, each with K / V buffers of its own,
 //           so there is no barrier between the first step and the merge of the partial results in LDS.
 //   wide    many row tiles: a work-group takes RT of them, whose waves go through the keys together and share every tile.
-#include "fsa_common.h"
+#include "attn_rows.h"
 
 #include <algorithm>
 #include <cmath>
@@ -35,16 +35,6 @@ struct DirectParams {
 
 constexpr int DIR_MAX_BLOCKS = 1024; // of a sequence: size of the tables in LDS
 
-// Four KB of a tile, global memory to LDS: lane l's 16 bytes at voff[j](l) + 1024 j of the buffer land at LDS byte
-// `lds` + 1024 j + 16 l (the instruction's offset moves both addresses).
-__device__ __forceinline__ void lds_dma4(__amdgpu_buffer_rsrc_t rsrc, const uint32_t* voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %5\n\ts_nop 0\n\t"
-               "buffer_load_dwordx4 %0, %4, 0 offen lds\n\t"
-               "buffer_load_dwordx4 %1, %4, 0 offen offset:1024 lds\n\t"
-               "buffer_load_dwordx4 %2, %4, 0 offen offset:2048 lds\n\t"
-               "buffer_load_dwordx4 %3, %4, 0 offen offset:3072 lds"
-               :: "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(rsrc), "s"(lds) : "memory");
-}
 // A row tile.  The rows of the whole buffer are dealt out, so that none of o and lse stays unwritten where the sequences do not
 // fill it: segment i runs from cu[i - 1] to cu[i], with the start of the buffer in front and its end behind.  Segment 0, in
 // front of the first sequence, has no keys; the last one holds the last sequence and, as queries at the positions behind it,
@@ -83,181 +73,13 @@ __device__ __forceinline__ bool direct_tile(const int32_t* __restrict__ cu, int 
   return false;
 }
 
-// Tiles of 32 K or V rows of a sequence and kv head on their way to LDS.
-template <typename T, int D> struct DirectLoads {
-  static constexpr int CPR = D / 8, RPI = 64 / CPR, N = 32 / RPI;   // 16-byte chunks per row, rows per load, loads per tile
-  static constexpr int NV = RPI >= 4 ? 4 : 16 / RPI;   // lane offsets: 16 rows or more, after which chunk_swizzle repeats itself
-  static constexpr int BYTES = 32 * D * 2;
-  const char* base;
-  uint32_t row_bytes, voff[NV];   // (host: a head's rows span < 2^31 bytes)
-  int len;
-  __device__ __forceinline__ DirectLoads(const void* x, int64_t sn, int64_t sh, int q0, int h, int len_) : len(len_) {
-    base = reinterpret_cast<const char*>(reinterpret_cast<const T*>(x) + (int64_t)q0 * sn + (int64_t)h * sh);
-    row_bytes = (uint32_t)sn * 2;
-    const int lane = threadIdx.x & 63, ld_row = lane / CPR, ld_chunk = lane % CPR;
-    // The loading lane picks its source so that the chunks land where chunk_swizzle wants them.  (host: rows are at least 2 D
-    // bytes apart, so the difference is not negative)
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      const int r = j * RPI + ld_row;
-      voff[j] = r * row_bytes + (ld_chunk ^ chunk_swizzle<D>(r)) * 16 - (j & 3) * 1024;
-    }
-  }
-  // PARTS > 1: one of as many equal shares of the loads.  Rows behind the end of the sequence are out of the range of the
-  // descriptors and arrive as zeros: no query of the sequence sees them; one at a position behind it does, with score 0, as in
-  // the block-major kernels.
-  template <int PARTS = 1> __device__ __forceinline__ void issue(int key, uint32_t to, int part = 0) const {
-    static_assert(N / PARTS >= NV, "a share has whole descriptors");
-#pragma unroll
-    for (int i = 0; i < N / PARTS; i += NV) {
-      const int j0 = part * (N / PARTS) + i, first = key + j0 * RPI;
-      const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<char*>(base + (uint64_t)(uint32_t)first * row_bytes), 0, (int)((uint32_t)max(len - first, 0) * row_bytes), 0x00020000);
-#pragma unroll
-      for (int j = 0; j < NV; j += 4) lds_dma4(rsrc, &voff[j], to + (j0 + j) * 1024);
-    }
-  }
-};
-
-// Fragments of the tiles, relative to a tile's start: k-step ks of K at k ^ 16 ks, 32 dims from 32 dt of V at v ^ 64 dt.
-template <int D> struct DirectFrags {
-  uint32_t k, v;
-  __device__ __forceinline__ DirectFrags() {
-    const int lane = threadIdx.x & 63, col = lane & 31, hh = lane >> 5, vr = 4 * hh + ((lane & 15) >> 2);
-    k = col * (D * 2) + (((hh * (D / 16)) ^ chunk_swizzle<D>(col)) << 4);
-    v = vr * (D * 2) + (((2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ chunk_swizzle<D>(vr)) << 4) + (lane & 1) * 8;
-  }
-};
-
-// What a wave keeps of its row tile: one row per pair of lanes (col, col + 32).
-template <typename T, int D> struct DirectRows {
-  typedef typename Elem<T>::vec8 vec8;
-  static constexpr int NKS = D / 16, NDT = D / 32;
-  float scale_log2;
-  int qpos;               // position of the lane's query
-  vec8 q[NKS];            // dims hh D/2 + 8 ks .. + 7
-  float mref, l;          // reference maximum (scaled scores), sum
-  f32x16 o[NDT];
-
-  __device__ __forceinline__ void load_q(const DirectParams& p, int q0, int h, int row) {
-    const T* r = reinterpret_cast<const T*>(p.q) + (int64_t)(q0 + qpos) * p.q_sn + (int64_t)(h * p.g + row - qpos * p.g) * p.q_sh +
-                 ((threadIdx.x & 63) >> 5) * (D / 2);
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) q[ks] = load16<vec8>(r + ks * 8);
-  }
-  // q settled: otherwise the compiler waits for it where it is used first, inside the loop and in every step of it, and with it
-  // for the tile that was requested a moment before
-  __device__ __forceinline__ void settle_q() {
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) asm volatile("" : "+v"(q[ks]));
-  }
-  __device__ __forceinline__ void clear() {
-    mref = -INFINITY;
-    l = 0.f;
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
-  }
-  __device__ __forceinline__ void causal(f32x16& s, int key) const {
-    const int limit = qpos - key, hh = (threadIdx.x & 63) >> 5;
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-      if (8 * (i >> 2) + 4 * hh + (i & 3) > limit) s[i] = -INFINITY;
-  }
-  static __device__ __forceinline__ float lane_max(const f32x16& s) {
-    float mx = s[0];
-#pragma unroll
-    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
-    return mx;
-  }
-  // the reference maximum after scores whose maximum over the lane's own keys is mx
-  __device__ __forceinline__ void raise(float mx, bool on) {
-    mx = max32(mx) * scale_log2;
-    asm volatile("" : "+v"(mx));   // (a select, not a branch over what was computed above)
-    mx = on ? mx : -INFINITY;
-    // a row that has seen no key yet takes its first maximum as it is: there is nothing to rescale
-    mref = mref == -INFINITY ? mx : mref;
-    // as in the dense kernels: the reference maximum moves only when some row outgrows it by more than 2^8
-    if (__builtin_expect(__any(mx > mref + 8.f), 0)) {
-      const float top = fmaxf(mref, mx), alpha = top == -INFINITY ? 1.f : fast_exp2(mref - top);
-      l *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
-      mref = top;
-    }
-  }
-  __device__ __forceinline__ float reference(bool on) const { return !on ? INFINITY : mref == -INFINITY ? 0.f : mref; }   // 2^(s - inf) = 0
-  __device__ __forceinline__ bool has_nan() const {
-    float x = l;
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) x += o[dt][i];
-    return x != x;
-  }
-  // A step of the second pass, K and V through the wave's own 2 tiles at LDS address `own`: a block that a query did not select
-  // must not reach it at all (a key or value of it that is infinite or NaN makes 0 * x NaN in the products), and a block that a
-  // list names several times (`times`) counts as often.
-  __device__ __forceinline__ void step_carefully(const DirectLoads<T, D>& k, const DirectLoads<T, D>& v, const DirectFrags<D>& f, uint32_t own,
-                                                 int key, bool on, float times) {
-    k.issue(key, own);
-    v.issue(key, own + k.BYTES);
-    vm_wait<0>();
-    f32x16 s;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) s = Elem<T>::mfma32(load16<vec8>(lds_ptr<T>(own + (f.k ^ (16u * ks)))), q[ks], s);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] = on ? s[i] : -INFINITY;
-    causal(s, key);
-    raise(lane_max(s), on);
-    const float ref = reference(on);
-    vec8 pk[2];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float pv = on ? fast_exp2(s[i] * scale_log2 - ref) * times : 0.f;
-      l += pv;
-      pk[i >> 3][i & 7] = (T)pv;
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int dt = 0; dt < NDT; ++dt) {
-        const f32x16 x = Elem<T>::mfma32(swizzled_tr_frag<T, D>(own + k.BYTES + (f.v ^ (64u * dt)), j), pk[j], o[dt]);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) o[dt][i] = on ? x[i] : o[dt][i];
-      }
-    lds_reads_done();
-  }
-  // the wave's partial result: [32][D] fp32, 16-byte chunk c of row r at c ^ r; reference and sum to st_m[r], st_l[r]
-  static constexpr int XM = D / 4 - 1 < 31 ? D / 4 - 1 : 31;
-  __device__ __forceinline__ void park(float* part, float* st_m, float* st_l) const {
-    const int lane = threadIdx.x & 63, col = lane & 31, hh = lane >> 5;
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int qd = 0; qd < 4; ++qd) {
-        const int c = (dt * 8 + 2 * qd + hh) ^ (col & XM);
-        *reinterpret_cast<f32x4*>(part + col * D + c * 4) = f32x4{o[dt][4 * qd], o[dt][4 * qd + 1], o[dt][4 * qd + 2], o[dt][4 * qd + 3]};
-      }
-    if (hh == 0) {
-      st_m[col] = mref;
-      st_l[col] = l;
-    }
-  }
-};
-
 // Chunk `sub` (8 dims) of row r of a row tile, from the partial results of KG waves: partial w at part + w * part_step bytes,
 // its statistics at st_m + w * st_step.
 template <typename T, int D, bool MERGE, int KG>
 __device__ __forceinline__ void direct_store(const DirectParams& p, int h, int q0, int row, int r, int sub, const unsigned char* part, int part_step,
                                              const float* st_m, const float* st_l, int st_step) {
   typedef typename Elem<T>::vec8 vec8;
-  constexpr int XM = DirectRows<T, D>::XM;
+  constexpr int XM = AttnRows<T, D>::XM;
   float mw[KG], mx = -INFINITY;
 #pragma unroll
   for (int w = 0; w < KG; ++w) {
@@ -328,7 +150,7 @@ __global__ void __launch_bounds__(64 * KG, D <= 128 ? 2 : 1)
 selattn_direct_narrow_kernel(DirectParams p) {
   typedef typename Elem<T>::vec8 vec8;
   typedef NarrowLds<D, KG> L;
-  typedef DirectLoads<T, D> Loads;
+  typedef TileLoads<T, D> Loads;
   constexpr int NKS = D / 16, NDT = D / 32, NT = 64 * KG, NLD = Loads::N;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   float* st_m = reinterpret_cast<float*>(smem + KG * L::WAVE_BYTES);   // [wave][row]
@@ -345,12 +167,12 @@ selattn_direct_narrow_kernel(DirectParams p) {
   const int n_blk = min((q_last >> bks) + 1, (len + (1 << bks) - 1) >> bks);
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 31;
 
-  DirectRows<T, D> r;
+  AttnRows<T, D> r;
   r.scale_log2 = p.scale_log2;
   {
     const int row = min(row0 + col, rows - 1);
     r.qpos = div_group(row, p.g, p.g_shift);
-    r.load_q(p, q0, h, row);
+    r.load_q(reinterpret_cast<const T*>(p.q) + (int64_t)(q0 + r.qpos) * p.q_sn + (int64_t)(h * p.g + row - r.qpos * p.g) * p.q_sh);
   }
   const int qoff = r.qpos - q_first;
   const Loads kl(p.k, p.k_sn, p.k_sh, q0, h, len), vl(p.v, p.v_sn, p.v_sh, q0, h, len);
@@ -409,7 +231,7 @@ selattn_direct_narrow_kernel(DirectParams p) {
   const int upb_shift = bks - 5;   // log2 of the steps of 32 keys per block
   const int n_units = __builtin_amdgcn_readfirstlane(info[0]) << upb_shift;
   const int n_steps = (n_units - wv + KG - 1) / KG;   // of this wave
-  const DirectFrags<D> f;
+  const TileFrags<D> f;
   auto place = [&](int t) { return wv + KG * min(t, n_steps - 1); };   // in the list of steps
   auto key_of = [&](int u, int b) { return (b << bks) + (u & ((1 << upb_shift) - 1)) * 32; };
 
@@ -514,7 +336,7 @@ __global__ void __launch_bounds__(64 * KG * RT, D <= 128 ? 2 : 1)
 selattn_direct_wide_kernel(DirectParams p) {
   typedef typename Elem<T>::vec8 vec8;
   typedef WideLds<D, KG, RT> L;
-  typedef DirectLoads<T, D> Loads;
+  typedef TileLoads<T, D> Loads;
   constexpr int ROWS = 32 * RT, NKS = D / 16, NDT = D / 32, NT = 64 * L::WAVES;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   float* st_m = reinterpret_cast<float*>(smem + KG * L::GROUP_BYTES);   // [wave][32]
@@ -532,12 +354,12 @@ selattn_direct_wide_kernel(DirectParams p) {
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 31;
   const int rt = wv % RT, kg = wv / RT;
 
-  DirectRows<T, D> r;
+  AttnRows<T, D> r;
   r.scale_log2 = p.scale_log2;
   {
     const int row = min(row0 + 32 * rt + col, rows - 1);
     r.qpos = div_group(row, p.g, p.g_shift);
-    r.load_q(p, q0, h, row);
+    r.load_q(reinterpret_cast<const T*>(p.q) + (int64_t)(q0 + r.qpos) * p.q_sn + (int64_t)(h * p.g + row - r.qpos * p.g) * p.q_sh);
   }
   const int q_tile = div_group(min(row0 + 32 * rt, rows - 1), p.g, p.g_shift), qoff = r.qpos - q_tile;
   const Loads kl(p.k, p.k_sn, p.k_sh, q0, h, len), vl(p.v, p.v_sn, p.v_sh, q0, h, len);
@@ -622,17 +444,14 @@ selattn_direct_wide_kernel(DirectParams p) {
     if (u >= n_units) x.mask = 0;
     return x;
   };
-  const DirectFrags<D> f;
+  const TileFrags<D> f;
 
-  // S of a step stands beside the exponentials of the step before, the products with V beside the maxima: a wave has work for
-  // the matrix and for the vector unit at any time.
   auto attend = [&]() {
     r.clear();
     if (n_steps <= 0) {
       vm_wait<0>();
       return;
     }
-    constexpr int KA = 2, VA = 3;   // fragments requested ahead
     Unit cur = unit(0), nx1 = unit(1);
     if (cur.key != guess) {
       vm_wait<0>();   // (what is on its way would land in what comes now)
@@ -641,58 +460,17 @@ selattn_direct_wide_kernel(DirectParams p) {
     }
     issue_k(nx1.key, 1);
     int key2 = unit(2).key, b2 = key2 >> bks;
-    vec8 kf[KA + 1], vf[VA + 1], pk[2];
-    float ref, sum;
-    auto arrived = [&]() {   // the loads of all waves, and the reads of all waves from what is overwritten next
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    };
-    auto scores = [&](f32x16& next, f32x16& s, int stage, auto exps_) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) next[i] = 0.f;
-      auto k_read = [&](int ks) { kf[ks % (KA + 1)] = load16<vec8>(lds_ptr<T>(k_lds + (f.k ^ (16u * ks)) + stage * L::TILE)); };
-#pragma unroll
-      for (int ks = 0; ks < KA; ++ks) k_read(ks);
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) {
-        if (ks + KA < NKS) k_read(ks + KA);
-        next = Elem<T>::mfma32(kf[ks % (KA + 1)], r.q[ks], next);
-        if constexpr (decltype(exps_)::value) {
-#pragma unroll
-          for (int i = ks * 16 / NKS; i < (ks + 1) * 16 / NKS; ++i) {
-            const float pv = fast_exp2(s[i] * r.scale_log2 - ref);
-            sum += pv;
-            pk[i >> 3][i & 7] = (T)pv;
-            if ((i & 7) == 7) asm volatile("" : "+v"(pk[i >> 3]), "+v"(sum));   // (here, not in front of its use)
-          }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    };
+    vec8 pk[2];
     auto step = [&](f32x16& s, f32x16& next, int t) {   // scores of this step in s, those of the next one into `next`
       const int odd = t & 1;
-      arrived();   // K of the next step, V of this one
+      tiles_arrived();   // K of the next step, V of this one
       issue_k(key2, odd);
       issue_v(nx1.key, odd ^ 1);
       // asked for here, looked at behind the products: the mask of step t + 2, the block of step t + 3
       const uint32_t mask2 = sel[RT * b2 + rt], u3 = min(kg + KG * (t + 3), n_units - 1), b3 = list[u3 >> upb_shift];
-      ref = r.reference(cur.mask >> qoff & 1);
-      sum = 0.f;
-      scores(next, s, odd ^ 1, std::true_type{});
-      r.l += sum;   // the lane's own keys: the two lanes of a row are added behind the loop
+      r.template scores<true>(next, s, r.reference(cur.mask >> qoff & 1), pk, k_lds + (odd ^ 1) * L::TILE, f);
       if (__builtin_expect(nx1.key + 31 > q_first, 0)) r.causal(next, nx1.key);   // some row may see the keys partly
-      auto v_read = [&](int i) { vf[i % (VA + 1)] = swizzled_tr_frag<T, D>(v_lds + (f.v ^ (64u * (i % NDT))) + odd * L::TILE, i / NDT); };
-#pragma unroll
-      for (int i = 0; i < VA; ++i) v_read(i);
-      float mx = -INFINITY;
-#pragma unroll
-      for (int i = 0; i < 2 * NDT; ++i) {
-        if (i + VA < 2 * NDT) v_read(i + VA);
-        r.o[i % NDT] = Elem<T>::mfma32(vf[i % (VA + 1)], pk[i / NDT], r.o[i % NDT]);
-#pragma unroll
-        for (int x = i * 8 / NDT; x < (i + 1) * 8 / NDT; ++x) mx = fmaxf(mx, next[x]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      r.raise(mx, nx1.mask >> qoff & 1);
+      r.raise(r.values(next, pk, v_lds + odd * L::TILE, f), nx1.mask >> qoff & 1);
       cur = nx1;
       nx1.key = key2;
       nx1.mask = kg + KG * (t + 2) < n_units ? (uint32_t)__builtin_amdgcn_readfirstlane((int)mask2) : 0u;
@@ -700,8 +478,8 @@ selattn_direct_wide_kernel(DirectParams p) {
       key2 = (b2 << bks) + (u3 & ((1 << upb_shift) - 1)) * 32;
     };
     f32x16 sa, sb;
-    arrived();
-    scores(sa, sb, 0, std::false_type{});
+    tiles_arrived();
+    r.template scores<false>(sa, sb, 0.f, pk, k_lds, f);
     if (cur.key + 31 > q_first) r.causal(sa, cur.key);
     r.raise(r.lane_max(sa), cur.mask >> qoff & 1);
     for (int t = 0;;) {

@@ -98,3 +98,33 @@ def test_winattn_drifting_scores(dev, direction):
         print(f"  {name}: rel Frobenius {rel:.2e}, max excess {excess:.3e}", flush=True)
         assert rel < 1e-2, name
         assert excess <= 2 * TOL[dtype] * max(1.0, ref.abs().max().item()), name
+
+
+@pytest.mark.parametrize("d,dtype", [(64, torch.float16), (128, torch.bfloat16), (256, torch.bfloat16)])
+@pytest.mark.parametrize("form", ["shifted", "padded", "one_row", "one_head"])
+def test_forms_of_keys_and_values(dev, form, d, dtype):
+    """Keys and values whose rows cannot be loaded straight into LDS (an address of one element's alignment, rows or heads that
+    lie on top of each other), and rows of a wider buffer, against contiguous copies of them."""
+    print(f"case {form} {d} {dtype}", flush=True)
+    cu, hq, hkv, window = [0, 31, 31, 161, 515], 6, 2, 70
+    n, max_len = cu[-1], 354
+    gen = torch.Generator().manual_seed(5)
+    cut = torch.tensor(cu, dtype=torch.int32, device=dev)
+    cuk = torch.tensor([0, 0, 0, 7, 28], dtype=torch.int32, device=dev)   # windows of 32, 16 apart
+    q = torch.randn(n, hq, d, generator=gen).to(dtype).to(dev)
+    flat = torch.randn(n * hkv * (d + 8) + 8, generator=gen).to(dtype).to(dev)
+
+    def rows(m):
+        if form == "shifted":
+            return flat[1:1 + m * hkv * d].view(m, hkv, d)
+        if form == "padded":
+            return flat[8:8 + m * hkv * (d + 8)].view(m, hkv, d + 8)[..., :d]
+        if form == "one_row":
+            return flat[:hkv * d].view(1, hkv, d).expand(m, hkv, d)
+        return flat[:m * d].view(m, 1, d).expand(m, hkv, d)
+
+    for call in (lambda k, v: ops.winattn_fwd(q, k, v, cut, max_len, window),
+                 lambda k, v: ops.cmpattn_fwd(q, k, v, 32, 16, cut, cuk, max_len)):
+        k, v = rows(n), rows(n).flip(0)
+        (o, lse), (o_c, lse_c) = call(k, v), call(k.contiguous().clone(), v.contiguous().clone())
+        assert torch.equal(o, o_c) and torch.equal(lse, lse_c)
