@@ -105,7 +105,7 @@ template <typename T, int D> struct AttnRows {
     const int lane = threadIdx.x & 63;
     vec8 x[L::N];
 #pragma unroll
-    for (int j = 0; j < L::N; ++j) x[j] = load16<vec8>(lane_ptr(row, j * L::RPI + lane / L::CPR) + lane % L::CPR * 8);
+    for (int j = 0; j < L::N; ++j) x[j] = load16_at<vec8>(shfl64((uint64_t)row, j * L::RPI + lane / L::CPR) + lane % L::CPR * 16);
 #pragma unroll
     for (int j = 0; j < L::N; ++j) {
       const int r = j * L::RPI + lane / L::CPR;
@@ -114,10 +114,6 @@ template <typename T, int D> struct AttnRows {
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) q[ks] = load16<vec8>(lds_ptr<T>(lds_addr(tile) + (f.k ^ (16u * ks))));
-  }
-  template <typename P> static __device__ __forceinline__ P* lane_ptr(P* x, int lane) {   // of that lane
-    const uint64_t v = (uint64_t)x;
-    return reinterpret_cast<P*>((uint64_t)(uint32_t)__shfl((int)(v >> 32), lane, WAVE) << 32 | (uint32_t)__shfl((int)(uint32_t)v, lane, WAVE));
   }
   // o * scale to the rows `row` of the lanes, by way of such a tile; rows whose lanes are not `valid` are left out
   __device__ __forceinline__ void store_rows(T* row, bool valid, float scale, T* tile) const {
@@ -138,8 +134,8 @@ template <typename T, int D> struct AttnRows {
     for (int j = 0; j < L::N; ++j) {
       const int r = j * L::RPI + lane / L::CPR;
       const vec8 x = load16<vec8>(tile + r * D + (lane % L::CPR ^ chunk_swizzle<D>(r)) * 8);
-      T* to = lane_ptr(row, r) + lane % L::CPR * 8;
-      if (live >> r & 1) store16(to, x);
+      const uint64_t to = shfl64((uint64_t)row, r) + lane % L::CPR * 16;
+      if (live >> r & 1) store16_at(to, x);
     }
   }
   // q settled: otherwise the compiler waits for it where it is used first, inside the loop and in every step of it, and with it

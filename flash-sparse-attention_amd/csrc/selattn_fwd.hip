@@ -93,12 +93,12 @@ selattn_fwd_main_kernel(SelFwdParams p, HeadOrder order) {
   const int seq_start = p.cu_seqlens[s], seq_end = p.cu_seqlens[s + 1];
   const int tok0 = seq_start + b_local * BK;
   const int rows = p.counts[h * p.max_blocks + gb] * p.g;
-  const int start = p.starts[h * nbp1 + gb];
+  const int start = __builtin_amdgcn_readfirstlane(p.starts[h * nbp1 + gb]);
   // equal shares of the block's rows (whole passes) for its work-groups
   const int ntile_b = tp[gb + 1] - tp[gb];
   const int share = ((rows + ntile_b - 1) / ntile_b + SEL_WG_ROWS - 1) / SEL_WG_ROWS * SEL_WG_ROWS;
-  const int row_lo = (w - tp[gb]) * share;
-  const int row_hi = min(rows, row_lo + share);
+  const int row_lo = __builtin_amdgcn_readfirstlane((w - tp[gb]) * share);
+  const int row_hi = __builtin_amdgcn_readfirstlane(min(rows, row_lo + share));
 
   const int tid = threadIdx.x;
   const T* kbase = reinterpret_cast<const T*>(p.k) + (int64_t)h * p.k_sh;
@@ -119,12 +119,11 @@ selattn_fwd_main_kernel(SelFwdParams p, HeadOrder order) {
   }
   __syncthreads();
 
-  const int lane = tid & 63, wv = tid >> 6;
+  const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31, hh = lane >> 5;
   const int32_t* toks = p.sel_tokens + (int64_t)h * p.cap + start;
   const T* qbase_row = reinterpret_cast<const T*>(p.q) + (int64_t)h * p.g * p.q_sh;
   const int64_t prow0 = ((int64_t)h * p.cap + start) * p.g;
-  T* opart = reinterpret_cast<T*>(p.o_part);
   // this lane's address inside V for the transposing reads of O^T = V^T P^T:
   // keys 4*hh + (lane%16)/4 (+ 16*j, + 8), dims 16*((lane/16)&1) + 4*(lane%4) (+ 32*dt)
   const T* vtr = Vs + (4 * hh + ((lane & 15) >> 2)) * VS + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
@@ -137,22 +136,35 @@ selattn_fwd_main_kernel(SelFwdParams p, HeadOrder order) {
   constexpr int RPI = 64 / CPR;   // rows per load / store instruction
   constexpr int NLD = 32 / RPI;   // instructions per 32-row tile
   const int srow = lane / CPR, schunk = lane % CPR;
-  const uint32_t q_sn32 = (uint32_t)p.q_sn, q_sh32 = (uint32_t)p.q_sh;
+  // Rows behind the end of the share are loaded again from its last one, and partial rows leave by buffer stores whose range
+  // ends with the share: no branch around a load or store in the loop.  With branches the compiler had to assume that nothing
+  // younger than the awaited rows was on its way, and the memory queue was empty once per two sub-tiles, row stores included.
+  // (head_dim 128, 65536 tokens, GQA 4 1245 -> 1200 us, GQA 1 361 -> 354, 8192 x 32 366 -> 350; 64, 16384 x 16 159 -> 141; 256 with
+  // blocks of 64, 9000 x 4 145 -> 126, of 128 unchanged.)  What is left of a sub-tile is the chain of its products, exponentials and
+  // staged rows on two waves per SIMD.
   auto row_token = [&](int sub_) {  // token id of row (sub_ + col), kept by lane col
     const int r_ = min(sub_ + col, row_hi - 1);
     return toks[div_group(r_, p.g, p.g_shift)];
   };
-  auto fetch_q = [&](vec8 (&dst)[NLD], int tok_lane, int sub_) {
-#pragma unroll
-    for (int j = 0; j < NLD; ++j) {
-      const int row = srow + RPI * j;
-      const int tok_ = __shfl(tok_lane, row, 64);
-      const int r_ = min(sub_ + row, row_hi - 1);
-      // strides and the head term fit 32 bits (checked by the host): one 32 x 32 -> 64 bit multiply-add per row
-      const uint32_t head_ = p.g_shift >= 0 ? (uint32_t)(r_ & (p.g - 1)) : (uint32_t)(r_ - div_group(r_, p.g, p.g_shift) * p.g);
-      dst[j] = load16<vec8>(qbase_row + ((uint64_t)(uint32_t)tok_ * q_sn32 + (head_ * q_sh32 + schunk * 8)));
-    }
+  auto row_at = [&](int token, int sub_) {   // address of q row (sub_ + col)
+    const int r_ = min(sub_ + col, row_hi - 1);
+    return reinterpret_cast<uint64_t>(qbase_row + (int64_t)token * p.q_sn + (int64_t)(r_ - div_group(r_, p.g, p.g_shift) * p.g) * p.q_sh);
   };
+  auto fetch_q = [&](vec8 (&dst)[NLD], int tok_lane, int sub_) {
+    const uint64_t mine = row_at(tok_lane, sub_);
+#pragma unroll
+    for (int j = 0; j < NLD; ++j) dst[j] = load16_at<vec8>(shfl64(mine, srow + RPI * j) + schunk * 16);
+  };
+  // partial rows [row_lo, row_hi) and their log-sum-exps
+  auto share_of = [&](void* base, int64_t row_bytes) {
+    const uint64_t at = (uint64_t)base + (uint64_t)((prow0 + row_lo) * row_bytes);
+    return __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<void*>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32 |
+                                (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at)),
+        0, (int)((row_hi - row_lo) * row_bytes), 0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t o_rsrc = share_of(p.o_part, D * 2), lse_rsrc = share_of(p.lse_part, 4);
+  constexpr int NT_STORE = 2;   // cache policy of buffer stores: non-temporal
   constexpr bool STAGED = SelLds<D, BK>::STAGE_OUT;  // false: LDS cannot hold the wave tiles, direct loads / stores
   vec8 qst[NLD], qst_b[NLD];   // staged mode: the rows of the next two sub-tiles wait here (two buffers in turn)
   // Direct mode: the Q fragments of a lane's row in the MFMA operand layout, straight from global memory.  k-step ks
@@ -161,26 +173,19 @@ selattn_fwd_main_kernel(SelFwdParams p, HeadOrder order) {
   // consumed them, while the softmax and the O^T products of the current sub-tile run.
   vec8 qdir[STAGED ? 1 : NKS];
   auto fetch_dir = [&](int token, int sub_) {
-    const int rc_ = min(sub_ + col, row_hi - 1);
-    const uint32_t head_ = (uint32_t)(rc_ - div_group(rc_, p.g, p.g_shift) * p.g);
-    const T* qrow = qbase_row + ((uint64_t)(uint32_t)token * q_sn32 + (head_ * q_sh32 + hh * 8));
+    const uint64_t qrow = row_at(token, sub_) + hh * 16;
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) qdir[STAGED ? 0 : ks] = load16<vec8>(qrow + ks * 16);
+    for (int ks = 0; ks < NKS; ++ks) qdir[STAGED ? 0 : ks] = load16_at<vec8>(qrow + ks * 32);
   };
   // one sub-tile: rows sub.. of the block (direct mode: tok_next = token ids of the next sub-tile)
   // staged mode: `qbuf` holds the rows of this sub-tile on entry and, once they are parked in LDS, takes the rows
-  // of the sub-tile after the next (token ids tok_next).  The gathers are requested two sub-tiles ahead; how long they stay
-  // in flight is up to the compiler's waits: gathers, token loads and row stores stand behind branches, so where the rows of
-  // an even sub-tile are parked it assumes that nothing younger was issued and counts 7 ... 0, which also waits for the odd
-  // sub-tile's gathers and the last row stores.  The memory queue is empty once per two sub-tiles.
+  // of the sub-tile after the next (token ids tok_next).
   auto step = [&](vec8 (&qbuf)[NLD], int token, int sub, int tok_next) {
-    const int r = sub + col;
-    const bool valid = r < row_hi;
     if (STAGED) {
 #pragma unroll
       for (int j = 0; j < NLD; ++j) store16(&Ost[(srow + RPI * j) * OS + schunk * 8], qbuf[j]);
       __builtin_amdgcn_wave_barrier();
-      if (sub + 2 * SEL_WG_ROWS < row_hi) fetch_q(qbuf, tok_next, sub + 2 * SEL_WG_ROWS);
+      fetch_q(qbuf, tok_next, sub + 2 * SEL_WG_ROWS);
     }
     f32x16 acc[NA];
 #pragma unroll
@@ -195,7 +200,7 @@ selattn_fwd_main_kernel(SelFwdParams p, HeadOrder order) {
       }
     }
     __builtin_amdgcn_wave_barrier();  // Q fragments consumed: the tile is reused for the output rows
-    if (!STAGED && sub + SEL_WG_ROWS < row_hi) fetch_dir(tok_next, sub + SEL_WG_ROWS);
+    if (!STAGED) fetch_dir(tok_next, sub + SEL_WG_ROWS);
     // causal mask: key index inside the block must be <= limit
     const int limit = (token - seq_start) - b_local * BK;
     float mx = -INFINITY;
@@ -227,7 +232,7 @@ selattn_fwd_main_kernel(SelFwdParams p, HeadOrder order) {
       }
     l = sum32(l);
     const float inv_l = l > 0.f ? 1.f / l : 0.f;
-    const int64_t prow = prow0 + r;
+    const int prow = sub - row_lo;   // first of the sub-tile, of the share
     // O^T accumulators -> this wave's LDS tile [row][d] -> 16-byte stores in which 16 lanes
     // cover one full 2*D-byte row (8 cache lines per store instruction instead of 64)
     // the products of the next 32 dims are issued before the current ones are converted and stored: the matrix
@@ -255,7 +260,7 @@ selattn_fwd_main_kernel(SelFwdParams p, HeadOrder order) {
         for (int e = 0; e < 4; ++e) x[e] = (T)(oacc[4 * qd + e] * inv_l);
         if (SelLds<D, BK>::STAGE_OUT) store8(&Ost[col * OS + dt * 32 + 8 * qd + 4 * hh], x);
         else if (SelLds<D, BK>::SLICE_OUT) store8(&Osl[col * SLS + 8 * qd + 4 * hh], x);
-        else if (valid) store8(opart + prow * D + dt * 32 + 8 * qd + 4 * hh, x);  // LDS too small: direct
+        else __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), o_rsrc, ((prow + col) * D + dt * 32 + 8 * qd + 4 * hh) * 2, 0, 0);  // LDS too small: direct
       }
       if (SelLds<D, BK>::SLICE_OUT) {  // the 32 dims of this accumulator: 4 lanes per row, 16 rows per store
         __builtin_amdgcn_wave_barrier();
@@ -264,7 +269,7 @@ selattn_fwd_main_kernel(SelFwdParams p, HeadOrder order) {
           const int row = (lane >> 2) + 16 * j;
           vec8 y = load16<vec8>(&Osl[row * SLS + (lane & 3) * 8]);
           // 64-byte pieces: left to the L2 to merge into whole lines (as non-temporal stores they cost 4 % more)
-          if (sub + row < row_hi) store16(opart + (prow0 + sub + row) * D + dt * 32 + (lane & 3) * 8, y);
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, y), o_rsrc, ((prow + row) * D + dt * 32 + (lane & 3) * 8) * 2, 0, 0);
         }
         __builtin_amdgcn_wave_barrier();
       }
@@ -278,24 +283,24 @@ selattn_fwd_main_kernel(SelFwdParams p, HeadOrder order) {
       for (int j = 0; j < 32 / RPI; ++j) {
         const int row = srow + RPI * j;
         vec8 x = load16<vec8>(&Ost[row * OS + schunk * 8]);
-        if (sub + row < row_hi) store16_stream(opart + (prow0 + sub + row) * D + schunk * 8, x);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), o_rsrc, ((prow + row) * D + schunk * 8) * 2, 0, NT_STORE);
       }
     }
     __builtin_amdgcn_wave_barrier();
     // (a sum that is NaN stays NaN)
-    if (valid && hh == 0) __builtin_nontemporal_store(l == 0.f ? -INFINITY : mref + log2f(l), &p.lse_part[prow]);
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, l == 0.f ? -INFINITY : mref + log2f(l)), lse_rsrc,
+                                          hh == 0 ? (prow + col) * 4 : 0x7ffffffc, 0, NT_STORE);
   };
 
   int sub = row_lo + wv * 32;
   if (sub >= row_hi) return;
-  int ta = row_token(sub);
+  int ta = row_token(sub), tb = row_token(sub + SEL_WG_ROWS);
   if (STAGED) {
-    auto tok_at = [&](int s_) { return s_ < row_hi ? row_token(s_) : 0; };
-    int tb = tok_at(sub + SEL_WG_ROWS), tc = tok_at(sub + 2 * SEL_WG_ROWS), td = tok_at(sub + 3 * SEL_WG_ROWS);
+    int tc = row_token(sub + 2 * SEL_WG_ROWS), td = row_token(sub + 3 * SEL_WG_ROWS);
     fetch_q(qst, ta, sub);
-    if (sub + SEL_WG_ROWS < row_hi) fetch_q(qst_b, tb, sub + SEL_WG_ROWS);
+    fetch_q(qst_b, tb, sub + SEL_WG_ROWS);
     for (;;) {  // two sub-tiles per round, one from each buffer
-      const int te = tok_at(sub + 4 * SEL_WG_ROWS), tf = tok_at(sub + 5 * SEL_WG_ROWS);
+      const int te = row_token(sub + 4 * SEL_WG_ROWS), tf = row_token(sub + 5 * SEL_WG_ROWS);
       step(qst, ta, sub, tc);
       if (sub + SEL_WG_ROWS >= row_hi) break;
       step(qst_b, tb, sub + SEL_WG_ROWS, td);
@@ -306,9 +311,8 @@ selattn_fwd_main_kernel(SelFwdParams p, HeadOrder order) {
     return;
   }
   fetch_dir(ta, sub);
-  int tb = sub + SEL_WG_ROWS < row_hi ? row_token(sub + SEL_WG_ROWS) : 0;
   for (; sub < row_hi; sub += SEL_WG_ROWS) {
-    const int tc = sub + 2 * SEL_WG_ROWS < row_hi ? row_token(sub + 2 * SEL_WG_ROWS) : 0;
+    const int tc = row_token(sub + 2 * SEL_WG_ROWS);
     step(qst, ta, sub, tb);
     ta = tb;
     tb = tc;
