@@ -27,6 +27,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 namespace fsa {
 
@@ -39,6 +40,8 @@ template <int D> struct DecOcc {
   static constexpr int WAVES_PER_SIMD = D >= 256 ? 1 : 2;
   static constexpr int WG_WAVES = 2;  // waves per work-group at most
 };
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 struct DecParams {
   const void* q;   // [B, Hq, D]
@@ -74,8 +77,39 @@ struct DecParams {
   float rope_scale;
   int n_groups;             // groups of hkv waves that share the tile sequence
   float* part;              // [hkv][n_groups + batch][g][4 + D]: base-2 scaled max, sum, 2 unused, unnormalised O
+                            // (layer form: [hkv][chunks[0] + chunks[1]][g][4 + D])
+  int chunks[2];            // layer form: work-groups per kv head of source 0 and 1
+  int* arrived;             // layer form: [2][hkv] work-groups of (source, kv head) that have left their partial; zero between calls
   int32_t* tile_prefix;     // [B+1]: tiles (of one kv head) of the requests before b; batches of more than 64 requests
 };
+
+// Loads and stores of what a work-group hands to another one of the same launch: as atomics of the device's scope they go past
+// the L2 copies of the XCDs, so that neither side has to write back or invalidate a cache (1.7 us a launch).  SHARED false: plain.
+template <bool SHARED, typename V> __device__ __forceinline__ V dec_load(const float* p) {
+  if constexpr (!SHARED) {
+    return *reinterpret_cast<const V*>(p);
+  } else if constexpr (sizeof(V) == 4) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  } else {
+    typedef uint64_t words __attribute__((ext_vector_type(sizeof(V) / 8)));
+    words w;
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(V) / 8); ++i)
+      w[i] = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p) + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __builtin_bit_cast(V, w);
+  }
+}
+template <bool SHARED> __device__ __forceinline__ void dec_store(float* p, f32x4 v) {
+  if constexpr (!SHARED) {
+    *reinterpret_cast<f32x4*>(p) = v;
+  } else {
+    typedef uint64_t words __attribute__((ext_vector_type(2)));
+    const words w = __builtin_bit_cast(words, v);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __hip_atomic_store(reinterpret_cast<uint64_t*>(p) + i, w[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
 
 template <int D> struct DecLds {
   static constexpr int VS = D + 8;
@@ -130,7 +164,7 @@ decode_plan_kernel(DecParams p) {
 // topk x tiles-per-block tiles, the prefix is a product.  Compressed mode: up to 64 requests are scanned by every wave
 // itself (lane b holds request b; a microsecond inside the kernel against a launch of its own), larger batches read
 // the prefix that decode_plan_kernel wrote.
-template <int MODE, bool LAYER = false> struct DecSeq {
+template <int MODE> struct DecSeq {
   int per_req = 0, incl = 0, nt = 0, total = 0;
   bool scanned = false;
   __device__ __forceinline__ void init(const DecParams& p) {
@@ -139,12 +173,10 @@ template <int MODE, bool LAYER = false> struct DecSeq {
       total = p.batch * per_req;
       return;
     }
-    scanned = LAYER || p.batch <= WAVE;
+    scanned = p.batch <= WAVE;
     if (scanned) {
       const int lane = threadIdx.x & (WAVE - 1);
-      if (LAYER) {
-        nt = lane < 2 ? ((lane ? p.src[1].n_keys : p.src[0].n_keys) + DEC_TK - 1) / DEC_TK : 0;
-      } else if (lane < p.batch) {
+      if (lane < p.batch) {
         int n_keys, tpb;
         nt = dec_tiles<MODE>(p, lane, p.cu_k[lane + 1] - p.cu_k[lane], n_keys, tpb);
       }
@@ -195,9 +227,9 @@ __device__ __forceinline__ void sincos_turns(float x, float& sn, float& cs) {
 // time, so that a row (all kv heads, contiguous in memory) is fetched whole instead of in hkv visits of 2 D bytes.
 // ONE > 0: a work-group of ONE waves serves one (request, kv head), its waves sharing the tiles and merging their partials
 // in LDS; no partial goes through memory and no merge kernel follows.
-template <typename T, int D, int MODE, bool LAYER = false, int ONE = 0>
-__global__ void __launch_bounds__(ONE ? WAVE * ONE : WAVE * DecOcc<D>::WG_WAVES, ONE ? 1 : DecOcc<D>::WAVES_PER_SIMD)
-decode_attn_kernel(DecParams p) {
+// LAYER: as ONE, but a (source, kv head) has p.chunks work-groups, each of which leaves the partial of its tiles.
+template <typename T, int D, int MODE, bool LAYER, int ONE>
+__device__ __forceinline__ void decode_attn_body(const DecParams& p) {
   typedef typename Elem<T>::vec8 vec8;
   constexpr int VS = DecLds<D>::VS;
   constexpr int NS = D / 32, NDT = D / 16, VCH = DEC_TK * (D / 8) / 64, PS = D + 4;
@@ -205,8 +237,12 @@ decode_attn_kernel(DecParams p) {
   T* Vs = reinterpret_cast<T*>(smem + (threadIdx.x / WAVE) * DecLds<D>::BYTES);
   const int lane = threadIdx.x & (WAVE - 1), l16 = lane & 15, kg = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE));
-  const int grp = ONE ? blockIdx.x / p.hkv : w / p.hkv, h = (ONE ? blockIdx.x : w) - grp * p.hkv;   // ONE: grp is the request
-  DecSeq<MODE, LAYER> seq;
+  int grp = ONE ? blockIdx.x / p.hkv : w / p.hkv;   // ONE: the request; LAYER: the chunk, from here on of its source
+  const int h = (ONE ? blockIdx.x : w) - grp * p.hkv;
+  static_assert(!LAYER || ONE, "layer form");
+  const int chunk = grp, source = LAYER && grp >= p.chunks[0];
+  if (LAYER) grp -= source ? p.chunks[0] : 0;
+  DecSeq<MODE> seq;
   int x_lo = 0, x_hi = 0;
   if constexpr (!ONE) {
     if (grp >= p.n_groups) return;
@@ -369,12 +405,12 @@ decode_attn_kernel(DecParams p) {
   for (int t = 0; t < NDT; ++t) oacc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   Req rq, rqn;
-  load_req(rq, ONE ? grp : seq.request_of(p, x_lo));
+  load_req(rq, LAYER ? source : ONE ? grp : seq.request_of(p, x_lo));
   rqn = rq;
   if constexpr (ONE) {
-    const int wv = w - blockIdx.x * ONE;
-    x_lo = rq.nt * wv / ONE;
-    x_hi = rq.nt * (wv + 1) / ONE;
+    const int wv = w - blockIdx.x * ONE, share = LAYER ? grp * ONE + wv : wv, shares = LAYER ? p.chunks[source] * ONE : ONE;
+    x_lo = (int)((int64_t)rq.nt * share / shares);
+    x_hi = (int)((int64_t)rq.nt * (share + 1) / shares);
   }
   int ttn = ONE ? x_lo : x_lo - seq.prefix(p, rq.b);
   int row0 = 0, n_valid = 0;
@@ -423,7 +459,7 @@ decode_attn_kernel(DecParams p) {
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
           const int key0 = a * 16 + 4 * kg;
-          if (row0 + key0 < p.raw_ld) *reinterpret_cast<f32x4*>(rs + key0) = acc[a];
+          if (row0 + key0 < p.raw_ld) dec_store<LAYER>(rs + key0, acc[a]);
         }
       }
       float mx = m;
@@ -515,10 +551,35 @@ decode_attn_kernel(DecParams p) {
           o += wgt * *reinterpret_cast<const f32x4*>(oc + 4 + 4 * lr);
         }
       }
-      o *= lt > 0.f ? 1.f / lt : 0.f;
-      dec_emit<T, D>(p, grp, h, col, lr, o, lt > 0.f ? mt + log2f(lt) : -INFINITY);
+      if constexpr (LAYER) {
+        float* out = p.part + ((int64_t)h * (p.chunks[0] + p.chunks[1]) + chunk) * (p.g * PS) + col * PS;
+        if (lr == 0) dec_store<true>(out, f32x4{mt, lt, 0.f, 0.f});
+        dec_store<true>(out + 4 + 4 * lr, o);
+      } else {
+        o *= lt > 0.f ? 1.f / lt : 0.f;
+        dec_emit<T, D>(p, grp, h, col, lr, o, lt > 0.f ? mt + log2f(lt) : -INFINITY);
+      }
     }
   }
+}
+template <typename T, int D, int MODE, int ONE = 0>
+__global__ void __launch_bounds__(ONE ? WAVE * ONE : WAVE * DecOcc<D>::WG_WAVES, ONE ? 1 : DecOcc<D>::WAVES_PER_SIMD)
+decode_attn_kernel(DecParams p) {
+  decode_attn_body<T, D, MODE, false, ONE>(p);
+}
+
+// Whether this work-group is the last of the `n` that count themselves in at `counter`: what the others stored with dec_store
+// before has arrived then and is seen by dec_load.  The last one leaves the counter at zero.
+__device__ __forceinline__ bool dec_last_to_arrive(int* counter, int n) {
+  __shared__ int last;
+  vm_wait<0>();      // this wave's stores
+  __syncthreads();   // those of all waves
+  if (threadIdx.x == 0) {
+    last = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
+    if (last) *counter = 0;
+  }
+  __syncthreads();
+  return last != 0;
 }
 
 // Partials of a (request, kv head) -> o, lse.  D/4 lanes hold a row of a partial; the row groups of the work-group are
@@ -527,20 +588,12 @@ decode_attn_kernel(DecParams p) {
 // output element walking through all partials - twice, for the maximum first - took 8 to 25 us of a 50 us step.)
 constexpr int DEC_MERGE_THREADS = 512;
 // emit(col, lr, o / l as f32x4, lse) is called by the D/4 lanes that hold the merged row of head `col` of the group.
-template <int D, int MODE, bool LAYER, int THREADS, typename EMIT>
-__device__ __forceinline__ void dec_merge_block(const DecParams& p, int b, int h, EMIT emit) {
+// `part`: the first of ns partials, `slot` floats apart.
+template <int D, int THREADS, bool SHARED, typename EMIT>
+__device__ __forceinline__ void dec_merge_slots(const DecParams& p, const float* part, int ns, int slot, EMIT emit) {
   constexpr int LPR = D / 4, NG = THREADS / LPR, PS = D + 4;
   __shared__ float part_m[NG], part_l[NG];
   __shared__ f32x4 part_o[NG][LPR];
-  DecSeq<MODE, LAYER> seq;
-  seq.init(p);
-  const int per = dec_share(seq.total, p.n_groups);
-  const int x0 = seq.prefix(p, b);
-  const int nt = (b + 1 < p.batch ? seq.prefix(p, b + 1) : seq.total) - x0;
-  const int g0 = x0 / per;
-  const int ns = nt > 0 ? (x0 + nt - 1) / per - g0 + 1 : 0;
-  const int slot = p.g * PS;
-  const float* part = p.part + (int64_t)(h * (p.n_groups + p.batch) + g0 + b) * slot;
   const int rg = threadIdx.x / LPR, lr = threadIdx.x % LPR;
   const int n_slice = max(1, NG / p.g);      // slices per head; row groups beyond g * n_slice have none
   const int cols = NG / n_slice;             // heads in flight
@@ -560,10 +613,10 @@ __device__ __forceinline__ void dec_merge_block(const DecParams& p, int b, int h
 #pragma unroll
         for (int u = 0; u < UB; ++u) {
           const float* ps = pc + (int64_t)min(sb + u, s_hi - 1) * slot;
-          const float2 ml = *reinterpret_cast<const float2*>(ps);
-          ms[u] = sb + u < s_hi ? ml.x : -INFINITY;
-          ls[u] = ml.y;
-          os[u] = *reinterpret_cast<const f32x4*>(ps + 4 + lr * 4);
+          const f32x2 ml = dec_load<SHARED, f32x2>(ps);
+          ms[u] = sb + u < s_hi ? ml[0] : -INFINITY;
+          ls[u] = ml[1];
+          os[u] = dec_load<SHARED, f32x4>(ps + 4 + lr * 4);
         }
         float mn = m;
 #pragma unroll
@@ -617,7 +670,16 @@ template <typename T, int D, int MODE>
 __global__ void __launch_bounds__(DEC_MERGE_THREADS)
 decode_merge_kernel(DecParams p) {
   const int b = blockIdx.x, h = blockIdx.y;
-  dec_merge_block<D, MODE, false, DEC_MERGE_THREADS>(p, b, h, [&](int col, int lr, f32x4 o, float lse) {
+  DecSeq<MODE> seq;
+  seq.init(p);
+  const int per = dec_share(seq.total, p.n_groups);
+  const int x0 = seq.prefix(p, b);
+  const int nt = (b + 1 < p.batch ? seq.prefix(p, b + 1) : seq.total) - x0;
+  const int g0 = x0 / per;
+  const int ns = nt > 0 ? (x0 + nt - 1) / per - g0 + 1 : 0;
+  const int slot = p.g * (D + 4);
+  const float* part = p.part + (int64_t)(h * (p.n_groups + p.batch) + g0 + b) * slot;
+  dec_merge_slots<D, DEC_MERGE_THREADS, false>(p, part, ns, slot, [&](int col, int lr, f32x4 o, float lse) {
     dec_emit<T, D>(p, b, h, col, lr, o, lse);
   });
 }
@@ -653,7 +715,8 @@ constexpr int DEC_TOPK_MAX_K = 16;   // finalists of the four waves fill one wav
 // NREG: candidates per lane in registers (blocks <= 256 NREG, topk <= DEC_TOPK_MAX_K); 0: any size, scores in LDS
 // (nc, qp, len: compressed rows, query position and cache length of request b; lse_r: lse of the scoring head)
 // Called by a whole work-group of at least DEC_TOPK_THREADS threads; the threads beyond those only keep the barriers.
-template <int NREG>
+// SHARED: the raw scores come from other work-groups of the launch.
+template <int NREG, bool SHARED>
 __device__ __forceinline__ void dec_topk_block(const DecTopkParams& p, int b, int h, int nc, int qp, int len, float lse_r,
                                                float* bs) {
   __shared__ uint64_t final_key[DEC_TOPK_WAVES * DEC_TOPK_MAX_K];
@@ -677,7 +740,7 @@ __device__ __forceinline__ void dec_topk_block(const DecTopkParams& p, int b, in
       const int c = c0 + o;
       if (c >= 0 && c < n_vis) {
         const int wgt = min(min(o, n_off - 1 - o), min(na, ne) - 1) + 1;
-        acc += (float)wgt * fast_exp2(rs[c] * p.scale_log2 - lse_r);
+        acc += (float)wgt * fast_exp2(dec_load<SHARED, float>(rs + c) * p.scale_log2 - lse_r);
       }
     }
     return finish(acc, blk);
@@ -700,8 +763,8 @@ __device__ __forceinline__ void dec_topk_block(const DecTopkParams& p, int b, in
 #pragma unroll
       for (int r = 0; r < NREG; ++r) {
         const int c = 4 * (tid + DEC_TOPK_THREADS * r);
-        x[r] = *reinterpret_cast<const f32x4*>(rs + min(c, last));
-        x0[r] = rs[min(max(c - 1, 0), last)];
+        x[r] = dec_load<SHARED, f32x4>(rs + min(c, last));
+        x0[r] = dec_load<SHARED, float>(rs + min(max(c - 1, 0), last));
       }
 #pragma unroll
       for (int r = 0; r < NREG; ++r) {
@@ -808,12 +871,12 @@ decode_topk_kernel(DecTopkParams p) {
   extern __shared__ float bs[];
   const int b = blockIdx.x, h = blockIdx.y;
   const int hq_s = p.as_written ? h : h * p.g;
-  dec_topk_block<NREG>(p, b, h, p.cu_ck[b + 1] - p.cu_ck[b], p.pos[b], p.seqlens[b], p.lse[(int64_t)hq_s * p.batch + b], bs);
+  dec_topk_block<NREG, false>(p, b, h, p.cu_ck[b + 1] - p.cu_ck[b], p.pos[b], p.seqlens[b], p.lse[(int64_t)hq_s * p.batch + b], bs);
 }
 
 // ------------------------------------------------------- one token through the layer ----
-// Six launches for a token of one request: projections + rotation of q; compressed and window attention; their merge and
-// the block selection; selected attention; its merge and the gated sum; output projection.  The caches stay as they are
+// Four launches for a token of one request: projections + rotation of q; compressed and window attention with their merge and
+// the block selection; selected attention with its merge and the gated sum; output projection.  The caches stay as they are
 // (un-rotated, without the new token): keys are rotated in registers on their way into LDS, the new row is read from
 // where the projection left it.  Copying and rotating the caches for a step, as a composition of the single operators
 // does, moves 32 times the bytes that the step needs (32K tokens: 740 us in 31 launches).
@@ -827,6 +890,7 @@ struct DecLayerParams {
   void *q_rot, *k_new, *v_new;   // [hq, D], [hkv, D], [hkv, D]
   void* gate;                    // [3] sigmoid values
   void *o_cmp, *o_win;           // [hq, D]
+  int* arrived;                  // [2][hkv], see DecParams
   void* attn;                    // [hq, D] gated sum
   void* y;                       // [hidden]
 };
@@ -871,6 +935,8 @@ __device__ __forceinline__ void dot2(const T* __restrict__ x, const T* __restric
 template <typename T>
 __global__ void __launch_bounds__(256)
 decode_project_kernel(DecLayerParams p) {
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < 2 * p.hkv; i += 256) p.arrived[i] = 0;
   const int u = blockIdx.x * 4 + threadIdx.x / WAVE, half = p.d / 2;
   const int nq = p.hq * half, nkv = p.hkv * half;
   const int m = u < nq ? 0 : u < nq + nkv ? 1 : u < nq + 2 * nkv ? 2 : 3;   // which matrix (uniform)
@@ -915,16 +981,23 @@ decode_out_kernel(DecLayerParams p) {
   y[r1] = (T)s1;
 }
 
-// merge of compressed (blockIdx.y == 0, then the block selection of the kv head) and window attention
-constexpr int DEC_LAYER_MERGE_THREADS = 1024;
+// Compressed and window attention, their merge and the block selection in one launch: the last work-group of a (source, kv head)
+// to leave its partial merges them, and, of the compressed branch, selects the blocks of that head.  A launch of its own for
+// that took 4 us more, most of them until its first loads had returned.
+template <int D> struct DecLayerWaves {
+  static constexpr int N = 4;   // DEC_TOPK_THREADS for the selection; more waves per work-group bring more rows into one CU
+};
 template <typename T, int D, int NREG>
-__global__ void __launch_bounds__(DEC_LAYER_MERGE_THREADS)
+__global__ void __launch_bounds__(WAVE * DecLayerWaves<D>::N, DecOcc<D>::WAVES_PER_SIMD)
 decode_layer_select_kernel(DecParams p, DecTopkParams tk, DecLayerParams lp) {
-  extern __shared__ float bs[];
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   __shared__ float lse_s;
-  const int h = blockIdx.x, b = blockIdx.y;
+  decode_attn_body<T, D, DEC_MODE_COMPRESSED, true, DecLayerWaves<D>::N>(p);
+  const int chunk = blockIdx.x / p.hkv, h = blockIdx.x - chunk * p.hkv, b = chunk >= p.chunks[0], slot = p.g * (D + 4);
+  if (!dec_last_to_arrive(p.arrived + b * p.hkv + h, p.chunks[b])) return;
   T* out = reinterpret_cast<T*>(b == 0 ? lp.o_cmp : lp.o_win);
-  dec_merge_block<D, DEC_MODE_COMPRESSED, true, DEC_LAYER_MERGE_THREADS>(p, b, h, [&](int col, int lr, f32x4 o, float lse) {
+  const float* part = p.part + ((int64_t)h * (p.chunks[0] + p.chunks[1]) + (b ? p.chunks[0] : 0)) * slot;
+  dec_merge_slots<D, WAVE * DecLayerWaves<D>::N, true>(p, part, p.chunks[b], slot, [&](int col, int lr, f32x4 o, float lse) {
     typename Elem<T>::vec4 x;
 #pragma unroll
     for (int i = 0; i < 4; ++i) x[i] = (T)o[i];
@@ -933,18 +1006,20 @@ decode_layer_select_kernel(DecParams p, DecTopkParams tk, DecLayerParams lp) {
   });
   if (b != 0) return;
   __syncthreads();
-  dec_topk_block<NREG>(tk, 0, h, p.src[0].n_keys, lp.pos, lp.pos + 1, lse_s, bs);
+  dec_topk_block<NREG, true>(tk, 0, h, p.src[0].n_keys, lp.pos, lp.pos + 1, lse_s, reinterpret_cast<float*>(smem));
 }
 
-// merge of selected attention and the gated sum of the three branches
+// Selected attention, its merge and the gated sum of the three branches, in the same way
 template <typename T, int D>
-__global__ void __launch_bounds__(DEC_LAYER_MERGE_THREADS)
+__global__ void __launch_bounds__(WAVE * DecLayerWaves<D>::N, DecOcc<D>::WAVES_PER_SIMD)
 decode_layer_combine_kernel(DecParams p, DecLayerParams lp) {
   typedef typename Elem<T>::vec4 vec4;
-  const int h = blockIdx.x;
+  decode_attn_body<T, D, DEC_MODE_SELECTED, true, DecLayerWaves<D>::N>(p);
+  const int h = blockIdx.x % p.hkv, slot = p.g * (D + 4);
+  if (!dec_last_to_arrive(p.arrived + h, p.chunks[0])) return;
   const T* gate = reinterpret_cast<const T*>(lp.gate);
   const float g0 = (float)gate[0], g1 = (float)gate[1], g2 = (float)gate[2];
-  dec_merge_block<D, DEC_MODE_SELECTED, true, DEC_LAYER_MERGE_THREADS>(p, 0, h, [&](int col, int lr, f32x4 o, float) {
+  dec_merge_slots<D, WAVE * DecLayerWaves<D>::N, true>(p, p.part + (int64_t)h * p.chunks[0] * slot, p.chunks[0], slot, [&](int col, int lr, f32x4 o, float) {
     const int at = (h * p.g + col) * D + lr * 4;
     const vec4 a = load8<vec4>(reinterpret_cast<const T*>(lp.o_cmp) + at), c = load8<vec4>(reinterpret_cast<const T*>(lp.o_win) + at);
     vec4 x;
@@ -964,8 +1039,8 @@ template <int D> struct DecOne {
 template <typename T, int D, int MODE> static int dec_one_launch(const DecParams& p, int pairs, int dev, hipStream_t stream) {
   constexpr int W = DecOne<D>::WAVES, LDS = W * DecLds<D>::BYTES;
   static LdsAllowed allowed;
-  if (int rc_ = allow_lds(allowed, (const void*)decode_attn_kernel<T, D, MODE, false, W>, LDS, dev)) return rc_;
-  decode_attn_kernel<T, D, MODE, false, W><<<pairs, WAVE * W, LDS, stream>>>(p);
+  if (int rc_ = allow_lds(allowed, (const void*)decode_attn_kernel<T, D, MODE, W>, LDS, dev)) return rc_;
+  decode_attn_kernel<T, D, MODE, W><<<pairs, WAVE * W, LDS, stream>>>(p);
   return 0;
 }
 
@@ -1058,8 +1133,9 @@ static size_t dec_ws_bytes(int batch, int hq, int hkv, int d) {
 }
 
 // ---- one token through the layer: host side ----
+constexpr int DEC_LAYER_CHUNKS = 64;   // work-groups per (source, kv head) at most
 struct DecLayerWs {
-  size_t q_rot, gate, o_cmp, o_win, attn, idx, raw, part, total;
+  size_t q_rot, gate, o_cmp, o_win, attn, idx, raw, part, arrived, total;
   int64_t raw_ld;
   int topk;
 };
@@ -1081,7 +1157,8 @@ static DecLayerWs dec_layer_ws(const fsa_decode_layer_args& a) {
   w.idx = take((size_t)a.num_kv_heads * w.topk * 4);
   w.raw_ld = (a.ck_len + 1 + 3) / 4 * 4;
   w.raw = take((size_t)a.num_kv_heads * w.raw_ld * 4);
-  w.part = take(((size_t)DEC_MAX_WAVES + 2 * a.num_kv_heads) * (a.num_q_heads / a.num_kv_heads) * (4 + a.head_dim) * 4);
+  w.part = take((size_t)2 * DEC_LAYER_CHUNKS * a.num_kv_heads * (a.num_q_heads / a.num_kv_heads) * (4 + a.head_dim) * 4);
+  w.arrived = take((size_t)2 * a.num_kv_heads * 4);
   w.total = at;
   return w;
 }
@@ -1122,6 +1199,7 @@ static DecLayerParams dec_layer_params(const fsa_decode_layer_args& a, const Dec
   p.hidden = a.hidden; p.hq = a.num_q_heads; p.hkv = a.num_kv_heads; p.d = a.head_dim; p.pos = (int)a.cache_len;
   p.inv_freq = a.inv_freq; p.rope_scale = a.rope_scale;
   p.q_rot = ws + w.q_rot; p.k_new = a.k_new; p.v_new = a.v_new; p.gate = ws + w.gate;
+  p.arrived = (int*)(ws + w.arrived);
   p.o_cmp = ws + w.o_cmp; p.o_win = ws + w.o_win; p.attn = ws + w.attn; p.y = a.y;
   return p;
 }
@@ -1132,10 +1210,6 @@ static int dec_layer_attend(const fsa_decode_layer_args& a, hipStream_t stream) 
   const DecLayerParams lp = dec_layer_params(a, w);
   char* ws = (char*)a.workspace;
   const int L = (int)a.cache_len, hkv = a.num_kv_heads;
-  int n_waves = 0, dev = -1;
-  int rc = dec_grid_waves<T, D, DEC_MODE_COMPRESSED>(&n_waves, &dev);
-  if (rc) return rc;
-  const int max_groups = std::max(1, n_waves / hkv), wg_waves = std::min(hkv, DecOcc<D>::WG_WAVES);
   DecParams p = {};
   p.q = lp.q_rot; p.q_sh = D;
   p.batch = 2; p.hq = a.num_q_heads; p.hkv = hkv; p.g = p.gq = a.num_q_heads / hkv;
@@ -1150,12 +1224,11 @@ static int dec_layer_attend(const fsa_decode_layer_args& a, hipStream_t stream) 
               a.kernel_stride};
   p.src[1] = {elem(a.k_cache, w0 * a.k_stride_n), elem(a.v_cache, w0 * a.v_stride_n), a.k_new, a.v_new, a.k_stride_n,
               a.k_stride_h, a.v_stride_n, a.v_stride_h, L - w0, L + 1 - w0, w0, 1};
-  auto attn_grid = [&](int tiles) {
-    p.n_groups = std::max(1, std::min(max_groups, tiles));
-    return (p.n_groups * hkv + wg_waves - 1) / wg_waves;
-  };
-  int grid = attn_grid((p.src[0].n_keys + DEC_TK - 1) / DEC_TK + (p.src[1].n_keys + DEC_TK - 1) / DEC_TK);
-  decode_attn_kernel<T, D, DEC_MODE_COMPRESSED, true><<<grid, WAVE * wg_waves, DecLds<D>::BYTES * wg_waves, stream>>>(p);
+  // a tile per wave, as long as the chip holds them all
+  constexpr int W = DecLayerWaves<D>::N, LDS = W * DecLds<D>::BYTES;
+  auto chunks = [&](int tiles) { return std::max(1, std::min({(tiles + W - 1) / W, DEC_LAYER_CHUNKS, std::max(1, 1024 / (W * hkv))})); };
+  p.arrived = lp.arrived;
+  for (int i = 0; i < 2; ++i) p.chunks[i] = chunks((p.src[i].n_keys + DEC_TK - 1) / DEC_TK);
 
   DecTopkParams tk = {};
   tk.raw_score = p.raw_score; tk.raw_ld = w.raw_ld; tk.batch = 1; tk.hkv = hkv; tk.g = p.g;
@@ -1163,19 +1236,27 @@ static int dec_layer_attend(const fsa_decode_layer_args& a, hipStream_t stream) 
   tk.init_blocks = a.init_blocks; tk.local_blocks = a.local_blocks; tk.scores_to_bf16 = 1;
   tk.scale_log2 = p.scale_log2; tk.topk_idx = (int32_t*)(ws + w.idx);
   const int nblk = (L + a.block_size) / a.block_size;
-  const dim3 sgrid(hkv, 2);
-  if (w.topk <= DEC_TOPK_MAX_K && nblk <= DEC_TOPK_THREADS)
-    decode_layer_select_kernel<T, D, 1><<<sgrid, DEC_LAYER_MERGE_THREADS, 0, stream>>>(p, tk, lp);
-  else if (w.topk <= DEC_TOPK_MAX_K && nblk <= 4 * DEC_TOPK_THREADS)
-    decode_layer_select_kernel<T, D, 4><<<sgrid, DEC_LAYER_MERGE_THREADS, 0, stream>>>(p, tk, lp);
-  else
-    decode_layer_select_kernel<T, D, 0><<<sgrid, DEC_LAYER_MERGE_THREADS, (size_t)nblk * 4, stream>>>(p, tk, lp);
+  const int grid = (p.chunks[0] + p.chunks[1]) * hkv;
+  auto select = [&](auto nreg, size_t lds) {
+    constexpr int NREG = decltype(nreg)::value;
+    static LdsAllowed allowed;
+    if (int rc_ = allow_lds(allowed, (const void*)decode_layer_select_kernel<T, D, NREG>, std::max(LDS, 64 * 1024))) return rc_;
+    decode_layer_select_kernel<T, D, NREG><<<grid, WAVE * W, std::max(lds, (size_t)LDS), stream>>>(p, tk, lp);
+    return 0;
+  };
+  int rc;
+  if (w.topk <= DEC_TOPK_MAX_K && nblk <= DEC_TOPK_THREADS) rc = select(std::integral_constant<int, 1>{}, 0);
+  else if (w.topk <= DEC_TOPK_MAX_K && nblk <= 4 * DEC_TOPK_THREADS) rc = select(std::integral_constant<int, 4>{}, 0);
+  else rc = select(std::integral_constant<int, 0>{}, (size_t)nblk * 4);
+  if (rc) return rc;
 
   p.batch = 1;
   p.src[0] = {a.k_cache, a.v_cache, a.k_new, a.v_new, a.k_stride_n, a.k_stride_h, a.v_stride_n, a.v_stride_h, L, L + 1, 0, 1};
-  grid = attn_grid(w.topk * ((a.block_size + DEC_TK - 1) / DEC_TK));
-  decode_attn_kernel<T, D, DEC_MODE_SELECTED, true><<<grid, WAVE * wg_waves, DecLds<D>::BYTES * wg_waves, stream>>>(p);
-  decode_layer_combine_kernel<T, D><<<hkv, DEC_LAYER_MERGE_THREADS, 0, stream>>>(p, lp);
+  p.chunks[0] = chunks(w.topk * ((a.block_size + DEC_TK - 1) / DEC_TK));
+  p.chunks[1] = 0;
+  static LdsAllowed allowed;
+  if (int rc_ = allow_lds(allowed, (const void*)decode_layer_combine_kernel<T, D>, LDS)) return rc_;
+  decode_layer_combine_kernel<T, D><<<p.chunks[0] * hkv, WAVE * W, LDS, stream>>>(p, lp);
   decode_out_kernel<T><<<(a.hidden + 7) / 8, 256, 0, stream>>>(lp);
   FSA_CHECK_LAUNCH("fsa_decode_layer_attend");
   return 0;
