@@ -17,7 +17,9 @@
 // 2*D-byte rows per instruction) and pass through a wave-private LDS tile: K
 // is read back as 16x16x32 MFMA operands, V transposed.  A wave writes one
 // fp32 partial (m, l, O) per pair it touches; a small merge kernel combines
-// the partials of a pair in a fixed order.  The query heads occupy the first
+// the partials of a pair in a fixed order.  Where there are few tiles, a pair
+// has a number of work-groups of its own and the last of them merges, or one
+// work-group, whose waves meet in LDS (dec_launch).  The query heads occupy the first
 // g of the 16 MFMA columns; column g carries the scoring head.
 //
 // Semantics: fsa_preview/ops/compressed_attention_decode.py:361-490 (attention),
@@ -26,6 +28,7 @@
 #include "fsa_common.h"
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <type_traits>
 
@@ -78,8 +81,11 @@ struct DecParams {
   int n_groups;             // groups of hkv waves that share the tile sequence
   float* part;              // [hkv][n_groups + batch][g][4 + D]: base-2 scaled max, sum, 2 unused, unnormalised O
                             // (layer form: [hkv][chunks[0] + chunks[1]][g][4 + D])
-  int chunks[2];            // layer form: work-groups per kv head of source 0 and 1
+                            // (chunked form: [batch][hkv][chunks[0]][g][4 + D])
+  int chunks[2];            // layer form: work-groups per kv head of source 0 and 1; chunked form: [0] per (request, kv head)
   int* arrived;             // layer form: [2][hkv] work-groups of (source, kv head) that have left their partial; zero between calls
+  uint64_t* stamps;         // chunked form: [batch][hkv][chunks[0]], `call` where the partial is there
+  uint64_t call;            // no other call's number
   int32_t* tile_prefix;     // [B+1]: tiles (of one kv head) of the requests before b; batches of more than 64 requests
 };
 
@@ -227,8 +233,9 @@ __device__ __forceinline__ void sincos_turns(float x, float& sn, float& cs) {
 // time, so that a row (all kv heads, contiguous in memory) is fetched whole instead of in hkv visits of 2 D bytes.
 // ONE > 0: a work-group of ONE waves serves one (request, kv head), its waves sharing the tiles and merging their partials
 // in LDS; no partial goes through memory and no merge kernel follows.
-// LAYER: as ONE, but a (source, kv head) has p.chunks work-groups, each of which leaves the partial of its tiles.
-template <typename T, int D, int MODE, bool LAYER, int ONE>
+// CHUNKED: as ONE, but a (request, kv head), or in the LAYER form a (source, kv head), has p.chunks work-groups, each of which
+// leaves the partial of its tiles.
+template <typename T, int D, int MODE, bool LAYER, int ONE, bool CHUNKED = LAYER>
 __device__ __forceinline__ void decode_attn_body(const DecParams& p) {
   typedef typename Elem<T>::vec8 vec8;
   constexpr int VS = DecLds<D>::VS;
@@ -239,9 +246,16 @@ __device__ __forceinline__ void decode_attn_body(const DecParams& p) {
   const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE));
   int grp = ONE ? blockIdx.x / p.hkv : w / p.hkv;   // ONE: the request; LAYER: the chunk, from here on of its source
   const int h = (ONE ? blockIdx.x : w) - grp * p.hkv;
-  static_assert(!LAYER || ONE, "layer form");
-  const int chunk = grp, source = LAYER && grp >= p.chunks[0];
-  if (LAYER) grp -= source ? p.chunks[0] : 0;
+  static_assert(!CHUNKED || ONE, "chunks are work-groups");
+  // LAYER: the place among the chunks of both sources, then in its source; CHUNKED: the request, the chunk of it
+  int chunk = grp;
+  const int source = LAYER && grp >= p.chunks[0];
+  if (LAYER) {
+    grp -= source ? p.chunks[0] : 0;
+  } else if (CHUNKED) {
+    grp = (uint32_t)grp / (uint32_t)p.chunks[0];
+    chunk -= grp * p.chunks[0];
+  }
   DecSeq<MODE> seq;
   int x_lo = 0, x_hi = 0;
   if constexpr (!ONE) {
@@ -408,7 +422,7 @@ __device__ __forceinline__ void decode_attn_body(const DecParams& p) {
   load_req(rq, LAYER ? source : ONE ? grp : seq.request_of(p, x_lo));
   rqn = rq;
   if constexpr (ONE) {
-    const int wv = w - blockIdx.x * ONE, share = LAYER ? grp * ONE + wv : wv, shares = LAYER ? p.chunks[source] * ONE : ONE;
+    const int wv = w - blockIdx.x * ONE, share = (LAYER ? grp : CHUNKED ? chunk : 0) * ONE + wv, shares = CHUNKED ? p.chunks[source] * ONE : ONE;
     x_lo = (int)((int64_t)rq.nt * share / shares);
     x_hi = (int)((int64_t)rq.nt * (share + 1) / shares);
   }
@@ -551,8 +565,9 @@ __device__ __forceinline__ void decode_attn_body(const DecParams& p) {
           o += wgt * *reinterpret_cast<const f32x4*>(oc + 4 + 4 * lr);
         }
       }
-      if constexpr (LAYER) {
-        float* out = p.part + ((int64_t)h * (p.chunks[0] + p.chunks[1]) + chunk) * (p.g * PS) + col * PS;
+      if constexpr (CHUNKED) {
+        const int64_t at = LAYER ? (int64_t)h * (p.chunks[0] + p.chunks[1]) + chunk : ((int64_t)grp * p.hkv + h) * p.chunks[0] + chunk;
+        float* out = p.part + at * (p.g * PS) + col * PS;
         if (lr == 0) dec_store<true>(out, f32x4{mt, lt, 0.f, 0.f});
         dec_store<true>(out + 4 + 4 * lr, o);
       } else {
@@ -580,6 +595,27 @@ __device__ __forceinline__ bool dec_last_to_arrive(int* counter, int n) {
   }
   __syncthreads();
   return last != 0;
+}
+
+// The same without a counter that somebody had to clear: every work-group leaves the number of the call beside its partial and
+// looks whether all n numbers are there.  Its own store is awaited before it looks, so that at least the last one sees them all;
+// if several do, they write the same results.  Numbers are not used twice, and they are cleared once all have been seen: a
+// recorded call that is replayed starts without them.
+__device__ __forceinline__ bool dec_all_arrived(uint64_t* stamps, int n, int mine, uint64_t call) {
+  __shared__ int all;
+  vm_wait<0>();
+  __syncthreads();
+  if (threadIdx.x < WAVE) {
+    if (threadIdx.x == 0) __hip_atomic_store(stamps + mine, call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    vm_wait<0>();
+    const bool there =
+        (int)threadIdx.x >= n || __hip_atomic_load(stamps + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == call;
+    const bool last = __all(there);
+    if (threadIdx.x == 0) all = last;
+    if (last && (int)threadIdx.x < n) __hip_atomic_store(stamps + threadIdx.x, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  return all != 0;
 }
 
 // Partials of a (request, kv head) -> o, lse.  D/4 lanes hold a row of a partial; the row groups of the work-group are
@@ -680,6 +716,20 @@ decode_merge_kernel(DecParams p) {
   const int slot = p.g * (D + 4);
   const float* part = p.part + (int64_t)(h * (p.n_groups + p.batch) + g0 + b) * slot;
   dec_merge_slots<D, DEC_MERGE_THREADS, false>(p, part, ns, slot, [&](int col, int lr, f32x4 o, float lse) {
+    dec_emit<T, D>(p, b, h, col, lr, o, lse);
+  });
+}
+
+// A (request, kv head) in p.chunks[0] work-groups, the last of which merges (dec_all_arrived).
+constexpr int DEC_CHUNK_WAVES = 4, DEC_MAX_CHUNKS = WAVE, DEC_CHUNK_SLOTS = 1024;   // work-groups of a launch at most
+template <typename T, int D, int MODE>
+__global__ void __launch_bounds__(WAVE * DEC_CHUNK_WAVES, DecOcc<D>::WAVES_PER_SIMD)
+decode_attn_chunked_kernel(DecParams p) {
+  decode_attn_body<T, D, MODE, false, DEC_CHUNK_WAVES, true>(p);
+  const int pair = blockIdx.x / p.hkv, h = blockIdx.x - pair * p.hkv, b = (uint32_t)pair / (uint32_t)p.chunks[0], slot = p.g * (D + 4);
+  const int64_t first = ((int64_t)b * p.hkv + h) * p.chunks[0];
+  if (!dec_all_arrived(p.stamps + first, p.chunks[0], pair - b * p.chunks[0], p.call)) return;
+  dec_merge_slots<D, WAVE * DEC_CHUNK_WAVES, true>(p, p.part + first * slot, p.chunks[0], slot, [&](int col, int lr, f32x4 o, float lse) {
     dec_emit<T, D>(p, b, h, col, lr, o, lse);
   });
 }
@@ -1030,9 +1080,10 @@ decode_layer_combine_kernel(DecParams p, DecLayerParams lp) {
 }
 
 // One work-group per (request, kv head): a tile takes a wave 3 us from end to end, so its waves may have few of them.  With
-// few pairs the shares spread the tiles over more of the chip, and two tiles per wave are the most that the saved merge
-// pays for (one request: one tile per wave 6.2 against 11.4 us, four 12.3 against 9.8); from 96 pairs on the shares are
-// that long themselves (32 requests x 8 heads, 1024 selected keys, a whole step: 41 -> 37 us).  512 pairs are resident.
+// few pairs chunks spread the tiles over more of the chip, and two tiles per wave are the most that the saved exchange
+// pays for (one request, two tiles: compressed keys of 6000 tokens 8.1 against 8.8 us); where there are pairs enough to leave
+// no chunks, shares would be that long themselves (32 requests x 8 heads, 1024 selected keys, a whole step: 41 -> 37 us).  512
+// pairs are resident.
 template <int D> struct DecOne {
   static constexpr int WAVES = D >= 256 ? 4 : 8;   // what the registers allow
 };
@@ -1070,6 +1121,23 @@ static int dec_grid_waves(int* n_waves, int* device) {
   return 0;
 }
 
+// Work-groups per (request, kv head) of the chunked form: a tile per wave while the chip holds them at once, 1 where the waves
+// would have more than DEC_CHUNK_TILES tiles (the shares of the persistent grid are the better ones then).  Against partials and
+// a merge launch, us, 32 + 8 heads of 128, compressed: one request of 16K 10.7 -> 8.8, 32K 12.0 -> 8.8, 128K 21.9 -> 16.8, four of
+// 32K 16.0 -> 12.7, 8 of 16K 14.8 -> 12.6; 16 of 32K 28.5 -> 27.4, with twice the work-groups 31.9; 1024 selected keys: one request
+// 9.1 -> 8.6, 12 requests, against a work-group for each pair, 16.5 -> 15.1.
+constexpr int DEC_CHUNK_TILES = 4;
+static int64_t dec_chunks(int64_t req_tiles, int64_t pairs) {
+  const int64_t most = std::min<int64_t>(DEC_MAX_CHUNKS, DEC_CHUNK_SLOTS / 2 / std::max<int64_t>(1, pairs));
+  const int64_t n = std::min((req_tiles + DEC_CHUNK_WAVES - 1) / DEC_CHUNK_WAVES, most);
+  return n > 1 && req_tiles <= n * DEC_CHUNK_WAVES * DEC_CHUNK_TILES ? n : 1;
+}
+static uint64_t dec_call_number() {
+  static std::atomic<uint64_t> next{0x5eed0fca115ull};
+  const uint64_t x = next.fetch_add(1, std::memory_order_relaxed) * 0x9e3779b97f4a7c15ull;   // odd: no number comes twice
+  return x ? x : dec_call_number();
+}
+
 // p0.g holds the whole group size on entry.  Scores of the scoring head: with the first head of the group as
 // scoring head they are the scores of column 0 of the first launch; with the head that the reference's kernel
 // actually reads (q head number h for kv head h) they need a column of their own, so that launch has 15 heads.
@@ -1085,10 +1153,12 @@ static int dec_launch(const DecParams& p0, hipStream_t stream) {
   const int64_t req_tiles = MODE == DEC_MODE_COMPRESSED ? ((int64_t)p.max_keys + DEC_TK - 1) / DEC_TK
                                                         : (int64_t)p.topk * ((p.block_size + DEC_TK - 1) / DEC_TK);
   const int64_t pairs = (int64_t)p.batch * p.hkv;
-  const bool one = req_tiles <= (pairs < 96 ? 2 : 4) * DecOne<D>::WAVES && pairs <= 512;
+  const int64_t chunks = dec_chunks(req_tiles, pairs);
+  const bool chunked = chunks > 1 && req_tiles > 2 * DecOne<D>::WAVES;
+  const bool one = !chunked && req_tiles <= (pairs < 96 ? 2 : 4) * DecOne<D>::WAVES && pairs <= 512;
   const int64_t most = std::max<int64_t>(1, req_tiles * p.batch);
   p.n_groups = (int)std::min<int64_t>(std::max(1, n_waves / p.hkv), most);
-  if (MODE == DEC_MODE_COMPRESSED && p.batch > WAVE && !one) decode_plan_kernel<<<1, WAVE, 0, stream>>>(p);
+  if (MODE == DEC_MODE_COMPRESSED && p.batch > WAVE && !one && !chunked) decode_plan_kernel<<<1, WAVE, 0, stream>>>(p);
   // two neighbouring kv heads per work-group (64 requests of 32K - 128K: 304 us a step with one, 288 / 291 / 293 with
   // two / four / eight)
   const int wg_waves = std::min(p.hkv, DecOcc<D>::WG_WAVES);
@@ -1102,6 +1172,14 @@ static int dec_launch(const DecParams& p0, hipStream_t stream) {
     if (one) {
       rc = dec_one_launch<T, D, MODE>(p, p.batch * p.hkv, dev, stream);
       if (rc) return rc;
+    } else if (chunked) {
+      constexpr int LDS = DEC_CHUNK_WAVES * DecLds<D>::BYTES;
+      static LdsAllowed allowed;
+      if (int rc_ = allow_lds(allowed, (const void*)decode_attn_chunked_kernel<T, D, MODE>, LDS, dev)) return rc_;
+      p.chunks[0] = (int)chunks;
+      p.stamps = reinterpret_cast<uint64_t*>(p.part + (int64_t)DEC_CHUNK_SLOTS * p0.g * (D + 4));   // behind the partials
+      p.call = dec_call_number();
+      decode_attn_chunked_kernel<T, D, MODE><<<(int)(pairs * chunks), WAVE * DEC_CHUNK_WAVES, LDS, stream>>>(p);
     } else {
       decode_attn_kernel<T, D, MODE><<<grid, WAVE * wg_waves, DecLds<D>::BYTES * wg_waves, stream>>>(p);
       decode_merge_kernel<T, D, MODE><<<dim3(p.batch, p.hkv), DEC_MERGE_THREADS, 0, stream>>>(p);
