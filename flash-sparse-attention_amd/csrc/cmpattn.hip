@@ -6,7 +6,7 @@
 //                   K/V tile serves the whole GQA group; S^T = K Q^T with one row
 //                   per lane, online softmax in registers, O^T += V^T P^T.
 //   cmpattn_bwd   : delta, a query-major dQ kernel of the same shape, and the
-//                   shared key-major dK/dV kernel (dkdv_kernel.h).
+//                   key-major dK/dV kernel (dense_dkdv.h, dkdv_kernel.h).
 //   cmp_score     : probabilities of the first head of every group, fp32.
 //   cmp_topk      : per query: weighted 5-tap re-binning into selection blocks,
 //                   forced blocks, cast to bf16, top-k by (value desc, id asc),
@@ -18,6 +18,7 @@
 // :1272-1315 (selection).
 #include "attn_rows.h"
 #include "dkdv_kernel.h"
+#include "dense_dkdv.h"
 
 #include <algorithm>
 
@@ -788,12 +789,22 @@ static dim3 dense_pair_grid(int nx, int hkv, int batch, int lists = 0) {   // bo
   return g;
 }
 
+// Rows per work-group of the dK/dV kernel.  A work-group alone on a CU takes 1.3 us for a pass of 64 rows of 128 dims, two there
+// 2.5, so one for every CU is as good as two, and every share of a key tile costs 64 KB of partial sums, written and read.  Kernel
+// and reduction of both branches, us, two per slot (as for gathered rows) | 384 work-groups a branch | 256: 2000 tokens x 8 heads of
+// 128, window 128, 30.1 | 29.7 | 29.1, 3000 x 16, window 512, 71.9 | 64.4 | 72.6, 4000 x 8 79 | 64 | 70, 5003 x 32 210 | 174 | 173,
+// 12000 x 32 421 | 400 | 398; 6000 x 32 heads of 64 162 | 140 | 122, 20000 x 32 244 | 220 | 221.
+static int dense_tile_rows(int64_t rows_total, int g, int d) {
+  if (!dense_kv_shape_ok(g, d)) return kv_tile_rows(rows_total, g, d, CMP_BK);
+  const int64_t r = rows_total / (d > 64 ? 384 : 256) / 64 * 64;
+  return (int)std::max<int64_t>(128, std::min<int64_t>(r, KV_TILE_ROWS_MAX));
+}
 // rows of all (key tile, query head) pairs: a key tile of a sequence is seen by about half of its queries
 static int cmp_tile_rows(int64_t max_blocks, int64_t max_q, int hq, int g, int d) {
-  return kv_tile_rows(max_blocks * max_q * hq / 2, g, d, CMP_BK);
+  return dense_tile_rows(max_blocks * max_q * hq / 2, g, d);
 }
 static int win_tile_rows(int64_t max_blocks, int window, int hq, int g, int d) {
-  return kv_tile_rows(max_blocks * (CMP_BK + window) * hq, g, d, CMP_BK);
+  return dense_tile_rows(max_blocks * (CMP_BK + window) * hq, g, d);
 }
 
 struct CmpBwdWs {
@@ -857,6 +868,9 @@ static int attn_bwd_launch(CmpParams p, const SelBwdParams& kv, int batch, int h
   if (int rc_ = allow_lds(lds1, (const void*)cmpattn_bwd_dq_kernel<T, D, MODE>, CmpLds<D>::BYTES)) return rc_;
   static LdsAllowed lds2;
   if (int rc_ = allow_lds(lds2, (const void*)attn_bwd_dkdv_kernel<T, D, CMP_BK, KVM>, KvCfg<D, CMP_BK>::BYTES)) return rc_;
+  static LdsAllowed lds3;
+  if constexpr (D <= 128)
+    if (int rc_ = allow_lds(lds3, (const void*)dense_dkdv_kernel<T, D, KVM>, DenseKv<D>::BYTES)) return rc_;
   p.hkv = hkv;
   p.nx = (int)((max_rows + CMP_ROWS - 1) / CMP_ROWS);
   {
@@ -873,8 +887,13 @@ static int attn_bwd_launch(CmpParams p, const SelBwdParams& kv, int batch, int h
   {
     const HeadOrder order = head_order(hkv, n * kv.g * D * 2);
     ProfScope ps_(MODE == CMP_MODE_WINDOW ? "winattn_bwd_dkdv" : "cmpattn_bwd_dkdv", stream);
-    attn_bwd_dkdv_kernel<T, D, CMP_BK, KVM>
-        <<<head_tile_grid(kv.max_tiles, order), KvCfg<D, CMP_BK>::NT, KvCfg<D, CMP_BK>::BYTES, stream>>>(kv, order);
+    bool done = false;
+    if constexpr (D <= 128)
+      if ((done = dense_kv_rows_ok(kv, D)))
+        dense_dkdv_kernel<T, D, KVM><<<head_tile_grid(kv.max_tiles, order), DenseKv<D>::NT, DenseKv<D>::BYTES, stream>>>(kv, order);
+    if (!done)
+      attn_bwd_dkdv_kernel<T, D, CMP_BK, KVM>
+          <<<head_tile_grid(kv.max_tiles, order), KvCfg<D, CMP_BK>::NT, KvCfg<D, CMP_BK>::BYTES, stream>>>(kv, order);
   }
   {
     ProfScope ps_(MODE == CMP_MODE_WINDOW ? "winattn_bwd_dkdv_reduce" : "cmpattn_bwd_dkdv_reduce", stream);
@@ -908,6 +927,9 @@ static int pair_bwd_launch(CmpParams a, CmpParams b, const SelBwdParams& ka, con
   typedef KvCfg<D, CMP_BK> C;
   static LdsAllowed lds2;
   if (int rc_ = allow_lds(lds2, (const void*)attn_bwd_dkdv_pair_kernel<T, D, CMP_BK>, C::BYTES)) return rc_;
+  static LdsAllowed lds3;
+  if constexpr (D <= 128)
+    if (int rc_ = allow_lds(lds3, (const void*)dense_dkdv_pair_kernel<T, D>, DenseKv<D>::BYTES)) return rc_;
   a.hkv = b.hkv = hkv;
   a.nx = b.nx = (int)((max_rows + CMP_ROWS - 1) / CMP_ROWS);
   {
@@ -917,8 +939,12 @@ static int pair_bwd_launch(CmpParams a, CmpParams b, const SelBwdParams& ka, con
   {
     const HeadOrder order = head_order(hkv, ka.n_tokens * ka.g * D * 2);
     ProfScope ps_("attn_bwd_dkdv_pair", stream);
-    attn_bwd_dkdv_pair_kernel<T, D, CMP_BK>
-        <<<head_tile_grid(ka.max_tiles + kb.max_tiles, order), C::NT, C::BYTES, stream>>>(ka, kb, (int)ka.max_tiles, order);
+    const dim3 grid = head_tile_grid(ka.max_tiles + kb.max_tiles, order);
+    bool done = false;
+    if constexpr (D <= 128)
+      if ((done = dense_kv_rows_ok(ka, D) && dense_kv_rows_ok(kb, D)))
+        dense_dkdv_pair_kernel<T, D><<<grid, DenseKv<D>::NT, DenseKv<D>::BYTES, stream>>>(ka, kb, (int)ka.max_tiles, order);
+    if (!done) attn_bwd_dkdv_pair_kernel<T, D, CMP_BK><<<grid, C::NT, C::BYTES, stream>>>(ka, kb, (int)ka.max_tiles, order);
   }
   {
     ProfScope ps_("attn_bwd_dkdv_pair_reduce", stream);

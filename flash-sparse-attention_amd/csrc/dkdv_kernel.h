@@ -1,6 +1,6 @@
 // dK/dV kernel shared by selected attention (gathered query rows of a kv block)
-// and compressed attention (the dense range of queries that can see a tile of
-// compressed keys).  Block-major, contraction over the rows: each wave owns 16
+// and, for the shapes that dense_dkdv.h does not take, compressed and window
+// attention (the range of queries that can see a tile of keys).  Block-major, contraction over the rows: each wave owns 16
 // keys and keeps their K / V fragments in registers; Q / dO tiles of 64 rows go
 // through LDS once and feed S = Q K^T, dP = dO V^T (16x16x32 MFMA) and, through
 // transposing LDS reads, dV^T += dO^T P and dK^T += Q^T dS.  The g heads of a
