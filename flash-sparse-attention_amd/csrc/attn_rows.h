@@ -99,13 +99,16 @@ template <typename T, int D> struct AttnRows {
     for (int ks = 0; ks < NKS; ++ks) q[ks] = load16<vec8>(row + ((threadIdx.x & 63) >> 5) * (D / 2) + ks * 8);
   }
   // The same by way of an LDS tile of the wave's own: a load instruction of whole rows touches 64 / (D / 8) rows instead of 32.
-  // `row`: the q row of lane col and of lane col + 32.
-  __device__ __forceinline__ void load_q_rows(const T* row, T* tile, const TileFrags<D>& f) {
+  // `row`: the row of lane col and of lane col + 32.
+  static __device__ __forceinline__ void rows_fetch(vec8 (&x)[TileLoads<T, D>::N], const T* row) {
     typedef TileLoads<T, D> L;
     const int lane = threadIdx.x & 63;
-    vec8 x[L::N];
 #pragma unroll
     for (int j = 0; j < L::N; ++j) x[j] = load16_at<vec8>(shfl64((uint64_t)row, j * L::RPI + lane / L::CPR) + lane % L::CPR * 16);
+  }
+  static __device__ __forceinline__ void rows_to_frags(vec8 (&frag)[NKS], const vec8 (&x)[TileLoads<T, D>::N], T* tile, const TileFrags<D>& f) {
+    typedef TileLoads<T, D> L;
+    const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int j = 0; j < L::N; ++j) {
       const int r = j * L::RPI + lane / L::CPR;
@@ -113,7 +116,12 @@ template <typename T, int D> struct AttnRows {
     }
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) q[ks] = load16<vec8>(lds_ptr<T>(lds_addr(tile) + (f.k ^ (16u * ks))));
+    for (int ks = 0; ks < NKS; ++ks) frag[ks] = load16<vec8>(lds_ptr<T>(lds_addr(tile) + (f.k ^ (16u * ks))));
+  }
+  __device__ __forceinline__ void load_q_rows(const T* row, T* tile, const TileFrags<D>& f) {
+    vec8 x[TileLoads<T, D>::N];
+    rows_fetch(x, row);
+    rows_to_frags(q, x, tile, f);
   }
   // o * scale to the rows `row` of the lanes, by way of such a tile; rows whose lanes are not `valid` are left out
   __device__ __forceinline__ void store_rows(T* row, bool valid, float scale, T* tile) const {

@@ -55,34 +55,27 @@ constexpr int CMP_MODE_WINDOW = 1;   // the same query-major kernels over raw ke
 constexpr int CMP_BK = 64;      // compressed keys per tile
 constexpr int CMP_ROWS = 128;   // rows per work-group (4 waves x 32)
 
-template <int D> struct CmpLds {
-  static constexpr int KS = D + 16;  // 32 B pad: the transposing reads of K^T (dQ kernel) run conflict-free, with 16 B they do not
-  static constexpr int VS = D + 16;
-  static constexpr int BYTES = (CMP_BK * KS + CMP_BK * VS) * 2;
+template <int D> struct CmpLds {   // keys of the score kernel
+  static constexpr int KS = D + 8;  // 16 B pad: fragments of 16 bytes from 32 rows without bank conflicts
+  static constexpr int BYTES = CMP_BK * KS * 2;
 };
 
-// A K / V tile of CMP_BK rows travels as 16-byte chunks, chunk c = tid + 256 j of thread tid: row c / (D / 8),
+// A tile of CMP_BK keys travels as 16-byte chunks, chunk c = tid + 256 j of thread tid: row c / (D / 8),
 // which is tid / (D / 8) + j * ROWS_PER_STEP.  The loads are buffer loads: step j has a scalar descriptor of its
 // own (first row of the step, as many bytes as the step has rows left in the sequence) and every step uses the
-// same 32-bit lane offset (kv_tile_offset), which never changes - no per-load vector arithmetic at all, and the
+// same 32-bit lane offset (k_tile_offset), which never changes - no per-load vector arithmetic at all, and the
 // rows past the end of the sequence (last tile only) come back as zeros from the descriptor's range check.
-template <typename T, int D> struct KvTileRegs {
-  static constexpr int CPR = D / 8;                  // 16-byte chunks per row
-  static constexpr int ROWS_PER_STEP = 256 / CPR;
-  static constexpr int N = CMP_BK / ROWS_PER_STEP;   // chunks per thread and tensor
-  typename Elem<T>::vec8 k[N], v[N];
-};
 template <typename T, int D>
-__device__ __forceinline__ uint32_t kv_tile_offset(int64_t sn, int tid) {
-  constexpr int CPR = KvTileRegs<T, D>::CPR;
+__device__ __forceinline__ uint32_t k_tile_offset(int64_t sn, int tid) {
+  constexpr int CPR = D / 8;
   return (uint32_t)((tid / CPR) * sn * (int64_t)sizeof(T)) + (tid % CPR) * 16;   // host: CMP_BK * sn * sizeof(T) < 2^32
 }
-template <typename T, int D, int N>
-__device__ __forceinline__ void kv_rows_load(typename Elem<T>::vec8 (&r)[N], const T* base, int64_t sn, uint32_t off,
-                                             int row0, int n_valid) {
-  constexpr int RPS = KvTileRegs<T, D>::ROWS_PER_STEP;
+template <typename T, int D>
+__device__ __forceinline__ void stage_k_tile(const T* base, int64_t sn, uint32_t off, int row0, int n_valid, T* Ks, int tid) {
+  constexpr int CPR = D / 8, RPS = 256 / CPR, N = CMP_BK / RPS;   // chunks per row, rows per step, steps
   const int64_t row_bytes = sn * (int64_t)sizeof(T);
   const char* tile = reinterpret_cast<const char*>(base) + row0 * row_bytes;
+  typename Elem<T>::vec8 r[N];
 #pragma unroll
   for (int j = 0; j < N; ++j) {
     const int rows = min(n_valid - j * RPS, RPS);  // rows of this step inside the sequence
@@ -91,33 +84,8 @@ __device__ __forceinline__ void kv_rows_load(typename Elem<T>::vec8 (&r)[N], con
         __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(tile + j * RPS * row_bytes), 0, (int)bytes, 0x00020000);
     r[j] = __builtin_bit_cast(typename Elem<T>::vec8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
   }
-}
-// kv_tile_load issues the global loads of a tile into registers, kv_tile_store parks them in LDS: in two steps,
-// so that the rows of the next tile can travel while the current one is used.
-template <typename T, int D, bool HAS_V = true>
-__device__ __forceinline__ void kv_tile_load(KvTileRegs<T, D>& r, const T* kbase, int64_t k_sn, uint32_t k_off,
-                                             const T* vbase, int64_t v_sn, uint32_t v_off, int row0, int n_valid,
-                                             int tid) {
-  kv_rows_load<T, D>(r.k, kbase, k_sn, k_off, row0, n_valid);
-  if (HAS_V) kv_rows_load<T, D>(r.v, vbase, v_sn, v_off, row0, n_valid);
-}
-template <typename T, int D, bool HAS_V = true>
-__device__ __forceinline__ void kv_tile_store(const KvTileRegs<T, D>& r, T* Ks, T* Vs, int tid) {
-  constexpr int KS = CmpLds<D>::KS, VS = CmpLds<D>::VS;
-  constexpr int CPR = KvTileRegs<T, D>::CPR, RPS = KvTileRegs<T, D>::ROWS_PER_STEP;
 #pragma unroll
-  for (int j = 0; j < KvTileRegs<T, D>::N; ++j) {
-    const int row = tid / CPR + j * RPS, col = tid % CPR;
-    store16(&Ks[row * KS + col * 8], r.k[j]);
-    if (HAS_V) store16(&Vs[row * VS + col * 8], r.v[j]);
-  }
-}
-template <typename T, int D, bool HAS_V = true>
-__device__ __forceinline__ void stage_kv_tile(const T* kbase, int64_t k_sn, uint32_t k_off, const T* vbase, int64_t v_sn,
-                                              uint32_t v_off, int row0, int n_valid, T* Ks, T* Vs, int tid) {
-  KvTileRegs<T, D> r;
-  kv_tile_load<T, D, HAS_V>(r, kbase, k_sn, k_off, vbase, v_sn, v_off, row0, n_valid, tid);
-  kv_tile_store<T, D, HAS_V>(r, Ks, Vs, tid);
+  for (int j = 0; j < N; ++j) store16(&Ks[(tid / CPR + j * RPS) * CmpLds<D>::KS + tid % CPR * 8], r[j]);
 }
 
 // Work-group -> (query tile, sequence, kv head).  Consecutive work-groups go to the eight XCDs in turn: with the kv head
@@ -238,15 +206,20 @@ __device__ __forceinline__ void attn_fwd_tile(const CmpParams& p, int id) {
 }
 
 // --------------------------------------------------------------------- dq ----
-template <typename T, int D, int MODE>
+// The structure of the forward: dP of a step beside its exponentials, scores of the next step beside dS of this one, then the products
+// of K^T and dS; K of two steps and what is on its way in three tiles.  A step of 24 products (768 clocks) on two waves per SIMD is
+// half of it matrix time.  Against 64-key tiles by way of the registers, phases in turn, q, dO and dQ in pieces of 16 bytes, both
+// branches of a layer, us: 4 x 8192 tokens x 32 heads of 128, window 512, 980 -> 778; 12000 x 32 336 -> 276; 5003 x 32 143 -> 118;
+// 2 x 1000 x 8, window 128, 21.3 -> 15.6; 6000 x 32 of 64 100 -> 84; window alone, 9000 x 8 of 256, 128 -> 127.
+template <typename T, int D> struct CmpDqLds {
+  static constexpr int TILE = TileLoads<T, D>::BYTES, BYTES = 9 * TILE;   // three tiles of K, two of V, one of q / dO / dQ for every wave
+};
+template <typename T, int D, int MODE, bool ANY>
 __device__ __forceinline__ void attn_bwd_dq_tile(const CmpParams& p, int id) {
   typedef typename Elem<T>::vec8 vec8;
-  typedef typename Elem<T>::vec4 vec4;
-  constexpr int KS = CmpLds<D>::KS, VS = CmpLds<D>::VS;
-  constexpr int NA = CMP_BK / 32, NKS = D / 16, NDT = D / 32, NJ = CMP_BK / 16;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  T* Ks = reinterpret_cast<T*>(smem);
-  T* Vs = Ks + CMP_BK * KS;
+  typedef TileLoads<T, D, ANY> Loads;
+  constexpr int TILE = Loads::BYTES, NKS = D / 16, NDT = D / 32;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
   int bx, s, h;
   tile_of(p, id, bx, s, h);
@@ -256,102 +229,128 @@ __device__ __forceinline__ void attn_bwd_dq_tile(const CmpParams& p, int id) {
   const int rows_total = lq * p.g;
   const int row_lo = bx * CMP_ROWS;
   if (row_lo >= rows_total) return;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int col = lane & 31, hh = lane >> 5;
-  const int r = row_lo + wv * 32 + col;
-  const bool valid = r < rows_total;
-  const int rr = valid ? r : rows_total - 1;
-  const int qi = rr / p.g, head = rr - qi * p.g;
-  const int hq_i = h * p.g + head;
-  const T* qrow = reinterpret_cast<const T*>(p.q) + (int64_t)(q0 + qi) * p.q_sn + (int64_t)hq_i * p.q_sh + hh * (D / 2);
-  const T* dorow = reinterpret_cast<const T*>(p.d_o) + (int64_t)(q0 + qi) * p.do_sn + (int64_t)hq_i * p.do_sh + hh * (D / 2);
-  vec8 qreg[NKS], doreg[NKS];
-#pragma unroll
-  for (int ks = 0; ks < NKS; ++ks) {
-    qreg[ks] = load16<vec8>(qrow + ks * 8);
-    doreg[ks] = load16<vec8>(dorow + ks * 8);
-  }
-  const int64_t stat = (int64_t)hq_i * p.n_tokens + q0 + qi;
-  // a row without any visible key has lse = -inf: +inf instead turns every probability of it into 0, not NaN
-  const float2 pair = p.stat2 ? p.stat2[(int64_t)(q0 + qi) * (p.g * p.hkv) + hq_i] : make_float2(p.lse[stat], p.delta[stat]);
-  const float lse_in = pair.x;
-  const float lse_r = lse_in == -INFINITY ? INFINITY : lse_in;
-  const float delta_s = pair.y * p.scale;
-  const int jmax = KeyRange<MODE>::hi(p, qi, nc), jmin = KeyRange<MODE>::lo(p, qi);
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 31, hh = lane >> 5;
+  const int row = row_lo + wv * 32 + col;
+  const bool valid = row < rows_total;
+  const int rr = valid ? row : rows_total - 1;
+  const int qi = rr / p.g, hq_i = h * p.g + rr - qi * p.g;
+  // the range of keys of the work-group, in steps of 32
   const int qi_first = row_lo / p.g, qi_last = (min(rows_total, row_lo + CMP_ROWS) - 1) / p.g;
-  const int n_keys = KeyRange<MODE>::hi(p, qi_last, nc) + 1;                 // end of the work-group's key range
-  const int jt0 = KeyRange<MODE>::lo(p, qi_first) / CMP_BK * CMP_BK;          // its tile-aligned start
-
-  const T* kbase = reinterpret_cast<const T*>(p.k) + (int64_t)h * p.k_sh;
-  const T* vbase = reinterpret_cast<const T*>(p.v) + (int64_t)h * p.v_sh;
-  const uint32_t k_off = kv_tile_offset<T, D>(p.k_sn, tid), v_off = kv_tile_offset<T, D>(p.v_sn, tid);
-  const T* ktr = Ks + (4 * hh + ((lane & 15) >> 2)) * KS + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-
-  f32x16 dacc[NDT];
-#pragma unroll
-  for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) dacc[dt][i] = 0.f;
-
-  for (int jt = jt0; jt < n_keys; jt += CMP_BK) {
-    if (jt != jt0) __syncthreads();
-    stage_kv_tile<T, D>(kbase, p.k_sn, k_off, vbase, p.v_sn, v_off, k0 + jt, nc - jt, Ks, Vs, tid);
-    __syncthreads();
-    f32x16 acc[NA], dp[NA];
-#pragma unroll
-    for (int a = 0; a < NA; ++a) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        acc[a][i] = 0.f;
-        dp[a][i] = 0.f;
-      }
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) {
-        vec8 kf = load16<vec8>(&Ks[(a * 32 + col) * KS + hh * (D / 2) + ks * 8]);
-        acc[a] = Elem<T>::mfma32(kf, qreg[ks], acc[a]);
-        vec8 vf = load16<vec8>(&Vs[(a * 32 + col) * VS + hh * (D / 2) + ks * 8]);
-        dp[a] = Elem<T>::mfma32(vf, doreg[ks], dp[a]);
-      }
-    }
-    const int limit = jmax - jt, limit_lo = jmin - jt;
-    vec8 dsk[NJ];
-    // tiles that every row of the wave sees completely need no mask
-    if (!__all(limit >= CMP_BK - 1 && limit_lo <= 0)) {
-#pragma unroll
-      for (int a = 0; a < NA; ++a)
+  const int jt0 = __builtin_amdgcn_readfirstlane(KeyRange<MODE>::lo(p, qi_first) & ~31);
+  const int n_steps = __builtin_amdgcn_readfirstlane((KeyRange<MODE>::hi(p, qi_last, nc) + 1 - jt0 + 31) >> 5);
+  const Loads kl(p.k, p.k_sn, p.k_sh, k0, h, nc), vl(p.v, p.v_sn, p.v_sh, k0, h, nc);
+  const uint32_t k_lds = lds_addr(smem), v_lds = k_lds + 3 * TILE;
+  // this wave's share of a tile: as in the forward
+  constexpr int PARTS = Loads::N >= 2 * Loads::NV ? 2 : 1;
+  auto issue_k = [&](int t, uint32_t to) {
+    if ((wv & 1) == 0 && wv < 2 * PARTS) kl.template issue<PARTS>(jt0 + 32 * t, to, wv >> 1);
+  };
+  auto issue_v = [&](int t) {
+    if ((wv & 1) == 1 && wv < 2 * PARTS) vl.template issue<PARTS>(jt0 + 32 * t, v_lds + (t & 1) * TILE, wv >> 1);
+  };
+  AttnRows<T, D> r;   // q, and dQ in its accumulators
+  r.clear();
+  T* rows_lds = reinterpret_cast<T*>(smem + (5 + wv) * TILE);
+  if (n_steps > 0) {
+    uint32_t k_old = k_lds + 2 * TILE, k_now = k_lds, k_next = k_lds + TILE;   // where K of the last, this and the next step lies
+    issue_k(0, k_now);
+    issue_v(0);
+    issue_k(1, k_next);
+    const TileFrags<D> f;
+    vec8 xq[Loads::N], xd[Loads::N], dorow[NKS];
+    r.rows_fetch(xq, reinterpret_cast<const T*>(p.q) + (int64_t)(q0 + qi) * p.q_sn + (int64_t)hq_i * p.q_sh);
+    r.rows_fetch(xd, reinterpret_cast<const T*>(p.d_o) + (int64_t)(q0 + qi) * p.do_sn + (int64_t)hq_i * p.do_sh);
+    const int64_t stat = (int64_t)hq_i * p.n_tokens + q0 + qi;
+    // a row without any visible key has lse = -inf: +inf instead turns every probability of it into 0, not NaN
+    const float2 pair = p.stat2 ? p.stat2[(int64_t)(q0 + qi) * (p.g * p.hkv) + hq_i] : make_float2(p.lse[stat], p.delta[stat]);
+    const float lse = pair.x == -INFINITY ? INFINITY : pair.x, delta = pair.y * p.scale;
+    const int jmax = KeyRange<MODE>::hi(p, qi, nc) - jt0, jmin = KeyRange<MODE>::lo(p, qi) - jt0;
+    auto mask = [&](f32x16& x, int t) {   // a step that every row of the wave sees completely needs none
+      const int limit = jmax - 32 * t, limit_lo = jmin - 32 * t;
+      if (!__all(limit >= 31 && limit_lo <= 0)) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const int key = a * 32 + 8 * (i >> 2) + 4 * hh + (i & 3);
-          if (!(key <= limit && key >= limit_lo)) acc[a][i] = -INFINITY;
+          const int key = 8 * (i >> 2) + 4 * hh + (i & 3);
+          if (!(key <= limit && key >= limit_lo)) x[i] = -INFINITY;
         }
+      }
+    };
+    r.rows_to_frags(r.q, xq, rows_lds, f);
+    r.rows_to_frags(dorow, xd, rows_lds, f);
+    r.settle_q();
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) asm volatile("" : "+v"(dorow[ks]));
+    auto step = [&](f32x16& x, f32x16& next, int t) {   // scores of this step in x, those of the next one into `next`
+      tiles_arrived();   // K of the next step, V of this one
+      issue_k(t + 2, k_old);    // (behind the last key: zeros, and nothing is read)
+      issue_v(t + 1);
+      const uint32_t v_tile = v_lds + (t & 1) * TILE;
+      constexpr int AHEAD = 2;
+      vec8 fr[AHEAD + 1], ds[2];
+      f32x16 dp;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) dp[i] = next[i] = 0.f;
+      auto read = [&](int i) { fr[i % (AHEAD + 1)] = load16<vec8>(lds_ptr<T>((i < NKS ? v_tile : k_next) + (f.k ^ (16u * (i % NKS))))); };
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) read(i);
+      // dP of this step beside its exponentials, then scores of the next step beside dS = P (dP - delta) scale of this one
+      constexpr int LATE = NKS / 4;   // dS starts that many products after the last one of dP
+#pragma unroll
+      for (int i = 0; i < 2 * NKS; ++i) {
+        if (i + AHEAD < 2 * NKS) read(i + AHEAD);
+        if (i < NKS) {
+          dp = Elem<T>::mfma32(fr[i % (AHEAD + 1)], dorow[i % NKS], dp);
+#pragma unroll
+          for (int e = i * 16 / NKS; e < (i + 1) * 16 / NKS; ++e) {
+            x[e] = fast_exp2(x[e] * p.scale_log2 - lse);
+            asm volatile("" : "+v"(x[e]));   // (here, not in front of its use)
+          }
+        } else {
+          next = Elem<T>::mfma32(fr[i % (AHEAD + 1)], r.q[i % NKS], next);
+          constexpr int SLOTS = NKS - LATE;
+          const int j = i - NKS - LATE;
+#pragma unroll
+          for (int e = j < 0 ? 0 : j * 16 / SLOTS; e < (j < 0 ? 0 : (j + 1) * 16 / SLOTS); ++e) {
+            ds[e >> 3][e & 7] = (T)(x[e] * (dp[e] * p.scale - delta));
+            if ((e & 7) == 7) asm volatile("" : "+v"(ds[e >> 3]));
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // dQ^T += K^T dS
+      constexpr int AH = 3;
+      vec8 tr[AH + 1];
+      auto readt = [&](int i) { tr[i % (AH + 1)] = swizzled_tr_frag<T, D>(k_now + (f.v ^ (64u * (i % NDT))), i / NDT); };
+#pragma unroll
+      for (int i = 0; i < AH; ++i) readt(i);
+#pragma unroll
+      for (int i = 0; i < 2 * NDT; ++i) {
+        if (i + AH < 2 * NDT) readt(i + AH);
+        r.o[i % NDT] = Elem<T>::mfma32(tr[i % (AH + 1)], ds[i / NDT], r.o[i % NDT]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      mask(next, t + 1);
+      const uint32_t k = k_old;
+      k_old = k_now;
+      k_now = k_next;
+      k_next = k;
+    };
+    f32x16 sa, sb;
+    tiles_arrived();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sa[i] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) sa = Elem<T>::mfma32(load16<vec8>(lds_ptr<T>(k_now + (f.k ^ (16u * ks)))), r.q[ks], sa);
+    mask(sa, 0);
+    for (int t = 0;;) {
+      step(sa, sb, t);
+      if (++t >= n_steps) break;
+      step(sb, sa, t);
+      if (++t >= n_steps) break;
     }
-    // dS = P (dP - delta) scale
-#pragma unroll
-    for (int a = 0; a < NA; ++a)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float pv = fast_exp2(acc[a][i] * p.scale_log2 - lse_r);
-        dsk[a * 2 + (i >> 3)][i & 7] = (T)(pv * (dp[a][i] * p.scale - delta_s));
-      }
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int dt = 0; dt < NDT; ++dt) {
-        vec8 kf = lds_read_tr8<T>(ktr + 16 * j * KS + dt * 32, 8 * KS);
-        dacc[dt] = Elem<T>::mfma32(kf, dsk[j], dacc[dt]);
-      }
+    vm_wait<0>();
   }
-  if (!valid) return;
-  T* orow = reinterpret_cast<T*>(p.dq) + ((int64_t)(q0 + qi) * (p.g * p.hkv) + hq_i) * D + 4 * hh;
-#pragma unroll
-  for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-    for (int qd = 0; qd < 4; ++qd) {
-      vec4 x;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] = (T)dacc[dt][4 * qd + e];
-      store8(orow + dt * 32 + 8 * qd, x);
-    }
+  r.store_rows(reinterpret_cast<T*>(p.dq) + ((int64_t)(q0 + qi) * (p.g * p.hkv) + hq_i) * D, valid, 1.f, rows_lds);
 }
 
 template <typename T, int D, int MODE, bool ANY>
@@ -359,10 +358,10 @@ __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1))
 cmpattn_fwd_kernel(CmpParams p) {
   attn_fwd_tile<T, D, MODE, ANY>(p, blockIdx.x);
 }
-template <typename T, int D, int MODE>
+template <typename T, int D, int MODE, bool ANY>
 __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1))
 cmpattn_bwd_dq_kernel(CmpParams p) {
-  attn_bwd_dq_tile<T, D, MODE>(p, blockIdx.x);
+  attn_bwd_dq_tile<T, D, MODE, ANY>(p, blockIdx.x);
 }
 // Compressed (blockIdx.z == 0, in front) and window attention of one layer in one launch.  At small sizes either alone
 // leaves most of the chip idle.
@@ -469,7 +468,7 @@ kv_tiles_kernel(KvTiles p, int batch, int g) {
 
 // dQ of a pair; the first 2 hkv work-groups write the two work lists that the dK/dV launch behind it needs (their places in
 // the other rows of the grid stay empty).
-template <typename T, int D>
+template <typename T, int D, bool ANY>
 __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1))
 attn_bwd_dq_pair_kernel(CmpParams a, CmpParams b, KvTiles ta, KvTiles tb, int batch) {
   const int hkv = a.hkv, id = (int)blockIdx.x - 2 * hkv;
@@ -478,9 +477,9 @@ attn_bwd_dq_pair_kernel(CmpParams a, CmpParams b, KvTiles ta, KvTiles tb, int ba
     if (id < -hkv) kv_tiles<CMP_MODE_COMPRESSED>(ta, batch, a.g, id + 2 * hkv);
     else kv_tiles<CMP_MODE_WINDOW>(tb, batch, a.g, id + hkv);
   } else if (blockIdx.z == 0) {
-    attn_bwd_dq_tile<T, D, CMP_MODE_COMPRESSED>(a, id);
+    attn_bwd_dq_tile<T, D, CMP_MODE_COMPRESSED, ANY>(a, id);
   } else {
-    attn_bwd_dq_tile<T, D, CMP_MODE_WINDOW>(b, id);
+    attn_bwd_dq_tile<T, D, CMP_MODE_WINDOW, ANY>(b, id);
   }
 }
 
@@ -523,7 +522,7 @@ cmp_score_kernel(CmpParams p) {
   const int n_keys = qi_last >= p.kernel_size - 1 ? min(nc, (qi_last - p.kernel_size + 1) / p.kernel_stride + 1) : 0;
   const T* kbase = reinterpret_cast<const T*>(p.k) + (int64_t)h * p.k_sh;
   float* srow = p.score + ((int64_t)h * p.n_tokens + q0 + qi) * p.score_ld;
-  const uint32_t k_off = kv_tile_offset<T, D>(p.k_sn, tid);
+  const uint32_t k_off = k_tile_offset<T, D>(p.k_sn, tid);
 
   // REBIN: one more tile when the visible keys end on a tile boundary - the block that starts there still owns the
   // last key before it
@@ -531,7 +530,7 @@ cmp_score_kernel(CmpParams p) {
   float carry = 0.f;  // REBIN, lower half of the wave: probability of the key just before this tile
   for (int jt = 0; jt < n_keys_loop; jt += CMP_BK) {
     if (jt) __syncthreads();
-    stage_kv_tile<T, D, false>(kbase, p.k_sn, k_off, (const T*)nullptr, 0, 0u, k0 + jt, nc - jt, Ks, (T*)nullptr, tid);
+    stage_k_tile<T, D>(kbase, p.k_sn, k_off, k0 + jt, nc - jt, Ks, tid);
     __syncthreads();
     f32x16 acc[NA];
 #pragma unroll
@@ -860,12 +859,18 @@ static int win_fwd_launch(const CmpParams& p, int batch, int hkv, int64_t max_ro
   return attn_fwd_launch<T, D, CMP_MODE_WINDOW>(p, batch, hkv, max_rows, stream);
 }
 
+template <typename T, int D, int MODE, bool ANY>
+static int attn_dq_launch_as(const CmpParams& p, int batch, hipStream_t stream) {
+  static LdsAllowed lds;
+  if (int rc_ = allow_lds(lds, (const void*)cmpattn_bwd_dq_kernel<T, D, MODE, ANY>, CmpDqLds<T, D>::BYTES)) return rc_;
+  ProfScope ps_(MODE == CMP_MODE_WINDOW ? "winattn_bwd_dq" : "cmpattn_bwd_dq", stream);
+  cmpattn_bwd_dq_kernel<T, D, MODE, ANY><<<dense_grid(p.nx, p.hkv, batch), 256, CmpDqLds<T, D>::BYTES, stream>>>(p);
+  return 0;
+}
 template <typename T, int D, int MODE>
 static int attn_bwd_launch(CmpParams p, const SelBwdParams& kv, int batch, int hq, int hkv,
                            int64_t max_rows, int64_t n, hipStream_t stream) {
   constexpr int KVM = MODE == CMP_MODE_WINDOW ? KV_MODE_WINDOW : KV_MODE_COMPRESSED;
-  static LdsAllowed lds1;
-  if (int rc_ = allow_lds(lds1, (const void*)cmpattn_bwd_dq_kernel<T, D, MODE>, CmpLds<D>::BYTES)) return rc_;
   static LdsAllowed lds2;
   if (int rc_ = allow_lds(lds2, (const void*)attn_bwd_dkdv_kernel<T, D, CMP_BK, KVM>, KvCfg<D, CMP_BK>::BYTES)) return rc_;
   static LdsAllowed lds3;
@@ -879,11 +884,9 @@ static int attn_bwd_launch(CmpParams p, const SelBwdParams& kv, int batch, int h
     cmp_delta_kernel<T, D><<<(unsigned)((n * hq + RPB - 1) / RPB), 256, 0, stream>>>(
         (const T*)p.o, p.o_sn, p.o_sh, (const T*)p.d_o, p.do_sn, p.do_sh, n, hq, (float*)p.delta);
   }
-  {
-    ProfScope ps_(MODE == CMP_MODE_WINDOW ? "winattn_bwd_dq" : "cmpattn_bwd_dq", stream);
-    const dim3 grid = dense_grid(p.nx, hkv, batch);
-    cmpattn_bwd_dq_kernel<T, D, MODE><<<grid, 256, CmpLds<D>::BYTES, stream>>>(p);
-  }
+  if (int rc_ = rows_go_straight(p, D) ? attn_dq_launch_as<T, D, MODE, false>(p, batch, stream)
+                                       : attn_dq_launch_as<T, D, MODE, true>(p, batch, stream))
+    return rc_;
   {
     const HeadOrder order = head_order(hkv, n * kv.g * D * 2);
     ProfScope ps_(MODE == CMP_MODE_WINDOW ? "winattn_bwd_dkdv" : "cmpattn_bwd_dkdv", stream);
@@ -919,11 +922,17 @@ static int pair_fwd_launch(const CmpParams& a, const CmpParams& b, int batch, in
   return rows_go_straight(a, D) && rows_go_straight(b, D) ? pair_fwd_launch_as<T, D, false>(a, b, batch, hkv, max_rows, stream)
                                                           : pair_fwd_launch_as<T, D, true>(a, b, batch, hkv, max_rows, stream);
 }
+template <typename T, int D, bool ANY>
+static int pair_dq_launch_as(const CmpParams& a, const CmpParams& b, const KvTiles& ta, const KvTiles& tb, int batch, hipStream_t stream) {
+  static LdsAllowed lds;
+  if (int rc_ = allow_lds(lds, (const void*)attn_bwd_dq_pair_kernel<T, D, ANY>, CmpDqLds<T, D>::BYTES)) return rc_;
+  ProfScope ps_("attn_bwd_dq_pair", stream);
+  attn_bwd_dq_pair_kernel<T, D, ANY><<<dense_pair_grid(a.nx, a.hkv, batch, 2 * a.hkv), 256, CmpDqLds<T, D>::BYTES, stream>>>(a, b, ta, tb, batch);
+  return 0;
+}
 template <typename T, int D>
 static int pair_bwd_launch(CmpParams a, CmpParams b, const SelBwdParams& ka, const SelBwdParams& kb, const KvTiles& ta,
                            const KvTiles& tb, int batch, int hkv, int64_t max_rows, hipStream_t stream) {
-  static LdsAllowed lds1;
-  if (int rc_ = allow_lds(lds1, (const void*)attn_bwd_dq_pair_kernel<T, D>, CmpLds<D>::BYTES)) return rc_;
   typedef KvCfg<D, CMP_BK> C;
   static LdsAllowed lds2;
   if (int rc_ = allow_lds(lds2, (const void*)attn_bwd_dkdv_pair_kernel<T, D, CMP_BK>, C::BYTES)) return rc_;
@@ -932,10 +941,9 @@ static int pair_bwd_launch(CmpParams a, CmpParams b, const SelBwdParams& ka, con
     if (int rc_ = allow_lds(lds3, (const void*)dense_dkdv_pair_kernel<T, D>, DenseKv<D>::BYTES)) return rc_;
   a.hkv = b.hkv = hkv;
   a.nx = b.nx = (int)((max_rows + CMP_ROWS - 1) / CMP_ROWS);
-  {
-    ProfScope ps_("attn_bwd_dq_pair", stream);
-    attn_bwd_dq_pair_kernel<T, D><<<dense_pair_grid(a.nx, hkv, batch, 2 * hkv), 256, CmpLds<D>::BYTES, stream>>>(a, b, ta, tb, batch);
-  }
+  if (int rc_ = rows_go_straight(a, D) && rows_go_straight(b, D) ? pair_dq_launch_as<T, D, false>(a, b, ta, tb, batch, stream)
+                                                                 : pair_dq_launch_as<T, D, true>(a, b, ta, tb, batch, stream))
+    return rc_;
   {
     const HeadOrder order = head_order(hkv, ka.n_tokens * ka.g * D * 2);
     ProfScope ps_("attn_bwd_dkdv_pair", stream);
@@ -972,8 +980,8 @@ static int cmp_score_launch(CmpParams p, int batch, int hkv, int64_t max_q, hipS
   p.hkv = hkv;
   p.nx = (int)((max_q + CMP_ROWS - 1) / CMP_ROWS);
   const dim3 grid = dense_grid(p.nx, hkv, batch);
-  if (p.rebin) cmp_score_kernel<T, D, true><<<grid, 256, CMP_BK * CmpLds<D>::KS * 2, stream>>>(p);
-  else cmp_score_kernel<T, D, false><<<grid, 256, CMP_BK * CmpLds<D>::KS * 2, stream>>>(p);
+  if (p.rebin) cmp_score_kernel<T, D, true><<<grid, 256, CmpLds<D>::BYTES, stream>>>(p);
+  else cmp_score_kernel<T, D, false><<<grid, 256, CmpLds<D>::BYTES, stream>>>(p);
   return 0;
 }
 

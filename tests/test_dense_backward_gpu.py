@@ -1,4 +1,4 @@
-"""GPU: dK / dV of window and compressed attention where q and dO go straight to LDS, against the kernel that takes any rows (the same
+"""GPU: dQ, dK and dV of window and compressed attention where q and dO go straight to LDS, against the kernel that takes any rows (the same
 tensors one element off their alignment): GQA groups that fill a pass of 64 rows in different ways, key tiles and passes that end early,
 tiles of one work-group and of several, rows of a head far apart or not, statistics of either type."""
 import pytest
@@ -48,9 +48,12 @@ def test_forms(dev, lens, hq, hkv, d, window, dtype, heads_first):
     tol = 4e-3 if dtype == torch.bfloat16 else 6e-4
     o, lse = ops.winattn_fwd(q, k, v, cu, max(lens), window)
     oc, lsec = ops.cmpattn_fwd(q, ck, cv, 32, 16, cu, cu_ck, max(lens))
-    for name, run in (("window", lambda q, do: ops.winattn_bwd(q, k, v, o, do, lse, cu, max(lens), window)),
-                      ("compressed", lambda q, do: ops.cmpattn_bwd(q, ck, cv, oc, do, lsec, 32, 16, cu, cu_ck, max(lens)))):
-        got, want = run(q, do), run(_off(q.contiguous()), _off(do.contiguous()))
+    for name, k_, v_, run in (
+            ("window", k, v, lambda q, k, v, do: ops.winattn_bwd(q, k, v, o, do, lse, cu, max(lens), window)),
+            ("compressed", ck, cv, lambda q, k, v, do: ops.cmpattn_bwd(q, k, v, oc, do, lsec, 32, 16, cu, cu_ck, max(lens)))):
+        got, want = run(q, k_, v_, do), run(_off(q.contiguous()), k_, v_, _off(do.contiguous()))
+        # keys and values that cannot go straight to LDS take the same steps through the registers
+        assert all(torch.equal(x, y) for x, y in zip(got, run(q, _off(k_), _off(v_), do))), name
         for part, x, y in zip(("dq", "dk", "dv"), got, want):
             assert torch.isfinite(x.float()).all(), (name, part)
             if y.numel():
