@@ -154,8 +154,11 @@ template <int W, bool HALVES = true> __device__ __forceinline__ int swz(int row,
 
 template <int D, int BK> struct KvCfg {
   static constexpr int NW = BK / 16;        // one wave per 16 keys
-  // gathered rows per pass; 32 where 8 waves of head_dim 256 leave no registers for a 64-row pass
-  static constexpr int KV_R = (D >= 256 && BK >= 128) ? 32 : 64;
+  // Gathered rows per pass; 32 where 8 waves of head_dim 256 leave no registers for a 64-row pass, and with two waves, which
+  // would have 16 pieces of every tensor in registers each (107 of them spilled at head_dim 128) and one wave on a SIMD: fused
+  // backward of 16 blocks of 32, 20000 tokens x 4 heads of 128 430 -> 136 us, 60000 x 8 2544 -> 996, 3000 x 4 of 256 523 -> 123;
+  // 30000 x 8 of 64, where they have eight pieces, 231 -> 238.
+  static constexpr int KV_R = (D >= 256 && BK >= 128) || (D >= 128 && BK <= 32) ? 32 : 64;
   static constexpr int NT = NW * 64;
   static constexpr int QS = D;             // LDS rows of the Q / dO tiles are unpadded and swizzled (swz<D>)
   static constexpr int CPR = D / 8;         // 16-byte chunks per row
@@ -671,30 +674,47 @@ __device__ __forceinline__ void attn_bwd_dkdv_tile(const SelBwdParams& p, const 
 #pragma unroll
     for (int t = 0; t < NDT; ++t) dvacc[t] *= P_UNDO;
   }
-  if (ntile_b == 1) {
-    if (key_ok) {
-      T* dkrow = reinterpret_cast<T*>(p.dk) + (int64_t)ktok * p.dk_sn + (int64_t)h * p.dk_sh + 4 * kg;
-      T* dvrow = reinterpret_cast<T*>(p.dv) + (int64_t)ktok * p.dk_sn + (int64_t)h * p.dk_sh + 4 * kg;
+  // Whole rows, by way of LDS: dK, then dV, EW dims at a time, as [16][EW] fp32 of every wave with 16-byte chunk c of row r at
+  // c ^ r.  (The pass loop ends with a barrier: nobody reads what is overwritten here.)  A work-group of a short problem has few
+  // passes in front of this: 2000 tokens x 8 heads, 8 blocks of 64, 32.0 -> 28.5 us against pieces of 8 and 64 bytes straight
+  // from the registers; 12000 x 8, 8 blocks of 128, 259 -> 256; no difference at the largest.
+  constexpr int EW = D < 128 ? D : 128, CH = EW / 4, XM = CH - 1 < 15 ? CH - 1 : 15;
+  static_assert(C::NW * 16 * EW * 4 <= (FUSE_DQ ? C::BYTES_FUSED : C::BYTES), "staging of the results");
+  f32x4* own = reinterpret_cast<f32x4*>(smem) + wv * (16 * CH);
+  auto leave = [&](const f32x4 (&acc)[NDT], void* out, int which) {
 #pragma unroll
-      for (int t = 0; t < NDT; ++t) {
-        vec4 a, b;
+    for (int d0 = 0; d0 < NDT; d0 += EW / 16) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          a[i] = (T)dkacc[t][i];
-          b[i] = (T)dvacc[t][i];
+      for (int t = 0; t < EW / 16; ++t) own[l16 * CH + ((4 * t + kg) ^ (l16 & XM))] = acc[d0 + t];
+      __builtin_amdgcn_wave_barrier();
+      if (ntile_b == 1) {
+        constexpr int CPW = EW / 8, RPI = 64 / CPW;
+        T* rows_out = reinterpret_cast<T*>(out) + (int64_t)(blk.key_row0 + wv * 16) * p.dk_sn + (int64_t)h * p.dk_sh + d0 * 16;
+#pragma unroll
+        for (int j = 0; j < 16 / RPI; ++j) {
+          const int r = j * RPI + lane / CPW, c = 2 * (lane % CPW);
+          const f32x4 lo = own[r * CH + (c ^ (r & XM))], hi = own[r * CH + ((c + 1) ^ (r & XM))];
+          vec8 y;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            y[e] = (T)lo[e];
+            y[4 + e] = (T)hi[e];
+          }
+          if (wv * 16 + r < blk.n_keys_valid) store16(rows_out + (int64_t)r * p.dk_sn + 4 * c, y);
         }
-        store8(dkrow + 16 * t, a);
-        store8(dvrow + 16 * t, b);
-      }
-    }
-  } else {
-    float* part = p.dkdv_part + ((int64_t)h * p.max_tiles + w) * (2 * BK * D) + key * D + 4 * kg;
+      } else {
+        float* part = p.dkdv_part + ((int64_t)h * p.max_tiles + w) * (2 * BK * D) + which * (BK * D) + wv * 16 * D + d0 * 16;
 #pragma unroll
-    for (int t = 0; t < NDT; ++t) {
-      __builtin_nontemporal_store(dkacc[t], reinterpret_cast<f32x4*>(part + 16 * t));
-      __builtin_nontemporal_store(dvacc[t], reinterpret_cast<f32x4*>(part + BK * D + 16 * t));
+        for (int j = 0; j < 16 * CH / 64; ++j) {
+          const int r = (j * 64 + lane) / CH, c = (j * 64 + lane) % CH;
+          __builtin_nontemporal_store(own[r * CH + (c ^ (r & XM))], reinterpret_cast<f32x4*>(part + r * D + 4 * c));
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
     }
-  }
+  };
+  leave(dkacc, p.dk, 0);
+  leave(dvacc, p.dv, 1);
 }
 
 template <typename T, int D, int BK, int MODE, bool FUSE_DQ = false, bool GATED = false>
