@@ -574,20 +574,25 @@ template <typename T, bool MERGE> static int dispatch_direct_fwd(int d, const Di
 }
 
 // Whether the forward of `n` tokens in sequences of at most `max_len` takes this path.  Both sides in us on one chip: these
-// kernels visit up to half of a sequence for every row; the block-major launches work on topk * block keys per row, behind 33 us
-// that do not depend on the size (index, two more launches and their gaps), 12 of them for the index, which is no loss where the
-// caller builds it all the same (training).  index + block-major / direct in us on the sizes above, head_dim 128: 3000 x 4
-// 13 + 40 / 28, 5000 x 4 17 + 54 / 46, 8000 x 4 23 + 77 / 100, 5000 x 32 27 + 288 / 222, 8000 x 32 33 + 460 / 503; GQA 4 5000 x 32
-// 18 + 269 / 212, 8000 x 32 24 + 428 / 485; 64: 8000 x 4 23 + 49 / 55, 5000 x 32 27 + 171 / 136, 8000 x 32 33 + 264 / 302; 256:
-// 3000 x 4 11 + 53 / 48, 3000 x 32 12 + 243 / 210, 5000 x 32 22 + 434 / 512.
+// kernels visit up to half of a sequence for every row; the block-major launches write and read a partial row for every (row,
+// block) and work on topk * block keys per row, behind a fixed part and, unless the caller builds it all the same (training), the
+// index.  index + block-major / direct in us, blocks of 64 and 16 to a list unless said otherwise, head_dim 128: 3000 x 4 13 + 40 /
+// 28, 5000 x 4 17 + 54 / 46, 8000 x 4 23 + 77 / 100, 5000 x 32 27 + 288 / 222, 8000 x 32 33 + 460 / 503, 5000 x 32, 16 blocks of
+// 32, 19 + 260 / 199, 8 of 64 14 + 155 / 199, 8 of 128 13 + 196 / 208; 64: 8000 x 4 23 + 49 / 55, 5000 x 32 27 + 171 / 136, 16
+// blocks of 32 19 + 148 / 121, 8 of 64 14 + 88 / 119; 256: 3000 x 32 13 + 361 / 203, 16 blocks of 32 14 + 321 / 200, 8 of 64 11 +
+// 219 / 202, 8 of 128 12 + 243 / 210; 5000 x 4 17 + 114 / 105, 8 of 64 13 + 78 / 102.
 bool selattn_direct_preferred(int64_t n, int64_t max_len, int hq, int d, int topk, int bk, bool index_needed) {
   if (!(d == 64 || d == 128 || d == 256) || !(bk == 32 || bk == 64 || bk == 128) || topk > 4096 ||
       max_len > (int64_t)bk * DIR_MAX_BLOCKS)
     return false;
   const double rows = (double)n * hq * d / 128, len = (double)max_len;
   const double keys = std::min<double>((double)topk * bk, len);
-  const double block_major = 33 + rows * keys / (d == 256 ? 7.8e5 : d == 128 ? 6.2e5 : 5.4e5);
-  return direct_us(direct_form(d, rows, len), d, rows, len) <= block_major - (index_needed ? 12 : 0);
+  struct Fit { double fixed, block, key; };   // per row of 128 dims
+  static constexpr Fit fits[3] = {{21, 8.7e-5, 4e-7}, {24, 8.1e-5, 3e-7}, {27, 8e-5, 4.5e-7}};
+  const Fit& f = fits[d <= 64 ? 0 : d <= 128 ? 1 : 2];
+  const double blocks = std::min<double>(topk, std::ceil(len / bk));
+  const double block_major = f.fixed + rows * (blocks * f.block + keys * f.key), index = index_needed ? 0 : 9.5 + 1.1e-4 * (double)n * topk;
+  return direct_us(direct_form(d, rows, len), d, rows, len) <= block_major + index;
 }
 
 int selattn_direct_fwd(const void* q, const void* k, const void* v, int32_t dtype, int64_t q_stride_n, int64_t q_stride_h,
