@@ -796,15 +796,11 @@ static dim3 dense_pair_grid(int nx, int hkv, int batch, int lists = 0) {   // bo
 static int dense_tile_rows(int64_t rows_total, int g, int d) {
   if (!dense_kv_shape_ok(g, d)) return kv_tile_rows(rows_total, g, d, CMP_BK);
   const int64_t r = rows_total / (d > 64 ? 384 : 256) / 64 * 64;
-  return (int)std::max<int64_t>(128, std::min<int64_t>(r, KV_TILE_ROWS_MAX));
+  return (int)std::max<int64_t>(kv_tile_rows(rows_total, g, d, CMP_BK), std::min<int64_t>(r, KV_TILE_ROWS_MAX));
 }
 // rows of all (key tile, query head) pairs: a key tile of a sequence is seen by about half of its queries
-static int cmp_tile_rows(int64_t max_blocks, int64_t max_q, int hq, int g, int d) {
-  return dense_tile_rows(max_blocks * max_q * hq / 2, g, d);
-}
-static int win_tile_rows(int64_t max_blocks, int window, int hq, int g, int d) {
-  return dense_tile_rows(max_blocks * (CMP_BK + window) * hq, g, d);
-}
+static int64_t cmp_rows_total(int64_t max_blocks, int64_t max_q, int hq) { return max_blocks * max_q * hq / 2; }
+static int64_t win_rows_total(int64_t max_blocks, int window, int hq) { return max_blocks * (CMP_BK + window) * hq; }
 
 struct CmpBwdWs {
   size_t off_delta, off_cu_tiles, off_counts, off_tiles, off_part, total;
@@ -812,19 +808,25 @@ struct CmpBwdWs {
   int tile_rows;
 };
 
+// The work list and the partial sums of key tiles that at most `rows` rows see each.  The room for the sums is that of the shares
+// that gathered rows would have, as callers know it: shares for one work-group per CU are never shorter.
+static void dense_tiles(CmpBwdWs& w, int64_t rows, int64_t rows_total, int g, int hkv, int d) {
+  const int64_t gathered = kv_tile_rows(rows_total, g, d, CMP_BK);
+  w.tile_rows = dense_tile_rows(rows_total, g, d);
+  w.max_tiles = w.max_blocks * ((rows + w.tile_rows - 1) / w.tile_rows);   // as kv_tiles deals them
+  w.total = w.off_part + align_up((size_t)hkv * w.max_blocks * ((rows + gathered - 1) / gathered) * 2 * CMP_BK * d * 4, 256);
+}
 static CmpBwdWs cmp_bwd_ws(int64_t n, int64_t n_k, int64_t max_q, int batch, int hq, int hkv, int d) {
   CmpBwdWs w;
   const int g = hq / hkv;
   w.max_blocks = (n_k + CMP_BK - 1) / CMP_BK + batch;
-  // a key tile is seen by at most max_q queries of its sequence; rows = queries * g
-  w.tile_rows = cmp_tile_rows(w.max_blocks, max_q, hq, g, d);
-  w.max_tiles = w.max_blocks * ((max_q * g + w.tile_rows - 1) / w.tile_rows);
   w.off_delta = 0;
   w.off_cu_tiles = align_up((size_t)n * hq * 4, 256);
   w.off_counts = w.off_cu_tiles + align_up((size_t)(batch + 1) * 4, 256);
   w.off_tiles = w.off_counts + align_up((size_t)hkv * w.max_blocks * 4, 256);
   w.off_part = w.off_tiles + align_up((size_t)hkv * (w.max_blocks + 1) * 4, 256);
-  w.total = w.off_part + align_up((size_t)hkv * w.max_tiles * 2 * CMP_BK * d * 4, 256);
+  // a key tile is seen by at most max_q queries of its sequence; rows = queries * g
+  dense_tiles(w, max_q * g, cmp_rows_total(w.max_blocks, max_q, hq), g, hkv, d);
   return w;
 }
 
@@ -1257,10 +1259,7 @@ extern "C" int fsa_winattn_fwd(const void* q, const void* k, const void* v, int3
 static CmpBwdWs win_bwd_ws(int64_t n, int64_t max_q, int window, int batch, int hq, int hkv, int d) {
   CmpBwdWs w = cmp_bwd_ws(n, n, max_q, batch, hq, hkv, d);
   const int g = hq / hkv;
-  const int64_t rows = (int64_t)(CMP_BK + window) * g;
-  w.tile_rows = win_tile_rows(w.max_blocks, window, hq, g, d);
-  w.max_tiles = w.max_blocks * ((rows + w.tile_rows - 1) / w.tile_rows);   // as kv_tiles deals them
-  w.total = w.off_part + align_up((size_t)hkv * w.max_tiles * 2 * CMP_BK * d * 4, 256);
+  dense_tiles(w, (int64_t)(CMP_BK + window) * g, win_rows_total(w.max_blocks, window, hq), g, hkv, d);
   return w;
 }
 
