@@ -1,8 +1,8 @@
 // Compressed attention (queries against the compressed keys / values), the
 // block-importance scores derived from it and the top-k block selection, gfx950.
 //
-//   cmpattn_fwd   : query-major flash attention over tiles of 64 compressed keys
-//                   staged in LDS; rows are (query, head-in-group) pairs so one
+//   cmpattn_fwd   : query-major flash attention over tiles of 32 compressed keys
+//                   that go straight to LDS; rows are (query, head-in-group) pairs so one
 //                   K/V tile serves the whole GQA group; S^T = K Q^T with one row
 //                   per lane, online softmax in registers, O^T += V^T P^T.
 //   cmpattn_bwd   : delta, a query-major dQ kernel of the same shape, and the
@@ -207,10 +207,10 @@ __device__ __forceinline__ void attn_fwd_tile(const CmpParams& p, int id) {
 
 // --------------------------------------------------------------------- dq ----
 // The structure of the forward: dP of a step beside its exponentials, scores of the next step beside dS of this one, then the products
-// of K^T and dS; K of two steps and what is on its way in three tiles.  A step of 24 products (768 clocks) on two waves per SIMD is
-// half of it matrix time.  Against 64-key tiles by way of the registers, phases in turn, q, dO and dQ in pieces of 16 bytes, both
-// branches of a layer, us: 4 x 8192 tokens x 32 heads of 128, window 512, 980 -> 778; 12000 x 32 336 -> 276; 5003 x 32 143 -> 118;
-// 2 x 1000 x 8, window 128, 21.3 -> 15.6; 6000 x 32 of 64 100 -> 84; window alone, 9000 x 8 of 256, 128 -> 127.
+// of K^T and dS; K of two steps and what is on its way in three tiles.  Matrix unit 50 %, vector issue 47 %, LDS 36 %: as in the kernel
+// of dK / dV, the chain of a step is the rest.  Against 64-key tiles by way of the registers, phases in turn, q, dO and dQ in pieces of
+// 16 bytes, both branches of a layer, us: 4 x 8192 tokens x 32 heads of 128, window 512, 980 -> 778; 12000 x 32 336 -> 276; 5003 x 32
+// 143 -> 118; 2 x 1000 x 8, window 128, 21.3 -> 15.6; 6000 x 32 of 64 100 -> 84; window alone, 9000 x 8 of 256, 128 -> 127.
 template <typename T, int D> struct CmpDqLds {
   static constexpr int TILE = TileLoads<T, D>::BYTES, BYTES = 9 * TILE;   // three tiles of K, two of V, one of q / dO / dQ for every wave
 };

@@ -6,10 +6,10 @@
 // and 32 keys, whose K (and, at head_dim 64, V) fragments stay in registers; the other V fragments lie in LDS in the order of the
 // lanes.  (16 keys a wave, as for gathered rows, read every row of Q and dO twice as often: 128 KB of LDS traffic for 64 keys x 32
 // rows, 1000 clocks beside 512 of products.)  Q, dO and the statistics of the next pass are on their way to LDS past the registers
-// while this one is computed; exponentials stand beside the products of dP, dS beside those of dV.  Bound by LDS reads (39 KB for
-// 1024 clocks of products) and by the chain of a pass on two waves per SIMD: 0.4 of the matrix rate.  Both branches of a layer, us,
-// before -> after: 4 x 8192 tokens x 32 heads of 128, window 512, 1550 -> 1070; 5003 233 -> 161; 2 x 1000 x 8, window 128, 21.1 -> 17.6;
-// 6000 x 32 heads of 64 152 -> 113.
+// while this one is computed; exponentials stand beside the products of dP, dS beside those of dV.  No unit is full (4 x 8192 tokens:
+// matrix 51 %, vector issue 49 %, LDS 40 %): the rest is the chain of a pass on two waves per SIMD, at the 1.7 GHz that the chip
+// keeps up under this load.  Both branches of a layer, us, before -> after: 4 x 8192 tokens x 32 heads of 128, window 512, 1550 ->
+// 1075; 5003 233 -> 161; 2 x 1000 x 8, window 128, 21.1 -> 17.4; 6000 x 32 heads of 64 152 -> 114.
 #pragma once
 #include "attn_rows.h"
 #include "dkdv_kernel.h"
