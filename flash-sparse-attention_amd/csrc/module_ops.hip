@@ -275,6 +275,12 @@ template <typename T> __device__ __forceinline__ void lc_dpe(const LcTensors& tp
 }
 
 // dX: one wave = 32 tokens of one phase (t % stride), so that the window offsets k_r are wave-uniform
+template <int D> struct LcDxLds {
+  static constexpr int WS = D + 8;                          // W of a step, rows 16 bytes apart in the banks
+  static constexpr int ROWS_BYTES = LC_ROWS * D * 2;        // the results of the four waves, in place of it (head_dim 64: the larger)
+  static constexpr int SUMS_BYTES = 64 * (LCB_COLS + 1) * 4;   // lc_dbias
+  static constexpr int BYTES = std::max({D * WS * 2, ROWS_BYTES, SUMS_BYTES});
+};
 template <typename T, int D>
 __global__ void __launch_bounds__(256)
 lc_dx_kernel(LcPair p, const int32_t* __restrict__ cu_x, const int32_t* __restrict__ cu_y, int nheads, int ks, int stride) {
@@ -309,7 +315,7 @@ lc_dx_kernel(LcPair p, const int32_t* __restrict__ cu_x, const int32_t* __restri
     for (int i = 0; i < 16; ++i) acc[i_][i] = 0.f;
   // W[h, k] ([d][dout], 2 D^2 bytes) of the step is staged in LDS: as the A operand every lane reads a different
   // row of it, which straight from global memory is 64 cache lines per load instruction
-  constexpr int WS = D + 8;
+  constexpr int WS = LcDxLds<D>::WS;
   T* Ws = reinterpret_cast<T*>(lc_smem);
   for (int r = 0; r < nrep; ++r) {
     const int nwin = m - r, k = phase + r * stride;
@@ -339,6 +345,7 @@ lc_dx_kernel(LcPair p, const int32_t* __restrict__ cu_x, const int32_t* __restri
   // Whole rows, by way of LDS (chunk c of row r in the place of chunk c ^ chunk_swizzle(r)).  Against pieces of 8 bytes of 32 rows,
   // us: 4 x 8192 tokens x 8 heads of 128 105 -> 92, 5003 x 8 26.7 -> 23.4, 6000 x 8 of 64 15.8 -> 12.3.
   __syncthreads();
+  static_assert(256 / WAVE * 32 * D * (int)sizeof(T) <= LcDxLds<D>::BYTES, "a tile of 32 rows for every wave");
   T* own = Ws + wv * (32 * D);
 #pragma unroll
   for (int i_ = 0; i_ < NT; ++i_)
@@ -619,7 +626,7 @@ template <typename T, int D>
 static int lc_bwd_t(const LcPair& p, int n, const int32_t* cu_x, const int32_t* cu_y, int batch, int64_t max_x, int h, int ks,
                     int stride, hipStream_t stream) {
   static LdsAllowed lds1;
-  if (int rc_ = allow_lds(lds1, (const void*)lc_dx_kernel<T, D>, D * (D + 8) * 2)) return rc_;
+  if (int rc_ = allow_lds(lds1, (const void*)lc_dx_kernel<T, D>, LcDxLds<D>::BYTES)) return rc_;
   static LdsAllowed lds2;
   if (int rc_ = allow_lds(lds2, (const void*)lc_dw_kernel<T, D>, LcDwLds<D>::BYTES)) return rc_;
   {
@@ -627,7 +634,7 @@ static int lc_bwd_t(const LcPair& p, int n, const int32_t* cu_x, const int32_t* 
     const int64_t m_per_phase = (max_x + stride - 1) / stride;
     // the grid is sized for the longest sequence; shorter sequences recompute their own tiling inside
     const dim3 grid((unsigned)(D / LCB_COLS + stride * ((m_per_phase + LC_ROWS - 1) / LC_ROWS)), batch, n * h);
-    lc_dx_kernel<T, D><<<grid, 256, D * (D + 8) * 2, stream>>>(p, cu_x, cu_y, h, ks, stride);
+    lc_dx_kernel<T, D><<<grid, 256, LcDxLds<D>::BYTES, stream>>>(p, cu_x, cu_y, h, ks, stride);
   }
   ProfScope ps_("linear_compress_dw", stream);
   const dim3 grid(LC_DPE_WGS + (D == 64 ? ks / 2 : ks), n * h, D == 64 ? 1 : D / 128);

@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 # head_dim 96 is not a size the kernels are built for (it runs zero-padded to 128), head_dim 64 is padded for the
 # weight gradient of the compression only
 @pytest.mark.parametrize("dtype,lens,hd", [(torch.bfloat16, [700, 1300], 128), (torch.float16, [40, 1000, 25], 128),
-                                           (torch.bfloat16, [600, 300], 96), (torch.bfloat16, [500], 64)])
+                                           (torch.bfloat16, [600, 300], 96), (torch.bfloat16, [500], 64),
+                                           (torch.bfloat16, [2150], 64)])
 def test_layer_forward_backward(dev, dtype, lens, hd):
     print(f"case {dtype} lens={lens} head_dim={hd}", flush=True)
     torch.manual_seed(0)

@@ -39,6 +39,12 @@ CASES = [
     ([0, 20, 700, 731, 2100, 3000], 2, 128, 32, 16, torch.bfloat16, True),
     ([0, 1500], 2, 128, 32, 16, torch.float16, False),
     ([0, 1100], 2, 256, 32, 16, torch.float16, True),
+    # head_dim 64, tokens of a phase (every 16th) in all four waves of a work-group: a whole tile of 128 and four more, then tiles
+    # that end in the first wave, the second, the third and the fourth
+    ([0, 2100], 2, 64, 32, 16, torch.bfloat16, True),
+    ([0, 2100], 2, 64, 32, 16, torch.float16, False),
+    ([0, 20, 660, 1960, 3720], 3, 64, 32, 16, torch.bfloat16, False),
+    ([0, 20, 660, 1960, 3720], 3, 64, 32, 16, torch.float16, True),
 ]
 
 
