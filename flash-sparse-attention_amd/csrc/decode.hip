@@ -1121,16 +1121,31 @@ static int dec_grid_waves(int* n_waves, int* device) {
   return 0;
 }
 
-// Work-groups per (request, kv head) of the chunked form: a tile per wave while the chip holds them at once, 1 where the waves
-// would have more than DEC_CHUNK_TILES tiles (the shares of the persistent grid are the better ones then).  Against partials and
-// a merge launch, us, 32 + 8 heads of 128, compressed: one request of 16K 10.7 -> 8.8, 32K 12.0 -> 8.8, 128K 21.9 -> 16.8, four of
-// 32K 16.0 -> 12.7, 8 of 16K 14.8 -> 12.6; 16 of 32K 28.5 -> 27.4, with twice the work-groups 31.9; 1024 selected keys: one request
-// 9.1 -> 8.6, 12 requests, against a work-group for each pair, 16.5 -> 15.1.
+// Work-groups per (request, kv head) of the chunked form: a tile per wave while the chip holds them at once, 1 where another form
+// is the better one.  Against partials and a merge launch, us, 32 + 8 heads of 128, compressed: one request of 16K 10.7 -> 8.8, 32K
+// 12.0 -> 8.8, 128K 21.9 -> 16.8, four of 32K 16.0 -> 12.7, 8 of 16K 14.8 -> 12.6; 16 of 32K 28.5 -> 27.4, with twice the work-groups
+// 31.9; 1024 selected keys: one request 9.1 -> 8.6.  What the chip does not hold waits for a place: 128 chunks beside 256 of head_dim
+// 256, one to a CU, make 12 pairs of 125 tiles 1.24 times as slow as without chunks, 256 in all 0.75 times.  With more than
+// DEC_CHUNK_TILES tiles per wave the shares of the persistent grid are better.
 constexpr int DEC_CHUNK_TILES = 4;
-static int64_t dec_chunks(int64_t req_tiles, int64_t pairs) {
-  const int64_t most = std::min<int64_t>(DEC_MAX_CHUNKS, DEC_CHUNK_SLOTS / 2 / std::max<int64_t>(1, pairs));
+template <int D> static int64_t dec_chunks(int64_t req_tiles, int64_t pairs) {
+  constexpr int64_t RESIDENT = 256 * DecOcc<D>::WAVES_PER_SIMD;   // a wave on every SIMD of a CU is a work-group
+  static_assert(RESIDENT <= DEC_CHUNK_SLOTS, "room for the partials");
+  const int64_t most = std::min<int64_t>(DEC_MAX_CHUNKS, RESIDENT / std::max<int64_t>(1, pairs));
   const int64_t n = std::min((req_tiles + DEC_CHUNK_WAVES - 1) / DEC_CHUNK_WAVES, most);
   return n > 1 && req_tiles <= n * DEC_CHUNK_WAVES * DEC_CHUNK_TILES ? n : 1;
+}
+// Which form.  One work-group for a pair, without an exchange, where its waves have at most two tiles, and four where there are
+// pairs enough that the chip is not left idle.  There chunks pay for their exchange only while they cut a pair into four and
+// more, and then from the fourth tile on; us, one work-group / chunks, compressed: 128 pairs of 17 tiles of 64 dims 5.8 / 8.3, of 32
+// 8.2 / 9.3, of 128 dims 17 tiles 9.9 / 11.3, 32 tiles 17.2 / 16.4, 200 pairs 18.3 / 22.7.
+enum DecForm { DEC_FORM_SHARES, DEC_FORM_ONE, DEC_FORM_CHUNKS };
+template <int D> static DecForm dec_form(int64_t req_tiles, int64_t pairs, int64_t* chunks) {
+  constexpr int W = DecOne<D>::WAVES;
+  *chunks = dec_chunks<D>(req_tiles, pairs);
+  if (req_tiles <= 2 * W && pairs <= 512) return DEC_FORM_ONE;
+  if (pairs >= 96 && req_tiles <= 4 * W && pairs <= 512 && !(D >= 128 && *chunks >= 4 && req_tiles > 3 * W)) return DEC_FORM_ONE;
+  return *chunks > 1 && req_tiles > 2 * W ? DEC_FORM_CHUNKS : DEC_FORM_SHARES;
 }
 static uint64_t dec_call_number() {
   static std::atomic<uint64_t> next{0x5eed0fca115ull};
@@ -1153,12 +1168,11 @@ static int dec_launch(const DecParams& p0, hipStream_t stream) {
   const int64_t req_tiles = MODE == DEC_MODE_COMPRESSED ? ((int64_t)p.max_keys + DEC_TK - 1) / DEC_TK
                                                         : (int64_t)p.topk * ((p.block_size + DEC_TK - 1) / DEC_TK);
   const int64_t pairs = (int64_t)p.batch * p.hkv;
-  const int64_t chunks = dec_chunks(req_tiles, pairs);
-  const bool chunked = chunks > 1 && req_tiles > 2 * DecOne<D>::WAVES;
-  const bool one = !chunked && req_tiles <= (pairs < 96 ? 2 : 4) * DecOne<D>::WAVES && pairs <= 512;
+  int64_t chunks = 0;
+  const DecForm form = dec_form<D>(req_tiles, pairs, &chunks);
   const int64_t most = std::max<int64_t>(1, req_tiles * p.batch);
   p.n_groups = (int)std::min<int64_t>(std::max(1, n_waves / p.hkv), most);
-  if (MODE == DEC_MODE_COMPRESSED && p.batch > WAVE && !one && !chunked) decode_plan_kernel<<<1, WAVE, 0, stream>>>(p);
+  if (MODE == DEC_MODE_COMPRESSED && p.batch > WAVE && form == DEC_FORM_SHARES) decode_plan_kernel<<<1, WAVE, 0, stream>>>(p);
   // two neighbouring kv heads per work-group (64 requests of 32K - 128K: 304 us a step with one, 288 / 291 / 293 with
   // two / four / eight)
   const int wg_waves = std::min(p.hkv, DecOcc<D>::WG_WAVES);
@@ -1169,10 +1183,10 @@ static int dec_launch(const DecParams& p0, hipStream_t stream) {
     const bool own_col = MODE == DEC_MODE_COMPRESSED && p.raw_score && p0.score_head_as_written;
     p.g = std::min(p0.g - head0, own_col ? 15 : 16);
     p.score_col = own_col ? p.g : 0;
-    if (one) {
+    if (form == DEC_FORM_ONE) {
       rc = dec_one_launch<T, D, MODE>(p, p.batch * p.hkv, dev, stream);
       if (rc) return rc;
-    } else if (chunked) {
+    } else if (form == DEC_FORM_CHUNKS) {
       constexpr int LDS = DEC_CHUNK_WAVES * DecLds<D>::BYTES;
       static LdsAllowed allowed;
       if (int rc_ = allow_lds(allowed, (const void*)decode_attn_chunked_kernel<T, D, MODE>, LDS, dev)) return rc_;

@@ -28,7 +28,16 @@ def _case(dev, n_keys, hq, hkv, d, dtype, seed=0):
     ([32768], 2, 1, 64, torch.float16),               # ... of four tiles per wave
     ([32769], 2, 1, 64, torch.float16),               # one key more: shares of the persistent grid
     ([1025, 700], 34, 2, 256, torch.bfloat16),        # two launches per group
-    ([1030] * 16, 16, 16, 128, torch.bfloat16),       # 256 pairs of two work-groups
+    ([1030] * 16, 16, 16, 128, torch.bfloat16),       # 256 pairs, a tile more than two work-groups of each would take: shares
+    ([1030] * 20, 8, 8, 128, torch.float16),          # 160 pairs of three work-groups
+    ([1000] * 12, 16, 8, 128, torch.bfloat16),        # 96 pairs of five, four tiles for a wave of a single one
+    ([700] * 12, 16, 8, 128, torch.float16),          # ... three tiles: a single one
+    ([1000] * 16, 16, 8, 64, torch.bfloat16),         # head_dim 64: a single one, too
+    ([700, 520] * 8, 12, 6, 64, torch.float16),       # 96 pairs of it
+    ([700] * 19, 10, 5, 64, torch.bfloat16),          # 95: five work-groups
+    ([530] * 24, 8, 4, 256, torch.bfloat16),          # head_dim 256, half as many in all: two for each of 96 pairs
+    ([1000, 600] * 16, 8, 4, 256, torch.float16),     # ... of 128
+    ([530] * 43, 6, 3, 256, torch.float16),           # 129 pairs: one would be left
 ])
 def test_compressed(dev, n_keys, hq, hkv, d, dtype):
     print(f"case n_keys={n_keys[:3]} x{len(n_keys)} hq={hq} hkv={hkv} d={d} {dtype}", flush=True)
