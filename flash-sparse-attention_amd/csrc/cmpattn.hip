@@ -792,9 +792,11 @@ static dim3 dense_pair_grid(int nx, int hkv, int batch, int lists = 0) {   // bo
 // 2.5, so one for every CU is as good as two, and every share of a key tile costs 64 KB of partial sums, written and read.  Kernel
 // and reduction of both branches, us, two per slot (as for gathered rows) | 384 work-groups a branch | 256: 2000 tokens x 8 heads of
 // 128, window 128, 30.1 | 29.7 | 29.1, 3000 x 16, window 512, 71.9 | 64.4 | 72.6, 4000 x 8 79 | 64 | 70, 5003 x 32 210 | 174 | 173,
-// 12000 x 32 421 | 400 | 398; 6000 x 32 heads of 64 162 | 140 | 122, 20000 x 32 244 | 220 | 221.
-static int dense_tile_rows(int64_t rows_total, int g, int d) {
-  if (!dense_kv_shape_ok(g, d)) return kv_tile_rows(rows_total, g, d, CMP_BK);
+// 12000 x 32 421 | 400 | 398; 6000 x 32 heads of 64 162 | 140 | 122, 20000 x 32 244 | 220 | 221.  `straight` false: the kernel for gathered
+// rows runs, and with these shares it would be slower (rows that are not aligned, 16384 x 32 of 128, window | compressed, 545 | 649
+// against 496 | 528, 16384 x 16 of 64 compressed 235 against 146).
+static int dense_tile_rows(int64_t rows_total, int g, int d, bool straight) {
+  if (!straight) return kv_tile_rows(rows_total, g, d, CMP_BK);
   const int64_t r = rows_total / (d > 64 ? 384 : 256) / 64 * 64;
   return (int)std::max<int64_t>(kv_tile_rows(rows_total, g, d, CMP_BK), std::min<int64_t>(r, KV_TILE_ROWS_MAX));
 }
@@ -810,13 +812,13 @@ struct CmpBwdWs {
 
 // The work list and the partial sums of key tiles that at most `rows` rows see each.  The room for the sums is that of the shares
 // that gathered rows would have, as callers know it: shares for one work-group per CU are never shorter.
-static void dense_tiles(CmpBwdWs& w, int64_t rows, int64_t rows_total, int g, int hkv, int d) {
+static void dense_tiles(CmpBwdWs& w, int64_t rows, int64_t rows_total, int g, int hkv, int d, bool straight) {
   const int64_t gathered = kv_tile_rows(rows_total, g, d, CMP_BK);
-  w.tile_rows = dense_tile_rows(rows_total, g, d);
+  w.tile_rows = dense_tile_rows(rows_total, g, d, straight);
   w.max_tiles = w.max_blocks * ((rows + w.tile_rows - 1) / w.tile_rows);   // as kv_tiles deals them
   w.total = w.off_part + align_up((size_t)hkv * w.max_blocks * ((rows + gathered - 1) / gathered) * 2 * CMP_BK * d * 4, 256);
 }
-static CmpBwdWs cmp_bwd_ws(int64_t n, int64_t n_k, int64_t max_q, int batch, int hq, int hkv, int d) {
+static CmpBwdWs cmp_bwd_ws(int64_t n, int64_t n_k, int64_t max_q, int batch, int hq, int hkv, int d, bool straight) {
   CmpBwdWs w;
   const int g = hq / hkv;
   w.max_blocks = (n_k + CMP_BK - 1) / CMP_BK + batch;
@@ -826,7 +828,7 @@ static CmpBwdWs cmp_bwd_ws(int64_t n, int64_t n_k, int64_t max_q, int batch, int
   w.off_tiles = w.off_counts + align_up((size_t)hkv * w.max_blocks * 4, 256);
   w.off_part = w.off_tiles + align_up((size_t)hkv * (w.max_blocks + 1) * 4, 256);
   // a key tile is seen by at most max_q queries of its sequence; rows = queries * g
-  dense_tiles(w, max_q * g, cmp_rows_total(w.max_blocks, max_q, hq), g, hkv, d);
+  dense_tiles(w, max_q * g, cmp_rows_total(w.max_blocks, max_q, hq), g, hkv, d, straight);
   return w;
 }
 
@@ -871,7 +873,7 @@ static int attn_dq_launch_as(const CmpParams& p, int batch, hipStream_t stream) 
 }
 template <typename T, int D, int MODE>
 static int attn_bwd_launch(CmpParams p, const SelBwdParams& kv, int batch, int hq, int hkv,
-                           int64_t max_rows, int64_t n, hipStream_t stream) {
+                           int64_t max_rows, int64_t n, bool straight, hipStream_t stream) {
   constexpr int KVM = MODE == CMP_MODE_WINDOW ? KV_MODE_WINDOW : KV_MODE_COMPRESSED;
   static LdsAllowed lds2;
   if (int rc_ = allow_lds(lds2, (const void*)attn_bwd_dkdv_kernel<T, D, CMP_BK, KVM>, KvCfg<D, CMP_BK>::BYTES)) return rc_;
@@ -894,7 +896,7 @@ static int attn_bwd_launch(CmpParams p, const SelBwdParams& kv, int batch, int h
     ProfScope ps_(MODE == CMP_MODE_WINDOW ? "winattn_bwd_dkdv" : "cmpattn_bwd_dkdv", stream);
     bool done = false;
     if constexpr (D <= 128)
-      if ((done = dense_kv_rows_ok(kv, D)))
+      if ((done = straight))
         dense_dkdv_kernel<T, D, KVM><<<head_tile_grid(kv.max_tiles, order), DenseKv<D>::NT, DenseKv<D>::BYTES, stream>>>(kv, order);
     if (!done)
       attn_bwd_dkdv_kernel<T, D, CMP_BK, KVM>
@@ -934,7 +936,7 @@ static int pair_dq_launch_as(const CmpParams& a, const CmpParams& b, const KvTil
 }
 template <typename T, int D>
 static int pair_bwd_launch(CmpParams a, CmpParams b, const SelBwdParams& ka, const SelBwdParams& kb, const KvTiles& ta,
-                           const KvTiles& tb, int batch, int hkv, int64_t max_rows, hipStream_t stream) {
+                           const KvTiles& tb, int batch, int hkv, int64_t max_rows, bool straight, hipStream_t stream) {
   typedef KvCfg<D, CMP_BK> C;
   static LdsAllowed lds2;
   if (int rc_ = allow_lds(lds2, (const void*)attn_bwd_dkdv_pair_kernel<T, D, CMP_BK>, C::BYTES)) return rc_;
@@ -952,7 +954,7 @@ static int pair_bwd_launch(CmpParams a, CmpParams b, const SelBwdParams& ka, con
     const dim3 grid = head_tile_grid(ka.max_tiles + kb.max_tiles, order);
     bool done = false;
     if constexpr (D <= 128)
-      if ((done = dense_kv_rows_ok(ka, D) && dense_kv_rows_ok(kb, D)))
+      if ((done = straight))
         dense_dkdv_pair_kernel<T, D><<<grid, DenseKv<D>::NT, DenseKv<D>::BYTES, stream>>>(ka, kb, (int)ka.max_tiles, order);
     if (!done) attn_bwd_dkdv_pair_kernel<T, D, CMP_BK><<<grid, C::NT, C::BYTES, stream>>>(ka, kb, (int)ka.max_tiles, order);
   }
@@ -967,13 +969,13 @@ static int pair_bwd_launch(CmpParams a, CmpParams b, const SelBwdParams& ka, con
 
 template <typename T, int D>
 static int cmp_bwd_launch(const CmpParams& p, const SelBwdParams& kv, int batch, int hq, int hkv,
-                          int64_t max_rows, int64_t n, hipStream_t stream) {
-  return attn_bwd_launch<T, D, CMP_MODE_COMPRESSED>(p, kv, batch, hq, hkv, max_rows, n, stream);
+                          int64_t max_rows, int64_t n, bool straight, hipStream_t stream) {
+  return attn_bwd_launch<T, D, CMP_MODE_COMPRESSED>(p, kv, batch, hq, hkv, max_rows, n, straight, stream);
 }
 template <typename T, int D>
 static int win_bwd_launch(const CmpParams& p, const SelBwdParams& kv, int batch, int hq, int hkv,
-                          int64_t max_rows, int64_t n, hipStream_t stream) {
-  return attn_bwd_launch<T, D, CMP_MODE_WINDOW>(p, kv, batch, hq, hkv, max_rows, n, stream);
+                          int64_t max_rows, int64_t n, bool straight, hipStream_t stream) {
+  return attn_bwd_launch<T, D, CMP_MODE_WINDOW>(p, kv, batch, hq, hkv, max_rows, n, straight, stream);
 }
 
 template <typename T, int D>
@@ -1017,16 +1019,16 @@ static int cmp_fwd_dispatch(int dtype, int head_dim, const CmpParams& p, int bat
   FSA_CMP_DISPATCH(cmp_fwd_launch, p, batch, hkv, max_rows, stream);
 }
 static int cmp_bwd_dispatch(int dtype, int head_dim, const CmpParams& p, const SelBwdParams& kv, int batch,
-                            int hq, int hkv, int64_t max_rows, int64_t n, hipStream_t stream) {
-  FSA_CMP_DISPATCH(cmp_bwd_launch, p, kv, batch, hq, hkv, max_rows, n, stream);
+                            int hq, int hkv, int64_t max_rows, int64_t n, bool straight, hipStream_t stream) {
+  FSA_CMP_DISPATCH(cmp_bwd_launch, p, kv, batch, hq, hkv, max_rows, n, straight, stream);
 }
 static int win_fwd_dispatch(int dtype, int head_dim, const CmpParams& p, int batch, int hkv,
                             int64_t max_rows, hipStream_t stream) {
   FSA_CMP_DISPATCH(win_fwd_launch, p, batch, hkv, max_rows, stream);
 }
 static int win_bwd_dispatch(int dtype, int head_dim, const CmpParams& p, const SelBwdParams& kv, int batch,
-                            int hq, int hkv, int64_t max_rows, int64_t n, hipStream_t stream) {
-  FSA_CMP_DISPATCH(win_bwd_launch, p, kv, batch, hq, hkv, max_rows, n, stream);
+                            int hq, int hkv, int64_t max_rows, int64_t n, bool straight, hipStream_t stream) {
+  FSA_CMP_DISPATCH(win_bwd_launch, p, kv, batch, hq, hkv, max_rows, n, straight, stream);
 }
 static int pair_fwd_dispatch(int dtype, int head_dim, const CmpParams& a, const CmpParams& b, int batch, int hkv,
                              int64_t max_rows, hipStream_t stream) {
@@ -1034,8 +1036,8 @@ static int pair_fwd_dispatch(int dtype, int head_dim, const CmpParams& a, const 
 }
 static int pair_bwd_dispatch(int dtype, int head_dim, const CmpParams& a, const CmpParams& b, const SelBwdParams& ka,
                              const SelBwdParams& kb, const KvTiles& ta, const KvTiles& tb, int batch, int hkv, int64_t max_rows,
-                             hipStream_t stream) {
-  FSA_CMP_DISPATCH(pair_bwd_launch, a, b, ka, kb, ta, tb, batch, hkv, max_rows, stream);
+                             bool straight, hipStream_t stream) {
+  FSA_CMP_DISPATCH(pair_bwd_launch, a, b, ka, kb, ta, tb, batch, hkv, max_rows, straight, stream);
 }
 static int cmp_score_dispatch(int dtype, int head_dim, const CmpParams& p, int batch, int hkv,
                               int64_t max_q, hipStream_t stream) {
@@ -1085,7 +1087,7 @@ extern "C" int fsa_cmpattn_fwd(const void* q, const void* ck, const void* cv, in
 extern "C" size_t fsa_cmpattn_bwd_workspace_bytes(int64_t total_q, int64_t total_k, int64_t max_seqlen_q,
                                                   int32_t batch, int32_t num_q_heads,
                                                   int32_t num_kv_heads, int32_t head_dim) {
-  return cmp_bwd_ws(total_q, total_k, max_seqlen_q, batch, num_q_heads, num_kv_heads, head_dim).total;
+  return cmp_bwd_ws(total_q, total_k, max_seqlen_q, batch, num_q_heads, num_kv_heads, head_dim, false).total;   // (of either kernel)
 }
 
 extern "C" int fsa_cmpattn_bwd(const void* q, const void* ck, const void* cv, const void* o,
@@ -1107,7 +1109,9 @@ extern "C" int fsa_cmpattn_bwd(const void* q, const void* ck, const void* cv, co
   if (rc) return rc;
   FSA_CHECK_ARG(total_k >= 1, "fsa_cmpattn_bwd: no compressed keys");
   FSA_CHECK_ARG(max_seqlen_q >= 1 && max_seqlen_q <= total_q, "fsa_cmpattn_bwd: bad max_seqlen_q");
-  CmpBwdWs ws = cmp_bwd_ws(total_q, total_k, max_seqlen_q, batch, num_q_heads, num_kv_heads, head_dim);
+  const bool straight = dense_kv_rows_ok(q, q_stride_n, q_stride_h, d_o, do_stride_n, do_stride_h, total_q,
+                                         num_q_heads / num_kv_heads, head_dim);
+  CmpBwdWs ws = cmp_bwd_ws(total_q, total_k, max_seqlen_q, batch, num_q_heads, num_kv_heads, head_dim, straight);
   if (!workspace || workspace_bytes < ws.total) {
     set_error("fsa_cmpattn_bwd: workspace too small (%zu < %zu)", workspace_bytes, ws.total);
     return FSA_ERR_WORKSPACE;
@@ -1147,7 +1151,7 @@ extern "C" int fsa_cmpattn_bwd(const void* q, const void* ck, const void* cv, co
   kv.cu_seqlens_k = cu_seqlens_k; kv.kernel_size = kernel_size; kv.kernel_stride = kernel_stride;
 
   rc = cmp_bwd_dispatch(dtype, head_dim, p, kv, batch, num_q_heads, num_kv_heads, max_seqlen_q * g, total_q,
-                        stream);
+                        straight, stream);
   if (rc) return rc;
   FSA_CHECK_LAUNCH("fsa_cmpattn_bwd");
   return 0;
@@ -1256,17 +1260,17 @@ extern "C" int fsa_winattn_fwd(const void* q, const void* k, const void* v, int3
   return 0;
 }
 
-static CmpBwdWs win_bwd_ws(int64_t n, int64_t max_q, int window, int batch, int hq, int hkv, int d) {
-  CmpBwdWs w = cmp_bwd_ws(n, n, max_q, batch, hq, hkv, d);
+static CmpBwdWs win_bwd_ws(int64_t n, int64_t max_q, int window, int batch, int hq, int hkv, int d, bool straight) {
+  CmpBwdWs w = cmp_bwd_ws(n, n, max_q, batch, hq, hkv, d, straight);
   const int g = hq / hkv;
-  dense_tiles(w, (int64_t)(CMP_BK + window) * g, win_rows_total(w.max_blocks, window, hq), g, hkv, d);
+  dense_tiles(w, (int64_t)(CMP_BK + window) * g, win_rows_total(w.max_blocks, window, hq), g, hkv, d, straight);
   return w;
 }
 
 extern "C" size_t fsa_winattn_bwd_workspace_bytes(int64_t total_tokens, int64_t max_seqlen, int32_t window,
                                                   int32_t batch, int32_t num_q_heads,
                                                   int32_t num_kv_heads, int32_t head_dim) {
-  return win_bwd_ws(total_tokens, max_seqlen, window, batch, num_q_heads, num_kv_heads, head_dim).total;
+  return win_bwd_ws(total_tokens, max_seqlen, window, batch, num_q_heads, num_kv_heads, head_dim, false).total;
 }
 
 extern "C" int fsa_winattn_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o,
@@ -1283,7 +1287,9 @@ extern "C" int fsa_winattn_bwd(const void* q, const void* k, const void* v, cons
   int rc = cmp_check_common("fsa_winattn_bwd", dtype, num_q_heads, num_kv_heads, 1, 1, batch, total_tokens);
   if (rc) return rc;
   FSA_CHECK_ARG(window >= 0 && max_seqlen >= 1 && max_seqlen <= total_tokens, "fsa_winattn_bwd: bad sizes");
-  CmpBwdWs ws = win_bwd_ws(total_tokens, max_seqlen, window, batch, num_q_heads, num_kv_heads, head_dim);
+  const bool straight = dense_kv_rows_ok(q, q_stride_n, q_stride_h, d_o, do_stride_n, do_stride_h, total_tokens,
+                                         num_q_heads / num_kv_heads, head_dim);
+  CmpBwdWs ws = win_bwd_ws(total_tokens, max_seqlen, window, batch, num_q_heads, num_kv_heads, head_dim, straight);
   if (!workspace || workspace_bytes < ws.total) {
     set_error("fsa_winattn_bwd: workspace too small (%zu < %zu)", workspace_bytes, ws.total);
     return FSA_ERR_WORKSPACE;
@@ -1321,7 +1327,7 @@ extern "C" int fsa_winattn_bwd(const void* q, const void* k, const void* v, cons
   kv.cu_seqlens_k = cu_seqlens; kv.kernel_size = 1; kv.kernel_stride = 1; kv.window = window;
 
   rc = win_bwd_dispatch(dtype, head_dim, p, kv, batch, num_q_heads, num_kv_heads, max_seqlen * g, total_tokens,
-                        stream);
+                        straight, stream);
   if (rc) return rc;
   FSA_CHECK_LAUNCH("fsa_winattn_bwd");
   return 0;
@@ -1353,13 +1359,15 @@ int fsa::layer_attn_fwd(const LayerAttn& l, hipStream_t stream) {
 }
 
 size_t fsa::layer_attn_bwd_workspace_bytes(int64_t n, int64_t total_ck, int64_t max_len, int window, int batch, int hq, int hkv, int d) {
-  return cmp_bwd_ws(n, total_ck, max_len, batch, hq, hkv, d).total + win_bwd_ws(n, max_len, window, batch, hq, hkv, d).total;
+  return cmp_bwd_ws(n, total_ck, max_len, batch, hq, hkv, d, false).total + win_bwd_ws(n, max_len, window, batch, hq, hkv, d, false).total;
 }
 
 int fsa::layer_attn_bwd(const LayerAttn& l, void* workspace, hipStream_t stream) {
   const int dtype = l.dtype, head_dim = l.head_dim, g = l.hq / l.hkv;
-  const CmpBwdWs w[2] = {cmp_bwd_ws(l.n, l.total_ck, l.max_len, l.batch, l.hq, l.hkv, head_dim),
-                         win_bwd_ws(l.n, l.max_len, l.window, l.batch, l.hq, l.hkv, head_dim)};
+  const int64_t row = (int64_t)l.hq * head_dim;
+  const bool straight = dense_kv_rows_ok(l.q, row, head_dim, l.d_out, row, head_dim, l.n, g, head_dim);
+  const CmpBwdWs w[2] = {cmp_bwd_ws(l.n, l.total_ck, l.max_len, l.batch, l.hq, l.hkv, head_dim, straight),
+                         win_bwd_ws(l.n, l.max_len, l.window, l.batch, l.hq, l.hkv, head_dim, straight)};
   CmpParams p[2];
   SelBwdParams kv[2] = {};
   KvTiles tiles[2];
@@ -1383,7 +1391,7 @@ int fsa::layer_attn_bwd(const LayerAttn& l, void* workspace, hipStream_t stream)
     ws += w[i].total;
   }
   FSA_CHECK_ARG(kv_qdo_strides_ok(kv[0].q_sn, kv[0].q_sh, kv[0].do_sn, kv[0].do_sh, g, head_dim), "fsa_layer: too many heads");
-  if (int rc = pair_bwd_dispatch(dtype, head_dim, p[0], p[1], kv[0], kv[1], tiles[0], tiles[1], l.batch, l.hkv, l.max_len * g, stream))
+  if (int rc = pair_bwd_dispatch(dtype, head_dim, p[0], p[1], kv[0], kv[1], tiles[0], tiles[1], l.batch, l.hkv, l.max_len * g, straight, stream))
     return rc;
   FSA_CHECK_LAUNCH("fsa_layer attention backward");
   return 0;

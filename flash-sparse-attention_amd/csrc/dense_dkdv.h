@@ -26,11 +26,12 @@ template <int D> struct DenseKv {
 
 inline bool dense_kv_shape_ok(int g, int d) { return d <= 128 && g <= 64 && (g & (g - 1)) == 0; }
 // Host: a pass has whole queries, rows are 16-byte aligned, and an offset from the first row of a pass to any of its rows has 32 bits
-inline bool dense_kv_rows_ok(const SelBwdParams& p, int d) {
+inline bool dense_kv_rows_ok(const void* q, int64_t q_sn, int64_t q_sh, const void* d_o, int64_t do_sn, int64_t do_sh, int64_t n_tokens,
+                             int g, int d) {
   auto ok = [&](const void* x, int64_t sn, int64_t sh) {
-    return ((uintptr_t)x % 16 | (sn | sh) % 8) == 0 && 2 * (66 * sn + p.g * sh + d) < (int64_t)0xFFFFFF00;
+    return ((uintptr_t)x % 16 | (sn | sh) % 8) == 0 && 2 * (66 * sn + g * sh + d) < (int64_t)0xFFFFFF00;
   };
-  return dense_kv_shape_ok(p.g, d) && (p.n_tokens + 64) * p.g < (1 << 30) && ok(p.q, p.q_sn, p.q_sh) && ok(p.d_o, p.do_sn, p.do_sh);
+  return dense_kv_shape_ok(g, d) && (n_tokens + 64) * g < (1 << 30) && ok(q, q_sn, q_sh) && ok(d_o, do_sn, do_sh);
 }
 
 // upper_seg by a whole wave: a look-up of a chain of log64 n loads, not log2 n
