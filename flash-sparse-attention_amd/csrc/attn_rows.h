@@ -21,7 +21,7 @@ __device__ __forceinline__ void lds_dma4(__amdgpu_buffer_rsrc_t rsrc, const uint
 __device__ __forceinline__ void tiles_arrived() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // Tiles of 32 K or V rows of a sequence and kv head on their way to LDS.  ANY: of rows that are not 16-byte aligned or lie on
-// top of each other; they go through the registers, and the wave waits for them.
+// top of each other; they go through the registers: fetch, and land once there is nothing else to do.
 template <typename T, int D, bool ANY = false> struct TileLoads {
   static constexpr int CPR = D / 8, RPI = 64 / CPR, N = 32 / RPI;   // 16-byte chunks per row, rows per load, loads per tile
   static constexpr int NV = RPI >= 4 ? 4 : 16 / RPI;   // lane offsets: 16 rows or more, after which chunk_swizzle repeats itself
@@ -46,18 +46,30 @@ template <typename T, int D, bool ANY = false> struct TileLoads {
   // PARTS > 1: one of as many equal shares of the loads.  Rows behind the end of the sequence are out of the range of the
   // descriptors and arrive as zeros: no query of the sequence sees them; one at a position behind it does, with score 0, as in
   // the block-major kernels.
+  typedef typename Elem<T>::vec8 vec8;
+  template <int PARTS> __device__ __forceinline__ void fetch(vec8 (&x)[N / PARTS], int key, int part) const {
+    const int lane = threadIdx.x & 63, c = lane % CPR;
+#pragma unroll
+    for (int i = 0; i < N / PARTS; ++i) {
+      const int r = key + (part * (N / PARTS) + i) * RPI + lane / CPR;
+      x[i] = load16_at<vec8>(reinterpret_cast<uint64_t>(base) + (uint64_t)(uint32_t)min(r, len - 1) * row_bytes + c * 16);
+      if (r >= len) x[i] = zero8<T>();
+    }
+  }
+  template <int PARTS> __device__ __forceinline__ void land(const vec8 (&x)[N / PARTS], uint32_t to, int part) const {
+    const int lane = threadIdx.x & 63, c = lane % CPR;
+#pragma unroll
+    for (int i = 0; i < N / PARTS; ++i) {
+      const int r = (part * (N / PARTS) + i) * RPI + lane / CPR;
+      store16(const_cast<T*>(lds_ptr<T>(to + r * (D * 2) + (c ^ chunk_swizzle<D>(r)) * 16)), x[i]);
+    }
+  }
   template <int PARTS = 1> __device__ __forceinline__ void issue(int key, uint32_t to, int part = 0) const {
     static_assert(N / PARTS >= NV, "a share has whole descriptors");
     if constexpr (ANY) {
-      const int lane = threadIdx.x & 63, c = lane % CPR;
-      typedef typename Elem<T>::vec8 vec8;
-#pragma unroll
-      for (int i = 0; i < N / PARTS; ++i) {
-        const int r = (part * (N / PARTS) + i) * RPI + lane / CPR;
-        vec8 x = zero8<T>();
-        if (key + r < len) x = load16<vec8>(base + (uint64_t)(uint32_t)(key + r) * row_bytes + c * 16);
-        store16(const_cast<T*>(lds_ptr<T>(to + r * (D * 2) + (c ^ chunk_swizzle<D>(r)) * 16)), x);
-      }
+      vec8 x[N / PARTS];
+      fetch<PARTS>(x, key, part);
+      land<PARTS>(x, to, part);
       return;
     }
 #pragma unroll

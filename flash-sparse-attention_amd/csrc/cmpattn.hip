@@ -157,6 +157,19 @@ __device__ __forceinline__ void attn_fwd_tile(const CmpParams& p, int id) {
   auto issue_v = [&](int t) {
     if ((wv & 1) == 1 && wv < 2 * PARTS) vl.template issue<PARTS>(jt0 + 32 * t, v_lds + (t & 1) * TILE, wv >> 1);
   };
+  // ANY: every wave requests a quarter of either tile at the start of a step and puts it into LDS at its end.  (Put there at once,
+  // as in front of the loop, the waves waited for every tile: keys and values one element off, window / compressed, us, 16384 x 32 of
+  // 128 285 / 296 -> 213 / 199, 16384 x 16 of 64 114 / 107 -> 64 / 58, 9000 x 8 of 256 215 / 104 -> 118 / 63; 64-key tiles 241 / 210, 72 /
+  // 60, 139 / 73.)
+  vec8 next_k[Loads::N / 4], next_v[Loads::N / 4];
+  auto fetch = [&](int t) {
+    kl.template fetch<4>(next_k, jt0 + 32 * (t + 2), wv);
+    vl.template fetch<4>(next_v, jt0 + 32 * (t + 1), wv);
+  };
+  auto land = [&](uint32_t k_to, uint32_t v_to) {
+    kl.template land<4>(next_k, k_to, wv);
+    vl.template land<4>(next_v, v_to, wv);
+  };
   AttnRows<T, D> r;
   r.scale_log2 = p.scale_log2;
   r.clear();
@@ -181,11 +194,16 @@ __device__ __forceinline__ void attn_fwd_tile(const CmpParams& p, int id) {
     vec8 pk[2];
     auto step = [&](f32x16& x, f32x16& next, int t) {   // scores of this step in x, those of the next one into `next`
       tiles_arrived();   // K of the next step, V of this one
-      issue_k(t + 2);    // (behind the last key: zeros, and nothing is read)
-      issue_v(t + 1);
+      if constexpr (ANY) {
+        fetch(t);
+      } else {
+        issue_k(t + 2);    // (behind the last key: zeros, and nothing is read)
+        issue_v(t + 1);
+      }
       r.template scores<true>(next, x, r.reference(true), pk, k_lds + ((t + 1) & 1) * TILE, f);
       mask(next, t + 1);
       r.raise(r.values(next, pk, v_lds + (t & 1) * TILE, f), true);
+      if constexpr (ANY) land(k_lds + (t & 1) * TILE, v_lds + ((t + 1) & 1) * TILE);
     };
     f32x16 sa, sb;
     tiles_arrived();
@@ -248,6 +266,17 @@ __device__ __forceinline__ void attn_bwd_dq_tile(const CmpParams& p, int id) {
   auto issue_v = [&](int t) {
     if ((wv & 1) == 1 && wv < 2 * PARTS) vl.template issue<PARTS>(jt0 + 32 * t, v_lds + (t & 1) * TILE, wv >> 1);
   };
+  // ANY: as in the forward; window / compressed, us, 16384 x 32 of 128 337 / 386 -> 297 / 261, 16384 x 16 of 64 121 / 130 -> 79 / 73,
+  // 9000 x 8 of 256 258 / 184 -> 158 / 83; 64-key tiles 304 / 286, 88 / 82, 155 / 83
+  vec8 next_k[Loads::N / 4], next_v[Loads::N / 4];
+  auto fetch = [&](int t) {
+    kl.template fetch<4>(next_k, jt0 + 32 * (t + 2), wv);
+    vl.template fetch<4>(next_v, jt0 + 32 * (t + 1), wv);
+  };
+  auto land = [&](uint32_t k_to, uint32_t v_to) {
+    kl.template land<4>(next_k, k_to, wv);
+    vl.template land<4>(next_v, v_to, wv);
+  };
   AttnRows<T, D> r;   // q, and dQ in its accumulators
   r.clear();
   T* rows_lds = reinterpret_cast<T*>(smem + (5 + wv) * TILE);
@@ -257,6 +286,9 @@ __device__ __forceinline__ void attn_bwd_dq_tile(const CmpParams& p, int id) {
     issue_v(0);
     issue_k(1, k_next);
     const TileFrags<D> f;
+    // ANY, head_dim 256: dO of the row tile stays in LDS.  Beside K and V on their way 73 registers were spilled, and dQ took 279 / 128
+    // us, window / compressed, in the last example above.
+    constexpr bool DO_LDS = ANY && D >= 256;
     vec8 xq[Loads::N], xd[Loads::N], dorow[NKS];
     r.rows_fetch(xq, reinterpret_cast<const T*>(p.q) + (int64_t)(q0 + qi) * p.q_sn + (int64_t)hq_i * p.q_sh);
     r.rows_fetch(xd, reinterpret_cast<const T*>(p.d_o) + (int64_t)(q0 + qi) * p.do_sn + (int64_t)hq_i * p.do_sh);
@@ -278,19 +310,29 @@ __device__ __forceinline__ void attn_bwd_dq_tile(const CmpParams& p, int id) {
     r.rows_to_frags(r.q, xq, rows_lds, f);
     r.rows_to_frags(dorow, xd, rows_lds, f);
     r.settle_q();
+    if constexpr (!DO_LDS) {
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) asm volatile("" : "+v"(dorow[ks]));
+      for (int ks = 0; ks < NKS; ++ks) asm volatile("" : "+v"(dorow[ks]));
+    }
+    const uint32_t do_lds = lds_addr(rows_lds);
     auto step = [&](f32x16& x, f32x16& next, int t) {   // scores of this step in x, those of the next one into `next`
       tiles_arrived();   // K of the next step, V of this one
-      issue_k(t + 2, k_old);    // (behind the last key: zeros, and nothing is read)
-      issue_v(t + 1);
+      if constexpr (ANY) {
+        fetch(t);
+      } else {
+        issue_k(t + 2, k_old);    // (behind the last key: zeros, and nothing is read)
+        issue_v(t + 1);
+      }
       const uint32_t v_tile = v_lds + (t & 1) * TILE;
       constexpr int AHEAD = 2;
       vec8 fr[AHEAD + 1], ds[2];
       f32x16 dp;
 #pragma unroll
       for (int i = 0; i < 16; ++i) dp[i] = next[i] = 0.f;
-      auto read = [&](int i) { fr[i % (AHEAD + 1)] = load16<vec8>(lds_ptr<T>((i < NKS ? v_tile : k_next) + (f.k ^ (16u * (i % NKS))))); };
+      auto read = [&](int i) {
+        fr[i % (AHEAD + 1)] = load16<vec8>(lds_ptr<T>((i < NKS ? v_tile : k_next) + (f.k ^ (16u * (i % NKS)))));
+        if (DO_LDS && i < NKS) dorow[i % (AHEAD + 1)] = load16<vec8>(lds_ptr<T>(do_lds + (f.k ^ (16u * i))));
+      };
 #pragma unroll
       for (int i = 0; i < AHEAD; ++i) read(i);
       // dP of this step beside its exponentials, then scores of the next step beside dS = P (dP - delta) scale of this one
@@ -299,7 +341,7 @@ __device__ __forceinline__ void attn_bwd_dq_tile(const CmpParams& p, int id) {
       for (int i = 0; i < 2 * NKS; ++i) {
         if (i + AHEAD < 2 * NKS) read(i + AHEAD);
         if (i < NKS) {
-          dp = Elem<T>::mfma32(fr[i % (AHEAD + 1)], dorow[i % NKS], dp);
+          dp = Elem<T>::mfma32(fr[i % (AHEAD + 1)], dorow[DO_LDS ? i % (AHEAD + 1) : i % NKS], dp);
 #pragma unroll
           for (int e = i * 16 / NKS; e < (i + 1) * 16 / NKS; ++e) {
             x[e] = fast_exp2(x[e] * p.scale_log2 - lse);
@@ -330,6 +372,7 @@ __device__ __forceinline__ void attn_bwd_dq_tile(const CmpParams& p, int id) {
         __builtin_amdgcn_sched_barrier(0);
       }
       mask(next, t + 1);
+      if constexpr (ANY) land(k_old, v_lds + ((t + 1) & 1) * TILE);
       const uint32_t k = k_old;
       k_old = k_now;
       k_now = k_next;

@@ -30,6 +30,8 @@ def _heads_first(x):
     ([5000], 32, 8, 128, 512, torch.bfloat16),             # key tiles of one work-group
     ([300], 128, 1, 64, 64, torch.float16),                # (no whole query in a pass: as gathered rows)
     ([900, 20], 6, 2, 128, 128, torch.bfloat16),           # (three heads to a group: the same)
+    ([900, 33], 8, 2, 256, 200, torch.bfloat16),           # (head_dim 256: the same; dQ of keys off their alignment keeps dO in LDS)
+    ([40, 31, 515], 4, 4, 256, 64, torch.float16),
 ])
 @pytest.mark.parametrize("heads_first", [False, True])
 def test_forms(dev, lens, hq, hkv, d, window, dtype, heads_first):

@@ -112,9 +112,9 @@ def test_forms_of_keys_and_values(dev, form, d, dtype):
     cut = torch.tensor(cu, dtype=torch.int32, device=dev)
     cuk = torch.tensor([0, 0, 0, 7, 28], dtype=torch.int32, device=dev)   # windows of 32, 16 apart
     q = torch.randn(n, hq, d, generator=gen).to(dtype).to(dev)
-    flat = torch.randn(n * hkv * (d + 8) + 8, generator=gen).to(dtype).to(dev)
+    flats = [torch.randn(n * hkv * (d + 8) + 8, generator=gen).to(dtype).to(dev) for _ in range(2)]
 
-    def rows(m):
+    def rows(m, flat):
         if form == "shifted":
             return flat[1:1 + m * hkv * d].view(m, hkv, d)
         if form == "padded":
@@ -125,6 +125,6 @@ def test_forms_of_keys_and_values(dev, form, d, dtype):
 
     for call in (lambda k, v: ops.winattn_fwd(q, k, v, cut, max_len, window),
                  lambda k, v: ops.cmpattn_fwd(q, k, v, 32, 16, cut, cuk, max_len)):
-        k, v = rows(n), rows(n).flip(0)
+        k, v = (rows(n, flat) for flat in flats)
         (o, lse), (o_c, lse_c) = call(k, v), call(k.contiguous().clone(), v.contiguous().clone())
         assert torch.equal(o, o_c) and torch.equal(lse, lse_c)
