@@ -1225,7 +1225,9 @@ static size_t dec_ws_bytes(int batch, int hq, int hkv, int d) {
 }
 
 // ---- one token through the layer: host side ----
-constexpr int DEC_LAYER_CHUNKS = 64;   // work-groups per (source, kv head) at most
+// work-groups per (source, kv head) at most: one for every CU by all kv heads of a source
+constexpr int DEC_LAYER_CHUNKS = 64;
+static int dec_layer_chunks(int hkv) { return std::min(DEC_LAYER_CHUNKS, std::max(1, 256 / hkv)); }
 struct DecLayerWs {
   size_t q_rot, gate, o_cmp, o_win, attn, idx, raw, part, arrived, total;
   int64_t raw_ld;
@@ -1249,7 +1251,7 @@ static DecLayerWs dec_layer_ws(const fsa_decode_layer_args& a) {
   w.idx = take((size_t)a.num_kv_heads * w.topk * 4);
   w.raw_ld = (a.ck_len + 1 + 3) / 4 * 4;
   w.raw = take((size_t)a.num_kv_heads * w.raw_ld * 4);
-  w.part = take((size_t)2 * DEC_LAYER_CHUNKS * a.num_kv_heads * (a.num_q_heads / a.num_kv_heads) * (4 + a.head_dim) * 4);
+  w.part = take((size_t)2 * dec_layer_chunks(a.num_kv_heads) * a.num_kv_heads * (a.num_q_heads / a.num_kv_heads) * (4 + a.head_dim) * 4);
   w.arrived = take((size_t)2 * a.num_kv_heads * 4);
   w.total = at;
   return w;
@@ -1316,9 +1318,9 @@ static int dec_layer_attend(const fsa_decode_layer_args& a, hipStream_t stream) 
               a.kernel_stride};
   p.src[1] = {elem(a.k_cache, w0 * a.k_stride_n), elem(a.v_cache, w0 * a.v_stride_n), a.k_new, a.v_new, a.k_stride_n,
               a.k_stride_h, a.v_stride_n, a.v_stride_h, L - w0, L + 1 - w0, w0, 1};
-  // a tile per wave, as long as the chip holds them all
+  // a tile per wave, as long as there are work-groups enough
   constexpr int W = DecLayerWaves<D>::N, LDS = W * DecLds<D>::BYTES;
-  auto chunks = [&](int tiles) { return std::max(1, std::min({(tiles + W - 1) / W, DEC_LAYER_CHUNKS, std::max(1, 1024 / (W * hkv))})); };
+  auto chunks = [&](int tiles) { return std::max(1, std::min((tiles + W - 1) / W, dec_layer_chunks(hkv))); };
   p.arrived = lp.arrived;
   for (int i = 0; i < 2; ++i) p.chunks[i] = chunks((p.src[i].n_keys + DEC_TK - 1) / DEC_TK);
 
