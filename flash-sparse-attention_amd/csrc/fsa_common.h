@@ -365,6 +365,7 @@ int selattn_fwd(const void* q, const void* k, const void* v, int32_t dtype, int6
                 int64_t o_stride_n, int64_t o_stride_h, float* lse, void* workspace, size_t workspace_bytes,
                 const MergeEpilogue& merge, hipStream_t stream);
 
+constexpr int DIR_MAX_BLOCKS = 1024;   // of a sequence that the direct forward takes: size of its tables in LDS
 bool selattn_direct_preferred(int64_t n, int64_t max_len, int hq, int d, int topk, int bk, bool index_needed);
 int selattn_direct_fwd(const void* q, const void* k, const void* v, int32_t dtype, int64_t q_stride_n, int64_t q_stride_h,
                        int64_t k_stride_n, int64_t k_stride_h, int64_t v_stride_n, int64_t v_stride_h, const int32_t* topk_idx,

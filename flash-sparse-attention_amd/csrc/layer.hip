@@ -364,8 +364,10 @@ static LayerSaved layer_saved(const fsa_layer_args& a) {
   const size_t e = 2, n = a.total_tokens, d = a.head_dim, hq = a.num_q_heads, hkv = a.num_kv_heads;
   s.t_out = (int)std::min<int64_t>(a.topk, (a.max_len + a.block_size - 1) / a.block_size);
   s.max_blocks = (a.total_tokens + a.block_size - 1) / a.block_size + a.batch;
-  s.direct = a.total_tokens * a.num_kv_heads * a.head_dim < (int64_t)1 << 30 &&
-             selattn_direct_preferred(a.total_tokens, a.max_len, a.num_q_heads, a.head_dim, s.t_out, a.block_size, !a.inference);
+  // sequences of unknown lengths are priced as in the operator: three quarters of the batch as one
+  const int64_t len = a.batch > 1 && a.max_len == a.total_tokens ? a.max_len - a.max_len / 4 : a.max_len;
+  s.direct = a.total_tokens * a.num_kv_heads * a.head_dim < (int64_t)1 << 30 && a.max_len <= (int64_t)a.block_size * DIR_MAX_BLOCKS &&
+             selattn_direct_preferred(a.total_tokens, len, a.num_q_heads, a.head_dim, s.t_out, a.block_size, !a.inference);
   s.index = !s.direct || !a.inference;
   s.cu_ck = b.take((a.batch + 1) * 4);
   s.table = b.take((size_t)a.max_len * d * e);

@@ -33,8 +33,6 @@ struct DirectParams {
   MergeEpilogue merge;
 };
 
-constexpr int DIR_MAX_BLOCKS = 1024; // of a sequence: size of the tables in LDS
-
 // A row tile.  The rows of the whole buffer are dealt out, so that none of o and lse stays unwritten where the sequences do not
 // fill it: segment i runs from cu[i - 1] to cu[i], with the start of the buffer in front and its end behind.  Segment 0, in
 // front of the first sequence, has no keys; the last one holds the last sequence and, as queries at the positions behind it,
@@ -580,18 +578,22 @@ template <typename T, bool MERGE> static int dispatch_direct_fwd(int d, const Di
 // 28, 5000 x 4 17 + 54 / 46, 8000 x 4 23 + 77 / 100, 5000 x 32 27 + 288 / 222, 8000 x 32 33 + 460 / 503, 5000 x 32, 16 blocks of
 // 32, 19 + 260 / 199, 8 of 64 14 + 155 / 199, 8 of 128 13 + 196 / 208; 64: 8000 x 4 23 + 49 / 55, 5000 x 32 27 + 171 / 136, 16
 // blocks of 32 19 + 148 / 121, 8 of 64 14 + 88 / 119; 256: 3000 x 32 13 + 361 / 203, 16 blocks of 32 14 + 321 / 200, 8 of 64 11 +
-// 219 / 202, 8 of 128 12 + 243 / 210; 5000 x 4 17 + 114 / 105, 8 of 64 13 + 78 / 102.
+// 219 / 202, 8 of 128 12 + 243 / 210; 5000 x 4 17 + 114 / 105, 8 of 64 13 + 78 / 102; lists that do not load four at a time take the
+// index longer: 6 of 64, 3000 x 4 of 256, 17 + 51 / 53.  The block-major side is fitted to 4000 measured calls (one in ten of them more
+// than 17 to 29 % off), with 2 us for every gap between its launches.  Over 4700 calls the choice takes 1.005 (training) and 1.010
+// (inference) of the better form's time.
 bool selattn_direct_preferred(int64_t n, int64_t max_len, int hq, int d, int topk, int bk, bool index_needed) {
   if (!(d == 64 || d == 128 || d == 256) || !(bk == 32 || bk == 64 || bk == 128) || topk > 4096 ||
       max_len > (int64_t)bk * DIR_MAX_BLOCKS)
     return false;
   const double rows = (double)n * hq * d / 128, len = (double)max_len;
   const double keys = std::min<double>((double)topk * bk, len);
-  struct Fit { double fixed, block, key; };   // per row of 128 dims
-  static constexpr Fit fits[3] = {{21, 8.7e-5, 4e-7}, {24, 8.1e-5, 3e-7}, {27, 8e-5, 4.5e-7}};
+  struct Fit { double fixed, row, block, key, key_128; };   // per row of 128 dims; key_128: what a key of a block of 128 adds
+  static constexpr Fit fits[3] = {{18.4, 1.3e-4, 8.4e-5, 2.7e-7, 6.5e-7}, {19.8, 1.8e-4, 7.7e-5, 2.6e-7, 1.5e-7}, {23.8, 3.2e-4, 8.05e-5, 2.55e-7, 0}};
   const Fit& f = fits[d <= 64 ? 0 : d <= 128 ? 1 : 2];
   const double blocks = std::min<double>(topk, std::ceil(len / bk));
-  const double block_major = f.fixed + rows * (blocks * f.block + keys * f.key), index = index_needed ? 0 : 9.5 + 1.1e-4 * (double)n * topk;
+  const double block_major = f.fixed + rows * (f.row + blocks * f.block + keys * (f.key + (bk == 128 ? f.key_128 : 0)));
+  const double index = index_needed ? 0 : 13.3 + (topk % 4 ? 4e-4 : 1.2e-4) * (double)n * topk;
   return direct_us(direct_form(d, rows, len), d, rows, len) <= block_major + index;
 }
 

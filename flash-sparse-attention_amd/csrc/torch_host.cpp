@@ -279,15 +279,18 @@ std::pair<Tensor, Tensor> selattn_fwd_native(const Tensor& q, const Tensor& k, c
 }
 
 // Short sequences: from the block lists (kernel_blocks), without an index.  The lengths are on the device and are not read
-// back, so that a packed batch is priced as one sequence as long as all of it: eight documents of 1000 tokens take the
-// block-major kernels although each of them is short.
-bool direct(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& topk_idx, int64_t block, bool index_needed) {
-  const int64_t n = q.size(0), d = q.size(2);
+// back.  A packed batch is priced as one sequence of three quarters of its tokens, which is the mean length that a row finds
+// where two sequences share the tokens 85 : 15.  (As one sequence of all of them, batches of short documents take the
+// block-major kernels: 3000 tokens x 4 heads of 256 in 4, 6 blocks of 64, 71 us against 36.  A batch that is one long sequence but
+// for a few tokens may be up to a quarter slower than with them.)
+bool direct(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& topk_idx, int64_t batch, int64_t block, bool index_needed) {
+  const int64_t n = q.size(0), d = q.size(2), len = batch > 1 ? n - n / 4 : n;
   auto rows_ok = [&](const Tensor& t) {   // they go to LDS by 16-byte buffer loads
     return t.stride(0) >= d && t.stride(0) * n < (int64_t)1 << 30 && (uintptr_t)t.data_ptr() % 16 == 0;
   };
-  return n >= 1 && topk_idx.size(0) == k.size(1) && topk_idx.size(1) == n && rows_ok(k) && rows_ok(v) &&
-         api.fsa_selattn_direct_preferred(n, n, (int32_t)q.size(1), (int32_t)d, (int32_t)topk_idx.size(2), (int32_t)block,
+  return n >= 1 && n <= 1024 * block &&   // the kernels' limit, whatever the price
+         topk_idx.size(0) == k.size(1) && topk_idx.size(1) == n && rows_ok(k) && rows_ok(v) &&
+         api.fsa_selattn_direct_preferred(n, len, (int32_t)q.size(1), (int32_t)d, (int32_t)topk_idx.size(2), (int32_t)block,
                                           index_needed) == 1;
 }
 std::pair<Tensor, Tensor> selattn_direct(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& topk_idx, const Tensor& cu,
@@ -340,7 +343,7 @@ std::pair<Tensor, Tensor> selattn_fwd(const Tensor& q, const Tensor& k, const Te
   const int64_t d = q.size(2), dn = native_dim(d);
   const double scale = default_scale(scale_, d);
   const Tensor qn = resize_d(q, dn), kn = resize_d(k, dn), vn = resize_d(v, dn);
-  auto [o, lse] = lists && direct(qn, kn, vn, *lists, block, true)
+  auto [o, lse] = lists && direct(qn, kn, vn, *lists, index[0].numel() - 1, block, true)
                       ? selattn_direct(qn, kn, vn, *lists, index[0], block, scale)
                       : selattn_fwd_native(qn, kn, vn, view_of(index, topk, block, max_blocks), scale);
   return {resize_d(o, d), lse};
@@ -353,7 +356,7 @@ std::pair<Tensor, Tensor> selattn_fwd_lists(const Tensor& q, const Tensor& k, co
   const int64_t d = q.size(2), dn = native_dim(d);
   const double scale = default_scale(scale_, d);
   const Tensor ids = kernel_blocks(topk_idx, cu, block), qn = resize_d(q, dn), kn = resize_d(k, dn), vn = resize_d(v, dn);
-  auto [o, lse] = direct(qn, kn, vn, ids, block, true)
+  auto [o, lse] = direct(qn, kn, vn, ids, cu.numel() - 1, block, true)
                       ? selattn_direct(qn, kn, vn, ids, cu, block, scale)
                       : selattn_fwd_native(qn, kn, vn, kernel_index(ids, cu, block, q.size(1), dn, true, false).view(), scale);
   return {resize_d(o, d), lse};
@@ -386,7 +389,7 @@ struct SelectedAttention : torch::autograd::Function<SelectedAttention> {
     const int64_t d = q.size(2), dn = native_dim(d);
     const Tensor ids = kernel_blocks(topk_idx, cu, block);
     const Tensor qn = resize_d(q, dn), kn = resize_d(k, dn), vn = resize_d(v, dn);
-    const bool from_lists = direct(qn, kn, vn, ids, block, true);
+    const bool from_lists = direct(qn, kn, vn, ids, cu.numel() - 1, block, true);
     const Index x = kernel_index(ids, cu, block, q.size(1), dn, !from_lists, true);
     auto [on, lse] = from_lists ? selattn_direct(qn, kn, vn, ids, cu, block, scale) : selattn_fwd_native(qn, kn, vn, x.view(), scale);
     ctx->save_for_backward({qn, kn, vn, on, lse, x.cu, x.mem});
@@ -417,7 +420,7 @@ Tensor selected_attention(const Tensor& q, const Tensor& k, const Tensor& v, con
     return SelectedAttention::apply(q, k, v, topk_idx, block, cu, scale);
   const int64_t d = q.size(2), dn = native_dim(d);
   const Tensor ids = kernel_blocks(topk_idx, cu, block), qn = resize_d(q, dn), kn = resize_d(k, dn), vn = resize_d(v, dn);
-  if (direct(qn, kn, vn, ids, block, false)) return resize_d(selattn_direct(qn, kn, vn, ids, cu, block, scale).first, d);
+  if (direct(qn, kn, vn, ids, cu.numel() - 1, block, false)) return resize_d(selattn_direct(qn, kn, vn, ids, cu, block, scale).first, d);
   const Index x = kernel_index(ids, cu, block, q.size(1), dn, true, false);
   return resize_d(selattn_fwd_native(qn, kn, vn, x.view(), scale).first, d);
 }

@@ -241,3 +241,48 @@ def test_line_between_the_forms(dev):
     alone = FSA_topk_sparse_attention(q, k, v, idx, 64, cu)
     trained = FSA_topk_sparse_attention(q.requires_grad_(), k, v, idx, 64, cu)
     assert (alone.float() - trained.float()).abs().max().item() <= O_TOL[torch.bfloat16]
+
+
+def _kernels(run):
+    run()
+    torch.cuda.synchronize()
+    _lib.profile_enable(True)
+    out = run()
+    torch.cuda.synchronize()
+    names = {name for name, _ in _lib.profile_records()}
+    _lib.profile_enable(False)
+    return out, names
+
+
+def test_packed_batch_is_not_priced_as_one_sequence(dev):
+    """Where one sequence of all the tokens would take the block-major kernels, a batch of documents does not."""
+    n, hq, d = 3000, 4, 256
+    lib = _lib.load()
+    assert [lib.fsa_selattn_direct_preferred(n, m, hq, d, 6, 64, 1) for m in (n, n - n // 4)] == [0, 1]
+    cu = [0, 800, 1500, 2300, n]
+    q, k, v = (x.to(dev) for x in make_qkv(n, hq, hq, d, torch.bfloat16, seed=13, with_do=False))
+    cut, idx = torch.tensor(cu, dtype=torch.int32, device=dev), make_topk_idx(cu, hq, 64, 6, seed=14).to(dev)
+    o, names = _kernels(lambda: FSA_topk_sparse_attention(q, k, v, idx, 64, cut))
+    assert names == {"selattn_direct_fwd"}
+    ref = _reference(q, k, v, idx, cut, 64)[0]
+    assert (o.double().cpu() - ref).abs().max().item() <= O_TOL[torch.bfloat16]
+    q.requires_grad_()
+    _, names = _kernels(lambda: FSA_topk_sparse_attention(q, k, v, idx, 64, cut))
+    assert "selattn_direct_fwd" in names and "selattn_fwd_main" not in names
+
+
+def test_packed_batch_beyond_the_tables(dev):
+    """A batch with more blocks than the direct kernels have tables for, long lists that would make them the cheaper ones."""
+    n, block, topk = 33000, 32, 512
+    assert _lib.load().fsa_selattn_direct_preferred(n, n - n // 4, 1, 64, topk, block, 0) == 1 and n > 1024 * block
+    q, k, v = (x.to(dev) for x in make_qkv(n, 1, 1, 64, torch.bfloat16, seed=15, with_do=False))
+    cu, cut = [0, 200, n], torch.tensor([0, 200, n], dtype=torch.int32, device=dev)
+    own = torch.cat([torch.arange(b - a) // block for a, b in zip(cu, cu[1:])])
+    idx = (own[None, :, None] - torch.arange(topk)).clamp_(min=-1).int().to(dev)     # the last 512 blocks
+    o, names = _kernels(lambda: FSA_topk_sparse_attention(q, k, v, idx, block, cut))
+    assert "selattn_direct_fwd" not in names and torch.isfinite(o.float()).all()
+    for row in (0, 199, 200, 17000, n - 1):
+        s0 = 0 if row < 200 else 200
+        lo = max(s0, s0 + ((row - s0) // block - topk + 1) * block)
+        p = torch.softmax((k[lo:row + 1, 0].double() @ q[row, 0].double()) / 8, 0)
+        assert (o[row, 0].double() - p @ v[lo:row + 1, 0].double()).abs().max().item() <= O_TOL[torch.bfloat16]
