@@ -1,6 +1,6 @@
 """GPU: dQ, dK and dV of window and compressed attention where q and dO go straight to LDS, against the kernel that takes any rows (the same
 tensors one element off their alignment): GQA groups that fill a pass of 64 rows in different ways, key tiles and passes that end early,
-tiles of one work-group and of several, rows of a head far apart or not, statistics of either type."""
+tiles of one work-group and of several, rows of a head far apart or not.  (Statistics as two arrays; a layer hands over pairs.)"""
 import pytest
 import torch
 
@@ -64,7 +64,8 @@ def test_forms(dev, lens, hq, hkv, d, window, dtype, heads_first):
 
 
 def test_rows_that_are_not_visible(dev):
-    """What a query that does not see a key holds reaches neither its dK nor its dV: infinite q and dO of the others."""
+    """A query whose q and log-sum-exp are NaN reaches dK and dV of no tile without a key that it sees, and in the other tiles dV of
+    no key that it does not see."""
     n, window, dtype = 400, 50, torch.bfloat16
     gen = torch.Generator().manual_seed(5)
     q, k, v, do = (torch.randn(n, 4, 128, generator=gen).to(dev, dtype) for _ in range(4))

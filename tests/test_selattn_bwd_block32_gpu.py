@@ -1,5 +1,5 @@
-"""GPU: selected attention backward with blocks of 32 (passes of 32 gathered rows) at the edges of a pass: blocks with fewer rows
-than one, exactly one, one more, and blocks that several work-groups share, against the CPU oracle."""
+"""GPU: selected attention backward with blocks of 32 (passes of 32 gathered rows, of 64 at head_dim 64) at the edges of a pass:
+blocks with fewer rows than one, exactly one, one more, and blocks that several work-groups share, against the CPU oracle."""
 import pytest
 import torch
 

@@ -100,7 +100,8 @@ def test_matches_reference(dev, cu, hq, hkv, d, block, topk, dtype):
 MANY_ROWS = [
     # cu_seqlens, Hq, Hkv, D, block, T, dtype, kv heads looked at
     ([0, 1501], 32, 32, 128, 64, 16, torch.bfloat16, [0, 31]),             # 2 x 2
-    ([0, 1990], 12, 12, 256, 128, 4, torch.float16, [0, 11]),              # 2 x 2
+    ([0, 1990], 12, 12, 256, 128, 4, torch.float16, [0, 11]),              # (one row tile still, of head_dim 256)
+    ([0, 2301], 20, 20, 256, 128, 4, torch.float16, [0, 19]),              # 2 x 2
     ([0, 3100], 24, 8, 64, 32, 8, torch.bfloat16, [3]),                    # 2 x 2, a query in two row tiles
     ([0, 33, 33, 240], 1536, 512, 128, 32, 5, torch.float16, [0, 511]),    # 1 x 4, the same, an empty sequence
     ([0, 129, 260], 1024, 1024, 128, 64, 3, torch.bfloat16, [0, 1023]),    # 1 x 4, a row tile of one row
