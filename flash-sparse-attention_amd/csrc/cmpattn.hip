@@ -228,7 +228,9 @@ __device__ __forceinline__ void attn_fwd_tile(const CmpParams& p, int id) {
 // of K^T and dS; K of two steps and what is on its way in three tiles.  Matrix unit 50 %, vector issue 47 %, LDS 36 %: as in the kernel
 // of dK / dV, the chain of a step is the rest.  Against 64-key tiles by way of the registers, phases in turn, q, dO and dQ in pieces of
 // 16 bytes, both branches of a layer, us: 4 x 8192 tokens x 32 heads of 128, window 512, 980 -> 778; 12000 x 32 336 -> 276; 5003 x 32
-// 143 -> 118; 2 x 1000 x 8, window 128, 21.3 -> 15.6; 6000 x 32 of 64 100 -> 84; window alone, 9000 x 8 of 256, 128 -> 127.
+// 143 -> 118; 2 x 1000 x 8, window 128, 21.3 -> 15.6; 6000 x 32 of 64 100 -> 84; window alone, 9000 x 8 of 256, 128 -> 127.  At head_dim
+// 256 the registers do not suffice: 28 of either branch and 52 of both in one launch are spilled, which leaves it level (both, 9000 x
+// 8 194 -> 194, 16384 x 16 720 -> 703).
 template <typename T, int D> struct CmpDqLds {
   static constexpr int TILE = TileLoads<T, D>::BYTES, BYTES = 9 * TILE;   // three tiles of K, two of V, one of q / dO / dQ for every wave
 };

@@ -91,6 +91,13 @@ struct DecParams {
 
 // Loads and stores of what a work-group hands to another one of the same launch: as atomics of the device's scope they go past
 // the L2 copies of the XCDs, so that neither side has to write back or invalidate a cache (1.7 us a launch).  SHARED false: plain.
+// The hand-over has no release and no acquire, whose cost that is.  It rests on how the chip orders these accesses: a wave's
+// s_waitcnt vmcnt(0) covers its stores until they are where all XCDs look (device scope: behind the L2s); a barrier collects
+// the waves; only then is the counter or the stamp touched, by an access of the same scope; and what the last work-group loads, it
+// loads behind that, past its own L2, in program order that neither the compiler (atomics, volatile statements between them)
+// nor the wave (the loads wait for the answer through a branch and a barrier) turns round.  Nobody waits for anybody, so a late
+// work-group costs nothing but its own time.  What plain stores leave, o_cmp, o_win and a counter set back to zero, is read by
+// later launches only.
 template <bool SHARED, typename V> __device__ __forceinline__ V dec_load(const float* p) {
   if constexpr (!SHARED) {
     return *reinterpret_cast<const V*>(p);

@@ -55,8 +55,6 @@ template <typename V> __device__ __forceinline__ V load16(const void* p) {
 template <typename V> __device__ __forceinline__ void store16(void* p, V v) {
   *reinterpret_cast<uint4*>(p) = __builtin_bit_cast(uint4, v);
 }
-// The same 16-byte moves for data that is written once and read once by a later kernel (partial rows):
-// marked non-temporal so that they do not displace the K / V blocks and query rows that are reused.
 // The same at an address that was put together from its halves: global memory, which the compiler cannot see (a flat access
 // would wait for LDS as well, and for everything that is on its way).
 template <typename V> __device__ __forceinline__ V load16_at(uint64_t at) {
@@ -71,6 +69,8 @@ template <typename V> __device__ __forceinline__ void store16_at(uint64_t at, V 
 __device__ __forceinline__ uint64_t shfl64(uint64_t x, int lane) {
   return (uint64_t)(uint32_t)__shfl((int)(x >> 32), lane, 64) << 32 | (uint32_t)__shfl((int)(uint32_t)x, lane, 64);
 }
+// The same 16-byte moves for data that is written once and read once by a later kernel (partial rows):
+// marked non-temporal so that they do not displace the K / V blocks and query rows that are reused.
 template <typename V> __device__ __forceinline__ V load16_stream(const void* p) {
   typedef unsigned int u4_ __attribute__((ext_vector_type(4)));
   u4_ r = __builtin_nontemporal_load(reinterpret_cast<const u4_*>(p));

@@ -382,7 +382,7 @@ selattn_direct_wide_kernel(DirectParams p) {
     qo[i] = (uint32_t)e / (uint32_t)p.topk;
     id[i] = ids[qo[i] * p.i_sn + (e - qo[i] * p.topk)];
   }
-  int guess = 32 * kg;   // as in the paired kernel
+  int guess = 32 * kg;   // as in the narrow kernel
   if (guess + 32 <= len) {
     issue_k(guess, 0);
     issue_v(guess, 0);

@@ -62,7 +62,7 @@ class FlashSparseAttentionDecode(torch.nn.Module):
         self.rope = RotaryEmbedding(self.rope_config)
 
     def _fused_step(self, x, *caches):
-        """The step as one native call (six launches, caches neither copied nor rotated), or None where it does not
+        """The step as one native call (four launches, caches neither copied nor rotated), or None where it does not
         apply: projections that are more than a plain Linear, tensor subclasses, head dims or layouts without kernels, no
         compressed key."""
         gate = self.gate
